@@ -179,3 +179,56 @@ def tolerance(case):
     # against float64 on unrounded weights the kernels that apply scale and zero in fp32 are at rel 2.1e-4, max 6e-4 (the
     # fp16 output's rounding); those that round each weight to fp16 twice, as the reference's decode does, at 3.3e-4, 1.9e-3
     return {"rel": 1.3e-3, "max": 8e-3}
+
+
+def _codes(bits, matrix, mask):
+    """uint8 [k, s] of a packed matrix; with a mask bool [k, s] of the rows kept, else None"""
+    words = matrix.to(torch.int64) & 0xFFFFFFFF
+    s = words.shape[1]
+    if mask is None and bits != 3:
+        shifts = torch.arange(0, 32, bits, device=words.device)[None, :, None]
+        return ((words[:, None] >> shifts) & (2 ** bits - 1)).to(torch.uint8).reshape(-1, s), None
+    if mask is None:
+        # 32 codes of a column are a stream of 96 bits in three words
+        words = words.reshape(-1, 3, s)
+        codes = torch.empty((words.shape[0], 32, s), dtype=torch.uint8, device=words.device)
+        for i in range(32):
+            word, bit = divmod(3 * i, 32)
+            value = words[:, word] >> bit
+            if bit > 29:
+                value = value | (words[:, word + 1] << (32 - bit))
+            codes[:, i] = (value & 7).to(torch.uint8)
+        return codes.reshape(-1, s), None
+    # sixteen codes of 32 rows, in the order of the mask's set bits
+    kept = ((mask[:, None].to(torch.int64) >> torch.arange(32, device=mask.device)[None, :, None]) & 1).to(torch.uint8)
+    rank = kept.cumsum(dim=1, dtype=torch.int16) - kept
+    stored = ((words[:, None] >> torch.arange(0, 32, 4, device=words.device)[None, :, None]) & 15).to(torch.uint8)
+    stored = stored.reshape(-1, 16, s)
+    codes = stored.gather(1, rank.clamp(max=15).to(torch.int64))
+    return codes.reshape(-1, s), kept.reshape(-1, s).bool()
+
+
+def exact(case, seed):
+    """The products in float64, of weights that are not rounded on the way; packing gives whole numbers and has none."""
+    if case["path"] == "pack":
+        return None
+    state, outs = prepare(case, seed), []
+    x = state["x"].double()
+    for layer in state["layers"]:
+        if case["path"] == "linear":
+            layer = layer.matrix, layer.scales.reshape(-1, case["s"]), layer.zeros.reshape(-1, case["s"]), layer.sparse_mask
+        matrix, scales, zeros, mask = layer
+        codes, kept = _codes(case["bits"], matrix, mask)
+        out = torch.zeros((case["batch"] * case["rows"], case["s"]), dtype=torch.float64, device=DEV)
+        step = case["k"] if case["group"] < 0 else case["group"]
+        for group, first in enumerate(range(0, case["k"], step)):
+            code = codes[first:first + step].double()
+            scale, zero = scales[group].double(), zeros[group].double()
+            half = 2 ** (case["bits"] - 1)
+            power = torch.where(code >= half, -1.0, 1.0) * 2.0 ** (code % half)
+            weight = torch.where(scale >= 0, (code - zero) * scale, zero - scale * power)
+            if kept is not None:
+                weight = weight * kept[first:first + step]
+            out += x.reshape(-1, case["k"])[:, first:first + step] @ weight
+        outs.append(out.reshape(case["batch"], case["rows"], case["s"]))
+    return outs
