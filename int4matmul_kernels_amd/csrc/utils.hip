@@ -139,24 +139,45 @@ __global__ __launch_bounds__(256) void dense_pack_kernel(uint32_t* __restrict__ 
     for (int i = 0; i < BITS; ++i) matrix_out[(BITS * blk + i) * S + s] = w[i];
 }
 
-// 16:32 packer.  Inputs are in the [S, K] orientation (row = output column): a thread takes four
-// consecutive 32-row cells of its column -- the 128 consecutive bytes of a whole cache line of each
-// input -- compacts the kept codes eight rows at a time (keep flags gathered by a multiply, code bytes moved to
-// the front by v_perm with selectors from a 256-entry table, squeezed to nibbles) and writes three words per cell
-// with lanes along the column index.  K = S = 16384: 180 us with one cell per thread and a 32-step loop per cell,
-// 174 with whole lines, 165 with this compaction; staging a 64-column tile through LDS so that a wave reads whole
-// 256-byte runs changed nothing (173 against 174) -- what remains is the transposition: a wave's 64 lanes read
-// lines K bytes apart.
-constexpr int SPARSE_PACK_CELLS = 4;
+// 16:32 packer.  Inputs are in the [S, K] orientation (row = output column), outputs have lanes along the column
+// index, so the job is a transposition.  It is done on the outputs, which are 3 / 16 of the inputs' bytes: a workgroup
+// takes a tile of 64 columns x SPARSE_PACK_ROWS input rows, a wave's load is whole runs of consecutive bytes of a column
+// (a lane: half a 32-row cell, 16 bytes of each input), and the packed words go through LDS, from where a wave
+// stores 64 columns of one word row, 256 bytes.  Kept codes are compacted eight rows at a time: keep flags gathered
+// by a multiply, code bytes moved to the front by v_perm with selectors from a 256-entry table, squeezed to nibbles;
+// the two lanes of a cell exchange rank, mask and one word each.  Consecutive workgroups walk along K: the runs in
+// flight are then consecutive in memory, where walking along S reads lines K bytes apart, which for a K that is a power
+// of two fall onto few memory channels.
+// Bound by memory traffic: a whole weight_matrix_packing call at K = S = 16384 (637 MB) took 166 us with one 128-byte
+// line of each input per thread, lanes K bytes apart, and takes 147 so.
+constexpr int SPARSE_PACK_LANES = 32;                               // lanes along K: 512 rows of a column
+constexpr int SPARSE_PACK_ROWS = 16 * SPARSE_PACK_LANES;
+constexpr int SPARSE_PACK_COLS = 64;
 __global__ __launch_bounds__(256) void sparse_pack_kernel(uint32_t* __restrict__ wt_outs,
                                                           uint32_t* __restrict__ msk_outs,
                                                           const uint8_t* __restrict__ wt_in,
                                                           const uint8_t* __restrict__ msk_in,
-                                                          int64_t S, int64_t K,
+                                                          int64_t S, int64_t K, uint32_t k_tiles,
                                                           int* __restrict__ bad_blocks) {
+    constexpr int LANES = SPARSE_PACK_LANES, CELLS = LANES / 2, COLS = SPARSE_PACK_COLS;
+    constexpr int COLS_PASS = 256 / LANES, PASSES = COLS / COLS_PASS;
     // compaction table: for a byte of eight keep flags, the v_perm selectors that move the kept rows' code bytes to
     // the front in row order (0 ... 7: that row of the eight; 0x0C: a zero byte)
     __shared__ u32x2 front[256];
+    __shared__ uint32_t tile[3][CELLS][COLS + 1];                   // low words, high words, masks
+    const int64_t k0 = (int64_t)(blockIdx.x % k_tiles) * SPARSE_PACK_ROWS, s0 = (int64_t)(blockIdx.x / k_tiles) * COLS;
+    const int lane = threadIdx.x % LANES, col0 = threadIdx.x / LANES;
+    const bool in_k = k0 + 16 * lane < K;                           // (K is a multiple of 32: both lanes of a cell or neither)
+    u32x4 wq[PASSES], mq[PASSES];
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) {
+        const int64_t s = s0 + col0 + i * COLS_PASS;
+        wq[i] = mq[i] = u32x4{0, 0, 0, 0};
+        if (in_k && s < S) {
+            wq[i] = *reinterpret_cast<const u32x4*>(wt_in + s * K + k0 + 16 * lane);
+            mq[i] = *reinterpret_cast<const u32x4*>(msk_in + s * K + k0 + 16 * lane);
+        }
+    }
     {
         uint32_t sel[2] = {0x0C0C0C0Cu, 0x0C0C0C0Cu};
         int p = 0;
@@ -168,17 +189,6 @@ __global__ __launch_bounds__(256) void sparse_pack_kernel(uint32_t* __restrict__
         front[threadIdx.x] = u32x2{sel[0], sel[1]};
     }
     __syncthreads();
-    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, blk0 = (int64_t)blockIdx.y * SPARSE_PACK_CELLS;
-    if (s >= S) return;
-    const int64_t cells = K / 32;
-    u32x4 wq[SPARSE_PACK_CELLS][2], mq[SPARSE_PACK_CELLS][2];
-#pragma unroll
-    for (int i = 0; i < SPARSE_PACK_CELLS; ++i) {
-        if (blk0 + i >= cells) break;
-        const u32x4* wp = reinterpret_cast<const u32x4*>(wt_in + s * K + (blk0 + i) * 32);
-        const u32x4* mp = reinterpret_cast<const u32x4*>(msk_in + s * K + (blk0 + i) * 32);
-        wq[i][0] = wp[0]; wq[i][1] = wp[1]; mq[i][0] = mp[0]; mq[i][1] = mp[1];
-    }
     // keep flags of four rows (bytes > 0) as four bits: the top bit of every non-zero byte, gathered by a multiply
     auto flags4 = [](uint32_t m) {
         const uint32_t nz = ((((m & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | m) & 0x80808080u) >> 7;
@@ -189,31 +199,48 @@ __global__ __launch_bounds__(256) void sparse_pack_kernel(uint32_t* __restrict__
         const uint32_t n = (o | (o >> 4)) & 0x00FF00FFu;
         return (n | (n >> 8)) & 0xFFFFu;
     };
+    auto other_lane = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true); };  // lane ^ 1
+    const bool odd = lane & 1;
     int bad = 0;
 #pragma unroll
-    for (int i = 0; i < SPARSE_PACK_CELLS; ++i) {
-        const int64_t blk = blk0 + i;
-        if (blk >= cells) break;
-        const uint32_t wv[8] = {wq[i][0].x, wq[i][0].y, wq[i][0].z, wq[i][0].w, wq[i][1].x, wq[i][1].y, wq[i][1].z, wq[i][1].w};
-        const uint32_t mv[8] = {mq[i][0].x, mq[i][0].y, mq[i][0].z, mq[i][0].w, mq[i][1].x, mq[i][1].y, mq[i][1].z, mq[i][1].w};
-        uint32_t bmsk = 0;
+    for (int i = 0; i < PASSES; ++i) {
+        uint32_t keep = 0;
         uint64_t v = 0;
         int rank = 0;
 #pragma unroll
-        for (int g8 = 0; g8 < 4; ++g8) {                            // eight rows at a time
-            const uint32_t m8 = flags4(mv[2 * g8]) | (flags4(mv[2 * g8 + 1]) << 4);
+        for (int g8 = 0; g8 < 2; ++g8) {                            // eight rows at a time
+            const uint32_t m8 = flags4(mq[i][2 * g8]) | (flags4(mq[i][2 * g8 + 1]) << 4);
             const u32x2 sel = front[m8];
-            const uint32_t clo = wv[2 * g8] & 0x0F0F0F0Fu, chi = wv[2 * g8 + 1] & 0x0F0F0F0Fu;
+            const uint32_t clo = wq[i][2 * g8] & 0x0F0F0F0Fu, chi = wq[i][2 * g8 + 1] & 0x0F0F0F0Fu;
             const uint32_t kept = nibbles4(__builtin_amdgcn_perm(chi, clo, sel.x)) |
                                   (nibbles4(__builtin_amdgcn_perm(chi, clo, sel.y)) << 16);
-            bmsk |= m8 << (8 * g8);
-            if (rank < 16) v |= (uint64_t)kept << (4 * rank);       // (codes beyond the sixteenth fall off the top)
+            keep |= m8 << (8 * g8);
+            v |= (uint64_t)kept << (4 * rank);
             rank += __builtin_popcount(m8);
         }
-        msk_outs[blk * S + s] = bmsk;
-        wt_outs[(2 * blk) * S + s] = (uint32_t)v;
-        wt_outs[(2 * blk + 1) * S + s] = (uint32_t)(v >> 32);
-        bad += rank != 16;
+        // the odd lane's codes follow the even lane's (those beyond the sixteenth fall off the top)
+        const int rank_other = (int)other_lane((uint32_t)rank);
+        if (odd) v = rank_other < 16 ? v << (4 * rank_other) : 0;
+        const uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
+        const uint32_t word = (odd ? hi : lo) | other_lane(odd ? lo : hi);
+        const uint32_t keep_other = other_lane(keep);
+        const int col = col0 + i * COLS_PASS;
+        tile[odd][lane / 2][col] = word;
+        if (!odd) {
+            tile[2][lane / 2][col] = keep | (keep_other << 16);
+            bad += in_k && s0 + col < S && rank + rank_other != 16;
+        }
+    }
+    __syncthreads();
+    const int64_t s = s0 + threadIdx.x % COLS;
+    const int cells = (int)min((int64_t)CELLS, (K - k0) / 32);
+    if (s < S) {
+        for (int c = threadIdx.x / COLS; c < cells; c += 256 / COLS) {
+            const int64_t blk = k0 / 32 + c;
+            wt_outs[(2 * blk) * S + s] = tile[0][c][threadIdx.x % COLS];
+            wt_outs[(2 * blk + 1) * S + s] = tile[1][c][threadIdx.x % COLS];
+            msk_outs[blk * S + s] = tile[2][c][threadIdx.x % COLS];
+        }
     }
     if (bad && bad_blocks) atomicAdd(bad_blocks, bad);
 }
@@ -233,11 +260,13 @@ int int4mm_sparse_pack(void* wt_outs, void* msk_outs, const void* wt_in, const v
     if (out_size == 0 || in_size == 0) return INT4MM_OK;
     if (!wt_outs || !msk_outs || !wt_in || !msk_in) return INT4MM_ERR_NULL;
     if (((uintptr_t)wt_in | (uintptr_t)msk_in) & 15u) return INT4MM_ERR_ALIGN;
-    const dim3 grid((unsigned)((out_size + 255) / 256), (unsigned)((in_size / 32 + SPARSE_PACK_CELLS - 1) / SPARSE_PACK_CELLS));
-    hipLaunchKernelGGL(sparse_pack_kernel, grid, dim3(256), 0,
+    const int64_t k_tiles = (in_size + SPARSE_PACK_ROWS - 1) / SPARSE_PACK_ROWS;
+    const int64_t tiles = k_tiles * ((out_size + SPARSE_PACK_COLS - 1) / SPARSE_PACK_COLS);
+    if (tiles > 0xFFFFFFFF / 256) return INT4MM_ERR_SHAPE;          // (inputs of 2 x 0.5 TB: beyond any device)
+    hipLaunchKernelGGL(sparse_pack_kernel, dim3((unsigned)tiles), dim3(256), 0,
                        (hipStream_t)stream, (uint32_t*)wt_outs, (uint32_t*)msk_outs,
                        (const uint8_t*)wt_in, (const uint8_t*)msk_in, out_size, in_size,
-                       (int*)bad_blocks);
+                       (uint32_t)k_tiles, (int*)bad_blocks);
     return check_launch("sparse_pack");
 }
 

@@ -95,6 +95,27 @@ def test_sparse_pack_bit_exact_capi_and_extension(H):
         assert np.array_equal(m.cpu().numpy(), want_m)
 
 
+@pytest.mark.parametrize("S,K", [(64, 64), (63, 96), (65, 512), (1, 544), (128, 1056), (200, 480), (320, 1600)])
+def test_sparse_pack_tile_edges(H, S, K):
+    """edges of the packer's tile of 64 columns x 512 rows; cells that keep more or fewer than 16 rows are counted once each"""
+    rng = np.random.default_rng(S * 10007 + K)
+    codes_sk = rng.integers(0, 256, (S, K), dtype=np.uint8)
+    keep_sk = (rng.random((S, K // 32, 32)).argsort(axis=2) < 16).astype(np.uint8)
+    want_w, want_m = O.sparse_pack(codes_sk & 15, keep_sk.reshape(S, K))
+    spoilt = rng.random((S, K // 32)) < 0.1
+    for extra in (False, True):
+        if extra:                                   # the last row of a cell flips: 15 or 17 kept, checked by count alone
+            keep_sk[..., 31][spoilt] ^= 1
+        w = torch.full((K // 16, S), -1, dtype=torch.int32, device=H.DEV)
+        m = torch.full((K // 32, S), -1, dtype=torch.int32, device=H.DEV)
+        bad = torch.zeros(1, dtype=torch.int32, device=H.DEV)
+        H.capi.sparse_pack(w, m, H.t(codes_sk), H.t(keep_sk.reshape(S, K)), bad)
+        assert int(bad.item()) == (int(spoilt.sum()) if extra else 0)
+        if not extra:
+            assert np.array_equal(w.cpu().numpy(), want_w)
+            assert np.array_equal(m.cpu().numpy(), want_m)
+
+
 def test_sparse_pack_flags_wrong_popcount(H):
     S, K = 64, 64
     keep = np.zeros((S, K), np.uint8)
