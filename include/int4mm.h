@@ -172,6 +172,13 @@ INT4MM_API int int4mm_matvec(int bits, void* outs, const void* matrix, const voi
                   const int4mm_shape* shape, void* workspace, size_t workspace_bytes,
                   void* stream);
 
+/* int4mm_matvec that overwrites outs instead of adding onto it: the same launches, bit for bit the result of
+ * int4mm_matvec on zeroed outs, without the fill and without reading outs back. */
+INT4MM_API int int4mm_matvec_overwrite(int bits, void* outs, const void* matrix, const void* multiplier,
+                  const void* scales, const void* zeros, const void* sparse_mask,
+                  const int4mm_shape* shape, void* workspace, size_t workspace_bytes,
+                  void* stream);
+
 /* int4mm_matvec for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc): same arguments without
  * the workspace, same kernels.  Results are bit for bit those of int4mm_matvec on a workspace

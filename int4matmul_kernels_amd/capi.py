@@ -15,7 +15,7 @@ LIB_NAME = "libint4mm_hip.so"
 EXPORTS = [
     "int4mm_error_string", "int4mm_last_hip_error", "int4mm_abi_version", "int4mm_tune",
     "int4mm_workspace_bytes", "int4mm_workspace_init", "int4mm_matmul_workspace_bytes", "int4mm_matvec", "int4mm_matmul",
-    "int4mm_matvec_static", "int4mm_workspace_status", "int4mm_describe_launch",
+    "int4mm_matvec_overwrite", "int4mm_matvec_static", "int4mm_workspace_status", "int4mm_describe_launch",
     "int4mm_sparse_pack", "int4mm_dense_pack", "int4mm_unpack", "int4mm_dequantize",
 ]
 
@@ -58,7 +58,7 @@ def lib():
     L.int4mm_matmul_workspace_bytes.argtypes = [C.POINTER(Shape), C.c_int]
     L.int4mm_workspace_init.restype = C.c_int
     L.int4mm_workspace_init.argtypes = [vp, sz, vp]
-    for name in ("int4mm_matvec", "int4mm_matmul"):
+    for name in ("int4mm_matvec", "int4mm_matvec_overwrite", "int4mm_matmul"):
         f = getattr(L, name)
         f.restype = C.c_int
         f.argtypes = [C.c_int, vp, vp, vp, vp, vp, vp, C.POINTER(Shape), vp, sz, vp]
@@ -153,6 +153,15 @@ def matvec(bits, outs, matrix, multiplier, scales, zeros, group_size, sparse_mas
     _check(lib().int4mm_matvec(bits, _ptr(outs), _ptr(matrix), _ptr(multiplier), _ptr(scales),
                                _ptr(zeros), _ptr(sparse_mask), C.byref(sh), _ptr(workspace), nws,
                                _stream()), "int4mm_matvec")
+
+
+def matvec_overwrite(bits, outs, matrix, multiplier, scales, zeros, group_size, sparse_mask=None, workspace=None):
+    """the matvec that overwrites ``outs`` instead of adding onto it"""
+    sh = _shape(outs, matrix, multiplier, scales, group_size)
+    nws = 0 if workspace is None else workspace.numel()
+    _check(lib().int4mm_matvec_overwrite(bits, _ptr(outs), _ptr(matrix), _ptr(multiplier), _ptr(scales),
+                                         _ptr(zeros), _ptr(sparse_mask), C.byref(sh), _ptr(workspace), nws,
+                                         _stream()), "int4mm_matvec_overwrite")
 
 
 def matvec_static(bits, outs, matrix, multiplier, scales, zeros, group_size, sparse_mask=None):

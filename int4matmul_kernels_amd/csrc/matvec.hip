@@ -1026,7 +1026,7 @@ bool i4::matvec_one_row(int bits, h16* outs, const uint32_t* matrix, const uint3
 
 static int matvec_impl(int bits, void* outs, const void* matrix, const void* multiplier,
                        const void* scales, const void* zeros, const void* sparse_mask,
-                       const int4mm_shape* shape, void* workspace, size_t workspace_bytes,
+                       const int4mm_shape* shape, bool accumulate, void* workspace, size_t workspace_bytes,
                        void* stream) {
     int rc = validate_product(bits, outs, matrix, multiplier, scales, zeros, sparse_mask, shape, true);
     if (rc != INT4MM_OK) return rc;
@@ -1040,11 +1040,11 @@ static int matvec_impl(int bits, void* outs, const void* matrix, const void* mul
     // several batch elements of one row each: one pass over the weights for all of them
     if (B >= 2 && B <= 4 && !sparse_mask && !tuning(TUNE_NO_SKINNY) &&
         matvec_rows(bits, (h16*)outs, (const uint32_t*)matrix, (const h16*)multiplier, (const h16*)scales, (const h16*)zeros,
-                    B, K, S, g, true, (hipStream_t)stream, workspace, workspace_bytes))
+                    B, K, S, g, accumulate, (hipStream_t)stream, workspace, workspace_bytes))
         return check_launch("matvec");
     if (B >= 2 && B <= SK_WIDE_MAX_ROWS && !tuning(TUNE_NO_SKINNY) &&
         skinny_rows(bits, (h16*)outs, (const uint32_t*)matrix, (const h16*)multiplier, (const h16*)scales,
-                    (const h16*)zeros, B, K, S, g, true, (hipStream_t)stream, (const uint32_t*)sparse_mask, workspace, workspace_bytes))
+                    (const h16*)zeros, B, K, S, g, accumulate, (hipStream_t)stream, (const uint32_t*)sparse_mask, workspace, workspace_bytes))
         return check_launch("matvec");
 
     // more batch elements than the few-row kernels take at once: chunks of up to 512 through them (they add onto outs
@@ -1055,7 +1055,7 @@ static int matvec_impl(int bits, void* outs, const void* matrix, const void* mul
         while (B - done >= 2) {
             const int64_t n = std::min<int64_t>(SK_WIDE_MAX_ROWS, B - done);
             if (!skinny_rows(bits, (h16*)outs + done * S, (const uint32_t*)matrix, (const h16*)multiplier + done * K, (const h16*)scales,
-                             (const h16*)zeros, n, K, S, g, true, (hipStream_t)stream, (const uint32_t*)sparse_mask, workspace,
+                             (const h16*)zeros, n, K, S, g, accumulate, (hipStream_t)stream, (const uint32_t*)sparse_mask, workspace,
                              workspace_bytes))
                 break;
             rc = check_launch("matvec");
@@ -1065,11 +1065,11 @@ static int matvec_impl(int bits, void* outs, const void* matrix, const void* mul
         if (done == B) return INT4MM_OK;
     }
     return matvec_plain(bits, (h16*)outs + done * S, matrix, (const h16*)multiplier + done * K, scales, zeros, sparse_mask, B - done, K, S, g,
-                        true, workspace, workspace_bytes, (hipStream_t)stream);
+                        accumulate, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 // One launch of the single-row kernel per batch row; `accumulate`: add onto outs (the matvec entry) or
-// overwrite it (a single row through the matmul entry).  A launch stages its share of the states in LDS and
+// overwrite it (int4mm_matvec_overwrite, a single row through the matmul entry).  A launch stages its share of the states in LDS and
 // cuts K at most MV_MAX_SPLITS ways, so it covers MV_MAX_SPLITS x MV_MAX_UNITS_WG units of K; a longer K (the
 // reference's grid covers any: matvec_kernel.cu:339-347) goes in ranges of that many units, each a whole
 // number of quantisation groups, the later ones adding onto the result of the earlier.
@@ -1134,7 +1134,14 @@ extern "C" int int4mm_matvec(int bits, void* outs, const void* matrix, const voi
                              const void* scales, const void* zeros, const void* sparse_mask,
                              const int4mm_shape* shape, void* workspace, size_t workspace_bytes,
                              void* stream) {
-    return matvec_impl(bits, outs, matrix, multiplier, scales, zeros, sparse_mask, shape, workspace, workspace_bytes, stream);
+    return matvec_impl(bits, outs, matrix, multiplier, scales, zeros, sparse_mask, shape, true, workspace, workspace_bytes, stream);
+}
+
+extern "C" int int4mm_matvec_overwrite(int bits, void* outs, const void* matrix, const void* multiplier,
+                                       const void* scales, const void* zeros, const void* sparse_mask,
+                                       const int4mm_shape* shape, void* workspace, size_t workspace_bytes,
+                                       void* stream) {
+    return matvec_impl(bits, outs, matrix, multiplier, scales, zeros, sparse_mask, shape, false, workspace, workspace_bytes, stream);
 }
 
 // ---- the same product for callers that cannot allocate.  The hand-over slots and split-K
@@ -1179,5 +1186,5 @@ extern "C" int int4mm_matvec_static(int bits, void* outs, const void* matrix, co
     void* ptr;
     size_t bytes;
     if (!static_scratch(&ptr, &bytes)) return INT4MM_ERR_LAUNCH;
-    return matvec_impl(bits, outs, matrix, multiplier, scales, zeros, sparse_mask, shape, ptr, bytes, stream);
+    return matvec_impl(bits, outs, matrix, multiplier, scales, zeros, sparse_mask, shape, true, ptr, bytes, stream);
 }

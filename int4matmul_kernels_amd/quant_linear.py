@@ -105,10 +105,10 @@ class QuantLinear(torch.nn.Module):
         ext = pkg.load_extension()
         lead = x.shape[:-1]
         x3 = x.reshape(1, -1, self.in_features) if x.dim() != 3 else x
-        x3 = x3.contiguous().half()
-        outs = torch.zeros((x3.shape[0], x3.shape[1], self.out_features), dtype=torch.float16, device=x3.device)
-        ext.quant_matmul(self.bits, outs, self.matrix, x3, self.scales, self.zeros, self.group_size, self.sparse_mask)
-        y = outs.reshape(*lead, self.out_features)
+        y = ext.linear_forward(self.bits, self.out_features, self.matrix, x3, self.scales, self.zeros, self.group_size,
+                               self.sparse_mask)
+        if x3 is not x:
+            y = y.reshape(*lead, self.out_features)
         return y + self.bias if self.bias is not None else y
 
     def dequantized_weight(self) -> torch.Tensor:

@@ -54,3 +54,29 @@ def test_from_packed_round_trip_and_state_dict():
     assert torch.equal(a(x), b(x)) and torch.equal(a(x), c(x))
     with pytest.raises(ValueError):
         QuantLinear(3, 256, 128, sparse=True)
+
+
+@pytest.mark.parametrize("bits,sparse", [(4, False), (3, False), (2, False), (4, True)])
+@pytest.mark.parametrize("shape", [(1, 1), (3, 1), (8, 1), (70, 1), (130, 1), (515, 1), (1, 2), (2, 5), (1, 45), (1, 300), (0, 1), (2, 0)])
+def test_forward_overwrites_as_quant_matmul_on_zeros(bits, sparse, shape):
+    """a layer's output is allocated without a fill: whatever the memory held, every element is written, with the bits that
+    quant_matmul gives on a zeroed tensor"""
+    import int4matmul_kernels_amd as pkg
+    from int4matmul_kernels_amd.quant_linear import QuantLinear
+
+    gen = torch.Generator(device="cuda").manual_seed(bits)
+    K, S = 8192, 320                                 # few columns, long K: K is split, partial sums are handed over
+    matrix = torch.randint(-2 ** 31, 2 ** 31, (K // 16 if sparse else K * bits // 32, S), dtype=torch.int32, generator=gen, device="cuda")
+    scales = (torch.rand((K // 64, S), generator=gen, device="cuda") * 0.02 + 0.001).half()
+    zeros = (torch.rand((K // 64, S), generator=gen, device="cuda") * 3).half()
+    mask = torch.full((K // 32, S), 0x0FF00FF0, dtype=torch.int32, device="cuda") if sparse else None
+    layer = QuantLinear.from_packed(bits, matrix, scales, zeros, 64, mask)
+    x = torch.randn((*shape, K), generator=gen, device="cuda").half()
+    want = torch.zeros((*shape, S), dtype=torch.float16, device="cuda")
+    pkg.load_extension().quant_matmul(bits, want, matrix, x, scales, zeros, 64, mask)
+    stale = torch.full((*shape, S), float("nan"), dtype=torch.float16, device="cuda")
+    del stale                                        # (the allocator hands the block back to the layer's output)
+    assert torch.equal(layer(x), want)
+    assert torch.equal(layer(x.float()), want)       # converted on the way in, as before
+    if shape[0] > 1 and shape[1] == 1:
+        assert torch.equal(layer(x.expand(shape[0], 1, K).transpose(0, 1).contiguous().transpose(0, 1)), want)
