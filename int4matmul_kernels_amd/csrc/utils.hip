@@ -149,7 +149,7 @@ __global__ __launch_bounds__(256) void dense_pack_kernel(uint32_t* __restrict__ 
 // flight are then consecutive in memory, where walking along S reads lines K bytes apart, which for a K that is a power
 // of two fall onto few memory channels.
 // Bound by memory traffic: a whole weight_matrix_packing call at K = S = 16384 (637 MB) took 166 us with one 128-byte
-// line of each input per thread, lanes K bytes apart, and takes 147 so.
+// line of each input per thread, lanes K bytes apart, 147 so, and 133 with non-temporal loads (every byte is read once).
 constexpr int SPARSE_PACK_LANES = 32;                               // lanes along K: 512 rows of a column
 constexpr int SPARSE_PACK_ROWS = 16 * SPARSE_PACK_LANES;
 constexpr int SPARSE_PACK_COLS = 64;
@@ -174,8 +174,8 @@ __global__ __launch_bounds__(256) void sparse_pack_kernel(uint32_t* __restrict__
         const int64_t s = s0 + col0 + i * COLS_PASS;
         wq[i] = mq[i] = u32x4{0, 0, 0, 0};
         if (in_k && s < S) {
-            wq[i] = *reinterpret_cast<const u32x4*>(wt_in + s * K + k0 + 16 * lane);
-            mq[i] = *reinterpret_cast<const u32x4*>(msk_in + s * K + k0 + 16 * lane);
+            wq[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wt_in + s * K + k0 + 16 * lane));
+            mq[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(msk_in + s * K + k0 + 16 * lane));
         }
     }
     {
