@@ -211,8 +211,8 @@ INT4MM_API int int4mm_matmul(int bits, void* outs, const void* matrix, const voi
 
 /* 16:32 sparse int4 packer.  wt_in / msk_in: uint8 [S, K] (row = output column;
  * msk_in > 0 keeps the row); wt_outs: int32 [K/16, S]; msk_outs: int32 [K/32, S].
- * Requires K % 32 == 0.  Replaces sparse_int4_pack / weight_matrix_packing
- * (utils_kernel.cu:19-119, int4matmul.cpp:50-63).
+ * Requires K % 32 == 0, K <= 32 * 65535 and 16-byte aligned inputs; any S, in several launches where one grid
+ * cannot hold it.  Replaces sparse_int4_pack / weight_matrix_packing (utils_kernel.cu:19-119, int4matmul.cpp:50-63).
  * bad_blocks (device int32[1], may be NULL) is incremented once for every
  * (column, 32-row block) whose mask does not keep exactly 16 rows -- the
  * condition the reference asserts on the device (utils_kernel.cu:41). */

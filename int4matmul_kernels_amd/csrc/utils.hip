@@ -4,6 +4,8 @@
 // [rows, S] matrices is coalesced.
 #include "common.h"
 
+#include <algorithm>
+
 namespace i4 {
 
 // 32 codes of one column, blocks of 32 rows: the shared decode step.
@@ -153,11 +155,12 @@ __global__ __launch_bounds__(256) void dense_pack_kernel(uint32_t* __restrict__ 
 constexpr int SPARSE_PACK_LANES = 32;                               // lanes along K: 512 rows of a column
 constexpr int SPARSE_PACK_ROWS = 16 * SPARSE_PACK_LANES;
 constexpr int SPARSE_PACK_COLS = 64;
+constexpr int64_t SPARSE_PACK_TILES_LAUNCH = 1 << 20;               // tiles of a launch: a grid has no more than 2^32 threads
 __global__ __launch_bounds__(256) void sparse_pack_kernel(uint32_t* __restrict__ wt_outs,
                                                           uint32_t* __restrict__ msk_outs,
                                                           const uint8_t* __restrict__ wt_in,
                                                           const uint8_t* __restrict__ msk_in,
-                                                          int64_t S, int64_t K, uint32_t k_tiles,
+                                                          int64_t S, int64_t K, int64_t s_first, uint32_t k_tiles,
                                                           int* __restrict__ bad_blocks) {
     constexpr int LANES = SPARSE_PACK_LANES, CELLS = LANES / 2, COLS = SPARSE_PACK_COLS;
     constexpr int COLS_PASS = 256 / LANES, PASSES = COLS / COLS_PASS;
@@ -165,7 +168,8 @@ __global__ __launch_bounds__(256) void sparse_pack_kernel(uint32_t* __restrict__
     // the front in row order (0 ... 7: that row of the eight; 0x0C: a zero byte)
     __shared__ u32x2 front[256];
     __shared__ uint32_t tile[3][CELLS][COLS + 1];                   // low words, high words, masks
-    const int64_t k0 = (int64_t)(blockIdx.x % k_tiles) * SPARSE_PACK_ROWS, s0 = (int64_t)(blockIdx.x / k_tiles) * COLS;
+    const int64_t k0 = (int64_t)(blockIdx.x % k_tiles) * SPARSE_PACK_ROWS;
+    const int64_t s0 = s_first + (int64_t)(blockIdx.x / k_tiles) * COLS;
     const int lane = threadIdx.x % LANES, col0 = threadIdx.x / LANES;
     const bool in_k = k0 + 16 * lane < K;                           // (K is a multiple of 32: both lanes of a cell or neither)
     u32x4 wq[PASSES], mq[PASSES];
@@ -261,12 +265,14 @@ int int4mm_sparse_pack(void* wt_outs, void* msk_outs, const void* wt_in, const v
     if (!wt_outs || !msk_outs || !wt_in || !msk_in) return INT4MM_ERR_NULL;
     if (((uintptr_t)wt_in | (uintptr_t)msk_in) & 15u) return INT4MM_ERR_ALIGN;
     const int64_t k_tiles = (in_size + SPARSE_PACK_ROWS - 1) / SPARSE_PACK_ROWS;
-    const int64_t tiles = k_tiles * ((out_size + SPARSE_PACK_COLS - 1) / SPARSE_PACK_COLS);
-    if (tiles > 0xFFFFFFFF / 256) return INT4MM_ERR_SHAPE;          // (inputs of 2 x 0.5 TB: beyond any device)
-    hipLaunchKernelGGL(sparse_pack_kernel, dim3((unsigned)tiles), dim3(256), 0,
-                       (hipStream_t)stream, (uint32_t*)wt_outs, (uint32_t*)msk_outs,
-                       (const uint8_t*)wt_in, (const uint8_t*)msk_in, out_size, in_size,
-                       (uint32_t)k_tiles, (int*)bad_blocks);
+    const int64_t cols_launch = SPARSE_PACK_TILES_LAUNCH / k_tiles * SPARSE_PACK_COLS;                       // (k_tiles <= 4096)
+    for (int64_t s_first = 0; s_first < out_size; s_first += cols_launch) {
+        const int64_t tiles = k_tiles * ((std::min(cols_launch, out_size - s_first) + SPARSE_PACK_COLS - 1) / SPARSE_PACK_COLS);
+        hipLaunchKernelGGL(sparse_pack_kernel, dim3((unsigned)tiles), dim3(256), 0,
+                           (hipStream_t)stream, (uint32_t*)wt_outs, (uint32_t*)msk_outs,
+                           (const uint8_t*)wt_in, (const uint8_t*)msk_in, out_size, in_size, s_first,
+                           (uint32_t)k_tiles, (int*)bad_blocks);
+    }
     return check_launch("sparse_pack");
 }
 

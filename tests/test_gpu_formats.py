@@ -116,6 +116,36 @@ def test_sparse_pack_tile_edges(H, S, K):
             assert np.array_equal(m.cpu().numpy(), want_m)
 
 
+@pytest.mark.parametrize("K,S", [(544, (1 << 25) + 336), (32, (1 << 30) + 4304)])
+def test_sparse_pack_more_columns_than_a_launch_takes(H, K, S):
+    """two launches and more; the second is 2^30 columns of one cell, more than 2^32 input bytes each"""
+    need = 2 * S * K + 3 * S * K // 8
+    if torch.cuda.mem_get_info()[0] < need + (16 << 30):
+        pytest.skip(f"needs {need >> 30} GB")
+    P = 16 * 13                                         # the columns repeat with a period that no tile's width divides
+    assert S % P == 0
+    rng = np.random.default_rng(K)
+    codes = rng.integers(0, 16, (P, K), dtype=np.uint8)
+    keep = (rng.random((P, K // 32, 32)).argsort(axis=2) < 16).astype(np.uint8).reshape(P, K)
+    want_w, want_m = O.sparse_pack(codes, keep)
+    codes_all = torch.empty((S // P, P, K), dtype=torch.uint8, device=H.DEV)
+    keep_all = torch.empty_like(codes_all)
+    codes_all.copy_(H.t(codes)[None])
+    keep_all.copy_(H.t(keep)[None])
+    w = torch.full((K // 16, S), -1, dtype=torch.int32, device=H.DEV)
+    m = torch.full((K // 32, S), -1, dtype=torch.int32, device=H.DEV)
+    bad = torch.zeros(1, dtype=torch.int32, device=H.DEV)
+    try:
+        H.capi.sparse_pack(w, m, codes_all.reshape(S, K), keep_all.reshape(S, K), bad)
+        assert int(bad.item()) == 0
+        for got, want in ((w, want_w), (m, want_m)):
+            for row, want_row in zip(got, H.t(want)):
+                assert bool((row.reshape(-1, P) == want_row).all())
+    finally:
+        del codes_all, keep_all, w, m
+        torch.cuda.empty_cache()
+
+
 def test_sparse_pack_flags_wrong_popcount(H):
     S, K = 64, 64
     keep = np.zeros((S, K), np.uint8)
