@@ -143,32 +143,41 @@ __global__ __launch_bounds__(256) void dense_pack_kernel(uint32_t* __restrict__ 
 
 // 16:32 packer.  Inputs are in the [S, K] orientation (row = output column), outputs have lanes along the column
 // index, so the job is a transposition.  It is done on the outputs, which are 3 / 16 of the inputs' bytes: a workgroup
-// takes a tile of 64 columns x SPARSE_PACK_ROWS input rows, a wave's load is whole runs of consecutive bytes of a column
-// (a lane: half a 32-row cell, 16 bytes of each input), and the packed words go through LDS, from where a wave
-// stores 64 columns of one word row, 256 bytes.  Kept codes are compacted eight rows at a time: keep flags gathered
-// by a multiply, code bytes moved to the front by v_perm with selectors from a 256-entry table, squeezed to nibbles;
-// the two lanes of a cell exchange rank, mask and one word each.  Consecutive workgroups walk along K: the runs in
-// flight are then consecutive in memory, where walking along S reads lines K bytes apart, which for a K that is a power
-// of two fall onto few memory channels.
-// Bound by memory traffic: a whole weight_matrix_packing call at K = S = 16384 (637 MB) took 166 us with one 128-byte
-// line of each input per thread, lanes K bytes apart, 147 so, and 133 with non-temporal loads (every byte is read once).
-constexpr int SPARSE_PACK_LANES = 32;                               // lanes along K: 512 rows of a column
-constexpr int SPARSE_PACK_ROWS = 16 * SPARSE_PACK_LANES;
-constexpr int SPARSE_PACK_COLS = 64;
+// takes a tile of 16 LANES input rows x COLS columns, LANES threads along K and PASSES loads of each input per thread (a
+// load: half a 32-row cell, 16 bytes), a wave's load is whole runs of consecutive bytes of a column, and the packed words
+// go through LDS, from where they are stored along the columns.  Kept codes are compacted eight rows at a time: keep flags
+// gathered by a multiply, code bytes moved to the front by v_perm with selectors from a 256-entry table, squeezed to
+// nibbles; the two lanes of a cell exchange rank, mask and one word each.  Consecutive workgroups walk along K, so that the
+// runs in flight are consecutive in memory.
+// Bound by memory traffic.  A kernel with one 128-byte line of each input per thread, lanes K bytes apart, and this one,
+// whose loads are non-temporal (every byte is read once), us a launch:
+//   K x S                    16384 x 16384   15968 x 16385   8192 x 8192   11008 x 4096   1024 x 1024
+//   a line per thread          146 ... 164             184            49             36           5.8
+//   this kernel (5.5 TB/s)             116             127            28             20           3.9
+// The tile follows K: the fewest lanes that span it, at most 32, so that a tile is more than half full whatever K is.
+// A line per thread / 32 lanes and eight loads at any K / the fewest lanes:
+//   S = 2^20, K = 32: 15 / 80 / 14; K = 64: 32 / 82 / 27; S = 2^18, K = 128: 21 / 26 / 15; S = 4096, K = 64: 3.4 / 4.6 / 3.3 us.
+// Two loads of each input in flight per thread, four at 32 lanes, so that a tile has at least 32 columns and a store
+// fills whole lines.  Eight leave a small matrix to too few workgroups (1024 x 1024 5.2 us, 8192 x 63 5.2 against 3.8) and
+// gain nothing on a large one; two at 32 lanes (16 columns) take 105 instead of 116 us at 16384 x 16384, but 16.4 instead of
+// 15.3 at K = 512, S = 65536 and 24.9 instead of 22.5 at K = 544.
+constexpr int SPARSE_PACK_MAX_LANES = 32;
 constexpr int64_t SPARSE_PACK_TILES_LAUNCH = 1 << 20;               // tiles of a launch: a grid has no more than 2^32 threads
+constexpr int sparse_pack_passes(int lanes) { return lanes == 32 ? 4 : 2; }
+constexpr int sparse_pack_cols(int lanes) { return 256 / lanes * sparse_pack_passes(lanes); }
+template <int LANES>
 __global__ __launch_bounds__(256) void sparse_pack_kernel(uint32_t* __restrict__ wt_outs,
                                                           uint32_t* __restrict__ msk_outs,
                                                           const uint8_t* __restrict__ wt_in,
                                                           const uint8_t* __restrict__ msk_in,
                                                           int64_t S, int64_t K, int64_t s_first, uint32_t k_tiles,
                                                           int* __restrict__ bad_blocks) {
-    constexpr int LANES = SPARSE_PACK_LANES, CELLS = LANES / 2, COLS = SPARSE_PACK_COLS;
-    constexpr int COLS_PASS = 256 / LANES, PASSES = COLS / COLS_PASS;
+    constexpr int PASSES = sparse_pack_passes(LANES), CELLS = LANES / 2, COLS_PASS = 256 / LANES, COLS = sparse_pack_cols(LANES);
     // compaction table: for a byte of eight keep flags, the v_perm selectors that move the kept rows' code bytes to
     // the front in row order (0 ... 7: that row of the eight; 0x0C: a zero byte)
     __shared__ u32x2 front[256];
     __shared__ uint32_t tile[3][CELLS][COLS + 1];                   // low words, high words, masks
-    const int64_t k0 = (int64_t)(blockIdx.x % k_tiles) * SPARSE_PACK_ROWS;
+    const int64_t k0 = (int64_t)(blockIdx.x % k_tiles) * (16 * LANES);
     const int64_t s0 = s_first + (int64_t)(blockIdx.x / k_tiles) * COLS;
     const int lane = threadIdx.x % LANES, col0 = threadIdx.x / LANES;
     const bool in_k = k0 + 16 * lane < K;                           // (K is a multiple of 32: both lanes of a cell or neither)
@@ -236,15 +245,15 @@ __global__ __launch_bounds__(256) void sparse_pack_kernel(uint32_t* __restrict__
         }
     }
     __syncthreads();
-    const int64_t s = s0 + threadIdx.x % COLS;
     const int cells = (int)min((int64_t)CELLS, (K - k0) / 32);
-    if (s < S) {
-        for (int c = threadIdx.x / COLS; c < cells; c += 256 / COLS) {
-            const int64_t blk = k0 / 32 + c;
-            wt_outs[(2 * blk) * S + s] = tile[0][c][threadIdx.x % COLS];
-            wt_outs[(2 * blk + 1) * S + s] = tile[1][c][threadIdx.x % COLS];
-            msk_outs[blk * S + s] = tile[2][c][threadIdx.x % COLS];
-        }
+#pragma unroll
+    for (int i = 0; i < CELLS * COLS / 256; ++i) {
+        const int at = i * 256 + (int)threadIdx.x, c = at / COLS, col = at % COLS;
+        const int64_t s = s0 + col, blk = k0 / 32 + c;
+        if (c >= cells || s >= S) continue;
+        wt_outs[(2 * blk) * S + s] = tile[0][c][col];
+        wt_outs[(2 * blk + 1) * S + s] = tile[1][c][col];
+        msk_outs[blk * S + s] = tile[2][c][col];
     }
     if (bad && bad_blocks) atomicAdd(bad_blocks, bad);
 }
@@ -264,14 +273,25 @@ int int4mm_sparse_pack(void* wt_outs, void* msk_outs, const void* wt_in, const v
     if (out_size == 0 || in_size == 0) return INT4MM_OK;
     if (!wt_outs || !msk_outs || !wt_in || !msk_in) return INT4MM_ERR_NULL;
     if (((uintptr_t)wt_in | (uintptr_t)msk_in) & 15u) return INT4MM_ERR_ALIGN;
-    const int64_t k_tiles = (in_size + SPARSE_PACK_ROWS - 1) / SPARSE_PACK_ROWS;
-    const int64_t cols_launch = SPARSE_PACK_TILES_LAUNCH / k_tiles * SPARSE_PACK_COLS;                       // (k_tiles <= 4096)
+    int lanes = 2;
+    while (lanes < SPARSE_PACK_MAX_LANES && 16 * lanes < in_size) lanes *= 2;
+    const int64_t k_tiles = (in_size + 16 * lanes - 1) / (16 * lanes);
+    const int64_t cols = sparse_pack_cols(lanes), cols_launch = SPARSE_PACK_TILES_LAUNCH / k_tiles * cols;   // (k_tiles <= 4096)
     for (int64_t s_first = 0; s_first < out_size; s_first += cols_launch) {
-        const int64_t tiles = k_tiles * ((std::min(cols_launch, out_size - s_first) + SPARSE_PACK_COLS - 1) / SPARSE_PACK_COLS);
-        hipLaunchKernelGGL(sparse_pack_kernel, dim3((unsigned)tiles), dim3(256), 0,
-                           (hipStream_t)stream, (uint32_t*)wt_outs, (uint32_t*)msk_outs,
-                           (const uint8_t*)wt_in, (const uint8_t*)msk_in, out_size, in_size, s_first,
-                           (uint32_t)k_tiles, (int*)bad_blocks);
+        const int64_t tiles = k_tiles * ((std::min(cols_launch, out_size - s_first) + cols - 1) / cols);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(256), 0,
+                               (hipStream_t)stream, (uint32_t*)wt_outs, (uint32_t*)msk_outs,
+                               (const uint8_t*)wt_in, (const uint8_t*)msk_in, out_size, in_size, s_first,
+                               (uint32_t)k_tiles, (int*)bad_blocks);
+        };
+        switch (lanes) {
+            case 2: launch(sparse_pack_kernel<2>); break;
+            case 4: launch(sparse_pack_kernel<4>); break;
+            case 8: launch(sparse_pack_kernel<8>); break;
+            case 16: launch(sparse_pack_kernel<16>); break;
+            default: launch(sparse_pack_kernel<32>); break;
+        }
     }
     return check_launch("sparse_pack");
 }

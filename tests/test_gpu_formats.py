@@ -97,7 +97,7 @@ def test_sparse_pack_bit_exact_capi_and_extension(H):
 
 @pytest.mark.parametrize("S,K", [(64, 64), (63, 96), (65, 512), (1, 544), (128, 1056), (200, 480), (320, 1600)])
 def test_sparse_pack_tile_edges(H, S, K):
-    """edges of the packer's tile of 64 columns x 512 rows; cells that keep more or fewer than 16 rows are counted once each"""
+    """edges of the packer's tiles; cells that keep more or fewer than 16 rows are counted once each"""
     rng = np.random.default_rng(S * 10007 + K)
     codes_sk = rng.integers(0, 256, (S, K), dtype=np.uint8)
     keep_sk = (rng.random((S, K // 32, 32)).argsort(axis=2) < 16).astype(np.uint8)
@@ -114,6 +114,54 @@ def test_sparse_pack_tile_edges(H, S, K):
         if not extra:
             assert np.array_equal(w.cpu().numpy(), want_w)
             assert np.array_equal(m.cpu().numpy(), want_m)
+
+
+@pytest.mark.parametrize("S,K", [(1, 32), (255, 32), (257, 32), (600, 32), (127, 64), (129, 64), (63, 128), (65, 128), (33, 160),
+                                 (31, 256), (33, 256), (31, 288), (33, 992)])
+def test_sparse_pack_tile_follows_narrow_k(H, S, K):
+    """a tile has the fewest lanes that span K, and as many more columns: edges of each of the five tiles"""
+    rng = np.random.default_rng(S * 10007 + K)
+    codes = rng.integers(0, 256, (S, K), dtype=np.uint8)
+    keep = (rng.random((S, K // 32, 32)).argsort(axis=2) < 16).astype(np.uint8).reshape(S, K)
+    want_w, want_m = O.sparse_pack(codes & 15, keep)
+    # a row of guard words before and behind each output
+    w = torch.full((K // 16 + 2, S), -1, dtype=torch.int32, device=H.DEV)
+    m = torch.full((K // 32 + 2, S), -1, dtype=torch.int32, device=H.DEV)
+    keep[S // 2, 0] ^= 1                                # one cell keeps 15 or 17 rows: counted once, its words are not compared
+    bad = torch.zeros(1, dtype=torch.int32, device=H.DEV)
+    H.capi.sparse_pack(w[1:-1], m[1:-1], H.t(codes), H.t(keep), bad)
+    assert int(bad.item()) == 1
+    w, m = w.cpu().numpy(), m.cpu().numpy()
+    assert (w[[0, -1]] == -1).all() and (m[[0, -1]] == -1).all()
+    spoilt = np.zeros(S, bool)
+    spoilt[S // 2] = True
+    assert np.array_equal(w[1:-1][:, ~spoilt], want_w[:, ~spoilt]) and np.array_equal(w[3:-1], want_w[2:])
+    assert np.array_equal(m[1:-1][:, ~spoilt], want_m[:, ~spoilt]) and np.array_equal(m[2:-1], want_m[1:])
+
+
+@pytest.mark.parametrize("K", [32, 64])
+def test_sparse_pack_narrow_k_is_as_fast_as_a_square(H, K):
+    """the same bytes in 2^20 columns of one or two cells and in columns of 2048 rows: within a factor of two (they take
+    equal time; a tile that is 512 rows deep whatever K is took five and three times as long)"""
+    def best_us(k, s):
+        codes = torch.randint(0, 16, (s, k), dtype=torch.uint8, device=H.DEV)
+        keep = torch.zeros((s, k // 32, 32), dtype=torch.uint8, device=H.DEV)
+        keep[..., ::2] = 1
+        w = torch.empty((k // 16, s), dtype=torch.int32, device=H.DEV)
+        m = torch.empty((k // 32, s), dtype=torch.int32, device=H.DEV)
+        times = []
+        for _ in range(8):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            for _ in range(20):
+                H.capi.sparse_pack(w, m, codes, keep.reshape(s, k))
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end) * 50)
+        return min(times)
+
+    narrow, square = best_us(K, 1 << 20), best_us(2048, (1 << 20) * K // 2048)
+    assert narrow < 2 * square + 5, (narrow, square)
 
 
 @pytest.mark.parametrize("K,S", [(544, (1 << 25) + 336), (32, (1 << 30) + 4304)])
