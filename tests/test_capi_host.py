@@ -49,6 +49,8 @@ def test_argument_validation_happens_on_the_host():
         "S not multiple of 64": (lib.int4mm_matmul, 4, (1, 4, 128, 96, 16, 2, 64), None, 3),
         "packed rows mismatch": (lib.int4mm_matmul, 4, (1, 4, 128, 64, 15, 2, 64), None, 3),
         "sparse rows mismatch": (lib.int4mm_matmul, 4, (1, 4, 128, 64, 16, 2, 64), 0x1000, 3),
+        "overwriting matvec with M=2": (lib.int4mm_matvec_overwrite, 4, (1, 2, 128, 64, 16, 2, 64), None, 3),
+        "overwriting matvec, bits": (lib.int4mm_matvec_overwrite, 5, ok_vec, None, 1),
         "too few groups": (lib.int4mm_matmul, 4, (1, 4, 128, 64, 16, 1, 64), None, 3),
         "group size 32": (lib.int4mm_matmul, 4, (1, 4, 128, 64, 16, 4, 32), None, 4),
         "group size 0": (lib.int4mm_matmul, 4, (1, 4, 128, 64, 16, 4, 0), None, 4),
@@ -93,6 +95,8 @@ def test_extension_surface_and_cpu_tensors_are_rejected():
         ext.quant_matmul(7, outs, matrix, x, sz, sz, 64, None)
     with pytest.raises(RuntimeError):     # no CPU path: tensors must be on the GPU
         ext.quant_matmul(4, outs, matrix, x, sz, sz, 64, None)
+    with pytest.raises(RuntimeError):
+        ext.linear_forward(4, 64, matrix, x, sz, sz, 64, None)
     with pytest.raises(RuntimeError):
         ext.weight_matrix_packing(matrix, matrix, torch.zeros((64, 128), dtype=torch.uint8),
                                   torch.zeros((64, 128), dtype=torch.uint8))
