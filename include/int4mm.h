@@ -172,8 +172,9 @@ INT4MM_API int int4mm_matvec(int bits, void* outs, const void* matrix, const voi
                   const int4mm_shape* shape, void* workspace, size_t workspace_bytes,
                   void* stream);
 
-/* int4mm_matvec that overwrites outs instead of adding onto it: the same launches, bit for bit the result of
- * int4mm_matvec on zeroed outs, without the fill and without reading outs back. */
+/* int4mm_matvec that overwrites outs instead of adding onto it: the same launches with the same workspace, bit for
+ * bit the result of int4mm_matvec on zeroed outs, whatever outs held, without the fill.  (Only a K of several launches reads outs
+ * back, as its own earlier ranges wrote it.)  No counterpart in the reference, whose callers clear outs. */
 INT4MM_API int int4mm_matvec_overwrite(int bits, void* outs, const void* matrix, const void* multiplier,
                   const void* scales, const void* zeros, const void* sparse_mask,
                   const int4mm_shape* shape, void* workspace, size_t workspace_bytes,

@@ -4,7 +4,7 @@ The compiled extension lives inside the ``int4matmul_kernels_amd`` package, besi
 C-ABI library it links to.  This file, next to the package on ``sys.path``, makes the
 reference's own import line work unchanged: it loads the compiled module and puts it
 in ``sys.modules`` under this name, so ``int4matmul.quant_matmul`` and the ten other
-entry points (int4matmul.cpp:65-82) are the compiled functions themselves.  torch is
+entry points of the reference (int4matmul.cpp:65-82) are the compiled functions themselves.  torch is
 imported first, as every torch extension needs.  No fallback: a missing build raises
 ImportError.
 """

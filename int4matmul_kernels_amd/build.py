@@ -3,8 +3,9 @@
 * ``libint4mm_hip.so`` -- the C-ABI library (include/int4mm.h): hand-written HIP
   kernels compiled by hipcc for gfx950 only.  No torch dependency.
 * ``int4matmul.*.so`` -- the Python extension module ``int4matmul`` with the
-  reference's eleven entry points (int4matmul.cpp:65-82), compiled by the host
-  C++ compiler against torch/pybind11 and linked to the library above.
+  reference's eleven entry points (int4matmul.cpp:65-82) and ``linear_forward``
+  for ``QuantLinear``, compiled by the host C++ compiler against torch/pybind11
+  and linked to the library above.
 
 Run ``python -m int4matmul_kernels_amd.build`` (or ``__graft_entry__.build()``).
 """

@@ -1,7 +1,7 @@
 // Python extension module `int4matmul`: the reference's eleven entry points
 // (int4matmul.cpp:65-82) with the same names, positional argument order and
-// in-place semantics, implemented as thin calls into the C ABI of
-// libint4mm_hip.so (include/int4mm.h).  This file is compiled by the host
+// in-place semantics, and linear_forward, which QuantLinear calls; implemented
+// as thin calls into the C ABI of libint4mm_hip.so (include/int4mm.h).  This file is compiled by the host
 // compiler only; torch appears here for tensor metadata, the current HIP
 // stream, the device guard and the scratch allocation -- nothing else.
 //
@@ -176,8 +176,10 @@ void quant_matmul(uint32_t bits, TENSOR_MULT_ARGS) {
 // The product of a layer that holds its weights: [batch, seq_len, in_size] states to a new [batch, seq_len, out_size]
 // tensor.  Both products overwrite, so the output is allocated without a fill: the products' kernels are the same as
 // quant_matmul's on a zeroed tensor, one launch less per call and, with the checks and allocation in one native call, less
-// host time (QuantLinear, us per pass: sixteen 1024 x 1024 matvecs 221 -> 119; four layers of K = 5120, S = 20480 with 1 / 8 /
-// 64 tokens 56 -> 48 / 88 -> 71 / 151 -> 118; one with 2048 rows 416 -> 403).
+// host time.  QuantLinear, us per pass, conversions, zeros and quant_matmul called one by one from Python / in this one call with
+// the output zeroed / unfilled: sixteen 1024 x 1024 matvecs 221 / 179 / 119; four layers of K = 5120, S = 20480 with one token
+// 56 / 56 / 48, 8 tokens 88 / 88 / 72, 64 tokens 154 / 153 / 118; one with 2048 rows 410 / 410 / 399: where kernels are long the
+// gain is the fill alone.
 torch::Tensor linear_forward(uint32_t bits, int64_t out_size, torch::Tensor matrix, torch::Tensor multiplier,
                              torch::Tensor scales, torch::Tensor zeros, int group_size,
                              c10::optional<torch::Tensor> sparse_mask) {

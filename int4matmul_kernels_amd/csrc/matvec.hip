@@ -57,7 +57,7 @@ struct MatvecArgs {
     uint32_t* sticky;       // hand-over error word of the workspace (non-zero: poisoned)
     int spin_limit;         // polls before a reader gives up
     int rows;               // several rows of states in one pass (NR = 4 kernels): how many (2 .. 4), K apart in x, S apart in outs
-    int accumulate;         // ... and whether they add onto outs (the matvec entry) or overwrite it (the matmul entry)
+    int accumulate;         // add onto outs (int4mm_matvec) or overwrite it (int4mm_matvec_overwrite, the matmul entry)
 };
 
 // ------------------------------------------------------------------ formats
@@ -1047,9 +1047,8 @@ static int matvec_impl(int bits, void* outs, const void* matrix, const void* mul
                     (const h16*)zeros, B, K, S, g, accumulate, (hipStream_t)stream, (const uint32_t*)sparse_mask, workspace, workspace_bytes))
         return check_launch("matvec");
 
-    // more batch elements than the few-row kernels take at once: chunks of up to 512 through them (they add onto outs
-    // as the matvec does; 1 100 elements at K=4096, S=4096: three launches instead of 1 100), the plain kernel for what
-    // they do not take
+    // more batch elements than the few-row kernels take at once: chunks of up to 512 through them (1 100 elements at
+    // K=4096, S=4096: three launches instead of 1 100), the plain kernel, a launch per element, for what they do not take
     int64_t done = 0;
     if (B > SK_WIDE_MAX_ROWS && !tuning(TUNE_NO_SKINNY)) {
         while (B - done >= 2) {

@@ -3,8 +3,9 @@
 The reference is driven by an out-of-tree caller (reduced-kobold, README.md:1)
 that keeps, per layer, the packed matrix, scales, zeros and optional 16:32 mask
 and calls ``int4matmul.quant_matmul`` (int4matmul.cpp:26-48) with a freshly
-zeroed output.  ``QuantLinear`` is that holder: buffers in the layouts the
-kernels read, the call convention of kernel_test.py:254-259, and two ways to
+zeroed output (kernel_test.py:254-259).  ``QuantLinear`` is that holder: buffers in the
+layouts the kernels read, a forward pass through ``int4matmul.linear_forward`` (the same
+product into a new output, which is not zeroed first), and two ways to
 fill it -- from already packed tensors, or by round-to-nearest quantisation of
 an fp16 ``[in, out]`` weight, packed on the device by the library's packers.
 """

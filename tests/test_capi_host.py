@@ -1,7 +1,7 @@
 """Host-only checks (no GPU): the C-ABI library loads, exports every symbol
 include/int4mm.h declares, and rejects bad arguments before touching the
 device; the ``int4matmul`` extension exposes the reference's eleven entry points
-(int4matmul.cpp:65-82) and fails loudly on CPU tensors."""
+(int4matmul.cpp:65-82) and the one that ``QuantLinear`` calls, and fails loudly on CPU tensors."""
 import ctypes as C
 import os
 import re
@@ -81,7 +81,7 @@ def test_argument_validation_happens_on_the_host():
 
 def test_extension_surface_and_cpu_tensors_are_rejected():
     ext = pkg.load_extension()
-    names = ["weight_matrix_packing", "quant_matmul"] + [
+    names = ["weight_matrix_packing", "quant_matmul", "linear_forward"] + [
         f"quant_int{b}_linear_mult{suffix}" for b in (4, 3, 2) for suffix in ("", "_mtx", "_vec")]
     for n in names:
         assert callable(getattr(ext, n)), n
