@@ -3,7 +3,7 @@
 TEST INFRASTRUCTURE ONLY.  This module restates, in numpy, what the reference
 CUDA kernels compute.  It is imported by ``tests/``, by
 ``__graft_entry__.smoke()`` and by the ``cpu_baseline`` leg of ``bench.py`` as
-the checker; the product (the HIP library and the ``int4matmul`` extension)
+the oracle; the product (the HIP library and the ``int4matmul`` extension)
 never imports it and has no CPU fallback.
 
 Every function cites the reference lines it follows (paths relative to the

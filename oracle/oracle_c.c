@@ -2,7 +2,7 @@
  * Scalar C restatement of the reference's decode loops and products.
  *
  * TEST INFRASTRUCTURE ONLY: built into oracle/liboracle_c.so and loaded by
- * tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg as a checker
+ * tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg as the oracle
  * and as the "port" CPU baseline.  Nothing in the product links or loads it.
  *
  * It deliberately follows the *loop structure* of the CUDA decoders (shift and
