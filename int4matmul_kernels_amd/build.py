@@ -21,7 +21,7 @@ PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG, "csrc")
 OBJ = os.path.join(PKG, "build")
 LIB = os.path.join(PKG, "libint4mm_hip.so")
-HIP_SOURCES = ["api.hip", "utils.hip", "matvec.hip", "matmul.hip", "skinny.hip"]
+HIP_SOURCES = ["api.hip", "utils.hip", "matvec.hip", "matmul.hip", "skinny.hip", "wide.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
@@ -52,7 +52,7 @@ def build_hip_library(verbose: bool = False) -> str:
         src, obj = pair
         return _run([HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, src), "-o", obj])
 
-    with ThreadPoolExecutor(max_workers=4) as ex:
+    with ThreadPoolExecutor(max_workers=8) as ex:
         outs = list(ex.map(one, zip(HIP_SOURCES, objs)))
     if verbose:
         print("".join(outs))

@@ -38,7 +38,7 @@
 // which the matrix core multiplies exactly; a second MFMA on the same operand
 // masked to 0x0010 gives 16 * 2^-24 * (sum of the kept rows' states), and
 //     y[m, n] += s[n] * (2^24 (accA - accM) - z[n] * 2^20 accM).
-#include "common.h"
+#include "rows.h"
 
 #include <algorithm>
 #include <atomic>
@@ -46,143 +46,9 @@
 
 namespace i4 {
 
-// magic numbers (div_magic) of the divisors of the balanced launch's range arithmetic: K / 64, the group's units, q, q + 1
-struct BalancedMagics { uint32_t units, group_units, share_lo, share_hi; };
-
-struct SkinnyArgs {
-    h16* outs;
-    const uint32_t* matrix;
-    const uint32_t* mask;   // 16:32 sparse only
-    const h16* x;
-    const h16* scales;
-    const h16* zeros;
-    int R, K, S;
-    int group_units;        // group size / 64
-    int units_per_wave;
-    int accumulate;         // 1: outs = fp16(fp32(outs) + product) (matvec semantics); 0: overwrite
-    // split-K across workgroups (gridDim.z > 1; narrow matrices with a long K): each workgroup takes
-    // `units_per_split` units, stores its fp32 partial tile to `part` and counts itself in; the last one
-    // to arrive adds the partials up in split order and writes the strip
-    int units_per_split;
-    float* part;
-    int* counters;
-    int block_rows;         // wide kernel: rows of states per workgroup (blockIdx.y), a multiple of 16
-    // balanced launch of the few-row kernel (more strips than CUs): 256 workgroups share the strips' units
-    // evenly, workgroup i takes [i q + i r / 256, (i + 1) q + (i + 1) r / 256) of strips x units, strip-major
-    int bal_q, bal_r;
-    BalancedMagics bal_magics;
-    // launch with a fifth column per lane: the first `wide_wgs` workgroups take 80 columns, the others 64
-    int wide_wgs;
-};
-
 constexpr int SK_PITCH = 144;                   // bytes between rows of a staged unit (128 + 16: conflict-free)
 constexpr int SK_XBUF = 32 * SK_PITCH;          // one staged unit: 32 rows x 64 k
 constexpr int SK_WAVE_LDS = 2 * SK_XBUF + 256;  // two unit buffers + the group sums of 32 rows
-
-template <int CW> struct Words;
-template <> struct Words<4> { typedef u32x4 type; };
-template <> struct Words<2> { typedef u32x2 type; };
-template <> struct Words<1> { typedef uint32_t type; };
-
-template <int CW>
-__device__ __forceinline__ uint32_t word_of(const typename Words<CW>::type& v, int c) {
-    if constexpr (CW == 1) return v;
-    else return v[c];
-}
-
-
-// Per format: the k order of the 8 halves of an operand chunk, the offsets the
-// magic-number decode leaves on the low / high half of operand register e, and
-// the packed rows of a 32-row block.
-//   int4: order 0,4,1,5,2,6,3,7; registers 0, 2 carry 1024 + q, registers 1, 3 carry 64 + q
-//   int2: natural order, {1024 + q_even, 256 + q_odd};  int3: natural order, {1024 + q_even, 128 + q_odd}
-template <int BITS, bool SPARSE = false> struct SkFmt;
-template <> struct SkFmt<4, true> {
-    static constexpr int ROWS = 2, LOADS = 6;            // per block: two words of codes and the mask word
-    __device__ static constexpr int order(int e) { return (e >> 1) + 4 * (e & 1); }
-    __device__ static constexpr uint32_t offs(int) { return 0u; }
-};
-template <> struct SkFmt<4> {
-    static constexpr int ROWS = 4, LOADS = 2;            // packed rows per block, loads per lane and unit
-    __device__ static constexpr int order(int e) { return (e >> 1) + 4 * (e & 1); }
-    __device__ static constexpr uint32_t offs(int e) { return (e & 1) ? 0x54005400u : 0x64006400u; }
-};
-template <> struct SkFmt<2> {
-    static constexpr int ROWS = 2, LOADS = 2;
-    __device__ static constexpr int order(int e) { return e; }
-    __device__ static constexpr uint32_t offs(int) { return 0x5C006400u; }
-};
-template <> struct SkFmt<3> {
-    static constexpr int ROWS = 3, LOADS = 4;
-    __device__ static constexpr int order(int e) { return e; }
-    __device__ static constexpr uint32_t offs(int) { return 0x58006400u; }
-};
-
-// The 8 codes of one chunk (`f`: BITS bits apart, LSB first, garbage above) -> MFMA
-// operand of magic numbers; m0/g0 (and m1/g1 for int4) are the format's mask and
-// magic constants held in VGPRs.
-template <int BITS>
-__device__ __forceinline__ h16x8 magic_operand(uint32_t f, uint32_t m0, uint32_t m1, uint32_t g0, uint32_t g1) {
-    u32x4 r;
-    if constexpr (BITS == 4) {
-        const uint32_t f8 = f >> 8;
-        r = u32x4{(f & m0) | g0, (f & m1) | g1, (f8 & m0) | g0, (f8 & m1) | g1};
-    } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const uint32_t u = f >> (2 * BITS * e);
-            r[e] = (__builtin_amdgcn_perm(u, u, 0x01000100u) & m0) | g0;       // low 16 bits in both halves
-        }
-    }
-    return bitcast<h16x8>(r);
-}
-
-// 16:32: `v` = the chunk's kept codes as consecutive nibbles, `sel` = the selectors of its mask byte
-__device__ __forceinline__ u32x4 sparse_operand(uint32_t v, const u32x4& sel, uint32_t nib, uint32_t flag) {
-    const uint32_t even = (v & nib) | flag, odd = ((v >> 4) & nib) | flag;
-    return u32x4{__builtin_amdgcn_perm(odd, even, sel.x), __builtin_amdgcn_perm(odd, even, sel.y),
-                 __builtin_amdgcn_perm(odd, even, sel.z), __builtin_amdgcn_perm(odd, even, sel.w)};
-}
-
-__device__ __forceinline__ h16x8 exact_operand_sparse(uint32_t v, uint32_t m8, h16 sc, h16 ze) {
-    h16 row[8];
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-        const bool kept = (m8 >> r) & 1u;
-        row[r] = kept ? dequant_code<4>(v & 15u, sc, ze) : (h16)0.0f;
-        v >>= kept ? 4 : 0;
-    }
-    h16x8 o;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = row[SkFmt<4, true>::order(e)];
-    return o;
-}
-
-// The chunk's 8 fp16 weights themselves, in the operand's k order, in either quantisation mode
-// (the mode belongs to the lane's column and group), bit-exact with dequant_code and without a
-// branch: from the magic-number pairs, P = the codes (offsets removed, exact) or +-2^e,
-//     A = P + N (one rounding),  w = fma(A, B, C) (one rounding)
-// with (N, B, C) = (-z, s, -0) for a linear group -- fp16(q - z), then fp16(. * s); adding -0
-// changes no bit -- and (-0, -s, z) for an exponent group, the reference's single-rounded fma.
-template <int BITS>
-__device__ __forceinline__ h16x8 exact_operand(uint32_t f, uint32_t m0, uint32_t m1, uint32_t g0, uint32_t g1,
-                                               h16 sc, h16 ze) {
-    const u32x4 h = bitcast<u32x4>(magic_operand<BITS>(f, m0, m1, g0, g1));
-    const bool expo = !(sc >= (h16)0.0f);
-    const h16x2 minus0 = as_h2(0x80008000u), s2 = {sc, sc}, z2 = {ze, ze};
-    const h16x2 N = expo ? minus0 : -z2, B = expo ? -s2 : s2, C = expo ? z2 : minus0;
-    u32x4 r;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const uint32_t offs = SkFmt<BITS>::offs(e);                    // {2^a, 2^b} as halves
-        const h16x2 q = as_h2(h[e]) - as_h2(offs);                     // exact
-        // the same offsets as integers, for the packed multiply: 2^(exponent field - 15)
-        const uint32_t ints = off2(1u << (((offs >> 10) & 31u) - 15u), 1u << (((offs >> 26) & 31u) - 15u));
-        const h16x2 P = expo ? as_h2(expo_operand<BITS>(h[e], ints)) : q;
-        r[e] = as_u32(__builtin_elementwise_fma(P + N, B, C));
-    }
-    return bitcast<h16x8>(r);
-}
 
 // Balanced launch: workgroup i of 256 takes the range [i q + i r / 256, (i + 1) q + (i + 1) r / 256) of
 // strips x units (strip-major; q, r = quotient and remainder of the total by 256).  The range is at least one
@@ -752,509 +618,6 @@ __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix,
     }
 }
 
-// ---- 17 ... 512 rows, every format: the eight waves of a workgroup share one staged copy of the states.
-// In the kernel above every wave stages the states of its own units, so a workgroup of 64 columns reads
-// all R x K states: with R = 64 that is four times the packed weights it reads.  Here the waves stand side
-// by side along the columns (32 each, 256 per workgroup), all walk the same units, and each unit's states
-// (16 MT rows x 128 bytes) are moved to LDS once per workgroup, by all 512 threads, a unit ahead of the
-// MFMAs: one barrier per unit.  Thread t stages chunk t % 8 (8 k) of row t / 8.  With this many rows the
-// kernel is bound by its vector instructions, and folding scale and zero into the accumulators once per
-// group (3 operations per accumulator element, plus the row sums at the staging) costs more of them than
-// dequantising each weight: the operand is the reference's fp16(fp16(q - z) s), three packed operations
-// per pair of weights on top of the magic-number decode, and the accumulators hold the product itself.
-// K is split across workgroups (blockIdx.z) with the hand-over above, one counter per wave.
-template <int BITS, int MT, bool SPARSE = false>
-__global__ __launch_bounds__(512) void wide_rows_kernel(const uint32_t* pre_matrix, const h16* pre_x, const h16* pre_scales, const h16* pre_zeros,
-                                                   int pre_S, int pre_K, int pre_group_units, int pre_units, SkinnyArgs a) {
-    // (what the first loads depend on, once more in front of the record: the first dwords of a kernel's arguments
-    // reach a wave in registers at its start, a record's fields are fetched by the wave itself)
-    a.matrix = pre_matrix; a.x = pre_x; a.scales = pre_scales; a.zeros = pre_zeros; a.S = pre_S; a.K = pre_K;
-    a.group_units = pre_group_units; a.units_per_split = pre_units;
-    using F = SkFmt<BITS, SPARSE>;
-    // (units of weights in flight per wave: four; two in the tall 16:32 blocks, whose registers are short)
-    constexpr int CW = 2, NL = F::LOADS, PF = (SPARSE && MT > 4) ? 2 : 4, ROWS = 16 * MT, STRIP = 16 * CW, WSTRIP = 8 * STRIP;
-    constexpr int XBUF = ROWS * SK_PITCH;
-    extern __shared__ __attribute__((aligned(16))) char lds[];
-    typedef typename Words<CW>::type words_t;
-    const int t = threadIdx.x, lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int j = lane & 15, h = lane >> 4;
-    const int col0 = blockIdx.x * WSTRIP + wave * STRIP + CW * j;
-    const int units = a.K / 64;
-    const int u0 = blockIdx.z * a.units_per_split, u1 = min(units, u0 + a.units_per_split);
-    const int row0 = blockIdx.y * a.block_rows;
-    const int R = min(a.block_rows, a.R - row0);
-    const int group_lo = u0 / a.group_units;
-    const int groups = (u1 + a.group_units - 1) / a.group_units - group_lo;
-
-    // (16:32: the selector table of the kernel above, same layout)
-    __shared__ __attribute__((aligned(16))) u32x4 lut_table[SPARSE ? 256 : 1];
-    const char* lut = reinterpret_cast<const char*>(lut_table);
-    if constexpr (SPARSE) {
-        for (int b = t; b < 256; b += 512) {
-            uint32_t selb[8];
-            int rank = 0;
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                const bool k = (b >> r) & 1;
-                selb[r] = k ? (uint32_t)((rank & 1) * 4 + (rank >> 1)) : 0x0Cu;
-                rank += k;
-            }
-            u32x4 e;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) e[q] = selb[q] | (0x0Cu << 8) | (selb[q + 4] << 16) | (0x0Cu << 24);
-            lut_table[((b & 15) << 4) | (b >> 4)] = e;
-        }
-    }
-    // LDS: two unit buffers, a flag, the strip's scales and zeros
-    char* const xb = lds;
-    int* const flag = reinterpret_cast<int*>(lds + 2 * XBUF);
-    uint32_t* const sz = reinterpret_cast<uint32_t*>(lds + 2 * XBUF + 16);
-    auto scan_scales = [&]() -> bool {
-        if (t == 0) *flag = 0;
-        __syncthreads();
-        bool bad = false;
-        const int n = groups * (WSTRIP / 2);
-        for (int i = t; i < n; i += 512) {
-            const int g = i / (WSTRIP / 2), c = i % (WSTRIP / 2);
-            const int64_t at = (int64_t)(group_lo + g) * a.S + blockIdx.x * WSTRIP + 2 * c;
-            const uint32_t two = *reinterpret_cast<const uint32_t*>(a.scales + at);
-            bad |= !(as_h2(two).x >= (h16)0.0f) || !(as_h2(two).y >= (h16)0.0f);
-            sz[i] = two;
-            sz[n + i] = *reinterpret_cast<const uint32_t*>(a.zeros + at);
-        }
-        if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) *flag = 1;
-        __syncthreads();
-        return *flag != 0;
-    };
-
-    f32x4 acc[CW][MT];
-#pragma unroll
-    for (int c = 0; c < CW; ++c)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[c][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    // weights of unit u: as in the kernel above (lane group h: chunk h of each of the unit's two blocks)
-    const int wrow = BITS == 4 ? h : (h >> 1);
-    const int wshift = BITS == 4 ? 0 : (BITS == 2 ? 16 * (h & 1) : (h == 0 ? 0 : h == 1 ? 24 : h == 2 ? 16 : 40));
-    const uint32_t* wbase = a.matrix + (int64_t)(SPARSE ? 0 : wrow) * a.S + col0;
-    const uint32_t* mbase = SPARSE ? a.mask + col0 : nullptr;
-    auto load_w = [&](words_t w[NL], int u) {
-        const uint32_t* p = wbase + (int64_t)u * (2 * F::ROWS) * a.S;
-        if constexpr (SPARSE) {          // every lane group: both words of kept codes and the mask word of each block
-            const uint32_t* pm = mbase + (int64_t)u * 2 * a.S;
-#pragma unroll
-            for (int blk = 0; blk < 2; ++blk) {
-                w[3 * blk] = __builtin_nontemporal_load(reinterpret_cast<const words_t*>(p + (int64_t)(2 * blk) * a.S));
-                w[3 * blk + 1] = __builtin_nontemporal_load(reinterpret_cast<const words_t*>(p + (int64_t)(2 * blk + 1) * a.S));
-                w[3 * blk + 2] = __builtin_nontemporal_load(reinterpret_cast<const words_t*>(pm + (int64_t)blk * a.S));
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < NL; ++i) {
-                const int row = BITS == 3 ? 3 * (i >> 1) + (i & 1) : F::ROWS * i;
-                w[i] = __builtin_nontemporal_load(reinterpret_cast<const words_t*>(p + (int64_t)row * a.S));
-            }
-        }
-    };
-    auto chunk_bits = [&](const words_t w[NL], int blk, int c) -> uint32_t {
-        if constexpr (BITS == 3)
-            return (uint32_t)((((uint64_t)word_of<CW>(w[2 * blk + 1], c) << 32) | word_of<CW>(w[2 * blk], c)) >> wshift);
-        else
-            return word_of<CW>(w[blk], c) >> wshift;
-    };
-    // states: thread t moves chunk t % 8 of row t / 8 (and of row t / 8 + 64 in blocks of more than 64 rows)
-    constexpr int XP = (ROWS + 63) / 64;
-    struct XRegs { u32x4 v[XP]; };
-    const int xrow = t >> 3, xchunk = t & 7;
-    const h16* xsrc[XP];
-#pragma unroll
-    for (int q = 0; q < XP; ++q) xsrc[q] = a.x + (int64_t)(row0 + min(xrow + 64 * q, R - 1)) * a.K + xchunk * 8;
-    // (every thread loads -- rows beyond R re-read row R - 1, their products are never written: a load
-    // under a branch would make the compiler wait for all loads in flight at every use of one)
-    auto load_x = [&](int u) -> XRegs {
-        XRegs r;
-#pragma unroll
-        for (int q = 0; q < XP; ++q) r.v[q] = *reinterpret_cast<const u32x4*>(xsrc[q] + u * 64);
-        return r;
-    };
-    auto stage_x = [&](const XRegs& x, int p) {
-#pragma unroll
-        for (int k = 0; k < XP; ++k) {
-            const u32x4 v = x.v[k];
-            u32x4 q = v;
-            if constexpr (BITS == 4)         // the k order inside the chunk that the operand decode produces
-                q = u32x4{__builtin_amdgcn_perm(v[2], v[0], 0x05040100u), __builtin_amdgcn_perm(v[2], v[0], 0x07060302u),
-                          __builtin_amdgcn_perm(v[3], v[1], 0x05040100u), __builtin_amdgcn_perm(v[3], v[1], 0x07060302u)};
-            if (xrow + 64 * k < ROWS) *reinterpret_cast<u32x4*>(xb + p * XBUF + (xrow + 64 * k) * SK_PITCH + xchunk * 16) = q;
-        }
-    };
-
-    words_t w[PF][NL];
-    XRegs xr[PF];
-    const uint32_t m0 = in_vgpr(BITS == 4 ? 0x000F000Fu : BITS == 2 ? 0x000C0003u : 0x00380007u);
-    const uint32_t g0 = in_vgpr(BITS == 4 ? 0x64006400u : BITS == 2 ? 0x5C006400u : 0x58006400u);
-    const uint32_t m1 = BITS == 4 ? in_vgpr(0x00F000F0u) : 0u, g1 = BITS == 4 ? in_vgpr(0x54005400u) : 0u;
-    h16 sc[CW], ze[CW];
-    h16x2 s2[CW], c2[CW];               // {s, s} and {z, z} of the lane's columns
-#pragma unroll
-    for (int c = 0; c < CW; ++c) { sc[c] = (h16)0.f; ze[c] = (h16)0.f; s2[c] = h16x2{(h16)0.f, (h16)0.f}; c2[c] = s2[c]; }
-    auto load_sz = [&](int gi) {
-        const h16* ps = reinterpret_cast<const h16*>(sz) + (gi - group_lo) * WSTRIP + wave * STRIP + CW * j;
-        const h16* pz = ps + groups * WSTRIP;
-        const uint32_t s1 = *reinterpret_cast<const uint32_t*>(ps), z1 = *reinterpret_cast<const uint32_t*>(pz);
-        sc[0] = as_h2(s1).x; sc[1] = as_h2(s1).y; ze[0] = as_h2(z1).x; ze[1] = as_h2(z1).y;
-#pragma unroll
-        for (int c = 0; c < CW; ++c) {
-            s2[c] = h16x2{sc[c], sc[c]};
-            c2[c] = h16x2{ze[c], ze[c]};
-        }
-    };
-    // 16:32: the expanded chunk (halves 0x001q for a kept row, 0 for a dropped one; see the kernel above)
-    // ORed with 1024 is 1040 + q; minus 1040 the code, exactly, or -16; then the same two roundings, and
-    // the dropped rows are multiplied by 0 -- bit 4 of the half, the "kept" flag, times 0x3C0 is fp16 1.0
-    const uint32_t below = SPARSE ? (1u << (8 * h)) - 1u : 0u, rep_h = 0x01010101u * h;
-    const uint32_t sp_nib = SPARSE ? in_vgpr(0x0F0F0F0Fu) : 0u, sp_flag = SPARSE ? in_vgpr(0x10101010u) : 0u;
-    const uint32_t sp_kept = SPARSE ? in_vgpr(0x00100010u) : 0u, sp_idx = SPARSE ? in_vgpr(0x00000FF0u) : 0u;
-    auto sparse_chunk = [&](const words_t w[NL], int blk, int c, uint32_t& v, uint32_t& mb4) {
-        const uint32_t m = word_of<CW>(w[3 * blk + 2], c);
-        const uint64_t st = ((uint64_t)word_of<CW>(w[3 * blk + 1], c) << 32) | word_of<CW>(w[3 * blk], c);
-        v = (uint32_t)(st >> ((uint32_t)__builtin_popcount(m & below) << 2));
-        mb4 = __builtin_amdgcn_perm(m, m, rep_h);           // mask byte h, four times
-    };
-    auto sparse_scaled_operand = [&](uint32_t v, uint32_t mb4, int c) -> h16x8 {
-        const u32x4 sel = *reinterpret_cast<const u32x4*>(lut + (mb4 & sp_idx));
-        u32x4 r = sparse_operand(v, sel, sp_nib, sp_flag);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const h16x2 kept = as_h2((r[e] & sp_kept) * 0x3C0u);
-            const h16x2 q = as_h2(r[e] | 0x64006400u) - as_h2(0x64106410u);
-            r[e] = bitcast<uint32_t>(((q - c2[c]) * kept) * s2[c]);
-        }
-        return bitcast<h16x8>(r);
-    };
-    // the chunk's magic numbers minus their offsets are the codes, exactly; then the reference's own
-    // two roundings: fp16(fp16(q - z) s) (matmul.cuh:115-125)
-    auto scaled_operand = [&](uint32_t f, int c) -> h16x8 {
-        u32x4 r = bitcast<u32x4>(magic_operand<BITS>(f, m0, m1, g0, g1));
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const h16x2 q = as_h2(r[e]) - as_h2(F::offs(e));
-            r[e] = bitcast<uint32_t>((q - c2[c]) * s2[c]);
-        }
-        return bitcast<h16x8>(r);
-    };
-
-    // set f holds the weights of unit u0 + f; xr[f] the states of unit u0 + 1 + f (unit u0 goes to LDS at once)
-#pragma unroll
-    for (int f = 0; f < PF; ++f) load_w(w[f], min(u0 + f, u1 - 1));
-    {
-        const XRegs first = load_x(u0);
-#pragma unroll
-        for (int f = 0; f < PF; ++f) xr[f] = load_x(min(u0 + 1 + f, u1 - 1));
-        const bool general = scan_scales();
-        stage_x(first, 0);
-        __syncthreads();
-
-        // p: the LDS buffer that holds unit u; xn: the states of unit u + 1
-        auto step = [&](auto mode, int u, int p, words_t wu[NL], XRegs& xn) {
-            constexpr bool general = decltype(mode)::value;
-            if (u == u0 || u % a.group_units == 0) load_sz(u / a.group_units);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                h16x8 xa[MT];
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-                    xa[mt] = *reinterpret_cast<const h16x8*>(xb + p * XBUF + (j + 16 * mt) * SK_PITCH + (i * 4 + h) * 16);
-#pragma unroll
-                for (int c = 0; c < CW; ++c) {
-                    h16x8 wb;
-                    if constexpr (SPARSE) {
-                        uint32_t v, mb4;
-                        sparse_chunk(wu, i, c, v, mb4);
-                        wb = general ? exact_operand_sparse(v, mb4 & 0xFFu, sc[c], ze[c]) : sparse_scaled_operand(v, mb4, c);
-                    } else {
-                        const uint32_t f = chunk_bits(wu, i, c);
-                        wb = general ? exact_operand<BITS>(f, m0, m1, g0, g1, sc[c], ze[c]) : scaled_operand(f, c);
-                    }
-#pragma unroll
-                    for (int mt = 0; mt < MT; ++mt)
-                        acc[c][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[mt], wb, acc[c][mt], 0, 0, 0);
-                }
-            }
-            load_w(wu, min(u + PF, u1 - 1));
-            if (u + 1 < u1) stage_x(xn, p ^ 1);
-            xn = load_x(min(u + 1 + PF, u1 - 1));
-            __syncthreads();
-        };
-        auto run = [&](auto mode) {
-            int u = u0;
-            for (; u + PF <= u1; u += PF) {               // (whole rounds without early exits, as above)
-#pragma unroll
-                for (int f = 0; f < PF; ++f) step(mode, u + f, f & 1, w[f], xr[f]);
-            }
-#pragma unroll
-            for (int f = 0; f < PF - 1; ++f) {
-                if (u + f >= u1) break;
-                step(mode, u + f, f & 1, w[f], xr[f]);
-            }
-        };
-        if (general) run(std::integral_constant<bool, true>{});
-        else run(std::integral_constant<bool, false>{});
-    }
-
-    if (gridDim.z > 1) {
-        // hand-over between the workgroups of a strip (see the kernel above): every wave stores its part of
-        // the workgroup's partial tile, one counter per strip and row block
-        constexpr int NV = CW * MT * 4, THROUGH = 17;
-        const int tile = blockIdx.y * gridDim.x + blockIdx.x, ks = gridDim.z;
-        char* const slots = reinterpret_cast<char*>(a.part) + ((int64_t)(tile * ks) * 8 + wave) * (NV * 256);
-        const __amdgpu_buffer_rsrc_t mine = __builtin_amdgcn_make_buffer_rsrc(
-            slots + (int64_t)blockIdx.z * (8 * NV * 256), 0, NV * 256, 0x00020000);
-#pragma unroll
-        for (int c = 0; c < CW; ++c)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float v = acc[c][mt][e];
-                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), mine,
-                                                          (((c * MT + mt) * 4 + e) * 64 + lane) * 4, 0, THROUGH);
-                }
-        __builtin_amdgcn_s_waitcnt(0);                 // every store of this thread has been acknowledged
-        __syncthreads();
-        if (t == 0) *flag = __hip_atomic_fetch_add(a.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        if (*flag != ks - 1) return;
-        if (t == 0) __hip_atomic_store(a.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-        for (int c = 0; c < CW; ++c)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) acc[c][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int sp = 0; sp < ks; ++sp) {
-            const __amdgpu_buffer_rsrc_t theirs = __builtin_amdgcn_make_buffer_rsrc(
-                slots + (int64_t)sp * (8 * NV * 256), 0, NV * 256, 0x00020000);
-#pragma unroll
-            for (int c = 0; c < CW; ++c)
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        acc[c][mt][e] += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                            theirs, (((c * MT + mt) * 4 + e) * 64 + lane) * 4, 0, THROUGH));
-        }
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int m = mt * 16 + 4 * h + e;
-            if (m < R) {
-                h16* o = a.outs + (int64_t)(row0 + m) * a.S + col0;
-#pragma unroll
-                for (int c = 0; c < CW; ++c) {
-                    float v = acc[c][mt][e];
-                    if (a.accumulate) v += (float)o[c];
-                    o[c] = (h16)v;
-                }
-            }
-        }
-}
-
-// Plan of the wide kernel: row blocks of 16 ... 64 rows, 256-column strips, K split over about as many
-// workgroups as there are CUs (at least 8 units each; one counter per strip and row block: at most 1024).
-struct WidePlan { bool use; int mt, row_blocks, block_rows, ksplit, units_per_split; size_t part_bytes; };
-// LDS of the wide kernel: two unit buffers of states, a flag, the selector table's alignment slack, and the
-// strip's scales and zeros for the workgroup's share of K (1 KB per quantisation group)
-static size_t wide_lds_bytes(int block_rows, int64_t groups) {
-    return 2 * (size_t)block_rows * SK_PITCH + 1024 + 16 + (size_t)groups * 256 * 4;
-}
-static int64_t wide_groups(int64_t units, int64_t units_per_split, int64_t ksplit, int64_t group_units) {
-    int64_t groups = (units + group_units - 1) / group_units;
-    if (ksplit > 1) groups = std::min(groups, (units_per_split + group_units - 1) / group_units + 1);
-    return groups;
-}
-constexpr size_t WIDE_LDS_LIMIT = 150 * 1024;
-
-// `group_units`: 64-row units per quantisation group (K / 64 and more: a single group)
-// Whether the few-row kernel above runs 33 ... 96 rows (two or three row blocks per strip) as one round of 128 ... 256
-// workgroups, or through its own split-K on a narrow output (the same conditions as unsplit_cw / plan_skinny_split).
-static bool skinny_one_round(int64_t R, int64_t S, bool sparse) {
-    const int64_t blocks = (R + 31) / 32;
-    if (S % 64 == 0 && S / 32 * blocks < 192) return true;
-    for (const int c : {4, 2, 1}) {
-        if (sparse && c == 4) continue;
-        const int64_t wgs = S / (16 * c) * blocks;
-        if (S % (16 * c) == 0 && wgs >= 128 && wgs <= 256) return true;
-    }
-    return false;
-}
-
-static WidePlan plan_wide(int64_t R, int64_t K, int64_t S, bool sparse, int64_t group_units) {
-    WidePlan p{false, 0, 0, 0, 1, 0, 0};
-    // (knob: 1 = never, n >= 2 = from n rows on whatever the shape)
-    const int64_t knob = tuning(TUNE_NO_WIDE), min_rows = knob >= 2 ? knob : 17;
-    if (R < min_rows || R > SK_WIDE_MAX_ROWS || S % 256 != 0 || K % 64 != 0 || knob == 1) return p;
-    // Row blocks of up to 64 rows, or of up to 128 (16:32: with two units of weights in flight per wave instead
-    // of four, for the registers): every row block decodes the strip's weights again, so two blocks of 64 rows
-    // cost nearly twice one block of 128 --
-    // unless halving the number of workgroups means splitting K more than about six ways to fill the GPU, or
-    // into shares of less than 20 units, where the hand-over of the partial tiles (twice as large, twice as
-    // many) takes the gain back (measured: K=5120, S=20480, 128 rows 70 -> 52 us, int3 76 -> 58; K=8192,
-    // S=28672, 128 rows 127 -> 95 us; K=28672, S=8192, 192 rows 172 -> 132 us; K=S=8192, 128 rows, 8 splits
-    // instead of 4: 41 -> 46 us; K=2048, S=16384, 128 rows, shares of 8 units: 25 -> 30 us; 16:32, K=5120,
-    // S=20480: 96 rows 92 -> 51 us, 128 rows 79 (256-row tiles) -> 60 us)
-    const int64_t units = K / 64, forced = tuning(TUNE_MM_SPLIT);
-    int64_t wgs = 0, ks = 1;
-    auto shape = [&](int64_t tallest) {
-        p.row_blocks = (int)((R + tallest - 1) / tallest);
-        p.block_rows = (int)(((R + p.row_blocks - 1) / p.row_blocks + 15) / 16 * 16);
-        p.mt = p.block_rows / 16;
-        if (p.mt == 5) p.mt = 6;                      // (instantiated: 1, 2, 3, 4, 6, 8 tiles of 16 rows)
-        if (p.mt == 7) p.mt = 8;
-        p.block_rows = p.mt * 16;
-        wgs = S / 256 * p.row_blocks;
-        // (one workgroup per CU: as many splits as keep the grid within one round of 256 -- a grid a little
-        // larger than that runs a second round -- and four when even the unsplit grid leaves a third of the
-        // CUs idle)
-        ks = 256 / wgs;
-        if (ks <= 1 && wgs > 128 && wgs < 256) ks = 4;
-        ks = std::max<int64_t>(1, std::min<int64_t>(ks, units / 8));
-        if (forced >= 1) ks = std::min<int64_t>(forced, std::max<int64_t>(1, units / 4));
-        if (wgs > 1024) ks = 1;
-        // (a long share of K with small groups: more splits, within one round of workgroups, until the share's
-        // scales and zeros fit the LDS)
-        const size_t room = WIDE_LDS_LIMIT - (sparse ? 4096 : 0);
-        while (wgs * (ks + 1) <= 256 && ks < units / 8 &&
-               wide_lds_bytes(p.block_rows, wide_groups(units, (units + ks - 1) / ks, ks, group_units)) > room)
-            ++ks;
-    };
-    shape(128);
-    if (R <= 64 || ks > 6 || (ks > 1 && units / ks < 20)) shape(64);
-    // (49 ... 64 rows on a narrow output: two blocks of 32 rows with half the splits instead of one block of 64 --
-    // K=11008, S=4096: 28.7 -> 23.0 us; K=14336, S=4096: 31.3 -> 26.9; from 5120 columns on the single block wins on a long K)
-    if (!sparse && R > 48 && R <= 64 && S <= 4096 && forced < 1) shape(32);
-    // 65 ... 512 rows of a dense format against 1024 ... 32768 columns: block height
-    // (up to 128, 96, 64 or 48 rows) and split by a cost model fitted to 4 900 timed launches (int4, K = 2048 ...
-    // 28672, S = 4096 ... 8192, 72 ... 512 rows; its pick is within 0.3 % of the best measured candidate on average,
-    // 6.6 % at worst -- on 1 800 more launches at S = 2048 and 3072 with up to 16 splits, not used in the fit: 0.3 / 3.8 %
-    // (and it is used from 1024 columns on: K=8192, S=1280, 104 rows 27.8 -> 21.9 us);
-    // on 1 900 more at S = 11008 ... 28672, where it serves up to 192 rows: 0.3 / 10 %, the
-    // rules above 6.7 / 70 %: K=2048, S=28672, 128 rows 50 -> 30 us --,
-    // where the rules above were 8 % off on K <= 8192 and up to 73 % -- e.g. K=2048, S=8192, 416 rows: seven blocks
-    // of 64 rows split four ways, 49 us, against 28 us unsplit; int3, int2 and other group sizes rank alike):
-    // a workgroup takes a[row tiles] us per 64-row unit of its share plus 3.9 us; a split costs 0.8 us per way
-    // and 1.9 us per row tile, less 4.2; workgroups run in rounds of 256, the last one charged 3.5 us x its fill.
-    // (16:32, fitted apart to 2 300 launches at S = 4096 ... 8192: 1.12 / 1.20 / 1.32 / 1.54 us per unit, 4.2 us per
-    // workgroup, a split 0.9 us per way + 1.7 per row tile - 3.7, the last round 5.3 us x its fill; the pick is within
-    // 0.1 % of the best candidate on average, 2.8 % at worst, where the rules above were 5 % / 27 % off -- K=4096,
-    // S=8192, 160 rows 50 -> 39 us; K=14336, S=8192, 128 rows 82 -> 69)
-    struct WideCost { double per_unit[9], workgroup, split, per_way, per_tile, last_round; };
-    static const WideCost dense_cost = {{0, 0, 0, 0.617, 0.707, 0, 0.912, 0, 1.059}, 3.92, -4.164, 0.798, 1.915, 3.544};
-    static const WideCost sparse_cost = {{0, 0, 0, 1.12, 1.203, 0, 1.32, 0, 1.537}, 4.17, -3.744, 0.921, 1.701, 5.284};
-    if (R > 64 && S >= (sparse ? 4096 : 1024) && S <= (sparse ? 8192 : 32768) && forced < 1) {
-        const WideCost& wc = sparse ? sparse_cost : dense_cost;
-        const size_t room = WIDE_LDS_LIMIT - (sparse ? 4096 : 0);
-        double best = 1e30;
-        int64_t best_tall = 0, best_ks = 1;
-        for (const int64_t tallest : {128, 96, 64, 48}) {
-            shape(tallest);
-            const int64_t tiles = wgs;
-            for (int64_t k = 1; k <= 16 && (k == 1 || units / k >= 8) && tiles * k <= 1024; ++k) {
-                const int64_t share = (units + k - 1) / k, rounds = (tiles * k + 255) / 256, last = tiles * k - (rounds - 1) * 256;
-                if (wide_lds_bytes(p.block_rows, wide_groups(units, share, (units + share - 1) / share, group_units)) > room) continue;
-                const double t = rounds * (wc.per_unit[p.mt] * share + wc.workgroup) +
-                                 (k > 1 ? wc.split + wc.per_way * k + wc.per_tile * p.mt : 0.0) +
-                                 (rounds > 1 ? wc.last_round * last / 256.0 : 0.0);
-                if (t < best) { best = t; best_tall = tallest; best_ks = k; }
-            }
-        }
-        if (best_tall != 0) { shape(best_tall); ks = best_ks; }
-    }
-    p.units_per_split = (int)((units + ks - 1) / ks);
-    p.ksplit = (int)((units + p.units_per_split - 1) / p.units_per_split);
-    if (wide_lds_bytes(p.block_rows, wide_groups(units, p.units_per_split, p.ksplit, group_units)) >
-        WIDE_LDS_LIMIT - (sparse ? 4096 : 0))
-        return p;
-    // measured against the kernel above (K = 2048 ... 20480, S = 1024 ... 28672): with 17 ... 32 rows it
-    // needs 32 ... 96 strips and long shares of K, with 33 ... 64 rows matrices of 32 M weights and more
-    // and from 129 rows on the tile kernels win on wide outputs (beyond 14336 columns; from 193 rows beyond
-    // 10240, from 257 rows beyond 8192 -- K=8192, S=10240, 192 rows: 52 against 64 us; K=4096, S=14336, 192
-    // rows: 42.5 against 49, 256 rows: 52 against 50)
-    // (16:32, whose decode costs more here and in the tile kernels alike: 17 ... 32 rows from 64 M weights
-    // on, 33 ... 64 rows from 32 M, 65 ... 128 rows always, up to 256 rows for outputs of at most 8192 columns
-    // -- K=S=8192, 192 rows: 59 against 71 us --, beyond that of at most 4096)
-    if (knob < 2 && forced < 1) {
-        if (sparse) {
-            if (R <= 32 && K * S < (1ll << 26)) return p;
-            // (33 ... 64 rows: the kernel above while its two row blocks per strip make one round of workgroups -- outputs
-            // of at most 4096 columns -- up to K = 8192: K=S=4096, 40 / 64 rows 16.3 / 16.3 against 20.9 / 23.4 us; K=8192,
-            // S=4096 25.3 / 24.8 against 27.5 / 31.1; beyond that only on a short K: K=4096, S=5120 28.3 / 29.3 against
-            // 22.5 / 24.8; K=5120, S=6144 33.5 / 33.9 against 23.3 / 26.7)
-            if (R > 32 && R <= 64 &&
-                (skinny_one_round(R, S, true) ? (K <= 8192 || S < 3072) : (K < 4096 && K * S < (1ll << 25))))
-                return p;
-            // (the padded 256-row tiles win on very wide outputs against two row blocks)
-            if (R > 96 && R <= 128 && S > 16384 && p.row_blocks > 1) return p;
-            if (R > 128 && (S > 8192 || (R > 256 && S > 4096))) return p;
-        } else {
-            // (24 ... 31 strips only on a long K: K=14336, S=6144, 20 / 32 rows 24.5 / 24.5 against 29.6 / 32.3 us for the
-            // kernel above; K=8192, S=6144 18.9 / 19.0 against 18.7 / 19.5)
-            if (R <= 32 && (wgs < (units >= 160 ? 24 : 32) || wgs > 96 || p.units_per_split < 16)) return p;
-            // (one round of 129 ... 256 strips of 64 columns: the kernel above up to K = 6144 -- K=4096, S=14336, 20 / 32
-            // rows 16.3 / 17.7 against 18.4 / 18.3 us; K=5120, S=16384 19.4 / 21.8 against 22.7 / 22.8; K=8192, S=12288
-            // 25.8 / 27.1 against 25.1 / 25.1)
-            if (R <= 32 && S % 64 == 0 && S / 64 > 128 && S / 64 <= 256 && K <= 6144) return p;
-            // (33 ... 64 rows are two row blocks of the kernel above: where its strips can be cut to give one round of
-            // 128 ... 256 workgroups -- or its own split-K serves a narrow output -- it wins up to K = 5120, on outputs
-            // of at most 4096 columns up to K = 8192 and below 3072 columns always: K=S=4096, 40 / 64 rows 13.0 / 13.2
-            // against 16.1 / 18.7 us; K=5120, S=8192 18.5 / 18.9 against 19.4 / 22.3; K=8192, S=4096 19.5 / 19.6 against
-            // 22.3 / 26.6; K=8192, S=6144 24.7 / 25.0 against 21.9 / 25.4; K=14336, S=5120 36.9 against 27.6 / 31.3)
-            if (R > 32 && R <= 64 &&
-                (skinny_one_round(R, S, false) ? (K <= 5120 || (K <= 8192 && S <= 4096) || S < 3072) : K * S < (1ll << 25)))
-                return p;
-            // (with the plan from the cost model, up to 192 rows on any width it covers: K=4096, S=20480, 160 rows 50 us
-            // against 71 for the tiles, K=8192, S=20480, 192 rows 97 against 114, K=2048, S=20480 29 against 40)
-            // (193 ... 256 rows: on a K of at most 4096 as well -- K=4096, S=20480, 256 rows 64 against 74 us; K=8192: 122
-            // against 114)
-            if (R > 128 && S > 8192 && S > (R <= 192 ? 32768 : R <= 256 ? (K <= 4096 ? 32768 : 10240) : 8192)) return p;
-        }
-    }
-    p.part_bytes = p.ksplit > 1 ? (size_t)wgs * 8 * p.ksplit * (2 * p.mt * 4 * 256) : 0;
-    p.use = true;
-    return p;
-}
-
-template <int BITS, bool SPARSE = false>
-static bool launch_wide(SkinnyArgs a, const WidePlan& p, hipStream_t st) {
-    const size_t lds = wide_lds_bytes(p.block_rows, wide_groups(a.K / 64, p.units_per_split, p.ksplit, a.group_units));
-    if (lds > WIDE_LDS_LIMIT - (SPARSE ? 4096 : 0)) return false;
-    a.block_rows = p.block_rows;
-    a.units_per_split = p.units_per_split;
-    const dim3 grid((unsigned)(a.S / 256), (unsigned)p.row_blocks, (unsigned)p.ksplit), block(512);
-    if (noting("wide_rows_kernel<bits=%d,%s,row_tiles=%d> strips=%u row_blocks=%u ksplit=%u", BITS, SPARSE ? "16:32" : "dense", p.mt,
-               grid.x, grid.y, grid.z))
-        return true;
-    auto go = [&](auto kernel, int slot) {
-        static std::atomic<uint64_t> done[6];
-        int dev = 0;
-        hipGetDevice(&dev);
-        const uint64_t bit = 1ull << (dev & 63);
-        if (!(done[slot].load(std::memory_order_relaxed) & bit)) {
-            hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);
-            done[slot].fetch_or(bit, std::memory_order_relaxed);
-        }
-        hipLaunchKernelGGL(kernel, grid, block, lds, st, a.matrix, a.x, a.scales, a.zeros, a.S, a.K, a.group_units, a.units_per_split, a);
-    };
-    if (p.mt == 1) go(wide_rows_kernel<BITS, 1, SPARSE>, 0);
-    else if (p.mt == 2) go(wide_rows_kernel<BITS, 2, SPARSE>, 1);
-    else if (p.mt == 3) go(wide_rows_kernel<BITS, 3, SPARSE>, 2);
-    else if (p.mt == 4) go(wide_rows_kernel<BITS, 4, SPARSE>, 3);
-    else if (p.mt == 6) go(wide_rows_kernel<BITS, 6, SPARSE>, 4);
-    else go(wide_rows_kernel<BITS, 8, SPARSE>, 5);
-    return true;
-}
-
 template <int BITS, int CW, bool SPARSE>
 static bool launch_skinny(const SkinnyArgs& a, int waves, int ksplit, hipStream_t st) {
     const int strips = a.S / (16 * CW);
@@ -1445,12 +808,7 @@ static SkinnySplit plan_skinny_split(int64_t R, int64_t K, int64_t S, bool spars
 
 size_t skinny_workspace_bytes(int64_t R, int64_t K, int64_t S, bool sparse) {
     const SkinnySplit p = plan_skinny_split(R, K, S, sparse);
-    // (the split of the wide kernel can depend on the group size: room for whichever needs most)
-    size_t wide = 0;
-    for (const int64_t group_units : {1, 2, 3, 4, 6, 8, 16, 0x7FFFFFF}) {
-        const WidePlan w = plan_wide(R, K, S, sparse, group_units);
-        if (w.use) wide = std::max(wide, w.part_bytes);
-    }
+    const size_t wide = wide_workspace_bytes(R, K, S, sparse);
     const size_t balanced = balanced_shape(R, K, S) ? skinny_balanced_part_bytes(S) : 0;
     return std::max(std::max<size_t>(p.ksplit > 1 ? p.part_bytes : 0, wide), balanced);
 }
@@ -1469,24 +827,12 @@ bool skinny_rows(int bits, h16* outs, const uint32_t* matrix, const h16* x, cons
     const int64_t gu = group_size / 64;
     a.group_units = (int)(gu > 0x7FFFFFF ? 0x7FFFFFF : gu);
     a.accumulate = accumulate ? 1 : 0;
-    a.block_rows = 32;
     a.part = nullptr;
     a.counters = nullptr;
     a.bal_q = 0; a.bal_r = 0;
     a.wide_wgs = 0;
-    // 33 rows and more, dense: the kernel whose waves share the staged states
-    {
-        const WidePlan wp = plan_wide(R, K, S, sparse_mask != nullptr, a.group_units);
-        const WorkspaceParts ws = workspace_parts(workspace, workspace_bytes);
-        if (wp.use && (wp.ksplit == 1 || (ws.counters != nullptr && ws.scratch_bytes >= wp.part_bytes))) {
-            a.units_per_wave = 0;
-            a.counters = reinterpret_cast<int*>(ws.counters);
-            a.part = reinterpret_cast<float*>(ws.scratch);
-            const bool ok = sparse_mask ? launch_wide<4, true>(a, wp, st)
-                          : bits == 4 ? launch_wide<4>(a, wp, st) : bits == 3 ? launch_wide<3>(a, wp, st) : launch_wide<2>(a, wp, st);
-            if (ok) return true;
-        }
-    }
+    // 17 rows and more: the kernel whose waves share the staged states, where its plan says so
+    if (wide_rows(bits, a, workspace, workspace_bytes, st)) return true;
     if (R > 96) return false;
     // four waves split K when there are more workgroups than CUs (three of them fit a CU) and K
     // is short (each wave should walk a dozen units or more), eight otherwise -- also at exactly one

@@ -631,3 +631,57 @@ def test_few_rows_shared_strips_take_turns_on_one_workspace(H):
         H.assert_product_close(ov.cpu().numpy(), ev, fv, kind="vec")
         H.assert_product_close(om.cpu().numpy(), em, fm, kind="vec")
     capi.workspace_status(ws)
+
+
+# ---- the kernel with shared staging at the edges of its tiles: rows around the blocks of 32, K of one to eleven units (a K
+# group with fewer units than the others, or none), groups that end inside a K group, one to three strips, every way of splitting K
+WIDE_EDGES = [(17, 64, 256, 64), (32, 128, 256, 64), (33, 192, 512, 128), (63, 320, 256, 192), (64, 576, 768, 64), (65, 704, 256, 128),
+              (97, 448, 512, -1), (128, 1088, 256, 192), (129, 1024, 768, 256), (255, 640, 256, 128), (385, 1344, 512, 64)]
+
+
+@pytest.mark.parametrize("bits,sparse", [(4, False), (3, False), (2, False), (4, True)])
+@pytest.mark.parametrize("M,K,S,g", WIDE_EDGES)
+@pytest.mark.parametrize("expo", [False, True])
+def test_shared_staging_edges(H, bits, sparse, M, K, S, g, expo):
+    p = _problem(bits, K=K, S=S, M=M, group_size=g, sparse=sparse, seed=M + K)
+    if expo:
+        p["scales"].reshape(-1, S)[-1, 5:70] *= np.float16(-1)
+        p["zeros"].reshape(-1, S)[-1, 5:70] = np.float16(0.5)
+    d = H.dev_problem(p)
+    exact, f32 = H.oracles(p)
+    H.capi.tune(8, 2)                            # this kernel from two rows on, whatever the shape
+    try:
+        for split in (0, 1, 2, 5):               # the launcher's own choice, then so many ways as the shape allows
+            H.capi.tune(6, split)
+            line = H.capi.describe_launch("mtx", bits, 1, M, K, S, g, sparse)
+            assert line.startswith("wide_rows_kernel"), line
+            got = H.run_capi(p, d, "mtx", outs_init=np.full((1, M, S), np.nan, np.float16))
+            H.assert_product_close(got, exact, f32, kind="mtx")
+            assert np.array_equal(got, H.run_capi(p, d, "mtx")), line
+    finally:
+        H.capi.tune(6, 0)
+        H.capi.tune(8, 0)
+
+
+@pytest.mark.parametrize("bits,sparse", [(4, False), (3, False), (2, False), (4, True)])
+def test_shared_staging_keeps_infinite_and_nan_states_in_their_rows(H, bits, sparse):
+    """seven units on four K groups (the last group's second step has no unit): an infinite state gives its row the
+    infinities of the dequantised weights' signs, a NaN makes its row NaN, and no other row notices"""
+    M, K, S, g = 40, 448, 512, 64
+    p = _problem(bits, K=K, S=S, M=M, group_size=g, sparse=sparse, seed=5)
+    q = dict(p, states=p["states"].copy())
+    q["states"][0, 3, 400] = np.inf
+    q["states"][0, 20, 447] = np.nan
+    H.capi.tune(8, 2)
+    try:
+        clean = H.run_capi(p, H.dev_problem(p), "mtx")
+        got = H.run_capi(q, H.dev_problem(q), "mtx")
+    finally:
+        H.capi.tune(8, 0)
+    w = O.dequantize_matrix(bits, p["matrix"], p["scales"], p["zeros"], g, p["sparse_mask"])[400].astype(np.float32)
+    with np.errstate(invalid="ignore"):
+        want = np.float32(np.inf) * w
+    assert np.array_equal(got[0, 3].astype(np.float32), want, equal_nan=True)
+    assert np.all(np.isnan(got[0, 20]))
+    others = [m for m in range(M) if m not in (3, 20)]
+    assert np.array_equal(got[0, others], clean[0, others])
