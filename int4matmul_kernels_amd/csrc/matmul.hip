@@ -451,9 +451,9 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
                                           h16* outs, h16* As, h16* Bs, uint32_t* lut, const int tile, const int split,
                                           const int nsplit) {
     constexpr int BM = TM * 64, BN = NW * 64, WM = TM * 32, WN = 64, TN = 2, T = 2 * NW * 64;
-    constexpr int A_STAGE = BM * PK, B_STAGE = PK * BN;            // halves per stage
     constexpr int A_ROWS = T / 4;                                  // rows covered by one 16-byte load per thread
-    constexpr int A_LOADS = BM / A_ROWS;                           // such loads per thread and step
+    constexpr int A_LOADS = (BM + A_ROWS - 1) / A_ROWS;            // such loads per thread and step (192 rows: the second half full)
+    constexpr int A_STAGE = A_LOADS * A_ROWS * PK, B_STAGE = PK * BN;            // halves per stage
 
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int wm0 = (wave / NW) * WM, wn0 = (wave % NW) * WN;
@@ -477,7 +477,7 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
     uint32_t a_off[A_LOADS];
 #pragma unroll
     for (int i = 0; i < A_LOADS; ++i)
-        a_off[i] = (uint32_t)((min(a_row + A_ROWS * i, a.M - 1 - m0) * a.K + a_chunk * 8) * 2);
+        a_off[i] = (uint32_t)((min(a_row + A_ROWS * i, min(a.M - m0, BM) - 1) * a.K + a_chunk * 8) * 2);
     const int a_dst = a_row * PK + ((a_chunk ^ ((a_row >> 2) & 3)) << 3);       // halves; rows + A_ROWS: same swizzle
     auto load_a = [&](AStage& r, uint32_t step_off) {
 #pragma unroll
@@ -717,7 +717,7 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
 #pragma unroll
                     for (int e = 0; e < TM * TN; ++e) {
                         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                        __builtin_amdgcn_sched_group_barrier(0x002, TM == 4 ? 6 : 12, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x002, 24 / TM, 0);
                         if (e < A_LOADS + NWORDS + (SPARSE ? 3 : 2)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
                     }
                     __builtin_amdgcn_sched_group_barrier(0x200, 2, 0);
@@ -762,7 +762,7 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
 #pragma unroll
                 for (int e = 0; e < 2 * TM * TN; ++e) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, TM == 4 ? 3 : 4, 0);
                 }
                 __builtin_amdgcn_sched_group_barrier(0x100, 2 * (TM + TN) + (SPARSE ? 4 : 0), 0);
                 __builtin_amdgcn_sched_group_barrier(0x020, A_LOADS + NWORDS + (SPARSE ? 3 : 2), 0);
@@ -774,7 +774,7 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
 #pragma unroll
                 for (int e = 0; e < 2 * TM * TN; ++e) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, TM == 4 ? 3 : 4, 0);
                 }
                 __builtin_amdgcn_sched_group_barrier(0x200, 2, 0);
             }
@@ -854,7 +854,7 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
 #pragma unroll
                     for (int e = 0; e < TM * TN; ++e) {
                         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                        __builtin_amdgcn_sched_group_barrier(0x002, TM == 4 ? 14 : 28, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x002, TM == 4 ? 14 : TM == 3 ? 19 : 28, 0);
                         if (e < A_LOADS + NWORDS + 2) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
                     }
                     __builtin_amdgcn_sched_group_barrier(0x200, 2, 0);
@@ -993,7 +993,8 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
 template <int BITS, bool SPARSE, int NW, int TM, bool PING, bool SPLIT>
 __global__ __launch_bounds__(NW * 128, NW == 2 ? 2 : 1) void matmul_kernel_pipe(MatmulArgs a) {
     constexpr int BM = TM * 64, BN = NW * 64;
-    __shared__ __attribute__((aligned(16))) h16 As[P_STAGES * BM * PK];
+    constexpr int A_ROWS = NW * 32;
+    __shared__ __attribute__((aligned(16))) h16 As[P_STAGES * ((BM + A_ROWS - 1) / A_ROWS) * A_ROWS * PK];
     __shared__ __attribute__((aligned(16))) h16 Bs[P_STAGES * PK * BN];
     __shared__ __attribute__((aligned(16))) uint32_t Lut[SPARSE ? SPARSE_LUT_WORDS : 4];
     // (split-K: the workgroups of a tile are neighbours in the grid, so they run at about the same time;
@@ -1044,9 +1045,11 @@ static void launch_pipe(MatmulArgs a, int64_t B, hipStream_t st) {
     if (noting("matmul_kernel_pipe<bits=%d,%s,tile=%dx%d,%s> tiles=%d ksplit=%d split_from=%d workgroups=%u batch=%d", BITS,
                SPARSE ? "16:32" : "dense", TM * 64, NW * 64, PING ? "two-phase" : "plain", total, a.ksplit, a.split_from, grid.x, (int)B))
         return;
-    if (a.ksplit > 1) {
-        hipLaunchKernelGGL((matmul_kernel_pipe<BITS, SPARSE, NW, TM, PING, true>), grid, block, 0, st, a);
-        return;
+    if constexpr (TM != 3) {
+        if (a.ksplit > 1) {
+            hipLaunchKernelGGL((matmul_kernel_pipe<BITS, SPARSE, NW, TM, PING, true>), grid, block, 0, st, a);
+            return;
+        }
     }
     hipLaunchKernelGGL((matmul_kernel_pipe<BITS, SPARSE, NW, TM, PING, false>), grid, block, 0, st, a);
 }
@@ -1162,9 +1165,9 @@ static void launch(MatmulArgs a, int64_t B, hipStream_t st, void* workspace, siz
                             (SPARSE ? odd_rows && tiles_128 >= 192 : tiles_128 >= (odd_rows ? 128 : 144));
     const bool pipe2_ok = !SPARSE && m_ok && a.S % 128 == 0;
     const bool pipe4_ok = m_ok && a.S % 256 == 0;
-    if (variant != 1 && variant != 3 && variant != 5 && variant != 6 && variant != 7 && variant != 9) variant = 0;
+    if (variant != 1 && variant != 3 && variant != 5 && variant != 6 && variant != 7 && variant != 8 && variant != 9) variant = 0;
     if ((variant == 5 && !pipe2_ok) || ((variant == 6 || variant == 9) && !pipe4_ok) ||
-        (variant == 7 && !(shape_ok && a.S % 256 == 0))) variant = 0;
+        ((variant == 7 || variant == 8) && !(shape_ok && a.S % 256 == 0))) variant = 0;
     // (a last round of large tiles that fills at most half of the GPU is split along K when the
     // workspace has room for its partial tiles: better than small tiles then)
     const TailPlan tp = plan_tail(B, a.M, a.K, a.S);
@@ -1221,11 +1224,21 @@ static void launch(MatmulArgs a, int64_t B, hipStream_t st, void* workspace, siz
         a.counters = reinterpret_cast<int*>(wsp.counters);
         a.part = reinterpret_cast<float*>(wsp.scratch);
     }
+    // 192 x 256 tiles instead of whole 256 x 256 ones, where they take no more rounds of 256 workgroups and pad no more
+    // rows: a round of them costs five sixths to seven eighths (us, 256 / 192 rows: int3, K=4096, S=11008, 777 rows 104 / 97; int4,
+    // S=20480, 520 rows 132 / 103; 1152 rows -- two rounds both ways -- 227 / 205; K=S=8192, 1300 rows 216 / 192; 16:32,
+    // K=8192, S=20480, 520 rows 269 / 234; a round more loses up to a third: int3, K=4096, S=11008, 1152 rows 115 / 175).  A grid
+    // whose last round is split along K keeps the large tiles, 1 - 15 % faster.
+    if (variant == 6 && tuning(TUNE_MM_VARIANT) == 0 && a.ksplit == 1) {
+        const int64_t rows_192 = (a.M + 191) / 192, t256 = m_pad / 256 * (a.S / 256) * B, t192 = rows_192 * (a.S / 256) * B;
+        if (rows_192 * 192 <= m_pad && (t192 + 255) / 256 == (t256 + 255) / 256) variant = 8;
+    }
     if (variant == 1) launch_tile<BITS, SPARSE, 128, 128, 64, 64>(a, B, st);
     else if (variant == 3) launch_tile<BITS, SPARSE, 128, 256, 128, 64>(a, B, st);
     // (256 x 256: the dense formats run the two halves of the workgroup in opposite phases, 2-3 %
     // faster; the 16:32 decode has no registers to spare for it.  Variant 9 forces the plain order.)
     else if (variant == 7) launch_pipe<BITS, SPARSE, 4, 2>(a, B, st);
+    else if (variant == 8) launch_pipe<BITS, SPARSE, 4, 3, !SPARSE>(a, B, st);
     else if (variant == 6 && !SPARSE) launch_pipe<BITS, SPARSE, 4, 4, true>(a, B, st);
     else if (variant == 6 || variant == 9) launch_pipe<BITS, SPARSE, 4>(a, B, st);
     else if constexpr (!SPARSE) launch_pipe<BITS, false, 2>(a, B, st);

@@ -305,6 +305,43 @@ def test_matmul_five_rows_of_128_row_tiles_default_rule(H, bits, sparse):
     H.assert_product_close(got, exact, f32, kind="mtx")
 
 
+# ---- 192 x 256 tiles (tuning key 3 = 8 forces them): one row, a row more than a tile, full tiles and remainders; one trip of the
+# unrolled loop, two trips and a remainder; with and without exponent-mode groups, which take the general loop
+@pytest.mark.parametrize("bits,sparse", FORMATS)
+@pytest.mark.parametrize("M,K,S,g,B,expo", [(1, 192, 256, 64, 1, False), (193, 448, 512, 64, 1, True),
+                                            (384, 2048, 256, -1, 1, False), (191, 512, 512, 128, 3, True),
+                                            (577, 1088, 768, 64, 1, False)])
+def test_matmul_tiles_of_192_rows(H, bits, sparse, M, K, S, g, B, expo):
+    p = _problem(bits, sparse, K=K, S=S, M=M, group_size=g, seed=M + S, B=B)
+    if expo:
+        sc = p["scales"].reshape(-1, S)
+        sc[sc.shape[0] // 2, S - 60:S - 50] *= np.float16(-1)
+    d = H.dev_problem(p)
+    exact, f32 = H.oracles(p)
+    try:
+        H.capi.tune(3, 8)
+        got = H.run_capi(p, d, "mtx", outs_init=np.full((B, M, S), 4.0, np.float16))
+    finally:
+        H.capi.tune(3, 0)
+    H.assert_product_close(got, exact, f32, kind="mtx")
+
+
+@pytest.mark.parametrize("bits,sparse", [(4, False), (3, False), (2, False), (4, True)])
+def test_matmul_tiles_of_192_rows_default_rule(H, bits, sparse):
+    """700 rows against S=14336 take them by default (168 tiles of 256 rows, 224 of 192: one round either way); 1025 rows
+    do not where there is room to split the last round of the large tiles along K"""
+    K, S = 2048, 14336
+    line = H.capi.describe_launch("mtx", bits, 1, 700, K, S, 128, sparse, 0)
+    assert "tile=192x256" in line, line
+    line = H.capi.describe_launch("mtx", bits, 1, 1025, K, S, 128, sparse, 1 << 30)
+    assert "tile=192x256" not in line, line
+    p = _problem(bits, sparse, K=K, S=S, M=700, group_size=128, seed=31)
+    d = H.dev_problem(p)
+    exact, f32 = H.oracles(p)
+    got = H.run_capi(p, d, "mtx", outs_init=np.full((1, 700, S), 4.0, np.float16))
+    H.assert_product_close(got, exact, f32, kind="mtx")
+
+
 @pytest.mark.parametrize("bits,sparse", FORMATS)
 @pytest.mark.parametrize("B,M,K,S", [(5, 130, 512, 512), (32, 20, 256, 1024), (3, 300, 320, 256), (2, 600, 1024, 384)])
 def test_batches_are_one_product_of_all_their_rows(H, bits, sparse, B, M, K, S):
