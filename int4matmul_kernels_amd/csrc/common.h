@@ -149,6 +149,18 @@ bool matvec_one_row(int bits, _Float16* outs, const uint32_t* matrix, const uint
                     void* workspace, size_t workspace_bytes, int* rc);
 // most rows the few-row path takes (beyond 96: only its kernel with shared staging, for the shapes it serves)
 constexpr int SK_WIDE_MAX_ROWS = 512;
+constexpr int FEW_ROWS_MAX = 96;                     // rows that the few-row kernel with its sums of exact codes takes at once
+// Batch elements that the matvec entry hands to the few-row kernels at once: up to 512; on outputs of more than 512 columns
+// that are not whole strips of 256, which the kernel for more than 96 rows serves in the matmul entry alone (its weights are
+// rounded to fp16, the matvec sums exact codes), even shares of at most 96 (us, one matvec per element / so: int4, K=9280,
+// S=1600, 110 elements 760 / 48; 16:32, K=4096, S=1600, 128 elements 900 / 29; int2, K=3072, S=1856, 300 elements 1530 / 60)
+inline int64_t matvec_rows_at_once(int64_t B, int64_t S) {
+    if (S % 256 == 0) return SK_WIDE_MAX_ROWS;
+    if (B <= FEW_ROWS_MAX) return FEW_ROWS_MAX;
+    if (S <= 512) return 0;                          // (one matvec per element)
+    const int64_t chunks = (B + FEW_ROWS_MAX - 1) / FEW_ROWS_MAX;
+    return (B + chunks - 1) / chunks;
+}
 // bytes of partial tiles with which the few-row kernel splits K across workgroups (0: no split)
 size_t skinny_workspace_bytes(int64_t R, int64_t K, int64_t S, bool sparse);
 

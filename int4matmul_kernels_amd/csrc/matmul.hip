@@ -500,7 +500,8 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
     using F = PipeFmt<BITS, SPARSE>;
     constexpr int NWORDS = F::NWORDS;
     const int bn = t % BN, bhb = t / BN;
-    const int bcol = s0 + bn;
+    // (a last tile that is not full: the columns beyond the last repeat the last 64 and are not written)
+    const int bcol = min(s0 + bn, a.S - 64 + (bn & 63));
     struct Stage { uint32_t w[NWORDS]; uint32_t m; uint32_t sc, ze; };
     const uint32_t half_sel = (bcol & 1) ? 0x03020302u : 0x01000100u;
     uint32_t b_off[NWORDS];
@@ -665,12 +666,13 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
         const int total = groups * (BN / 2);
         const uint32_t* tile_scales = reinterpret_cast<const uint32_t*>(a.scales + s0);
         const int64_t row_words = a.S / 2;
+        const int last_word = (a.S - s0) / 2 - 1;
         for (int i0 = t; i0 < total; i0 += 4 * T) {
             uint32_t v[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const int i = min(i0 + k * T, total - 1);
-                v[k] = tile_scales[(int64_t)(i / (BN / 2)) * row_words + i % (BN / 2)];
+                v[k] = tile_scales[(int64_t)(i / (BN / 2)) * row_words + min(i % (BN / 2), last_word)];
             }
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
@@ -977,6 +979,7 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
                     }
         }
     }
+    if (s0 + wn0 >= a.S) return;                       // (a wave's 64 columns are inside or outside as one)
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -1038,7 +1041,7 @@ __global__ __launch_bounds__(NW * 128, NW == 2 ? 2 : 1) void matmul_kernel_pipe(
 template <int BITS, bool SPARSE, int NW, int TM = 4, bool PING = false>
 static void launch_pipe(MatmulArgs a, int64_t B, hipStream_t st) {
     a.tiles_m = (a.M + TM * 64 - 1) / (TM * 64);
-    a.tiles_n = a.S / (NW * 64);
+    a.tiles_n = (a.S + NW * 64 - 1) / (NW * 64);
     const int total = a.tiles_m * a.tiles_n;
     const dim3 grid(a.split_from + (total - a.split_from) * a.ksplit, 1, (unsigned)B), block(NW * 128);
     a.by_columns = a.tiles_n % 8 == 0;
@@ -1054,6 +1057,15 @@ static void launch_pipe(MatmulArgs a, int64_t B, hipStream_t st) {
     hipLaunchKernelGGL((matmul_kernel_pipe<BITS, SPARSE, NW, TM, PING, false>), grid, block, 0, st, a);
 }
 
+// The pipelined kernel takes any whole number of 64 columns; the last tile may be partly empty, up to an eighth of the
+// columns in all (16:32: half, its general tiles are the slowest).  Before, such outputs went to the general tiles, which hide
+// less of their loads and cannot split K (us, general / here: int4, K=9280, S=1600, 700 rows 135 / 54, S=14400, 1100 rows 422 /
+// 351; int2 there 239 / 54 and 699 / 341; 16:32 280 / 73 and 846 / 385; int4, K=9280, S=9344 -- 256 x 128 tiles before --
+// 1100 rows 280 / 214).
+static bool tile_columns(int64_t S, int width, bool sparse) {
+    return S % 64 == 0 && (S + width - 1) / width * width * 8 <= S * (sparse ? 12 : 9);
+}
+
 // ---- split-K plan.  Shapes with at most 128 tiles of 256 x 256 leave more than half of the GPU
 // idle; they run as 256 x 128 tiles (16:32: 256 x 256) with `ksplit` workgroups per tile.  The factor
 // minimises a cost in K steps fitted to measurements (K = 4096 ... 20480, 32 ... 240 tiles):
@@ -1063,10 +1075,10 @@ constexpr int64_t MM_SPLIT_MAX_BYTES = 192ll << 20;      // cap of the partial t
 struct SplitPlan { int ksplit; int64_t tiles; int64_t tile_bytes; };
 static SplitPlan plan_split(bool sparse, int64_t B, int64_t M, int64_t K, int64_t S) {
     const SplitPlan none{1, 0, 0};
-    if (S % (sparse ? 256 : 128) != 0) return none;
+    if (!tile_columns(S, sparse ? 256 : 128, sparse)) return none;
     const int64_t m_pad = (M + 255) / 256 * 256, tiles4 = m_pad / 256 * ((S + 255) / 256) * B;
     if (tiles4 > 128) return none;
-    SplitPlan p{1, m_pad / 256 * (S / (sparse ? 256 : 128)) * B, sparse ? 256 * 256 * 4 : 256 * 128 * 4};
+    SplitPlan p{1, m_pad / 256 * ((S + (sparse ? 255 : 127)) / (sparse ? 256 : 128)) * B, sparse ? 256 * 256 * 4 : 256 * 128 * 4};
     if (p.tiles > MM_SPLIT_MAX_TILES) return none;
     const int64_t steps = K / 32, forced = tuning(TUNE_MM_SPLIT);
     // (16:32, whose 256 x 256 tiles run one per CU: a GPU filled to the last CU runs its K steps 39 % slower than a
@@ -1096,10 +1108,10 @@ static SplitPlan plan_split(bool sparse, int64_t B, int64_t M, int64_t K, int64_
 // would fill at most half of the GPU, its tiles -- and only they -- are split along K over as many
 // workgroups as fit half of the GPU (at least two per tile, at least 32 K steps each).
 struct TailPlan { int ksplit; int64_t split_from, tiles; };
-static TailPlan plan_tail(int64_t B, int64_t M, int64_t K, int64_t S) {
+static TailPlan plan_tail(bool sparse, int64_t B, int64_t M, int64_t K, int64_t S) {
     const TailPlan none{1, 0, 0};
-    if (B != 1 || S % 256 != 0 || tuning(TUNE_MM_TAIL) == 1) return none;
-    const int64_t total = (M + 255) / 256 * (S / 256), tail = total % 256;
+    if (B != 1 || !tile_columns(S, 256, sparse) || tuning(TUNE_MM_TAIL) == 1) return none;
+    const int64_t total = (M + 255) / 256 * ((S + 255) / 256), tail = total % 256;
     if (total <= 256 || tail == 0 || tail > 128) return none;
     // (measured, K = 2048 ... 8192, tails of 16 ... 128 tiles: the split pays while its workgroups fill at most half of
     // the GPU -- two per tile from 64 tiles on, where the second adds the first one's partial tile to its registers
@@ -1124,7 +1136,7 @@ static void launch_tile(MatmulArgs a, int64_t B, hipStream_t st) {
 
 template <int BITS, bool SPARSE>
 static void launch(MatmulArgs a, int64_t B, hipStream_t st, void* workspace, size_t workspace_bytes) {
-    // variant 0 = automatic.  Tile-aligned shapes take the pipelined kernel, as
+    // variant 0 = automatic.  Shapes that fill their tiles well enough take the pipelined kernel, as
     // 256 x 256 tiles (one eight-wave workgroup per CU) or 256 x 128 tiles (two
     // four-wave workgroups per CU).  Measured on MI355X (K = 4096 ... 20480, S = 5120
     // ... 28672, M = 256 ... 4096): the small tiles win when at most half of the CUs
@@ -1155,22 +1167,22 @@ static void launch(MatmulArgs a, int64_t B, hipStream_t st, void* workspace, siz
     // same kernel with half the rows per wave) instead of 256 x 256 tiles padded by another 128 rows -- when
     // they give the GPU at most one round of at least half (16:32: three quarters) of its CUs; smaller grids
     // are better off with split-K
-    const int64_t rows_128 = (a.M + 127) / 128, tiles_128 = rows_128 * (a.S / 256) * B;
+    const int64_t rows_128 = (a.M + 127) / 128, tiles_128 = rows_128 * ((a.S + 255) / 256) * B;
     // (dense: also with an even number of rows when the 128 x 256 tiles fill nine sixteenths of the GPU and more --
     // better than half as many 256 x 256 tiles or 256 x 128 tiles with split-K, by 5 - 10 %)
     // (K=S=3072, eleven to thirteen rows of 128: 132 - 156 tiles of 128 x 256 in 49 - 50 us against 56 - 59 for the
     // 256 x 128 tiles that used to serve 1408 ... 1664 rows there)
     const bool odd_rows = rows_128 % 2 == 1 && rows_128 <= (SPARSE ? 9 : 13);
-    const bool three_rows = a.M > 256 && shape_ok && a.S % 256 == 0 && tiles_128 <= 256 &&
+    const bool three_rows = a.M > 256 && shape_ok && tile_columns(a.S, 256, SPARSE) && tiles_128 <= 256 &&
                             (SPARSE ? odd_rows && tiles_128 >= 192 : tiles_128 >= (odd_rows ? 128 : 144));
-    const bool pipe2_ok = !SPARSE && m_ok && a.S % 128 == 0;
-    const bool pipe4_ok = m_ok && a.S % 256 == 0;
+    const bool pipe2_ok = !SPARSE && m_ok && tile_columns(a.S, 128, SPARSE);
+    const bool pipe4_ok = m_ok && tile_columns(a.S, 256, SPARSE);
     if (variant != 1 && variant != 3 && variant != 5 && variant != 6 && variant != 7 && variant != 8 && variant != 9) variant = 0;
     if ((variant == 5 && !pipe2_ok) || ((variant == 6 || variant == 9) && !pipe4_ok) ||
-        ((variant == 7 || variant == 8) && !(shape_ok && a.S % 256 == 0))) variant = 0;
+        ((variant == 7 || variant == 8) && !(shape_ok && tile_columns(a.S, 256, SPARSE)))) variant = 0;
     // (a last round of large tiles that fills at most half of the GPU is split along K when the
     // workspace has room for its partial tiles: better than small tiles then)
-    const TailPlan tp = plan_tail(B, a.M, a.K, a.S);
+    const TailPlan tp = plan_tail(SPARSE, B, a.M, a.K, a.S);
     const WorkspaceParts wsp = workspace_parts(workspace, workspace_bytes);
     const bool tail_ok = pipe4_ok && tp.ksplit > 1 && wsp.counters != nullptr &&
                          wsp.scratch_bytes >= (size_t)(tp.tiles * tp.ksplit * (256 * 256 * 4));
@@ -1230,7 +1242,7 @@ static void launch(MatmulArgs a, int64_t B, hipStream_t st, void* workspace, siz
     // K=8192, S=20480, 520 rows 269 / 234; a round more loses up to a third: int3, K=4096, S=11008, 1152 rows 115 / 175).  A grid
     // whose last round is split along K keeps the large tiles, 1 - 15 % faster.
     if (variant == 6 && tuning(TUNE_MM_VARIANT) == 0 && a.ksplit == 1) {
-        const int64_t rows_192 = (a.M + 191) / 192, t256 = m_pad / 256 * (a.S / 256) * B, t192 = rows_192 * (a.S / 256) * B;
+        const int64_t rows_192 = (a.M + 191) / 192, t256 = m_pad / 256 * ((a.S + 255) / 256) * B, t192 = rows_192 * ((a.S + 255) / 256) * B;
         if (rows_192 * 192 <= m_pad && (t192 + 255) / 256 == (t256 + 255) / 256) variant = 8;
     }
     if (variant == 1) launch_tile<BITS, SPARSE, 128, 128, 64, 64>(a, B, st);
@@ -1314,14 +1326,15 @@ extern "C" size_t int4mm_matmul_workspace_bytes(const int4mm_shape* shape, int s
     size_t need = int4mm_workspace_bytes(S);
     if (B <= 0 || M <= 0 || K < 64 || S < 128) return need;
     if (B > 1 && B * M <= ((int64_t)1 << 31) - 256) { M *= B; B = 1; }           // (as int4mm_matmul does)
-    // (the matvec entry takes more than 512 batch elements of one row in chunks of up to 512 through the few-row kernels)
-    const size_t few_rows = B * M <= SK_WIDE_MAX_ROWS ? skinny_workspace_bytes(B * M, K, S, sparse != 0)
-                          : shape->seq_len == 1 ? skinny_workspace_bytes(SK_WIDE_MAX_ROWS, K, S, sparse != 0) : 0;
-    if (B * M <= 96) return need + 2 * round_to_page(few_rows);
+    size_t few_rows = B * M <= SK_WIDE_MAX_ROWS ? skinny_workspace_bytes(B * M, K, S, sparse != 0) : 0;
+    // (the matvec entry takes many batch elements of one row in chunks through the few-row kernels)
+    const int64_t at_once = shape->seq_len == 1 ? matvec_rows_at_once(B * M, S) : 0;
+    if (at_once > 0 && at_once < B * M) few_rows = std::max(few_rows, skinny_workspace_bytes(at_once, K, S, sparse != 0));
+    if (B * M <= FEW_ROWS_MAX) return need + 2 * round_to_page(few_rows);
     const SplitPlan sp = plan_split(sparse != 0, B, M, K, S);
     if (sp.ksplit > 1 || few_rows > 0)
         need += 2 * round_to_page(std::max(few_rows, sp.ksplit > 1 ? (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes) : 0));
-    const TailPlan tp = plan_tail(B, M, K, S);
+    const TailPlan tp = plan_tail(sparse != 0, B, M, K, S);
     if (sp.ksplit == 1 && tp.ksplit > 1) need += 2 * round_to_page((size_t)(tp.tiles * tp.ksplit * (256 * 256 * 4)));
     return need;
 }

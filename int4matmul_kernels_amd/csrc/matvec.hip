@@ -1042,17 +1042,18 @@ static int matvec_impl(int bits, void* outs, const void* matrix, const void* mul
         matvec_rows(bits, (h16*)outs, (const uint32_t*)matrix, (const h16*)multiplier, (const h16*)scales, (const h16*)zeros,
                     B, K, S, g, accumulate, (hipStream_t)stream, workspace, workspace_bytes))
         return check_launch("matvec");
-    if (B >= 2 && B <= SK_WIDE_MAX_ROWS && !tuning(TUNE_NO_SKINNY) &&
+    const int64_t at_once = matvec_rows_at_once(B, S);
+    if (B >= 2 && B <= at_once && !tuning(TUNE_NO_SKINNY) &&
         skinny_rows(bits, (h16*)outs, (const uint32_t*)matrix, (const h16*)multiplier, (const h16*)scales,
                     (const h16*)zeros, B, K, S, g, accumulate, (hipStream_t)stream, (const uint32_t*)sparse_mask, workspace, workspace_bytes))
         return check_launch("matvec");
 
-    // more batch elements than the few-row kernels take at once: chunks of up to 512 through them (1 100 elements at
-    // K=4096, S=4096: three launches instead of 1 100), the plain kernel, a launch per element, for what they do not take
+    // more batch elements than the few-row kernels take at once: in chunks through them (1 100 elements at K=4096, S=4096:
+    // three launches instead of 1 100), the plain kernel, a launch per element, for what they do not take
     int64_t done = 0;
-    if (B > SK_WIDE_MAX_ROWS && !tuning(TUNE_NO_SKINNY)) {
+    if (B > at_once && at_once > 0 && !tuning(TUNE_NO_SKINNY)) {
         while (B - done >= 2) {
-            const int64_t n = std::min<int64_t>(SK_WIDE_MAX_ROWS, B - done);
+            const int64_t n = std::min<int64_t>(at_once, B - done);
             if (!skinny_rows(bits, (h16*)outs + done * S, (const uint32_t*)matrix, (const h16*)multiplier + done * K, (const h16*)scales,
                              (const h16*)zeros, n, K, S, g, accumulate, (hipStream_t)stream, (const uint32_t*)sparse_mask, workspace,
                              workspace_bytes))

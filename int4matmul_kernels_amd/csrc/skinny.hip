@@ -833,7 +833,7 @@ bool skinny_rows(int bits, h16* outs, const uint32_t* matrix, const h16* x, cons
     a.wide_wgs = 0;
     // 17 rows and more: the kernel whose waves share the staged states, where its plan says so
     if (wide_rows(bits, a, workspace, workspace_bytes, st)) return true;
-    if (R > 96) return false;
+    if (R > FEW_ROWS_MAX) return false;
     // four waves split K when there are more workgroups than CUs (three of them fit a CU) and K
     // is short (each wave should walk a dozen units or more), eight otherwise -- also at exactly one
     // workgroup per CU, where eight waves keep twice the bytes in flight (K=5120, S=16384, 8 rows:

@@ -1,4 +1,4 @@
-// Products of 17 ... 512 rows, every format, S a multiple of 256: wide_rows_kernel.  Every weight is dequantised once per
+// Products of 17 ... 512 rows, every format, S a multiple of 256 (more than 96 rows: of 64): wide_rows_kernel.  Every weight is dequantised once per
 // block of up to 128 rows, with the reference's own two roundings fp16(fp16(q - z) s) (matmul.cuh:115-125) or, in exponent
 // mode, its single-rounded fma (matmul.cuh:127-136), and multiplied on v_mfma_f32_32x32x16_f16 into accumulators that hold
 // the product itself.
@@ -78,7 +78,8 @@ __global__ __launch_bounds__(512, MT == 1 && !SPARSE && !(BITS == 4 && WN == 2) 
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int j = lane & 31, h = lane >> 5;
     const int cg = wave % WN, kg = wave / WN;
-    const int scol = blockIdx.x * STRIP, wcol = scol + cg * 64;
+    // (a last strip that is not full: the waves beyond the last column repeat the last 64 and write nothing)
+    const int wcol = min((int)blockIdx.x * STRIP + cg * 64, S - 64);
     const int units = K / 64;
     const int z0 = blockIdx.z * units_per_split, share = min(units - z0, units_per_split);
     // K group kg takes units kg steps ... of the share; the last ones may get fewer
@@ -473,8 +474,8 @@ __global__ __launch_bounds__(512, MT == 1 && !SPARSE && !(BITS == 4 && WN == 2) 
 #pragma unroll
         for (int v = 0; v < NV; ++v) val[v] = sum[v];
     }
-    // ---- (rows beyond R lie beyond the buffer: their stores do nothing)
-    const __amdgpu_buffer_rsrc_t o_rsrc = __builtin_amdgcn_make_buffer_rsrc(a.outs + (int64_t)row0 * S, 0, (int)((uint32_t)R * row2), RSRC_FLAGS);
+    // ---- (rows beyond R lie beyond the buffer: their stores do nothing; a wave beyond the last column has an empty one)
+    const __amdgpu_buffer_rsrc_t o_rsrc = __builtin_amdgcn_make_buffer_rsrc(a.outs + (int64_t)row0 * S, 0, (int)(blockIdx.x * STRIP + cg * 64 < (unsigned)S ? (uint32_t)R * row2 : 0u), RSRC_FLAGS);
     const int m0 = WK == 2 ? 16 * kg : 8 * kg;         // first row of register kg OWN, in lane group 0
     const uint32_t o_off = (uint32_t)(m0 + 4 * h) * row2 + (uint32_t)(wcol + 2 * j) * 2u;
 #pragma unroll
@@ -562,11 +563,17 @@ static bool few_row_sums(int64_t R, int64_t K, int64_t S, bool sparse) {
     return S / 64 > 128 && S / 64 <= 256 && K <= 6144;
 }
 
+// Whole strips of 256 columns; beyond 96 rows, which the few-row kernel does not take, any number of whole 64 (the general
+// tiles that served them cannot split K: int2, K=9280, S=1600, 220 rows 238 us there, 21 here; the matvec entry, whose sums are of
+// the exact codes, does not come here with such a shape: matvec_rows_at_once).
+static bool wide_columns(int64_t R, int64_t S) { return S % 256 == 0 || (R > FEW_ROWS_MAX && S % 64 == 0); }
+static int64_t wide_strips(int64_t S, int wn) { return (S + 64 * wn - 1) / (64 * wn); }
+
 static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S, bool can_split) {
     WidePlan p{false, 0, 0, 0, 1, 0, 0};
     // (knob: 1 = never, n >= 2 = from n rows on whatever the shape)
     const int64_t knob = tuning(TUNE_NO_WIDE), min_rows = knob >= 2 ? knob : 17, forced = tuning(TUNE_MM_SPLIT);
-    if (R < min_rows || R > SK_WIDE_MAX_ROWS || S % 256 != 0 || K % 64 != 0 || knob == 1) return p;
+    if (R < min_rows || R > SK_WIDE_MAX_ROWS || !wide_columns(R, S) || K % 64 != 0 || knob == 1) return p;
     const int64_t units = K / 64;
     // (32-bit byte offsets into buffer resources: a share of the packed matrix, its scales and the block's rows of states and
     // outputs stay below 2 GB)
@@ -580,7 +587,7 @@ static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S
         if (32 * (c.mt - 1) >= R || (R > 64 && units <= 8 && c.mt != tallest)) continue;
         // (49 ... 64 rows on 2048 ... 4096 columns and a long K: two blocks of 32 rows)
         if (!sparse && R > 48 && R <= 64 && S > 2048 && S <= 4096 && K > 8192 && forced < 1 && (c.mt != 1 || c.wn != 4)) continue;
-        const int64_t blocks = (R + 32 * c.mt - 1) / (32 * c.mt), tiles = S / (64 * c.wn) * blocks;
+        const int64_t blocks = (R + 32 * c.mt - 1) / (32 * c.mt), tiles = wide_strips(S, c.wn) * blocks;
         // (below 1024 columns, where nothing was fitted: as many ways as leave shares of eight units)
         const int64_t only = forced >= 1 ? std::min<int64_t>(forced, std::max<int64_t>(1, units / 4))
                            : S < 1024 && can_split ? std::max<int64_t>(1, std::min<int64_t>({256 / tiles, units / 8, 16})) : 0;
@@ -600,9 +607,9 @@ static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S
     // 227 in tiles; int3, K=20480, S=11008 324 / 295; int4 K=8192, S=20480, 384 rows stays, 140 / 196)
     if (knob < 2 && forced < 1 && R > 256 && S > 10240 && K > 1024 && p.ksplit == 1) {
         const double flops = 2.0 * ((R + 255) / 256 * 256) * K * S;
-        if (best > 5.0 + flops / (S / (64 * p.wn) * p.row_blocks > 256 ? 1.05e9 : 0.75e9)) return p;
+        if (best > 5.0 + flops / (wide_strips(S, p.wn) * p.row_blocks > 256 ? 1.05e9 : 0.75e9)) return p;
     }
-    p.part_bytes = p.ksplit > 1 ? (size_t)p.ksplit * p.row_blocks * 32 * p.mt * S * 4 : 0;
+    p.part_bytes = p.ksplit > 1 ? (size_t)p.ksplit * p.row_blocks * 32 * p.mt * wide_strips(S, p.wn) * 64 * p.wn * 4 : 0;
     p.use = true;
     return p;
 }
@@ -610,17 +617,17 @@ static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S
 // An upper bound of any plan's partial tiles, cheap enough for every call: at most 512 workgroups of 32 KB per 32 rows, and
 // no more than the split's limit (16 ways, four units each) of the rows rounded up to whole blocks.
 size_t wide_workspace_bytes(int64_t R, int64_t K, int64_t S, bool sparse) {
-    if (R < 2 || R > SK_WIDE_MAX_ROWS || S % 256 != 0 || K % 64 != 0) return 0;
+    if (R < 2 || R > SK_WIDE_MAX_ROWS || !wide_columns(R, S) || K % 64 != 0) return 0;
     if (tuning(TUNE_NO_WIDE) < 2 && (R < 17 || few_row_sums(R, K, S, sparse))) return 0;
     const int64_t ways = std::min<int64_t>(16, K / 256), mt = std::min<int64_t>(4, (R + 31) / 32);
     if (ways < 2) return 0;
-    return (size_t)std::min<int64_t>(WIDE_MAX_SPLIT_WGS * mt * 32768, ways * ((R + 32 * mt - 1) / 32 * 32) * S * 4);
+    return (size_t)std::min<int64_t>(WIDE_MAX_SPLIT_WGS * mt * 32768, ways * ((R + 32 * mt - 1) / 32 * 32) * ((S + 255) / 256 * 256) * 4);
 }
 
 template <int BITS, int MT, bool SPARSE, int WN>
 static void launch_wide(const SkinnyArgs& s, const WidePlan& p, hipStream_t st) {
     constexpr size_t bytes = wide_lds_bytes(MT, WN);
-    const dim3 grid(s.S / (64 * WN), p.row_blocks, p.ksplit), block(512);
+    const dim3 grid((unsigned)wide_strips(s.S, WN), p.row_blocks, p.ksplit), block(512);
     auto kernel = wide_rows_kernel<BITS, MT, SPARSE, WN>;
     if constexpr (bytes > 64 * 1024) {                   // more than 64 KB of dynamic LDS has to be requested once per kernel and device
         static std::atomic<uint64_t> done;
@@ -640,7 +647,7 @@ static void launch_wide(const SkinnyArgs& s, const WidePlan& p, hipStream_t st) 
 template <int BITS, bool SPARSE>
 static bool launch_wide(const SkinnyArgs& a, const WidePlan& p, hipStream_t st) {
     if (noting("wide_rows_kernel<bits=%d,%s,row_tiles=%d> strips=%d row_blocks=%d ksplit=%d columns=%d", BITS, SPARSE ? "16:32" : "dense",
-               2 * p.mt, a.S / (64 * p.wn), p.row_blocks, p.ksplit, 64 * p.wn))
+               2 * p.mt, (int)wide_strips(a.S, p.wn), p.row_blocks, p.ksplit, 64 * p.wn))
         return true;
     if (p.wn == 2) {
         if (p.mt == 1) launch_wide<BITS, 1, SPARSE, 2>(a, p, st);

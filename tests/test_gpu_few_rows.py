@@ -685,3 +685,17 @@ def test_shared_staging_keeps_infinite_and_nan_states_in_their_rows(H, bits, spa
     assert np.all(np.isnan(got[0, 20]))
     others = [m for m in range(M) if m not in (3, 20)]
     assert np.array_equal(got[0, others], clean[0, others])
+
+
+# ---- the matvec entry with more batch elements than the few-row kernel takes at once, on outputs that are not whole strips of 256
+# columns: even shares of at most 96 elements, the last one shorter
+@pytest.mark.parametrize("bits,sparse", [(4, False), (3, False), (2, False), (4, True)])
+@pytest.mark.parametrize("B,K,S", [(97, 512, 576), (193, 1088, 704), (520, 256, 1088)])
+def test_matvec_many_batch_elements_ragged_outputs(H, bits, sparse, B, K, S):
+    p = O.make_problem(K=K, S=S, M=1, bits=bits, group_size=64, sparse=sparse, seed=B + bits, B=B)
+    p["scales"].reshape(-1, S)[1, S - 9:S - 2] *= np.float16(-1)
+    line = H.capi.describe_launch("vec", bits, B, 1, K, S, 64, sparse)
+    assert "skinny_kernel" in line and "matvec_kernel" not in line and "wide_rows" not in line, line
+    d = H.dev_problem(p)
+    exact, f32 = H.oracles(p)
+    H.assert_product_close(H.run_capi(p, d, "vec"), exact, f32, kind="vec")

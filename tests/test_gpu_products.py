@@ -342,6 +342,29 @@ def test_matmul_tiles_of_192_rows_default_rule(H, bits, sparse):
     H.assert_product_close(got, exact, f32, kind="mtx")
 
 
+# ---- a last strip or tile that is partly beyond the last column (S a multiple of 64, not of the strip's 128 or 256): one to three
+# quarters of it full, K split and not, exponent-mode groups in the last columns, and 0 = whatever the dispatch picks
+@pytest.mark.parametrize("bits,sparse", FORMATS)
+@pytest.mark.parametrize("variant,M,K,S,g,B", [(0, 97, 512, 320, 128, 1), (0, 220, 4160, 1600, 64, 1), (0, 512, 448, 1088, 64, 1),
+                                               (0, 130, 2048, 64, -1, 1), (0, 400, 1024, 3008, 128, 2), (5, 300, 2048, 704, 128, 1),
+                                               (6, 250, 2048, 704, 128, 1), (7, 300, 1024, 1600, -1, 1), (8, 200, 448, 2240, 64, 1),
+                                               (9, 512, 512, 704, 128, 2), (0, 600, 512, 1088, 64, 1)])
+@pytest.mark.parametrize("expo", [False, True], ids=["linear", "mixed"])
+def test_matmul_last_strip_partly_empty(H, bits, sparse, variant, M, K, S, g, B, expo):
+    p = _problem(bits, sparse, K=K, S=S, M=M, group_size=g, seed=M + S + variant, B=B)
+    if expo:
+        sc = p["scales"].reshape(-1, S)
+        sc[sc.shape[0] // 2, S - 20:S - 3] *= np.float16(-1)
+    d = H.dev_problem(p)
+    exact, f32 = H.oracles(p)
+    try:
+        H.capi.tune(3, variant)
+        got = H.run_capi(p, d, "mtx", outs_init=np.full((B, M, S), 4.0, np.float16))
+    finally:
+        H.capi.tune(3, 0)
+    H.assert_product_close(got, exact, f32, kind="mtx")
+
+
 @pytest.mark.parametrize("bits,sparse", FORMATS)
 @pytest.mark.parametrize("B,M,K,S", [(5, 130, 512, 512), (32, 20, 256, 1024), (3, 300, 320, 256), (2, 600, 1024, 384)])
 def test_batches_are_one_product_of_all_their_rows(H, bits, sparse, B, M, K, S):
