@@ -7,8 +7,8 @@
 
 namespace i4 {
 
-// magic numbers (div_magic) of the divisors of the balanced launch's range arithmetic: K / 64, the group's units, q, q + 1
-struct BalancedMagics { uint32_t units, group_units, share_lo, share_hi; };
+// magic numbers (div_magic) of the divisors of the balanced launch's range arithmetic: K / 64, the group's units
+struct BalancedMagics { uint32_t units, group_units; };
 
 struct SkinnyArgs {
     h16* outs;

@@ -1,8 +1,7 @@
-// Few-row products for gfx950, two kernels.  skinny_kernel (described first): 2 .. 96 rows of states (32 per
+// Few-row products for gfx950: 2 .. 96 rows of states (32 per
 // workgroup) against a dense int4 / int3 / int2 or 16:32 sparse int4 weight matrix, HBM-bound like the
-// matvec (every packed word is read once and used for all rows).  wide_rows_kernel (further down): 17 .. 256
-// rows, whose waves share one staged copy of the states and dequantise each weight.  skinny_rows() at the
-// end picks one by shape.  The reference has no such path: it sends M >= 2 to its
+// matvec (every packed word is read once and used for all rows).  17 .. 512 rows: wide_rows_kernel (csrc/wide.hip), which
+// skinny_rows() at the end asks first.  The reference has no such path: it sends M >= 2 to its
 // 64-row matmul tiles (int4matmul.cpp:27) and M == 1 with B > 1 to one matvec
 // per batch element, re-reading the weights each time (matvec_kernel.cu:346).
 //
@@ -50,16 +49,17 @@ constexpr int SK_PITCH = 144;                   // bytes between rows of a stage
 constexpr int SK_XBUF = 32 * SK_PITCH;          // one staged unit: 32 rows x 64 k
 constexpr int SK_WAVE_LDS = 2 * SK_XBUF + 256;  // two unit buffers + the group sums of 32 rows
 
+constexpr int SK_BAL_WAVES = 8;
+
 // Balanced launch: workgroup i of 256 takes the range [i q + i r / 256, (i + 1) q + (i + 1) r / 256) of
 // strips x units (strip-major; q, r = quotient and remainder of the total by 256).  The range is at least one
 // strip and less than two strips long, so it touches at most three strips: three segments, segment k on strip
 // strip0 + k.  The workgroup's waves are dealt to the segments in proportion to their units (at least one each).
 // For one wave: its segment (`mine`), the segment's units [lo, hi) within its strip, the segment's first wave
-// and number of waves; for the workgroup's copy of scales and zeros in LDS: the first group of each segment
-// and where each segment's groups start (goff3: all groups).
-struct BalancedShare { int strip0, mine, lo, hi, wave0, waves, glo0, glo1, glo2, goff1, goff2, goff3; };
-// (A dozen quotients stand between a wave's start and its first loads: they are taken with the divisors' magic
-// numbers, which the host passes -- magic_div, csrc/common.h.)
+// and number of waves; of all segments: the first unit of the first one and the units of each.
+struct BalancedShare { int strip0, mine, lo, hi, wave0, waves, first, n0, n1, n2; };
+// (The quotients stand between a wave's start and its first loads, in code that every launch fetches anew: they are taken with
+// magic numbers, which the host passes -- magic_div, csrc/common.h -- or through the float reciprocal.)
 // a / b for 0 <= a < 2^22 through the float reciprocal, for a divisor without a magic number at hand
 __device__ __forceinline__ int small_div(int a, int b, float inv_b) {
     int q = (int)((float)a * inv_b);
@@ -68,57 +68,32 @@ __device__ __forceinline__ int small_div(int a, int b, float inv_b) {
     if (r >= b) ++q;
     return q;
 }
-__device__ __forceinline__ BalancedShare balanced_share(int q, int r, const BalancedMagics& mg, int i, int units, int group_units,
-                                                        int nwaves, int wave) {
+__device__ __forceinline__ BalancedShare balanced_share(int q, int r, uint32_t units_magic, int i, int units, int wave) {
     BalancedShare b{};
     const int lo = i * q + ((i * r) >> 8), hi = (i + 1) * q + (((i + 1) * r) >> 8);           // (/ 256 workgroups)
     const int share = hi - lo;
-    const uint32_t share_magic = share == q ? mg.share_lo : mg.share_hi;
-    b.strip0 = magic_div(lo, units, mg.units);
-    int seg_lo[3], seg_n[3], seg_w[3], dealt = 0;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const int s0 = (b.strip0 + k) * units;
-        const int from = max(lo, s0), to = min(hi, s0 + units);
-        seg_lo[k] = from - s0;
-        seg_n[k] = max(0, to - from);
-        seg_w[k] = seg_n[k] > 0 ? max(1, magic_div(seg_n[k] * nwaves + share / 2, share, share_magic)) : 0;
-        dealt += seg_w[k];
-    }
-    // the rounding may deal a wave or two too many or too few: take from the segment with the fewest units per
-    // wave, give to the one with the most (the pick's units and waves are kept by value: no indexed registers)
-#pragma unroll
-    for (int it = 0; it < 3; ++it) {
-        if (dealt > nwaves) {
-            int k = -1, kn = 0, kw = 1;
-#pragma unroll
-            for (int c = 0; c < 3; ++c)
-                if (seg_w[c] > 1 && (k < 0 || seg_n[c] * kw < kn * seg_w[c])) { k = c; kn = seg_n[c]; kw = seg_w[c]; }
-#pragma unroll
-            for (int c = 0; c < 3; ++c) if (c == k) --seg_w[c];
-            --dealt;
-        } else if (dealt < nwaves) {
-            int k = -1, kn = 0, kw = 1;
-#pragma unroll
-            for (int c = 0; c < 3; ++c)
-                if (seg_n[c] > 0 && (k < 0 || seg_n[c] * kw > kn * seg_w[c])) { k = c; kn = seg_n[c]; kw = seg_w[c]; }
-#pragma unroll
-            for (int c = 0; c < 3; ++c) if (c == k) ++seg_w[c];
-            ++dealt;
-        }
-    }
-    int w0 = 0;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        if (wave >= w0 && wave < w0 + seg_w[k]) { b.mine = k; b.wave0 = w0; b.waves = seg_w[k]; b.lo = seg_lo[k]; b.hi = seg_lo[k] + seg_n[k]; }
-        w0 += seg_w[k];
-    }
-    const int g0 = magic_div(seg_lo[0], group_units, mg.group_units), g1 = magic_div(seg_lo[1], group_units, mg.group_units),
-              g2 = magic_div(seg_lo[2], group_units, mg.group_units);
-    b.glo0 = g0; b.glo1 = g1; b.glo2 = g2;
-    b.goff1 = seg_n[0] > 0 ? magic_div(seg_lo[0] + seg_n[0] - 1, group_units, mg.group_units) + 1 - g0 : 0;
-    b.goff2 = b.goff1 + (seg_n[1] > 0 ? magic_div(seg_lo[1] + seg_n[1] - 1, group_units, mg.group_units) + 1 - g1 : 0);
-    b.goff3 = b.goff2 + (seg_n[2] > 0 ? magic_div(seg_lo[2] + seg_n[2] - 1, group_units, mg.group_units) + 1 - g2 : 0);
+    const float per_unit = (float)SK_BAL_WAVES * __builtin_amdgcn_rcpf((float)share);
+    b.strip0 = magic_div(lo, units, units_magic);
+    b.first = lo - b.strip0 * units;
+    b.n0 = min(share, units - b.first);
+    b.n1 = min(share - b.n0, units);
+    b.n2 = share - b.n0 - b.n1;
+    // waves in proportion, at least one each: the outer segments' are rounded, the middle one, a whole strip and more than half
+    // of the range where there are three, has the rest (any deal is right; a rounding that differs moves a wave)
+    const int w2 = b.n2 > 0 ? max(1, (int)((float)b.n2 * per_unit + 0.5f)) : 0;
+    const int w0 = b.n1 > 0 ? min(max(1, (int)((float)b.n0 * per_unit + 0.5f)), SK_BAL_WAVES - 1 - w2) : SK_BAL_WAVES;
+    const int w1 = SK_BAL_WAVES - w0 - w2;
+    b.mine = wave < w0 ? 0 : wave < w0 + w1 ? 1 : 2;
+    b.wave0 = b.mine == 0 ? 0 : b.mine == 1 ? w0 : w0 + w1;
+    b.waves = b.mine == 0 ? w0 : b.mine == 1 ? w1 : w2;
+    b.lo = b.mine == 0 ? b.first : 0;
+    b.hi = b.mine == 0 ? b.first + b.n0 : b.mine == 1 ? b.n1 : b.n2;
+    // (the same in every lane, which the compiler cannot see behind the float arithmetic)
+    b.mine = __builtin_amdgcn_readfirstlane(b.mine);
+    b.wave0 = __builtin_amdgcn_readfirstlane(b.wave0);
+    b.waves = __builtin_amdgcn_readfirstlane(b.waves);
+    b.lo = __builtin_amdgcn_readfirstlane(b.lo);
+    b.hi = __builtin_amdgcn_readfirstlane(b.hi);
     return b;
 }
 
@@ -131,11 +106,19 @@ __device__ __forceinline__ BalancedShare balanced_share(int q, int r, const Bala
 // 16, the lane's four adjacent columns in the first four and column j of the fifth (a.wide_wgs workgroups have one)
 template <int BITS, int CW, int RT, bool SPARSE, bool BAL = false, int XC = 0>
 __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix, const h16* pre_x, const h16* pre_scales, const h16* pre_zeros,
-                                                   int pre_S, int pre_K, int pre_group_units, int pre_units, SkinnyArgs a) {
+                                                   int pre_S, int pre_K, int pre_group_units, int pre_units, uint32_t pre_rows,
+                                                   uint32_t pre_more, SkinnyArgs a) {
     // (what the first loads depend on, once more in front of the record: the first dwords of a kernel's arguments
-    // reach a wave in registers at its start, a record's fields are fetched by the wave itself)
+    // reach a wave in registers at its start, a record's fields are fetched by the wave itself; with the rows, the ranges and the
+    // waves among them nothing waits for the record before the loads: int4, K=5120, S=20480, 8 rows 18.2 -> 17.8 us a layer,
+    // int3, K=4864, S=2304 10.1 -> 9.9)
     a.matrix = pre_matrix; a.x = pre_x; a.scales = pre_scales; a.zeros = pre_zeros; a.S = pre_S; a.K = pre_K;
-    a.group_units = pre_group_units; a.units_per_wave = pre_units;
+    a.group_units = pre_group_units;
+    // (pre_units, pre_rows, pre_more -- BAL: q, rows and r, the magic number of the units; XC: units per wave, rows and waves,
+    // workgroups with a fifth sliver; else units per wave, rows and waves, units per split)
+    a.R = (int)(pre_rows & 0xFFFF);
+    if constexpr (BAL) { a.bal_q = pre_units; a.bal_r = (int)(pre_rows >> 16); a.bal_magics.units = pre_more; }
+    else { a.units_per_wave = pre_units; if constexpr (XC != 0) a.wide_wgs = (int)pre_more; else a.units_per_split = (int)pre_more; }
     using F = SkFmt<BITS, SPARSE>;
     constexpr int NL = F::LOADS;
     constexpr int PF = (BITS == 3 && CW == 4) || (SPARSE && CW == 4) ? 2 : 4, MT = RT == 4 ? 2 : 1;
@@ -144,7 +127,7 @@ __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix,
     constexpr int STRIP = 16 * CT;
     extern __shared__ __attribute__((aligned(16))) char lds[];
     typedef typename Words<CW>::type words_t;
-    const int t = threadIdx.x, lane = t & 63, nwaves = blockDim.x >> 6;
+    const int t = threadIdx.x, lane = t & 63, nwaves = BAL ? SK_BAL_WAVES : (int)(pre_rows >> 16);
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);   // scalar: the unit loop runs on SGPRs
     const int j = lane & 15, h = lane >> 4;
     const int units = a.K / 64;
@@ -154,7 +137,7 @@ __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix,
     int seg_wave0 = 0, seg_waves = nwaves;                      // the waves that work on the same strip
     BalancedShare bs{};
     if constexpr (BAL) {
-        bs = balanced_share(a.bal_q, a.bal_r, a.bal_magics, blockIdx.x, units, a.group_units, nwaves, wave);
+        bs = balanced_share(a.bal_q, a.bal_r, a.bal_magics.units, blockIdx.x, units, wave);
         strip = bs.strip0 + bs.mine;
         split_lo = bs.lo;
         split_hi = bs.hi;
@@ -164,8 +147,8 @@ __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix,
         u0 = min(split_hi, split_lo + (wave - seg_wave0) * upw);
         u1 = min(split_hi, u0 + upw);
     } else {
-        split_lo = blockIdx.z * a.units_per_split;
-        split_hi = min(units, split_lo + a.units_per_split);
+        split_lo = XC != 0 ? 0 : blockIdx.z * a.units_per_split;
+        split_hi = XC != 0 ? units : min(units, split_lo + a.units_per_split);
         u0 = min(split_hi, split_lo + wave * a.units_per_wave);
         u1 = min(split_hi, u0 + a.units_per_wave);
     }
@@ -185,11 +168,9 @@ __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix,
     // weights and states.  Exponent-mode scales (negative or NaN) anywhere in the
     // strip switch the whole workgroup to the exact per-weight decode.  (The copy
     // runs after the first loads have been issued, under their latency.)
-    // (of the groups that the workgroup's share of K touches: group_lo onwards)
-    const int group_lo = split_lo / a.group_units;
-    const int groups = (split_hi + a.group_units - 1) / a.group_units - group_lo;
-    // (BAL: the copies of the workgroup's segments one after the other; this wave's starts at group sz_goff)
-    const int sz_groups = BAL ? bs.goff3 : groups, sz_goff = BAL ? (bs.mine == 0 ? 0 : bs.mine == 1 ? bs.goff1 : bs.goff2) : 0;
+    // (of the groups that the workgroup's share of K touches)
+    // (BAL: the copies of the workgroup's segments one after the other; this wave's group gi is at sz_goff + gi)
+    int sz_groups = 0, sz_goff = 0;
     // (16:32: the selector table is allocated statically: its LDS address is a compile-time constant)
     __shared__ __attribute__((aligned(16))) u32x4 lut_table[SPARSE ? 256 : 1];
     const char* lut = reinterpret_cast<const char*>(lut_table);
@@ -216,6 +197,21 @@ __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix,
     auto scan_scales = [&]() __attribute__((always_inline)) -> bool {
         int* flag = reinterpret_cast<int*>(lds + nwaves * SK_WAVE_LDS);
         if (t == 0) *flag = 0;
+        // (BAL: the first group of the first segment -- the others start with their strip -- and where each segment's copy starts)
+        int glo0 = 0, goff1 = 0, goff2 = 0;
+        if constexpr (BAL) {
+            const uint32_t magic = a.bal_magics.group_units;
+            const int gu = a.group_units;
+            glo0 = magic_div(bs.first, gu, magic);
+            goff1 = magic_div(bs.first + bs.n0 - 1, gu, magic) + 1 - glo0;
+            goff2 = goff1 + (bs.n1 > 0 ? magic_div(bs.n1 - 1, gu, magic) + 1 : 0);
+            sz_groups = goff2 + (bs.n2 > 0 ? magic_div(bs.n2 - 1, gu, magic) + 1 : 0);
+            sz_goff = bs.mine == 0 ? -glo0 : bs.mine == 1 ? goff1 : goff2;
+        } else {
+            glo0 = split_lo / a.group_units;
+            sz_groups = (split_hi + a.group_units - 1) / a.group_units - glo0;
+            sz_goff = -glo0;
+        }
         __syncthreads();
         bool bad = false;
         const int n = sz_groups * (STRIP / 2);
@@ -225,12 +221,12 @@ __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix,
             if constexpr (BAL) {
                 // (sums rather than selections among the three segments' values: the compiler turns a selection
                 // among fields into an indexed load, which puts the whole record into scratch memory)
-                const int k1 = g >= bs.goff1 ? 1 : 0, k2 = g >= bs.goff2 ? 1 : 0;
-                const int first = bs.glo0 + k1 * (bs.glo1 - bs.glo0) + k2 * (bs.glo2 - bs.glo1);
-                const int off = k1 * bs.goff1 + k2 * (bs.goff2 - bs.goff1);
+                const int k1 = g >= goff1 ? 1 : 0, k2 = g >= goff2 ? 1 : 0;
+                const int first = glo0 - k1 * glo0;
+                const int off = k1 * goff1 + k2 * (goff2 - goff1);
                 at = (int64_t)(first + g - off) * a.S + (bs.strip0 + k1 + k2) * STRIP + 2 * c;
             } else {
-                at = (int64_t)(group_lo + g) * a.S + colbase + ((XC != 0 && !has_extra && c >= 8 * CW) ? 2 * c - 16 * CW : 2 * c);
+                at = (int64_t)(glo0 + g) * a.S + colbase + ((XC != 0 && !has_extra && c >= 8 * CW) ? 2 * c - 16 * CW : 2 * c);
             }
             const uint32_t two = *reinterpret_cast<const uint32_t*>(a.scales + at);
             bad |= !(as_h2(two).x >= (h16)0.0f) || !(as_h2(two).y >= (h16)0.0f);
@@ -362,7 +358,7 @@ __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix,
 #pragma unroll
         for (int c = 0; c < CT; ++c) { sc[c] = (h16)0.f; ze[c] = (h16)0.f; }
         auto load_sz = [&](int gi) {
-            const h16* ps = reinterpret_cast<const h16*>(sz) + (sz_goff + gi - group_lo) * STRIP + CW * j;
+            const h16* ps = reinterpret_cast<const h16*>(sz) + (sz_goff + gi) * STRIP + CW * j;
             const h16* pz = ps + sz_groups * STRIP;
             if constexpr (CW == 4) {
                 const u32x2 s2 = *reinterpret_cast<const u32x2*>(ps), z2 = *reinterpret_cast<const u32x2*>(pz);
@@ -643,7 +639,8 @@ static bool launch_skinny(const SkinnyArgs& a, int waves, int ksplit, hipStream_
                                 150 * 1024);
             done[slot].fetch_or(bit, std::memory_order_relaxed);
         }
-        hipLaunchKernelGGL(kernel, grid, block, lds, st, a.matrix, a.x, a.scales, a.zeros, a.S, a.K, a.group_units, a.units_per_wave, a);
+        hipLaunchKernelGGL(kernel, grid, block, lds, st, a.matrix, a.x, a.scales, a.zeros, a.S, a.K, a.group_units, a.units_per_wave, (uint32_t)a.R | (uint32_t)waves << 16,
+                           (uint32_t)a.units_per_split, a);
     };
     if (rt <= 1) go(skinny_kernel<BITS, CW, 1, SPARSE>, 0);
     else if (rt <= 2) go(skinny_kernel<BITS, CW, 2, SPARSE>, 1);
@@ -668,13 +665,13 @@ static bool balanced_shape(int64_t R, int64_t K, int64_t S) {
 }
 template <int BITS, bool SPARSE>
 static bool launch_skinny_balanced(SkinnyArgs a, hipStream_t st) {
-    constexpr int CW = 4, WAVES = 8;
+    constexpr int CW = 4, WAVES = SK_BAL_WAVES;
     const int strips = a.S / 64, units = a.K / 64;
     const int rt = (a.R + 7) / 8;
     const int64_t total = (int64_t)strips * units;
     a.bal_q = (int)(total / SK_BAL_WGS);
     a.bal_r = (int)(total % SK_BAL_WGS);
-    a.bal_magics = {div_magic((uint32_t)units), div_magic((uint32_t)a.group_units), div_magic((uint32_t)a.bal_q), div_magic((uint32_t)a.bal_q + 1u)};
+    a.bal_magics = {div_magic((uint32_t)units), div_magic((uint32_t)a.group_units)};
     // scales in LDS: a workgroup's range is less than two strips long and touches at most three
     const int groups = 2 * ((units + a.group_units - 1) / a.group_units) + 3;
     size_t lds = (size_t)WAVES * SK_WAVE_LDS + 16 + (size_t)groups * 16 * CW * 4;
@@ -695,7 +692,8 @@ static bool launch_skinny_balanced(SkinnyArgs a, hipStream_t st) {
                                 150 * 1024);
             done.fetch_or(bit, std::memory_order_relaxed);
         }
-        hipLaunchKernelGGL(kernel, grid, block, lds, st, a.matrix, a.x, a.scales, a.zeros, a.S, a.K, a.group_units, a.units_per_wave, a);
+        hipLaunchKernelGGL(kernel, grid, block, lds, st, a.matrix, a.x, a.scales, a.zeros, a.S, a.K, a.group_units, a.bal_q, (uint32_t)a.R | (uint32_t)a.bal_r << 16,
+                           a.bal_magics.units, a);
     };
     if (rt <= 1) go(skinny_kernel<BITS, CW, 1, SPARSE, true>);
     else go(skinny_kernel<BITS, CW, 2, SPARSE, true>);            // (up to 16 rows: balanced_shape)
@@ -739,7 +737,8 @@ static bool launch_skinny_slivers(SkinnyArgs a, hipStream_t st) {
                                 150 * 1024);
             done.fetch_or(bit, std::memory_order_relaxed);
         }
-        hipLaunchKernelGGL(kernel, grid, block, lds, st, a.matrix, a.x, a.scales, a.zeros, a.S, a.K, a.group_units, a.units_per_wave, a);
+        hipLaunchKernelGGL(kernel, grid, block, lds, st, a.matrix, a.x, a.scales, a.zeros, a.S, a.K, a.group_units, a.units_per_wave, (uint32_t)a.R | (uint32_t)WAVES << 16,
+                           (uint32_t)a.wide_wgs, a);
     };
     if (rt <= 1) go(skinny_kernel<BITS, CW, 1, false, false, 1>);
     else go(skinny_kernel<BITS, CW, 2, false, false, 1>);
