@@ -135,7 +135,7 @@ enum TuneKey { TUNE_MV_WAVES = 0, TUNE_MV_UNITS = 1, TUNE_MV_LK = 2, TUNE_MM_VAR
 bool noting(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
 bool is_noting();
 
-// few-row product (2 .. 96 rows; sparse_mask != nullptr: 16:32 int4); false = shape not taken, use the general kernels
+// few-row product (2 .. 96 rows, 17 .. 512 through csrc/wide.hip; sparse_mask != nullptr: 16:32 int4); false = shape not taken, use the general kernels
 bool skinny_rows(int bits, _Float16* outs, const uint32_t* matrix, const _Float16* x, const _Float16* scales,
                  const _Float16* zeros, int64_t R, int64_t K, int64_t S, int64_t group_size, bool accumulate,
                  hipStream_t st, const uint32_t* sparse_mask, void* workspace, size_t workspace_bytes);
