@@ -93,10 +93,12 @@ __global__ __launch_bounds__(512, MT == 1 && !SPARSE && !(BITS == 4 && WN == 2) 
     const int u_first = z0 + min(u_base, share - 1), u_last = z0 + min(u_base + steps, share) - 1;       // (u_last < u_first: no unit)
     const int g_first = magic_div(u_first, group_units, group_magic);
     const int groups = magic_div(max(u_last, u_first), group_units, group_magic) + 1 - g_first;
+    // (a wave without a unit has empty buffers: everything reads as 0)
+    const int row_bytes = u_base < share ? (int)((uint32_t)(groups - 1) * row2 + 128) : 0;
     const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<h16*>(scales) + (int64_t)g_first * S + wcol, 0, (int)((uint32_t)(groups - 1) * row2 + 128), RSRC_FLAGS);
+        const_cast<h16*>(scales) + (int64_t)g_first * S + wcol, 0, row_bytes, RSRC_FLAGS);
     const __amdgpu_buffer_rsrc_t z_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<h16*>(zeros) + (int64_t)g_first * S + wcol, 0, (int)((uint32_t)(groups - 1) * row2 + 128), RSRC_FLAGS);
+        const_cast<h16*>(zeros) + (int64_t)g_first * S + wcol, 0, row_bytes, RSRC_FLAGS);
     constexpr int BATCH = 4;                          // of two groups each
     uint32_t vs[BATCH], scan_off = (uint32_t)h * row2 + 4u * j;
     auto ask_scales = [&]() __attribute__((always_inline)) {
@@ -348,6 +350,7 @@ __global__ __launch_bounds__(512, MT == 1 && !SPARSE && !(BITS == 4 && WN == 2) 
     // of step s + 4 (tall blocks: s + 3) and, as each slice's registers fall free, for the weights of step s + 2; the fragments of a slice are
     // fetched during the one before it, across the barrier too: what a step reads was complete a barrier earlier.
     int group_end = g_first * group_units;             // first unit (of the matrix) beyond the current group
+    const int own_end = z0 + min(u_base + steps, share);                // and beyond the wave's
     const char* const xa = lds + j * PITCH + kg * 128 + h * 16;
     h16x8 fa[LEAN ? 1 : 2][MT];
     auto fetch = [&](h16x8 (&f)[MT], const char* from, int i) __attribute__((always_inline)) {
@@ -356,8 +359,9 @@ __global__ __launch_bounds__(512, MT == 1 && !SPARSE && !(BITS == 4 && WN == 2) 
     };
     uint32_t buf0 = 0, buf1 = XBUF, buf2 = 2 * XBUF;
     auto step = [&](auto mode, int s, Packed& wu, XRegs& xn) __attribute__((always_inline)) {
-        const int u = z0 + min(u_base + s, share - 1);
-        if (u >= group_end) {
+        // (a step without a unit multiplies states and codes of 0; its scale and zero are those beyond the wave's last group, which
+        // read as 0: a group's own may make an infinity of code 0)
+        if (z0 + u_base + s >= min(group_end, own_end)) {
             group_end += group_units;
             take_sz(mode);
             ask_sz();

@@ -687,6 +687,45 @@ def test_shared_staging_keeps_infinite_and_nan_states_in_their_rows(H, bits, spa
     assert np.array_equal(got[0, others], clean[0, others])
 
 
+# ---- a code 0 that overflows although no stored code is 0: fp16(fp16(0 - z) s) is infinite, every other code's weight is finite.
+# What a K group without a unit multiplies adds nothing at all then (not 0 x infinity)
+OVERFLOWS_AT_0 = {4: (8.0, 9000.0), 3: (4.0, 20000.0), 2: (2.0, 33000.0)}          # zero, scale
+
+
+def _problem_overflowing_at_0(bits, sparse, K, S, M, g):
+    rng = np.random.default_rng(K + S + M + bits)
+    zero, scale = OVERFLOWS_AT_0[bits]
+    p = O.make_problem(bits=bits, K=K, S=S, M=M, group_size=g, sparse=sparse, seed=K)
+    codes = rng.integers(1, 1 << bits, size=(K, S), dtype=np.uint8)
+    if sparse:
+        p["matrix"], p["sparse_mask"] = O.sparse_pack(np.ascontiguousarray(codes.T), np.ascontiguousarray(p["keep"].T).astype(np.uint8))
+    else:
+        p["matrix"] = O.pack_dense(bits, codes)
+    p["codes"] = codes
+    p["zeros"][...] = np.float16(zero)
+    p["scales"][...] = np.float16(scale)
+    p["states"] = (p["states"].astype(np.float32) / 512).astype(np.float16)        # (outputs within fp16)
+    return p
+
+
+@pytest.mark.parametrize("bits", [4, 3, 2])
+@pytest.mark.parametrize("M,K,S,g", [(20, 64, 256, 64), (40, 448, 512, 64), (65, 576, 256, -1), (128, 704, 768, 192), (300, 320, 320, 128)])
+def test_k_groups_without_a_unit_add_nothing(H, bits, M, K, S, g):
+    p = _problem_overflowing_at_0(bits, False, K, S, M, g)
+    d = H.dev_problem(p)
+    exact, f32 = H.oracles(p)
+    H.capi.tune(8, 2)
+    try:
+        for split in (0, 1, 2):
+            H.capi.tune(6, split)
+            assert H.capi.describe_launch("mtx", bits, 1, M, K, S, g).startswith("wide_rows_kernel")
+            got = H.run_capi(p, d, "mtx")
+            H.assert_product_close(got, exact, f32, kind="mtx")
+    finally:
+        H.capi.tune(6, 0)
+        H.capi.tune(8, 0)
+
+
 # ---- the matvec entry with more batch elements than the few-row kernel takes at once, on outputs that are not whole strips of 256
 # columns: even shares of at most 96 elements, the last one shorter
 @pytest.mark.parametrize("bits,sparse", [(4, False), (3, False), (2, False), (4, True)])
