@@ -291,7 +291,7 @@ __global__ __launch_bounds__(512, MT == 1 && !SPARSE && !(BITS == 4 && WN == 2) 
             }
         } else {
             uint32_t b0, b1;                      // the codes as bytes
-            h16x2 kept[4];
+            h16x2 kept[4];                        // 16:32: 1.0 in the kept rows' halves; in the loop for both modes all ones, to be ANDed
             if constexpr (SPARSE) {
                 const int b = 3 * (i >> 1);
                 const uint32_t w0 = wu.w[b][c], w1 = wu.w[b + 1][c], m = wu.w[b + 2][c];
@@ -304,8 +304,14 @@ __global__ __launch_bounds__(512, MT == 1 && !SPARSE && !(BITS == 4 && WN == 2) 
                 const uint32_t r0 = __builtin_amdgcn_perm(odd_, even, sel.x), r1 = __builtin_amdgcn_perm(odd_, even, sel.y);
                 b0 = r0 & 0x0F0F0F0Fu; b1 = r1 & 0x0F0F0F0Fu;
                 const uint32_t k0 = r0 & 0x10101010u, k1 = r1 & 0x10101010u;        // the byte 0x10 is 2^-5
-                kept[0] = from_fp8<false>(k0, 32.f); kept[1] = from_fp8<true>(k0, 32.f);
-                kept[2] = from_fp8<false>(k1, 32.f); kept[3] = from_fp8<true>(k1, 32.f);
+                if constexpr (gen) {
+                    const uint32_t f0 = (k0 << 4) - (k0 >> 4), f1 = (k1 << 4) - (k1 >> 4);        // 0x10 -> 0xFF, byte by byte
+                    kept[0] = as_h2(__builtin_amdgcn_perm(f0, f0, 0x01010000u)); kept[1] = as_h2(__builtin_amdgcn_perm(f0, f0, 0x03030202u));
+                    kept[2] = as_h2(__builtin_amdgcn_perm(f1, f1, 0x01010000u)); kept[3] = as_h2(__builtin_amdgcn_perm(f1, f1, 0x03030202u));
+                } else {
+                    kept[0] = from_fp8<false>(k0, 32.f); kept[1] = from_fp8<true>(k0, 32.f);
+                    kept[2] = from_fp8<false>(k1, 32.f); kept[3] = from_fp8<true>(k1, 32.f);
+                }
             } else {
                 const uint32_t word = wu.w[i][c];
                 b0 = word & 0x0F0F0F0Fu; b1 = (word >> 4) & 0x0F0F0F0Fu;
@@ -326,7 +332,8 @@ __global__ __launch_bounds__(512, MT == 1 && !SPARSE && !(BITS == 4 && WN == 2) 
                 h16x2 o;
                 if constexpr (gen) {
                     o = __builtin_elementwise_fma(q[e] + cN[c], cB[c], cC[c]);
-                    if constexpr (SPARSE) o = o * kept[e];
+                    // (a dropped row is 0, not 0 times its code 0's weight, which may be infinite)
+                    if constexpr (SPARSE) o = as_h2(as_u32(o) & as_u32(kept[e]));
                 } else if constexpr (SPARSE) {
                     o = __builtin_elementwise_fma(-kept[e], cN[c], q[e]) * cB[c];
                 } else {

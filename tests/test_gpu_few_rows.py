@@ -688,7 +688,7 @@ def test_shared_staging_keeps_infinite_and_nan_states_in_their_rows(H, bits, spa
 
 
 # ---- a code 0 that overflows although no stored code is 0: fp16(fp16(0 - z) s) is infinite, every other code's weight is finite.
-# What a K group without a unit multiplies adds nothing at all then (not 0 x infinity)
+# What a K group without a unit multiplies, and the rows that 16:32 drops, add nothing at all then (not 0 x infinity)
 OVERFLOWS_AT_0 = {4: (8.0, 9000.0), 3: (4.0, 20000.0), 2: (2.0, 33000.0)}          # zero, scale
 
 
@@ -724,6 +724,29 @@ def test_k_groups_without_a_unit_add_nothing(H, bits, M, K, S, g):
     finally:
         H.capi.tune(6, 0)
         H.capi.tune(8, 0)
+
+
+@pytest.mark.parametrize("M,K,S", [(20, 128, 256), (40, 512, 512), (128, 448, 256)])
+def test_dropped_rows_add_nothing_beside_exponent_mode(H, M, K, S):
+    """16:32, waves whose scales hold a negative one: a third of the columns as above, a third in exponent mode with a zero next
+    to fp16's largest value (code 0, the sum of both, is infinite; the kept codes' weights are not), the others ordinary"""
+    p = _problem_overflowing_at_0(4, True, K, S, M, 64)
+    rng = np.random.default_rng(S)
+    codes = p["codes"]
+    codes[:, 1::3] = rng.integers(8, 12, size=codes[:, 1::3].shape)                  # -1, -2, -4, -8 times the scale
+    p["matrix"], p["sparse_mask"] = O.sparse_pack(np.ascontiguousarray(codes.T), np.ascontiguousarray(p["keep"].T).astype(np.uint8))
+    p["zeros"][:, 1::3], p["scales"][:, 1::3] = np.float16(60000), np.float16(-10000)
+    p["zeros"][:, 2::3], p["scales"][:, 2::3] = np.float16(7.5), np.float16(100)
+    d = H.dev_problem(p)
+    exact, f32 = H.oracles(p)
+    H.capi.tune(8, 2)
+    try:
+        assert H.capi.describe_launch("mtx", 4, 1, M, K, S, 64, True).startswith("wide_rows_kernel")
+        got = H.run_capi(p, d, "mtx")
+    finally:
+        H.capi.tune(8, 0)
+    for c in range(3):                                # (each third on its own scale)
+        H.assert_product_close(got[..., c::3], exact[..., c::3], f32[..., c::3], kind="mtx")
 
 
 # ---- the matvec entry with more batch elements than the few-row kernel takes at once, on outputs that are not whole strips of 256
