@@ -906,6 +906,11 @@ static MatvecShape plan_matvec(int64_t S, int units_total) {
         if (want_splits < 1) want_splits = 1;
         upwg = (units_total + want_splits - 1) / want_splits;
         if (upwg < 4) upwg = 4;
+        // (a long K on a wide output: more splits, so that a workgroup's units fit its staged states)
+        if (upwg > MV_MAX_UNITS_WG) {
+            want_splits = (units_total + MV_MAX_UNITS_WG - 1) / MV_MAX_UNITS_WG;
+            upwg = (units_total + want_splits - 1) / want_splits;
+        }
     }
     if (upwg > units_total) upwg = units_total;
     // The workgroup of a strip's last split sums the strip up once the others have handed

@@ -159,6 +159,16 @@ def test_matvec_of_a_k_beyond_one_launch():
     assert d("vec", 4, 1, 1, 1 << 20, 256, -1).count("matvec_kernel<") == 3       # one group: any cut will do
 
 
+@pytest.mark.parametrize("k,s", [(28736, 32768), (32192, 16896), (46656, 26624), (60544, 11008), (430144, 1344), (14400, 109312), (458752, 32768)])
+def test_matvec_of_a_long_k_on_a_wide_output(k, s):
+    # K is split more ways than the output's width asks for, so that a workgroup's units fit its staged states
+    for bits, sparse in ((4, False), (3, False), (2, False), (4, True)):
+        line = d("vec", bits, 1, 1, k, s, 128, sparse)
+        name, f, _ = fields(line)
+        assert name == "matvec_kernel" and line.count("matvec_kernel<") == 1 and f["units_per_workgroup"] <= 224 and f["splits"] <= 32, line
+        assert f["splits"] * f["units_per_workgroup"] >= k // 64 > (f["splits"] - 1) * f["units_per_workgroup"], line
+
+
 def test_matvec_needs_its_workspace_whatever_the_shape():
     # K = 64: a single unit, nothing to hand over -- the documented rule holds all the same
     with pytest.raises(capi.Int4mmError) as e:

@@ -57,6 +57,35 @@ def test_matvec_of_a_k_longer_than_one_launch_covers(H, bits, sparse, g):
     H.assert_product_close(got, exact, f32, prior=prior)
 
 
+@pytest.mark.parametrize("bits,sparse,K,S,splits", [(4, False, 28736, 32768, 3), (2, False, 430144, 1344, 31), (4, True, 60544, 11008, 5)])
+def test_matvec_of_a_long_k_on_a_wide_output(H, bits, sparse, K, S, splits):
+    """an output so wide that K would be cut into shares beyond a workgroup's staged states: more shares; against the
+    dequantised matrix in slabs of K"""
+    g = 64
+    capi = H.capi
+    assert f"splits={splits} " in capi.describe_launch("vec", bits, 1, 1, K, S, g, sparse)
+    gen = torch.Generator(device="cuda").manual_seed(K)
+    matrix = torch.randint(-2 ** 31, 2 ** 31, (K // 16 if sparse else K * bits // 32, S), dtype=torch.int32, generator=gen, device="cuda")
+    # (16:32: the same sixteen rows of every 32, another sixteen in every other column)
+    mask = torch.tensor([0x0F0F3355, -0x0F0F3356], dtype=torch.int32, device="cuda").repeat(K // 32, S // 2) if sparse else None
+    scales = torch.empty((K // g, S), device="cuda").uniform_(0.001, 0.02, generator=gen).half()
+    zeros = torch.empty((K // g, S), device="cuda").uniform_(0.0, 2 ** bits - 1.0, generator=gen).half()
+    x = torch.randn((1, 1, K), generator=gen, device="cuda").half()
+    out = torch.zeros((1, 1, S), dtype=torch.float16, device="cuda")
+    capi.matvec(bits, out, matrix, x, scales, zeros, g, mask, capi.new_matmul_workspace(1, 1, K, S, sparse))
+    want = torch.zeros(S, dtype=torch.float64, device="cuda")
+    slab = g * max(1, (1 << 26) // (g * S))
+    for k0 in range(0, K, slab):
+        k1 = min(K, k0 + slab)
+        w = torch.empty((k1 - k0, S), dtype=torch.float16, device="cuda")
+        rows = (lambda k: k // 16) if sparse else (lambda k: k * bits // 32)
+        capi.dequantize(bits, w, matrix[rows(k0):rows(k1)], scales[k0 // g:k1 // g], zeros[k0 // g:k1 // g], g,
+                        mask[k0 // 32:k1 // 32] if sparse else None)
+        want += x[0, 0, k0:k1].double() @ w.double()
+    torch.cuda.synchronize()
+    assert O.max_rel_error(want.cpu().numpy(), out.cpu().numpy()[0, 0]) < H.TOL_EXACT
+
+
 @pytest.mark.parametrize("bits,sparse", FORMATS)
 def test_matvec_accumulates_onto_prior_outs_and_batches(H, bits, sparse):
     p = _problem(bits, sparse, K=512, S=192, M=1, B=3, group_size=64, seed=4)
