@@ -547,31 +547,83 @@ static const WideCost wide_cost[4][6] = {             // int4, int3, int2, 16:32
      {4, 4, 1.76, 0.352, 1.84, 7.15, 6.6, 2.45, 1.26, 5.45}}};
 constexpr int64_t WIDE_MAX_SPLIT_WGS = 512;              // workgroups of a launch that splits K (bounds its partial tiles)
 
-// 17 ... 64 rows that stay with the few-row kernel, whose sums are of the exact codes (scale and zero applied in fp32): what a
-// weight rounded twice to fp16 would cost in precision is not given for speed.  (The lines were drawn by the speed of an
-// earlier form of the kernel above, which took the others.)
-static bool few_row_sums(int64_t R, int64_t K, int64_t S, bool sparse) {
-    if (R > 64) return false;
-    const int64_t units = K / 64, strips = S / 256;
-    const bool one_round = [&] {                          // the few-row kernel runs two row blocks as one round, or splits K itself
+// Which products of up to 96 rows may take the kernel above.  Elsewhere they are sums of the exact codes, scale and zero applied in
+// fp32; here each weight is rounded to fp16 twice (error against float64, 2-norm: 2.1e-4 of the result there, 3.2e-4 here).
+// Hence this is a line of precision and not of speed, and is not to be fitted to timings: it admits what an earlier form of
+// the kernel took -- with its split of K, if its partial tiles have `room` in the workspace and a share's scales have room in the
+// LDS, as that form kept them there -- so that no product that had the exact codes' sums loses them.
+struct RoundedLine { bool admitted; size_t room; };
+static RoundedLine rounded_line(bool sparse, int64_t R, int64_t K, int64_t S, int64_t group_units) {
+    const RoundedLine none{false, 0};
+    if (R < 17 || R > SK_WIDE_MAX_ROWS || S % 256 != 0) return none;
+    const int64_t units = K / 64, strips = S / 256, lds_limit = 150 * 1024 - (sparse ? 4096 : 0);
+    int64_t tiles = 0, blocks = 0, wgs = 0, ks = 1;         // row tiles of 16 in a block, blocks, unsplit workgroups, ways
+    auto fits = [&](int64_t share) {
+        int64_t groups = (units + group_units - 1) / group_units;
+        if (share < units) groups = std::min(groups, (share + group_units - 1) / group_units + 1);
+        return 16 * tiles * 288 + 1040 + groups * 1024 <= lds_limit;
+    };
+    auto shape = [&](int64_t tallest) {
+        blocks = (R + tallest - 1) / tallest;
+        tiles = ((R + blocks - 1) / blocks + 15) / 16;
+        if (tiles == 5 || tiles == 7) ++tiles;
+        wgs = strips * blocks;
+    };
+    auto shape_and_split = [&](int64_t tallest) {
+        shape(tallest);
+        ks = wgs > 128 && wgs < 256 ? 4 : 256 / wgs;
+        ks = wgs > 1024 ? 1 : std::max<int64_t>(1, std::min<int64_t>(ks, units / 8));
+        while (wgs * (ks + 1) <= 256 && ks < units / 8 && !fits((units + ks - 1) / ks)) ++ks;
+    };
+    shape_and_split(128);
+    if (R <= 64 || ks > 6 || (ks > 1 && units / ks < 20)) shape_and_split(64);
+    if (!sparse && R > 48 && R <= 64 && S <= 4096) shape_and_split(32);
+    if (R > 64 && S >= (sparse ? 4096 : 1024) && S <= (sparse ? 8192 : 32768)) {
+        struct Cost { double unit[9], workgroup, split, way, tile, last; };
+        static const Cost costs[2] = {{{0, 0, 0, 0.617, 0.707, 0, 0.912, 0, 1.059}, 3.92, -4.164, 0.798, 1.915, 3.544},
+                                      {{0, 0, 0, 1.12, 1.203, 0, 1.32, 0, 1.537}, 4.17, -3.744, 0.921, 1.701, 5.284}};
+        const Cost& c = costs[sparse];
+        double best = 1e30;
+        int64_t best_tallest = 0, best_ks = 1;
+        for (const int64_t tallest : {128, 96, 64, 48}) {
+            shape(tallest);
+            for (int64_t k = 1; k <= 16 && (k == 1 || units / k >= 8) && wgs * k <= 1024; ++k) {
+                const int64_t share = (units + k - 1) / k, rounds = (wgs * k + 255) / 256, last = wgs * k - (rounds - 1) * 256;
+                if (!fits(share)) continue;
+                const double t = rounds * (c.unit[tiles] * share + c.workgroup) + (k > 1 ? c.split + c.way * k + c.tile * tiles : 0.0) +
+                                 (rounds > 1 ? c.last * last / 256.0 : 0.0);
+                if (t < best) { best = t; best_tallest = tallest; best_ks = k; }
+            }
+        }
+        if (best_tallest != 0) { shape(best_tallest); ks = best_ks; }
+        else shape_and_split(48);
+    }
+    const int64_t share = (units + ks - 1) / ks;
+    ks = (units + share - 1) / share;
+    if (!fits(share)) return none;
+    // one round of two row blocks of the few-row kernel, or that kernel's own split of K
+    const bool one_round = [&] {
         if (S / 32 * 2 < 192) return true;
         for (const int c : {4, 2, 1}) {
             if (sparse && c == 4) continue;
-            const int64_t wgs = S / (16 * c) * 2;
-            if (wgs >= 128 && wgs <= 256) return true;
+            if (S / (16 * c) * 2 >= 128 && S / (16 * c) * 2 <= 256) return true;
         }
         return false;
     }();
-    if (R > 32) {
-        if (sparse) return one_round ? (K <= 8192 || S < 3072) : (K < 4096 && K * S < (1ll << 25));
-        return one_round ? (K <= 5120 || (K <= 8192 && S <= 4096) || S < 3072) : K * S < (1ll << 25);
+    bool few_row;                                           // the few-row kernel or, beyond 96 rows, the matvec
+    if (sparse) {
+        few_row = R <= 32 ? K * S < (1ll << 26)
+                : R <= 64 ? (one_round ? K <= 8192 || S < 3072 : K < 4096 && K * S < (1ll << 25))
+                : R <= 96 ? false
+                : R <= 128 ? S > 16384 && blocks > 1 : S > 8192 || (R > 256 && S > 4096);
+    } else {
+        few_row = R <= 32 ? wgs < (units >= 160 ? 24 : 32) || wgs > 96 || share < 16 || (S / 64 > 128 && S / 64 <= 256 && K <= 6144)
+                : R <= 64 ? (one_round ? K <= 5120 || (K <= 8192 && S <= 4096) || S < 3072 : K * S < (1ll << 25))
+                : R <= 128 ? false
+                : S > 8192 && S > (R <= 192 || (R <= 256 && K <= 4096) ? 32768 : R <= 256 ? 10240 : 8192);
     }
-    if (sparse) return K * S < (1ll << 26);
-    int64_t ks = 256 / std::max<int64_t>(strips, 1);
-    if (ks <= 1 && strips > 128 && strips < 256) ks = 4;
-    ks = std::max<int64_t>(1, std::min<int64_t>(ks, units / 8));
-    if (strips < (units >= 160 ? 24 : 32) || strips > 96 || (units + ks - 1) / ks < 16) return true;
-    return S / 64 > 128 && S / 64 <= 256 && K <= 6144;
+    if (few_row) return none;
+    return {true, ks > 1 ? (size_t)(wgs * ks * tiles * 16384) : 0};
 }
 
 // Whole strips of 256 columns; beyond 96 rows, which the few-row kernel does not take, any number of whole 64 (the general
@@ -580,7 +632,8 @@ static bool few_row_sums(int64_t R, int64_t K, int64_t S, bool sparse) {
 static bool wide_columns(int64_t R, int64_t S) { return S % 256 == 0 || (R > FEW_ROWS_MAX && S % 64 == 0); }
 static int64_t wide_strips(int64_t S, int wn) { return (S + 64 * wn - 1) / (64 * wn); }
 
-static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S, bool can_split) {
+// `scratch`: bytes for partial tiles; the splits that need more are no candidates
+static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S, size_t scratch) {
     WidePlan p{false, 0, 0, 0, 1, 0, 0};
     // (knob: 1 = never, n >= 2 = from n rows on whatever the shape)
     const int64_t knob = tuning(TUNE_NO_WIDE), min_rows = knob >= 2 ? knob : 17, forced = tuning(TUNE_MM_SPLIT);
@@ -589,7 +642,6 @@ static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S
     // (32-bit byte offsets into buffer resources: a share of the packed matrix, its scales and the block's rows of states and
     // outputs stay below 2 GB)
     if (K * S >= (sparse ? 1ll << 33 : (1ll << 34) / bits) || K >= (1 << 22) || S >= (1 << 22)) return p;
-    if (knob < 2 && few_row_sums(R, K, S, sparse)) return p;
     const int64_t few = (R + 127) / 128, tallest = ((R + few - 1) / few + 31) / 32;
     double best = 1e30;
     for (const WideCost& c : wide_cost[sparse ? 3 : 4 - bits]) {
@@ -599,11 +651,16 @@ static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S
         // (49 ... 64 rows on 2048 ... 4096 columns and a long K: two blocks of 32 rows)
         if (!sparse && R > 48 && R <= 64 && S > 2048 && S <= 4096 && K > 8192 && forced < 1 && (c.mt != 1 || c.wn != 4)) continue;
         const int64_t blocks = (R + 32 * c.mt - 1) / (32 * c.mt), tiles = wide_strips(S, c.wn) * blocks;
+        const auto too_large = [&](int64_t k) {
+            const int64_t share = (units + k - 1) / k;
+            return k > 1 && (size_t)((units + share - 1) / share * tiles * c.mt * c.wn) * 8192 > scratch;
+        };
         // (below 1024 columns, where nothing was fitted: as many ways as leave shares of eight units)
-        const int64_t only = forced >= 1 ? std::min<int64_t>(forced, std::max<int64_t>(1, units / 4))
-                           : S < 1024 && can_split ? std::max<int64_t>(1, std::min<int64_t>({256 / tiles, units / 8, 16})) : 0;
+        int64_t only = forced >= 1 ? std::min<int64_t>(forced, std::max<int64_t>(1, units / 4))
+                     : S < 1024 ? std::max<int64_t>(1, std::min<int64_t>({256 / tiles, units / 8, 16})) : 0;
+        while (too_large(only)) --only;
         for (int64_t k = only ? only : 1; k <= 16; ++k) {
-            if (k > 1 && (!can_split || units / k < 4 || tiles * k > WIDE_MAX_SPLIT_WGS)) break;
+            if (k > 1 && (units / k < 4 || tiles * k > WIDE_MAX_SPLIT_WGS || too_large(k))) break;
             const int64_t share = (units + k - 1) / k, steps = (share * c.wn + 7) / 8, wgs = tiles * k, rounds = (wgs + 255) / 256;
             const double t = steps * (c.step + c.filled * std::min(1.0, wgs / 256.0)) + c.workgroup + (k > 1 ? c.split + c.way * k : 0.0) +
                              (rounds > 1 ? (rounds - 1) * (c.more_step * steps + c.more_workgroup) + c.last * (wgs - (rounds - 1) * 256) / 256.0 : 0.0);
@@ -620,7 +677,7 @@ static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S
         const double flops = 2.0 * ((R + 255) / 256 * 256) * K * S;
         if (best > 5.0 + flops / (wide_strips(S, p.wn) * p.row_blocks > 256 ? 1.05e9 : 0.75e9)) return p;
     }
-    p.part_bytes = p.ksplit > 1 ? (size_t)p.ksplit * p.row_blocks * 32 * p.mt * wide_strips(S, p.wn) * 64 * p.wn * 4 : 0;
+    p.part_bytes = p.ksplit > 1 ? (size_t)p.ksplit * p.row_blocks * p.mt * wide_strips(S, p.wn) * p.wn * 8192 : 0;
     p.use = true;
     return p;
 }
@@ -629,10 +686,19 @@ static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S
 // no more than the split's limit (16 ways, four units each) of the rows rounded up to whole blocks.
 size_t wide_workspace_bytes(int64_t R, int64_t K, int64_t S, bool sparse) {
     if (R < 2 || R > SK_WIDE_MAX_ROWS || !wide_columns(R, S) || K % 64 != 0) return 0;
-    if (tuning(TUNE_NO_WIDE) < 2 && (R < 17 || few_row_sums(R, K, S, sparse))) return 0;
+    size_t room = 0;
+    if (R <= FEW_ROWS_MAX && tuning(TUNE_NO_WIDE) < 2) {
+        bool admitted = false;
+        for (const int64_t group_units : {1, 2, 3, 4, 6, 8, 16, 0x7FFFFFF}) {
+            const RoundedLine line = rounded_line(sparse, R, K, S, group_units);
+            admitted = admitted || line.admitted;
+            room = std::max(room, line.room);
+        }
+        if (!admitted) return 0;
+    }
     const int64_t ways = std::min<int64_t>(16, K / 256), mt = std::min<int64_t>(4, (R + 31) / 32);
-    if (ways < 2) return 0;
-    return (size_t)std::min<int64_t>(WIDE_MAX_SPLIT_WGS * mt * 32768, ways * ((R + 32 * mt - 1) / 32 * 32) * ((S + 255) / 256 * 256) * 4);
+    if (ways < 2) return room;
+    return std::max(room, (size_t)std::min<int64_t>(WIDE_MAX_SPLIT_WGS * mt * 32768, ways * ((R + 32 * mt - 1) / 32 * 32) * ((S + 255) / 256 * 256) * 4));
 }
 
 template <int BITS, int MT, bool SPARSE, int WN>
@@ -673,8 +739,11 @@ static bool launch_wide(const SkinnyArgs& a, const WidePlan& p, hipStream_t st) 
 bool wide_rows(int bits, const SkinnyArgs& args, void* workspace, size_t workspace_bytes, hipStream_t st) {
     const bool sparse = args.mask != nullptr;
     const WorkspaceParts ws = workspace_parts(workspace, workspace_bytes);
-    WidePlan p = plan_wide(bits, sparse, args.R, args.K, args.S, ws.counters != nullptr);
-    if (p.use && p.ksplit > 1 && ws.scratch_bytes < p.part_bytes) p = plan_wide(bits, sparse, args.R, args.K, args.S, false);
+    if (args.R <= FEW_ROWS_MAX && tuning(TUNE_NO_WIDE) < 2) {
+        const RoundedLine line = rounded_line(sparse, args.R, args.K, args.S, args.group_units);
+        if (!line.admitted || ws.scratch_bytes < line.room) return false;
+    }
+    const WidePlan p = plan_wide(bits, sparse, args.R, args.K, args.S, ws.scratch_bytes);
     if (!p.use) return false;
     SkinnyArgs a = args;
     a.counters = reinterpret_cast<int*>(ws.counters);

@@ -111,6 +111,21 @@ def test_every_shape_gets_a_kernel_within_its_limits(fmt):
             assert n2 in KERNELS and f2.get("ksplit", 1) == 1 and f2.get("splits", 1) == 1, bare
 
 
+# ---- the kernels that sum exact codes keep the products that they had: a workspace too small for the split of K that the kernel with
+# rounded weights was admitted with, and a long K with small groups
+@pytest.mark.parametrize("product", ["mtx", "vec"])
+@pytest.mark.parametrize("bits,sparse,rows,k,s,g,ws", [(4, False, 64, 8192, 8192, 128, "matvec"), (3, False, 40, 20480, 4096, 64, "matvec"),
+                                                       (2, False, 96, 8192, 4096, -1, "matvec"), (4, True, 90, 8192, 8192, 64, "matvec"),
+                                                       (4, True, 72, 14016, 768, 64, 3 << 20), (4, False, 52, 16896, 23296, 64, None),
+                                                       (4, True, 18, 17920, 23808, 64, None)])
+def test_few_rows_keep_the_sums_of_exact_codes(product, bits, sparse, rows, k, s, g, ws):
+    nbytes = capi.lib().int4mm_workspace_bytes(s) if ws == "matvec" else ws
+    line = d(product, bits, *((rows, 1) if product == "vec" else (1, rows)), k, s, g, sparse, nbytes)
+    assert line.startswith("skinny_kernel"), line
+    if ws is not None:                                     # (with the workspace that the size query asks for they are rounded, as before)
+        assert d("mtx", bits, 1, rows, k, s, g, sparse).startswith("wide_rows_kernel")
+
+
 def evenly_shared(line):
     return "balanced" in line or "columns_per_lane=4+1" in line
 
