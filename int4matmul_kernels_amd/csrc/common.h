@@ -135,10 +135,12 @@ enum TuneKey { TUNE_MV_WAVES = 0, TUNE_MV_UNITS = 1, TUNE_MV_LK = 2, TUNE_MM_VAR
 bool noting(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
 bool is_noting();
 
-// few-row product (2 .. 96 rows, 17 .. 512 through csrc/wide.hip; sparse_mask != nullptr: 16:32 int4); false = shape not taken, use the general kernels
+// Few-row product (2 .. 96 rows, 17 .. 512 through csrc/wide.hip; sparse_mask != nullptr: 16:32 int4); false = shape not taken, use
+// the general kernels.  FOR_MATVEC: beyond 96 rows too only where weights rounded to fp16 may serve; EXACT_SUMS: never those
+enum RowsCall { FOR_MATMUL, FOR_MATVEC, EXACT_SUMS };
 bool skinny_rows(int bits, _Float16* outs, const uint32_t* matrix, const _Float16* x, const _Float16* scales,
                  const _Float16* zeros, int64_t R, int64_t K, int64_t S, int64_t group_size, bool accumulate,
-                 hipStream_t st, const uint32_t* sparse_mask, void* workspace, size_t workspace_bytes);
+                 hipStream_t st, const uint32_t* sparse_mask, void* workspace, size_t workspace_bytes, RowsCall call);
 // two to four rows through the matvec kernel (dense formats; csrc/matvec.hip): false when it does not take the shape
 bool matvec_rows(int bits, _Float16* outs, const uint32_t* matrix, const _Float16* x, const _Float16* scales,
                  const _Float16* zeros, int64_t R, int64_t K, int64_t S, int64_t group_size, bool accumulate,
@@ -150,19 +152,18 @@ bool matvec_one_row(int bits, _Float16* outs, const uint32_t* matrix, const uint
 // most rows the few-row path takes (beyond 96: only its kernel with shared staging, for the shapes it serves)
 constexpr int SK_WIDE_MAX_ROWS = 512;
 constexpr int FEW_ROWS_MAX = 96;                     // rows that the few-row kernel with its sums of exact codes takes at once
-// Batch elements that the matvec entry hands to the few-row kernels at once: up to 512; on outputs of more than 512 columns
-// that are not whole strips of 256, which the kernel for more than 96 rows serves in the matmul entry alone (its weights are
-// rounded to fp16, the matvec sums exact codes), even shares of at most 96 (us, one matvec per element / so: int4, K=9280,
-// S=1600, 110 elements 760 / 48; 16:32, K=4096, S=1600, 128 elements 900 / 29; int2, K=3072, S=1856, 300 elements 1530 / 60)
-inline int64_t matvec_rows_at_once(int64_t B, int64_t S) {
-    if (S % 256 == 0) return SK_WIDE_MAX_ROWS;
-    if (B <= FEW_ROWS_MAX) return FEW_ROWS_MAX;
-    if (S <= 512) return 0;                          // (one matvec per element)
-    const int64_t chunks = (B + FEW_ROWS_MAX - 1) / FEW_ROWS_MAX;
-    return (B + chunks - 1) / chunks;
+// Batch elements of the matvec entry that go through the few-row kernel at once where the kernel for more rows, whose weights are
+// rounded, is not admitted (rounded_line, csrc/wide.hip): even shares of at most 96 of those that are left (us, one matvec per element / so:
+// int4, K=9280, S=1600, 110 elements 760 / 48; 16:32, K=4096, S=1600, 128 elements 900 / 29; int2, K=3072, S=1856, 300 elements
+// 1530 / 60).  0: one matvec per element, as narrow outputs that are not whole strips of 256 run (int4, K=4096, S=192, 97 elements
+// 508 us, where shares would take 26)
+inline int64_t exact_sums_at_once(int64_t left, int64_t S) {
+    if (S <= 512 && S % 256 != 0) return 0;
+    const int64_t chunks = (left + FEW_ROWS_MAX - 1) / FEW_ROWS_MAX;
+    return (left + chunks - 1) / chunks;
 }
-// bytes of partial tiles with which the few-row kernel splits K across workgroups (0: no split)
-size_t skinny_workspace_bytes(int64_t R, int64_t K, int64_t S, bool sparse);
+// bytes of partial tiles with which such a product splits K across workgroups (0: no split)
+size_t skinny_workspace_bytes(int64_t R, int64_t K, int64_t S, bool sparse, RowsCall call);
 
 // Layout of a caller's workspace, a function of its size alone so that calls with different shapes may
 // share one buffer.  The lower half (down to a page boundary) is kept zero between calls: the matvec's

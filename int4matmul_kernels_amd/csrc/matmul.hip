@@ -1289,7 +1289,7 @@ extern "C" int int4mm_matmul(int bits, void* outs, const void* matrix, const voi
         return check_launch("matmul");
     if (B * M >= 2 && B * M <= SK_WIDE_MAX_ROWS && !tuning(TUNE_NO_SKINNY) && !tuning(TUNE_MM_VARIANT) &&
         skinny_rows(bits, (h16*)outs, (const uint32_t*)matrix, (const h16*)multiplier, (const h16*)scales,
-                    (const h16*)zeros, B * M, K, S, g, false, st, (const uint32_t*)sparse_mask, workspace, workspace_bytes))
+                    (const h16*)zeros, B * M, K, S, g, false, st, (const uint32_t*)sparse_mask, workspace, workspace_bytes, FOR_MATMUL))
         return check_launch("matmul");
 
     MatmulArgs a;
@@ -1326,10 +1326,18 @@ extern "C" size_t int4mm_matmul_workspace_bytes(const int4mm_shape* shape, int s
     size_t need = int4mm_workspace_bytes(S);
     if (B <= 0 || M <= 0 || K < 64 || S < 128) return need;
     if (B > 1 && B * M <= ((int64_t)1 << 31) - 256) { M *= B; B = 1; }           // (as int4mm_matmul does)
-    size_t few_rows = B * M <= SK_WIDE_MAX_ROWS ? skinny_workspace_bytes(B * M, K, S, sparse != 0) : 0;
-    // (the matvec entry takes many batch elements of one row in chunks through the few-row kernels)
-    const int64_t at_once = shape->seq_len == 1 ? matvec_rows_at_once(B * M, S) : 0;
-    if (at_once > 0 && at_once < B * M) few_rows = std::max(few_rows, skinny_workspace_bytes(at_once, K, S, sparse != 0));
+    size_t few_rows = B * M <= SK_WIDE_MAX_ROWS ? skinny_workspace_bytes(B * M, K, S, sparse != 0, FOR_MATMUL) : 0;
+    // (the matvec entry takes many batch elements of one row in chunks through the few-row kernels: as many as the kernel
+    // for more rows takes, else even shares, which may be one fewer towards the end)
+    if (shape->seq_len == 1)
+        for (const int64_t n : {std::min<int64_t>(B * M, SK_WIDE_MAX_ROWS), B * M % SK_WIDE_MAX_ROWS}) {
+            if (n < 2) continue;
+            few_rows = std::max(few_rows, skinny_workspace_bytes(n, K, S, sparse != 0, FOR_MATVEC));
+            for (const int64_t share : {exact_sums_at_once(n, S), exact_sums_at_once(B * M, S)})
+                if (n > FEW_ROWS_MAX && share > 2)
+                    few_rows = std::max({few_rows, skinny_workspace_bytes(share, K, S, sparse != 0, EXACT_SUMS),
+                                         skinny_workspace_bytes(share - 1, K, S, sparse != 0, EXACT_SUMS)});
+        }
     if (B * M <= FEW_ROWS_MAX) return need + 2 * round_to_page(few_rows);
     const SplitPlan sp = plan_split(sparse != 0, B, M, K, S);
     if (sp.ksplit > 1 || few_rows > 0)

@@ -1047,28 +1047,26 @@ static int matvec_impl(int bits, void* outs, const void* matrix, const void* mul
         matvec_rows(bits, (h16*)outs, (const uint32_t*)matrix, (const h16*)multiplier, (const h16*)scales, (const h16*)zeros,
                     B, K, S, g, accumulate, (hipStream_t)stream, workspace, workspace_bytes))
         return check_launch("matvec");
-    const int64_t at_once = matvec_rows_at_once(B, S);
-    if (B >= 2 && B <= at_once && !tuning(TUNE_NO_SKINNY) &&
-        skinny_rows(bits, (h16*)outs, (const uint32_t*)matrix, (const h16*)multiplier, (const h16*)scales,
-                    (const h16*)zeros, B, K, S, g, accumulate, (hipStream_t)stream, (const uint32_t*)sparse_mask, workspace, workspace_bytes))
-        return check_launch("matvec");
-
-    // more batch elements than the few-row kernels take at once: in chunks through them (1 100 elements at K=4096, S=4096:
-    // three launches instead of 1 100), the plain kernel, a launch per element, for what they do not take
+    // more batch elements: in chunks of up to 512 through the kernels for that many rows where these may serve them (1 100
+    // elements at K=4096, S=4096: three launches), else in even shares through the few-row kernel with its sums of exact codes -- all of
+    // the rest then --, and the plain kernel, a launch per element, for what that does not take
     int64_t done = 0;
-    if (B > at_once && at_once > 0 && !tuning(TUNE_NO_SKINNY)) {
-        while (B - done >= 2) {
-            const int64_t n = std::min<int64_t>(at_once, B - done);
-            if (!skinny_rows(bits, (h16*)outs + done * S, (const uint32_t*)matrix, (const h16*)multiplier + done * K, (const h16*)scales,
-                             (const h16*)zeros, n, K, S, g, accumulate, (hipStream_t)stream, (const uint32_t*)sparse_mask, workspace,
-                             workspace_bytes))
-                break;
-            rc = check_launch("matvec");
-            if (rc != INT4MM_OK) return rc;
-            done += n;
+    RowsCall call = FOR_MATVEC;
+    while (B - done >= 2 && !tuning(TUNE_NO_SKINNY)) {
+        const int64_t left = B - done, n = call == FOR_MATVEC ? std::min<int64_t>(left, SK_WIDE_MAX_ROWS) : exact_sums_at_once(left, S);
+        if (n == 0) break;
+        if (!skinny_rows(bits, (h16*)outs + done * S, (const uint32_t*)matrix, (const h16*)multiplier + done * K, (const h16*)scales,
+                         (const h16*)zeros, n, K, S, g, accumulate, (hipStream_t)stream, (const uint32_t*)sparse_mask, workspace,
+                         workspace_bytes, call)) {
+            if (call == EXACT_SUMS) break;
+            call = EXACT_SUMS;
+            continue;
         }
-        if (done == B) return INT4MM_OK;
+        rc = check_launch("matvec");
+        if (rc != INT4MM_OK) return rc;
+        done += n;
     }
+    if (done == B) return INT4MM_OK;
     return matvec_plain(bits, (h16*)outs + done * S, matrix, (const h16*)multiplier + done * K, scales, zeros, sparse_mask, B - done, K, S, g,
                         accumulate, workspace, workspace_bytes, (hipStream_t)stream);
 }

@@ -805,9 +805,9 @@ static SkinnySplit plan_skinny_split(int64_t R, int64_t K, int64_t S, bool spars
     return p;
 }
 
-size_t skinny_workspace_bytes(int64_t R, int64_t K, int64_t S, bool sparse) {
+size_t skinny_workspace_bytes(int64_t R, int64_t K, int64_t S, bool sparse, RowsCall call) {
     const SkinnySplit p = plan_skinny_split(R, K, S, sparse);
-    const size_t wide = wide_workspace_bytes(R, K, S, sparse);
+    const size_t wide = wide_workspace_bytes(R, K, S, sparse, call);
     const size_t balanced = balanced_shape(R, K, S) ? skinny_balanced_part_bytes(S) : 0;
     return std::max(std::max<size_t>(p.ksplit > 1 ? p.part_bytes : 0, wide), balanced);
 }
@@ -817,7 +817,7 @@ size_t skinny_workspace_bytes(int64_t R, int64_t K, int64_t S, bool sparse) {
 // uses the general kernels).
 bool skinny_rows(int bits, h16* outs, const uint32_t* matrix, const h16* x, const h16* scales, const h16* zeros,
                  int64_t R, int64_t K, int64_t S, int64_t group_size, bool accumulate, hipStream_t st,
-                 const uint32_t* sparse_mask, void* workspace, size_t workspace_bytes) {
+                 const uint32_t* sparse_mask, void* workspace, size_t workspace_bytes, RowsCall call) {
     if (R < 2 || R > SK_WIDE_MAX_ROWS || S % 16 != 0 || K % 64 != 0 || K > (1 << 30) || S > (1 << 28)) return false;
     if (sparse_mask && bits != 4) return false;
     SkinnyArgs a;
@@ -831,7 +831,7 @@ bool skinny_rows(int bits, h16* outs, const uint32_t* matrix, const h16* x, cons
     a.bal_q = 0; a.bal_r = 0;
     a.wide_wgs = 0;
     // 17 rows and more: the kernel whose waves share the staged states, where its plan says so
-    if (wide_rows(bits, a, workspace, workspace_bytes, st)) return true;
+    if (wide_rows(bits, a, call, workspace, workspace_bytes, st)) return true;
     if (R > FEW_ROWS_MAX) return false;
     // four waves split K when there are more workgroups than CUs (three of them fit a CU) and K
     // is short (each wave should walk a dozen units or more), eight otherwise -- also at exactly one

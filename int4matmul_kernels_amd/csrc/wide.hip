@@ -547,7 +547,7 @@ static const WideCost wide_cost[4][6] = {             // int4, int3, int2, 16:32
      {4, 4, 1.76, 0.352, 1.84, 7.15, 6.6, 2.45, 1.26, 5.45}}};
 constexpr int64_t WIDE_MAX_SPLIT_WGS = 512;              // workgroups of a launch that splits K (bounds its partial tiles)
 
-// Which products of up to 96 rows may take the kernel above.  Elsewhere they are sums of the exact codes, scale and zero applied in
+// Which products of up to 96 rows, and which of the matvec entry, may take the kernel above.  Elsewhere they are sums of the exact codes, scale and zero applied in
 // fp32; here each weight is rounded to fp16 twice (error against float64, 2-norm: 2.1e-4 of the result there, 3.2e-4 here).
 // Hence this is a line of precision and not of speed, and is not to be fitted to timings: it admits what an earlier form of
 // the kernel took -- with its split of K, if its partial tiles have `room` in the workspace and a share's scales have room in the
@@ -626,9 +626,10 @@ static RoundedLine rounded_line(bool sparse, int64_t R, int64_t K, int64_t S, in
     return {true, ks > 1 ? (size_t)(wgs * ks * tiles * 16384) : 0};
 }
 
+static bool needs_admission(int64_t R, RowsCall call) { return (R <= FEW_ROWS_MAX || call == FOR_MATVEC) && tuning(TUNE_NO_WIDE) < 2; }
+
 // Whole strips of 256 columns; beyond 96 rows, which the few-row kernel does not take, any number of whole 64 (the general
-// tiles that served them cannot split K: int2, K=9280, S=1600, 220 rows 238 us there, 21 here; the matvec entry, whose sums are of
-// the exact codes, does not come here with such a shape: matvec_rows_at_once).
+// tiles that served them cannot split K: int2, K=9280, S=1600, 220 rows 238 us there, 21 here).
 static bool wide_columns(int64_t R, int64_t S) { return S % 256 == 0 || (R > FEW_ROWS_MAX && S % 64 == 0); }
 static int64_t wide_strips(int64_t S, int wn) { return (S + 64 * wn - 1) / (64 * wn); }
 
@@ -684,10 +685,10 @@ static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S
 
 // An upper bound of any plan's partial tiles, cheap enough for every call: at most 512 workgroups of 32 KB per 32 rows, and
 // no more than the split's limit (16 ways, four units each) of the rows rounded up to whole blocks.
-size_t wide_workspace_bytes(int64_t R, int64_t K, int64_t S, bool sparse) {
-    if (R < 2 || R > SK_WIDE_MAX_ROWS || !wide_columns(R, S) || K % 64 != 0) return 0;
+size_t wide_workspace_bytes(int64_t R, int64_t K, int64_t S, bool sparse, RowsCall call) {
+    if (call == EXACT_SUMS || R < 2 || R > SK_WIDE_MAX_ROWS || !wide_columns(R, S) || K % 64 != 0) return 0;
     size_t room = 0;
-    if (R <= FEW_ROWS_MAX && tuning(TUNE_NO_WIDE) < 2) {
+    if (needs_admission(R, call)) {
         bool admitted = false;
         for (const int64_t group_units : {1, 2, 3, 4, 6, 8, 16, 0x7FFFFFF}) {
             const RoundedLine line = rounded_line(sparse, R, K, S, group_units);
@@ -736,10 +737,11 @@ static bool launch_wide(const SkinnyArgs& a, const WidePlan& p, hipStream_t st) 
     return true;
 }
 
-bool wide_rows(int bits, const SkinnyArgs& args, void* workspace, size_t workspace_bytes, hipStream_t st) {
+bool wide_rows(int bits, const SkinnyArgs& args, RowsCall call, void* workspace, size_t workspace_bytes, hipStream_t st) {
     const bool sparse = args.mask != nullptr;
     const WorkspaceParts ws = workspace_parts(workspace, workspace_bytes);
-    if (args.R <= FEW_ROWS_MAX && tuning(TUNE_NO_WIDE) < 2) {
+    if (call == EXACT_SUMS) return false;
+    if (needs_admission(args.R, call)) {
         const RoundedLine line = rounded_line(sparse, args.R, args.K, args.S, args.group_units);
         if (!line.admitted || ws.scratch_bytes < line.room) return false;
     }

@@ -126,6 +126,26 @@ def test_few_rows_keep_the_sums_of_exact_codes(product, bits, sparse, rows, k, s
         assert d("mtx", bits, 1, rows, k, s, g, sparse).startswith("wide_rows_kernel")
 
 
+# ---- the matvec entry with more batch elements than the few-row kernel takes at once: the kernel with rounded weights where it is
+# admitted, else shares of at most 96 elements with sums of exact codes; never a launch per element
+@pytest.mark.parametrize("bits,sparse,batch,k,s", [(4, False, 256, 5120, 20480), (4, False, 256, 8192, 28672), (4, False, 300, 4096, 11008),
+                                                   (4, False, 512, 4096, 14336), (4, True, 133, 4096, 11008), (4, True, 100, 2048, 20480),
+                                                   (4, False, 385, 5120, 20480), (4, False, 1000, 5120, 20480), (3, False, 481, 4096, 11008),
+                                                   (4, True, 257, 8192, 28672), (2, False, 330, 4096, 11008), (3, False, 97, 4096, 576)])
+def test_many_batch_elements_keep_the_sums_of_exact_codes(bits, sparse, batch, k, s):
+    line = d("vec", bits, batch, 1, k, s, 64 if sparse else 128, sparse)
+    assert line.startswith("skinny_kernel") and "row_tiles=4>" in line and "wide_rows" not in line, line
+
+
+@pytest.mark.parametrize("bits,sparse", [(4, False), (3, False), (2, False), (4, True)])
+def test_many_batch_elements_never_run_one_by_one(bits, sparse):
+    for k, s in ((512, 256), (4096, 512), (2048, 1600), (4096, 11008), (5120, 20480), (8192, 28672), (2048, 40960)):
+        for batch in (5, 17, 96, 97, 128, 193, 320, 384, 385, 481, 512, 513, 777, 1000):
+            for ws in (None, capi.lib().int4mm_workspace_bytes(s)):
+                line = d("vec", bits, batch, 1, k, s, 64 if sparse else 128, sparse, ws)
+                assert line.startswith(("skinny_kernel", "wide_rows_kernel")), (batch, k, s, line)
+
+
 def evenly_shared(line):
     return "balanced" in line or "columns_per_lane=4+1" in line
 
