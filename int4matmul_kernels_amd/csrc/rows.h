@@ -140,6 +140,25 @@ __device__ __forceinline__ h16x8 exact_operand(uint32_t f, uint32_t m0, uint32_t
     return bitcast<h16x8>(r);
 }
 
+// The chunk's codes as they are or, TWO_MODES and a negative (or NaN) scale, as +-2^e: both exact in fp16
+template <int BITS, bool TWO_MODES>
+__device__ __forceinline__ h16x8 plain_operand(uint32_t f, uint32_t m0, uint32_t m1, uint32_t g0, uint32_t g1, h16 sc) {
+    const u32x4 h = bitcast<u32x4>(magic_operand<BITS>(f, m0, m1, g0, g1));
+    const bool expo = TWO_MODES && !(sc >= (h16)0.0f);
+    u32x4 r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t offs = SkFmt<BITS>::offs(e);                    // {2^a, 2^b} as halves
+        r[e] = as_u32(as_h2(h[e]) - as_h2(offs));
+        if constexpr (TWO_MODES) {
+            // the same offsets as integers, for the packed multiply: 2^(exponent field - 15)
+            const uint32_t ints = off2(1u << (((offs >> 10) & 31u) - 15u), 1u << (((offs >> 26) & 31u) - 15u));
+            r[e] = expo ? expo_operand<BITS>(h[e], ints) : r[e];
+        }
+    }
+    return bitcast<h16x8>(r);
+}
+
 // the kernel whose waves share the staged states (csrc/wide.hip): false when its plan does not take the product
 bool wide_rows(int bits, const SkinnyArgs& a, RowsCall call, void* workspace, size_t workspace_bytes, hipStream_t st);
 size_t wide_workspace_bytes(int64_t R, int64_t K, int64_t S, bool sparse, RowsCall call);

@@ -104,7 +104,13 @@ __device__ __forceinline__ BalancedShare balanced_share(int q, int r, uint32_t u
 // on one strip, and a strip that two workgroups share is summed through the hand-over below.
 // XC = 1: a fifth column per lane (CW = 4 only, dense formats): the workgroup's columns are four or five slivers of
 // 16, the lane's four adjacent columns in the first four and column j of the fifth (a.wide_wgs workgroups have one)
-template <int BITS, int CW, int RT, bool SPARSE, bool BAL = false, int XC = 0>
+// PLAIN: the operand is the codes themselves or, in exponent mode, their powers of two -- no offsets to be removed from the sums, no
+// weight that is rounded in a strip with a negative scale.  For the shares of a batch that would otherwise run one matvec per
+// element (17 rows and more, a batch that the kernel with rounded weights does not take) and lose nothing to it.  2-norm of the error
+// against float64 (1e-4), one matvec per element / shares with offsets and rounded weights / PLAIN, 110 ... 180 elements, S=1088: int3, K=4096, one
+// group 2.07 / 2.13 / 2.06; int2, K=8192, g=128 2.11 / 2.16 / 2.08; one (group, column) in 40 in exponent mode, K=4096: int4, g=128 2.07 / 3.25 /
+// 2.07 (1615 / 32 / 29 us), 16:32 2.06 / 3.24 / 2.06 (1102 / 45 / 32)
+template <int BITS, int CW, int RT, bool SPARSE, bool BAL = false, int XC = 0, bool PLAIN = false>
 __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix, const h16* pre_x, const h16* pre_scales, const h16* pre_zeros,
                                                    int pre_S, int pre_K, int pre_group_units, int pre_units, uint32_t pre_rows,
                                                    uint32_t pre_more, SkinnyArgs a) {
@@ -327,7 +333,7 @@ __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix,
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         sx = dot2(q[e], ONES, sx);
-                        so = dot2(q[e], F::offs(e), so);
+                        if constexpr (!PLAIN) so = dot2(q[e], F::offs(e), so);
                     }
                 }
                 *reinterpret_cast<u32x4*>(my + p * SK_XBUF + xm * SK_PITCH + (xpart * RT + i) * 16) = q;
@@ -406,7 +412,7 @@ __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix,
                         // skip of 64 bits only happens when no row of the chunk is kept)
                         const uint32_t v = (uint32_t)(st >> ((uint32_t)__builtin_popcount(m & below) << 2));
                         const uint32_t mb4 = __builtin_amdgcn_perm(m, m, rep_h);           // mask byte h, four times
-                        if constexpr (general) {
+                        if constexpr (general && !PLAIN) {
                             const h16x8 wb = exact_operand_sparse(v, mb4 & 0xFFu, sc[c], ze[c]);
 #pragma unroll
                             for (int mt = 0; mt < MT; ++mt)
@@ -414,8 +420,16 @@ __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix,
                         } else {
                             // (table entries sit under the nibble-swapped byte = bits 4 .. 11 of mb4)
                             const u32x4 sel = *reinterpret_cast<const u32x4*>(lut + (mb4 & sp_idx));
-                            const u32x4 b = sparse_operand(v, sel, sp_nib, sp_flag);
+                            u32x4 b = sparse_operand(v, sel, sp_nib, sp_flag);
                             const u32x4 bm = u32x4{b.x & sp_kept, b.y & sp_kept, b.z & sp_kept, b.w & sp_kept};
+                            if constexpr (general) {        // q 2^-24, or +-2^e, of the kept rows
+                                const bool expo = !(sc[c] >= (h16)0.0f);
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) {
+                                    const uint32_t power = ((b[e] & 0x00080008u) << 12) | (((b[e] & 0x00070007u) << 10) + 0x3C003C00u);
+                                    b[e] = expo ? power & ((bm[e] << 12) - (bm[e] >> 4)) : b[e] & 0x000F000Fu;
+                                }
+                            }
 #pragma unroll
                             for (int mt = 0; mt < MT; ++mt) {
                                 acc[c][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[mt], bitcast<h16x8>(b), acc[c][mt], 0, 0, 0);
@@ -424,8 +438,10 @@ __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix,
                         }
                     } else {
                         const uint32_t f = chunk_bits(w, wx, i, c);
-                        const h16x8 wb = general ? exact_operand<BITS>(f, m0, m1, g0, g1, sc[c], ze[c])
-                                                 : magic_operand<BITS>(f, m0, m1, g0, g1);
+                        h16x8 wb;
+                        if constexpr (PLAIN) wb = plain_operand<BITS, general>(f, m0, m1, g0, g1, sc[c]);
+                        else if constexpr (general) wb = exact_operand<BITS>(f, m0, m1, g0, g1, sc[c], ze[c]);
+                        else wb = magic_operand<BITS>(f, m0, m1, g0, g1);
 #pragma unroll
                         for (int mt = 0; mt < MT; ++mt)
                             acc[c][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[mt], wb, acc[c][mt], 0, 0, 0);
@@ -438,13 +454,18 @@ __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix,
             load_x(xn, min(u + 1 + PFX, u1 - 1));
             // group complete (or this wave's range ends): fold it into y
             if ((u + 1) % a.group_units == 0 || u + 1 == u1) {
-                if constexpr (SPARSE && !general) {
-                    load_sz(u / a.group_units);
+                if constexpr (SPARSE && (PLAIN || !general)) {
+                    if constexpr (!general) load_sz(u / a.group_units);
 #pragma unroll
                     for (int c = 0; c < CW; ++c) {
                         // y += s (A - z M) with A = 2^24 (acc - accm), M = 2^20 accm
-                        const float ka = (float)sc[c] * 16777216.f;
-                        const float km = -(ka + (float)sc[c] * (float)ze[c] * 1048576.f);
+                        float ka = (float)sc[c] * 16777216.f;
+                        float km = -(ka + (float)sc[c] * (float)ze[c] * 1048576.f);
+                        if constexpr (general) {            // A = 2^24 acc, or z M - s acc
+                            const bool expo = !(sc[c] >= (h16)0.0f);
+                            km = (expo ? 1048576.f : (float)sc[c] * -1048576.f) * (float)ze[c];
+                            ka = expo ? -(float)sc[c] : ka;
+                        }
 #pragma unroll
                         for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
@@ -463,12 +484,19 @@ __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix,
                     const f32x4 o4 = *reinterpret_cast<const f32x4*>(&sums[32 + 16 * mt + 4 * h]);
 #pragma unroll
                     for (int c = 0; c < CT; ++c) {
-                        const float sf = general ? 1.f : (float)sc[c];
-                        const float z = general ? 0.f : (float)ze[c];
+                        if constexpr (general && PLAIN) {   // y += s (acc - z X), or z X - s acc
+                            const bool expo = !(sc[c] >= (h16)0.0f);
+                            const float ka = expo ? -(float)sc[c] : (float)sc[c], kx = (expo ? 1.f : -(float)sc[c]) * (float)ze[c];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const float off = general ? 0.f : o4[e] + z * s4[e];
-                            y[c][mt][e] += sf * (acc[c][mt][e] - off);
+                            for (int e = 0; e < 4; ++e) y[c][mt][e] = __builtin_fmaf(ka, acc[c][mt][e], __builtin_fmaf(kx, s4[e], y[c][mt][e]));
+                        } else {
+                            const float sf = general ? 1.f : (float)sc[c];
+                            const float z = general ? 0.f : (float)ze[c];
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                const float off = general ? 0.f : PLAIN ? z * s4[e] : o4[e] + z * s4[e];
+                                y[c][mt][e] += sf * (acc[c][mt][e] - off);
+                            }
                         }
                         acc[c][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
                     }
@@ -615,7 +643,7 @@ __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix,
 }
 
 template <int BITS, int CW, bool SPARSE>
-static bool launch_skinny(const SkinnyArgs& a, int waves, int ksplit, hipStream_t st) {
+static bool launch_skinny(const SkinnyArgs& a, int waves, int ksplit, bool plain, hipStream_t st) {
     const int strips = a.S / (16 * CW);
     const int rt = ((a.R > 32 ? 32 : a.R) + 7) / 8;
     int groups = (a.K / 64 + a.group_units - 1) / a.group_units;
@@ -625,12 +653,13 @@ static bool launch_skinny(const SkinnyArgs& a, int waves, int ksplit, hipStream_
     if (red > lds) lds = red;
     if (lds > 150 * 1024 - (SPARSE ? 4096 : 0)) return false;      // (16:32: 4 KB of static LDS for the selector table)
     const dim3 grid(strips, (a.R + 31) / 32, ksplit), block(waves * 64);
-    if (noting("skinny_kernel<bits=%d,%s,columns_per_lane=%d,row_tiles=%d> strips=%d row_blocks=%u ksplit=%d waves=%d", BITS,
-               SPARSE ? "16:32" : "dense", CW, rt <= 1 ? 1 : (rt <= 2 ? 2 : 4), strips, grid.y, ksplit, waves))
+    plain = plain && rt > 2;
+    if (noting("skinny_kernel<bits=%d,%s,columns_per_lane=%d,row_tiles=%d%s> strips=%d row_blocks=%u ksplit=%d waves=%d", BITS,
+               SPARSE ? "16:32" : "dense", CW, rt <= 1 ? 1 : (rt <= 2 ? 2 : 4), plain ? ",plain" : "", strips, grid.y, ksplit, waves))
         return true;
     auto go = [&](auto kernel, int slot) {
         // more than 64 KB of dynamic LDS has to be requested once per kernel and device
-        static std::atomic<uint64_t> done[3];
+        static std::atomic<uint64_t> done[4];
         int dev = 0;
         hipGetDevice(&dev);
         const uint64_t bit = 1ull << (dev & 63);
@@ -642,6 +671,9 @@ static bool launch_skinny(const SkinnyArgs& a, int waves, int ksplit, hipStream_
         hipLaunchKernelGGL(kernel, grid, block, lds, st, a.matrix, a.x, a.scales, a.zeros, a.S, a.K, a.group_units, a.units_per_wave, (uint32_t)a.R | (uint32_t)waves << 16,
                            (uint32_t)a.units_per_split, a);
     };
+    if constexpr (!(SPARSE && CW == 4)) {                           // (which up to 16 rows have alone)
+        if (plain) { go(skinny_kernel<BITS, CW, 4, SPARSE, false, 0, true>, 3); return true; }
+    }
     if (rt <= 1) go(skinny_kernel<BITS, CW, 1, SPARSE>, 0);
     else if (rt <= 2) go(skinny_kernel<BITS, CW, 2, SPARSE>, 1);
     else go(skinny_kernel<BITS, CW, 4, SPARSE>, 2);
@@ -746,10 +778,10 @@ static bool launch_skinny_slivers(SkinnyArgs a, hipStream_t st) {
 }
 
 template <int BITS, bool SPARSE = false>
-static bool launch_skinny_cw(const SkinnyArgs& a, int cw, int waves, int ksplit, hipStream_t st) {
-    if (cw == 4) return launch_skinny<BITS, 4, SPARSE>(a, waves, ksplit, st);
-    if (cw == 2) return launch_skinny<BITS, 2, SPARSE>(a, waves, ksplit, st);
-    return launch_skinny<BITS, 1, SPARSE>(a, waves, ksplit, st);
+static bool launch_skinny_cw(const SkinnyArgs& a, int cw, int waves, int ksplit, bool plain, hipStream_t st) {
+    if (cw == 4) return launch_skinny<BITS, 4, SPARSE>(a, waves, ksplit, plain, st);
+    if (cw == 2) return launch_skinny<BITS, 2, SPARSE>(a, waves, ksplit, plain, st);
+    return launch_skinny<BITS, 1, SPARSE>(a, waves, ksplit, plain, st);
 }
 
 // Columns per lane of the unsplit kernel: the widest strips (64, 32 or 16 columns) that still give at
@@ -849,10 +881,10 @@ bool skinny_rows(int bits, h16* outs, const uint32_t* matrix, const h16* x, cons
     while (waves > 1 && units < 2 * waves) waves >>= 1;
     auto launch = [&](int cw_, int waves_, int ksplit_) {
         a.units_per_wave = (a.units_per_split + waves_ - 1) / waves_;
-        if (sparse_mask) return launch_skinny_cw<4, true>(a, cw_, waves_, ksplit_, st);
-        if (bits == 4) return launch_skinny_cw<4>(a, cw_, waves_, ksplit_, st);
-        if (bits == 3) return launch_skinny_cw<3>(a, cw_, waves_, ksplit_, st);
-        return launch_skinny_cw<2>(a, cw_, waves_, ksplit_, st);
+        if (sparse_mask) return launch_skinny_cw<4, true>(a, cw_, waves_, ksplit_, call == EXACT_SUMS, st);
+        if (bits == 4) return launch_skinny_cw<4>(a, cw_, waves_, ksplit_, call == EXACT_SUMS, st);
+        if (bits == 3) return launch_skinny_cw<3>(a, cw_, waves_, ksplit_, call == EXACT_SUMS, st);
+        return launch_skinny_cw<2>(a, cw_, waves_, ksplit_, call == EXACT_SUMS, st);
     };
     // split-K across workgroups where the plan asks for it and the scratch half of the workspace has room
     // for the partial tiles (per-strip counters: last page of the half that is kept zero)

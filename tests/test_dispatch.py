@@ -134,7 +134,7 @@ def test_few_rows_keep_the_sums_of_exact_codes(product, bits, sparse, rows, k, s
                                                    (4, True, 257, 8192, 28672), (2, False, 330, 4096, 11008), (3, False, 97, 4096, 576)])
 def test_many_batch_elements_keep_the_sums_of_exact_codes(bits, sparse, batch, k, s):
     line = d("vec", bits, batch, 1, k, s, 64 if sparse else 128, sparse)
-    assert line.startswith("skinny_kernel") and "row_tiles=4>" in line and "wide_rows" not in line, line
+    assert line.startswith("skinny_kernel") and "row_tiles=4,plain>" in line and "wide_rows" not in line, line
 
 
 @pytest.mark.parametrize("bits,sparse", [(4, False), (3, False), (2, False), (4, True)])
