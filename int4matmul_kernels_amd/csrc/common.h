@@ -162,8 +162,8 @@ inline int64_t exact_sums_at_once(int64_t left, int64_t S) {
     const int64_t chunks = (left + FEW_ROWS_MAX - 1) / FEW_ROWS_MAX;
     return (left + chunks - 1) / chunks;
 }
-// bytes of partial tiles with which such a product splits K across workgroups (0: no split)
-size_t skinny_workspace_bytes(int64_t R, int64_t K, int64_t S, bool sparse, RowsCall call);
+// bytes of partial tiles with which such a product splits K across workgroups (0: no split); bits = 0, group_units = 0: not known
+size_t skinny_workspace_bytes(int bits, int64_t R, int64_t K, int64_t S, bool sparse, int64_t group_units, RowsCall call);
 
 // Layout of a caller's workspace, a function of its size alone so that calls with different shapes may
 // share one buffer.  The lower half (down to a page boundary) is kept zero between calls: the matvec's

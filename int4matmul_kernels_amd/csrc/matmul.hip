@@ -1326,17 +1326,21 @@ extern "C" size_t int4mm_matmul_workspace_bytes(const int4mm_shape* shape, int s
     size_t need = int4mm_workspace_bytes(S);
     if (B <= 0 || M <= 0 || K < 64 || S < 128) return need;
     if (B > 1 && B * M <= ((int64_t)1 << 31) - 256) { M *= B; B = 1; }           // (as int4mm_matmul does)
-    size_t few_rows = B * M <= SK_WIDE_MAX_ROWS ? skinny_workspace_bytes(B * M, K, S, sparse != 0, FOR_MATMUL) : 0;
+    // (a caller who asks with the sizes alone leaves matrix_rows or group_size 0)
+    int bits = 0;
+    for (const int b : {4, 3, 2})
+        if (shape->matrix_rows * 32 == K * b) bits = b;
+    const int64_t g = shape->group_size, group_units = g < 0 ? ONE_GROUP / 64 : g / 64;
+    auto few = [&](int64_t rows, RowsCall call) { return skinny_workspace_bytes(bits, rows, K, S, sparse != 0, group_units, call); };
+    size_t few_rows = B * M <= SK_WIDE_MAX_ROWS ? few(B * M, FOR_MATMUL) : 0;
     // (the matvec entry takes many batch elements of one row in chunks through the few-row kernels: as many as the kernel
     // for more rows takes, else even shares, which may be one fewer towards the end)
-    if (shape->seq_len == 1)
+    if (shape->seq_len == 1 && B * M > FEW_ROWS_MAX)
         for (const int64_t n : {std::min<int64_t>(B * M, SK_WIDE_MAX_ROWS), B * M % SK_WIDE_MAX_ROWS}) {
             if (n < 2) continue;
-            few_rows = std::max(few_rows, skinny_workspace_bytes(n, K, S, sparse != 0, FOR_MATVEC));
+            few_rows = std::max(few_rows, few(n, FOR_MATVEC));
             for (const int64_t share : {exact_sums_at_once(n, S), exact_sums_at_once(B * M, S)})
-                if (n > FEW_ROWS_MAX && share > 2)
-                    few_rows = std::max({few_rows, skinny_workspace_bytes(share, K, S, sparse != 0, EXACT_SUMS),
-                                         skinny_workspace_bytes(share - 1, K, S, sparse != 0, EXACT_SUMS)});
+                if (n > FEW_ROWS_MAX && share > 2) few_rows = std::max({few_rows, few(share, EXACT_SUMS), few(share - 1, EXACT_SUMS)});
         }
     if (B * M <= FEW_ROWS_MAX) return need + 2 * round_to_page(few_rows);
     const SplitPlan sp = plan_split(sparse != 0, B, M, K, S);

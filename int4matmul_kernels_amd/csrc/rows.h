@@ -161,6 +161,6 @@ __device__ __forceinline__ h16x8 plain_operand(uint32_t f, uint32_t m0, uint32_t
 
 // the kernel whose waves share the staged states (csrc/wide.hip): false when its plan does not take the product
 bool wide_rows(int bits, const SkinnyArgs& a, RowsCall call, void* workspace, size_t workspace_bytes, hipStream_t st);
-size_t wide_workspace_bytes(int64_t R, int64_t K, int64_t S, bool sparse, RowsCall call);
+size_t wide_workspace_bytes(int bits, int64_t R, int64_t K, int64_t S, bool sparse, int64_t group_units, RowsCall call);
 
 }  // namespace i4

@@ -837,9 +837,9 @@ static SkinnySplit plan_skinny_split(int64_t R, int64_t K, int64_t S, bool spars
     return p;
 }
 
-size_t skinny_workspace_bytes(int64_t R, int64_t K, int64_t S, bool sparse, RowsCall call) {
+size_t skinny_workspace_bytes(int bits, int64_t R, int64_t K, int64_t S, bool sparse, int64_t group_units, RowsCall call) {
     const SkinnySplit p = plan_skinny_split(R, K, S, sparse);
-    const size_t wide = wide_workspace_bytes(R, K, S, sparse, call);
+    const size_t wide = wide_workspace_bytes(bits, R, K, S, sparse, group_units, call);
     const size_t balanced = balanced_shape(R, K, S) ? skinny_balanced_part_bytes(S) : 0;
     return std::max(std::max<size_t>(p.ksplit > 1 ? p.part_bytes : 0, wide), balanced);
 }

@@ -683,23 +683,27 @@ static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S
     return p;
 }
 
-// An upper bound of any plan's partial tiles, cheap enough for every call: at most 512 workgroups of 32 KB per 32 rows, and
-// no more than the split's limit (16 ways, four units each) of the rows rounded up to whole blocks.
-size_t wide_workspace_bytes(int64_t R, int64_t K, int64_t S, bool sparse, RowsCall call) {
+// What the plan's partial tiles take with room for any split and, where a product has to be admitted, the room that it takes to be;
+// bits = 0, group_units = 0: not known, the most of any
+size_t wide_workspace_bytes(int bits, int64_t R, int64_t K, int64_t S, bool sparse, int64_t group_units, RowsCall call) {
     if (call == EXACT_SUMS || R < 2 || R > SK_WIDE_MAX_ROWS || !wide_columns(R, S) || K % 64 != 0) return 0;
-    size_t room = 0;
+    size_t need = 0;
     if (needs_admission(R, call)) {
         bool admitted = false;
-        for (const int64_t group_units : {1, 2, 3, 4, 6, 8, 16, 0x7FFFFFF}) {
-            const RoundedLine line = rounded_line(sparse, R, K, S, group_units);
+        for (const int64_t units : {1, 2, 3, 4, 6, 8, 16, 0x7FFFFFF}) {
+            const RoundedLine line = rounded_line(sparse, R, K, S, group_units > 0 ? group_units : units);
             admitted = admitted || line.admitted;
-            room = std::max(room, line.room);
+            need = std::max(need, line.room);
+            if (group_units > 0) break;
         }
         if (!admitted) return 0;
     }
-    const int64_t ways = std::min<int64_t>(16, K / 256), mt = std::min<int64_t>(4, (R + 31) / 32);
-    if (ways < 2) return room;
-    return std::max(room, (size_t)std::min<int64_t>(WIDE_MAX_SPLIT_WGS * mt * 32768, ways * ((R + 32 * mt - 1) / 32 * 32) * ((S + 255) / 256 * 256) * 4));
+    for (const int b : {4, 3, 2}) {
+        if (sparse ? b != 4 : bits != 0 && b != bits) continue;
+        const WidePlan p = plan_wide(b, sparse, R, K, S, SIZE_MAX);
+        if (p.use) need = std::max(need, p.part_bytes);
+    }
+    return need;
 }
 
 template <int BITS, int MT, bool SPARSE, int WN>

@@ -184,6 +184,25 @@ def test_workspace_sizes_are_consistent():
                     assert capi.matmul_workspace_bytes(1, rows, k, s, sparse) >= n
 
 
+@pytest.mark.parametrize("s", [192, 512, 1600, 4096, 8192, 11008, 14400, 28672])
+def test_the_workspace_asked_for_is_all_that_a_product_uses(s):
+    # the launch with it is the launch with any amount more, whether the query knew the format and the group or only the sizes; and
+    # an unsplit product does not ask for partial tiles
+    for k in (512, 1088, 4096, 8192, 12352):
+        for rows in (2, 8, 17, 33, 60, 72, 96, 97, 128, 200, 256, 300, 384, 512, 600, 1000):
+            for bits, sparse, g in ((4, False, 128), (3, False, -1), (2, False, 64), (4, True, 64)):
+                for product, shape in (("mtx", (1, rows)), ("vec", (rows, 1))):
+                    plenty = d(product, bits, *shape, k, s, g, sparse, 1 << 34)
+                    assert d(product, bits, *shape, k, s, g, sparse) == plenty, (rows, k, s)
+                    nbytes = capi.matmul_workspace_bytes(*shape, k, s, sparse)
+                    assert d(product, bits, *shape, k, s, g, sparse, nbytes) == plenty, (rows, k, s)
+    # (K = 8192, S = 28672: 200 and 512 rows asked for 134 MB and used nothing of it)
+    if s == 28672:
+        for rows in (200, 512):
+            assert "ksplit=1" in d("mtx", 4, 1, rows, 8192, s, 128)
+            assert capi.matmul_workspace_bytes(1, rows, 8192, s) == capi.lib().int4mm_workspace_bytes(s)
+
+
 def test_matvec_of_a_k_beyond_one_launch():
     # 32 x 224 units of 64 rows is what one launch covers: a longer K runs as several launches (one line each)
     line = d("vec", 4, 1, 1, 1 << 20, 256, 128)
