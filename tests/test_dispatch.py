@@ -184,7 +184,7 @@ def test_workspace_sizes_are_consistent():
                     assert capi.matmul_workspace_bytes(1, rows, k, s, sparse) >= n
 
 
-@pytest.mark.parametrize("s", [192, 512, 1600, 4096, 8192, 11008, 14400, 28672])
+@pytest.mark.parametrize("s", [64, 192, 512, 1600, 4096, 8192, 11008, 14400, 28672])
 def test_the_workspace_asked_for_is_all_that_a_product_uses(s):
     # the launch with it is the launch with any amount more, whether the query knew the format and the group or only the sizes; and
     # an unsplit product does not ask for partial tiles
@@ -196,6 +196,8 @@ def test_the_workspace_asked_for_is_all_that_a_product_uses(s):
                     assert d(product, bits, *shape, k, s, g, sparse) == plenty, (rows, k, s)
                     nbytes = capi.matmul_workspace_bytes(*shape, k, s, sparse)
                     assert d(product, bits, *shape, k, s, g, sparse, nbytes) == plenty, (rows, k, s)
+    if s == 64:                                            # (one strip: K is all that there is to share out)
+        assert "ksplit=16" in d("mtx", 4, 1, 300, 18048, 64, 128) and "ksplit=5" in d("mtx", 4, 1, 44, 17728, 64, 128)
     # (K = 8192, S = 28672: 200 and 512 rows asked for 134 MB and used nothing of it)
     if s == 28672:
         for rows in (200, 512):

@@ -802,3 +802,17 @@ def test_matvec_many_batch_elements_as_exact_as_one(H, bits, sparse, B, K, S, g,
         w *= H.t(p["keep"])
     want = (d["states"][:, 0].double() @ w).cpu().numpy() + prior[:, 0].astype(np.float64)
     assert np.linalg.norm(got[:, 0] - want) / np.linalg.norm(want) < 2.0 ** -11 / 3 ** 0.5 + 5e-6
+
+
+@pytest.mark.parametrize("bits,sparse", [(4, False), (3, False), (2, False), (4, True)])
+@pytest.mark.parametrize("M,K", [(8, 16384), (44, 17728), (130, 2048), (401, 12352)])
+def test_one_strip_of_64_columns_splits_k(H, bits, sparse, M, K):
+    S, g = 64, 64
+    line = H.capi.describe_launch("mtx", bits, 1, M, K, S, g, sparse)
+    assert " strips=" in line and "ksplit=1 " not in line, line
+    p = _problem(bits, K=K, S=S, M=M, group_size=g, sparse=sparse, seed=M)
+    d = H.dev_problem(p)
+    exact, f32 = H.oracles(p)
+    got = H.run_capi(p, d, "mtx", outs_init=np.full((1, M, S), np.nan, np.float16))
+    H.assert_product_close(got, exact, f32, kind=H.matmul_kind(p))
+    assert np.array_equal(got, H.run_capi(p, d, "mtx"))
