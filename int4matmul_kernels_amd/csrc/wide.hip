@@ -643,12 +643,10 @@ static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S
     // (32-bit byte offsets into buffer resources: a share of the packed matrix, its scales and the block's rows of states and
     // outputs stay below 2 GB)
     if (K * S >= (sparse ? 1ll << 33 : (1ll << 34) / bits) || K >= (1 << 22) || S >= (1 << 22)) return p;
-    const int64_t few = (R + 127) / 128, tallest = ((R + few - 1) / few + 31) / 32;
     double best = 1e30;
     for (const WideCost& c : wide_cost[sparse ? 3 : 4 - bits]) {
-        // (a block of rows that would hold no row more than the one below; up to 512 k, where the launch is all prologue, the
-        // fewest blocks)
-        if (32 * (c.mt - 1) >= R || (R > 64 && units <= 8 && c.mt != tallest)) continue;
+        // (a block of rows that would hold no row more than the one below)
+        if (32 * (c.mt - 1) >= R) continue;
         // (49 ... 64 rows on 2048 ... 4096 columns and a long K: two blocks of 32 rows)
         if (!sparse && R > 48 && R <= 64 && S > 2048 && S <= 4096 && K > 8192 && forced < 1 && (c.mt != 1 || c.wn != 4)) continue;
         const int64_t blocks = (R + 32 * c.mt - 1) / (32 * c.mt), tiles = wide_strips(S, c.wn) * blocks;
@@ -673,8 +671,9 @@ static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S
     p.ksplit = (int)((units + p.units_per_split - 1) / p.units_per_split);
     // 257 rows and more on a wide output that is not split: the 256-row tiles, where the model's time is beyond what they
     // take (5 us and 0.75 PFLOP/s while the blocks fit one round of workgroups, 1.05 beyond: K=8192, S=28672, 512 rows 245 here,
-    // 227 in tiles; int3, K=20480, S=11008 324 / 295; int4 K=8192, S=20480, 384 rows stays, 140 / 196)
-    if (knob < 2 && forced < 1 && R > 256 && S > 10240 && K > 1024 && p.ksplit == 1) {
+    // 227 in tiles; int3, K=20480, S=11008 324 / 295; int4 K=8192, S=20480, 384 rows stays, 140 / 196; int3, K=512, S=17664, 442
+    // rows 29 / 20; K=192, S=28416, 435 rows 22 / 14)
+    if (knob < 2 && forced < 1 && R > 256 && S > 10240 && p.ksplit == 1) {
         const double flops = 2.0 * ((R + 255) / 256 * 256) * K * S;
         if (best > 5.0 + flops / (wide_strips(S, p.wn) * p.row_blocks > 256 ? 1.05e9 : 0.75e9)) return p;
     }

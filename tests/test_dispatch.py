@@ -146,6 +146,15 @@ def test_many_batch_elements_never_run_one_by_one(bits, sparse):
                 assert line.startswith(("skinny_kernel", "wide_rows_kernel")), (batch, k, s, line)
 
 
+def test_many_rows_on_a_short_k_are_not_left_to_few_workgroups():
+    # outputs wide enough for the tile kernels go to them from 257 rows on; narrower ones get more than the fewest blocks of rows
+    for bits, rows, k, s in ((3, 442, 512, 17664), (4, 435, 192, 28416), (4, 494, 192, 12288), (4, 476, 64, 14848)):
+        assert d("mtx", bits, 1, rows, k, s, 128).startswith("matmul_kernel"), (rows, k, s)
+    for bits, rows, k, s in ((4, 469, 448, 1920), (4, 363, 448, 1536), (4, 117, 448, 2560), (2, 441, 320, 1536)):
+        name, f, line = fields(d("mtx", bits, 1, rows, k, s, 128))
+        assert name == "wide_rows_kernel" and f["strips"] * f["row_blocks"] >= 40, line
+
+
 def evenly_shared(line):
     return "balanced" in line or "columns_per_lane=4+1" in line
 
