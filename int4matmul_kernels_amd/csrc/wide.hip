@@ -304,7 +304,14 @@ __global__ __launch_bounds__(512, MT == 1 && !SPARSE && !(BITS == 4 && WN == 2) 
                 const uint32_t r0 = __builtin_amdgcn_perm(odd_, even, sel.x), r1 = __builtin_amdgcn_perm(odd_, even, sel.y);
                 b0 = r0 & 0x0F0F0F0Fu; b1 = r1 & 0x0F0F0F0Fu;
                 const uint32_t k0 = r0 & 0x10101010u, k1 = r1 & 0x10101010u;        // the byte 0x10 is 2^-5
-                if constexpr (gen) {
+                if constexpr (gen && MT < 4) {
+                    // (a byte's flag becomes the sign of byte 1 or 3, which selectors 8 ... 11 spread over whole bytes: K=S=8192, 45 rows,
+                    // one group in 40 in exponent mode 26.9 us with the form below, 25.9 so.  Blocks of 128 rows have no registers for
+                    // it: K=5120, S=20480, 128 rows 50.4 / 49.0, but 43.9 / 45.3 without such groups)
+                    auto mask = [](uint32_t r, uint32_t sel) { return as_h2(__builtin_amdgcn_perm(r << 3, r << 11, sel)); };
+                    kept[0] = mask(r0, 0x0A0A0808u); kept[1] = mask(r0, 0x0B0B0909u);
+                    kept[2] = mask(r1, 0x0A0A0808u); kept[3] = mask(r1, 0x0B0B0909u);
+                } else if constexpr (gen) {
                     const uint32_t f0 = (k0 << 4) - (k0 >> 4), f1 = (k1 << 4) - (k1 >> 4);        // 0x10 -> 0xFF, byte by byte
                     kept[0] = as_h2(__builtin_amdgcn_perm(f0, f0, 0x01010000u)); kept[1] = as_h2(__builtin_amdgcn_perm(f0, f0, 0x03030202u));
                     kept[2] = as_h2(__builtin_amdgcn_perm(f1, f1, 0x01010000u)); kept[3] = as_h2(__builtin_amdgcn_perm(f1, f1, 0x03030202u));
