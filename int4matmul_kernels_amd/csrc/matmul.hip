@@ -1337,7 +1337,7 @@ extern "C" size_t int4mm_matmul_workspace_bytes(const int4mm_shape* shape, int s
     // for more rows takes, else even shares, which may be one fewer towards the end; its callers may ask with the flattened
     // shape too)
     if (B * M > FEW_ROWS_MAX && (shape->seq_len == 1 || B * M <= SK_WIDE_MAX_ROWS))
-        for (const int64_t n : {std::min<int64_t>(B * M, SK_WIDE_MAX_ROWS), B * M % SK_WIDE_MAX_ROWS}) {
+        for (const int64_t n : {std::min<int64_t>(B * M, SK_WIDE_MAX_ROWS), B * M > SK_WIDE_MAX_ROWS ? B * M % SK_WIDE_MAX_ROWS : 0}) {
             if (n < 2) continue;
             few_rows = std::max(few_rows, few(n, FOR_MATVEC));
             for (const int64_t share : {exact_sums_at_once(n, S), exact_sums_at_once(B * M, S)})

@@ -563,23 +563,25 @@ struct RoundedLine { bool admitted; size_t room; };
 static RoundedLine rounded_line(bool sparse, int64_t R, int64_t K, int64_t S, int64_t group_units) {
     const RoundedLine none{false, 0};
     if (R < 17 || R > SK_WIDE_MAX_ROWS || S % 256 != 0) return none;
-    const int64_t units = K / 64, strips = S / 256, lds_limit = 150 * 1024 - (sparse ? 4096 : 0);
-    int64_t tiles = 0, blocks = 0, wgs = 0, ks = 1;         // row tiles of 16 in a block, blocks, unsplit workgroups, ways
-    auto fits = [&](int64_t share) {
-        int64_t groups = (units + group_units - 1) / group_units;
-        if (share < units) groups = std::min(groups, (share + group_units - 1) / group_units + 1);
-        return 16 * tiles * 288 + 1040 + groups * 1024 <= lds_limit;
-    };
-    auto shape = [&](int64_t tallest) {
-        blocks = (R + tallest - 1) / tallest;
-        tiles = ((R + blocks - 1) / blocks + 15) / 16;
+    // (32-bit: a query of the workspace comes here as well as a launch)
+    const int rows = (int)R, units = (int)(K / 64), strips = (int)(S / 256), lds_limit = 150 * 1024 - (sparse ? 4096 : 0);
+    const int gu = (int)std::min<int64_t>(group_units, units);
+    int tiles = 0, blocks = 0, wgs = 0, ks = 1;             // row tiles of 16 in a block, blocks, unsplit workgroups, ways
+    const int all_groups = (units + gu - 1) / gu;
+    int64_t most_units = 0;                                 // of a share whose groups -- one more may be cut -- fit
+    auto fits = [&](int share) { return share <= most_units; };
+    auto shape = [&](int tallest) {
+        blocks = (rows + tallest - 1) / tallest;
+        tiles = ((rows + blocks - 1) / blocks + 15) / 16;
         if (tiles == 5 || tiles == 7) ++tiles;
         wgs = strips * blocks;
+        const int most_groups = (lds_limit - 1040 - 16 * tiles * 288) / 1024;
+        most_units = all_groups <= most_groups ? units : (int64_t)(most_groups - 1) * gu;
     };
-    auto shape_and_split = [&](int64_t tallest) {
+    auto shape_and_split = [&](int tallest) {
         shape(tallest);
         ks = wgs > 128 && wgs < 256 ? 4 : 256 / wgs;
-        ks = wgs > 1024 ? 1 : std::max<int64_t>(1, std::min<int64_t>(ks, units / 8));
+        ks = wgs > 1024 ? 1 : std::max(1, std::min(ks, units / 8));
         while (wgs * (ks + 1) <= 256 && ks < units / 8 && !fits((units + ks - 1) / ks)) ++ks;
     };
     shape_and_split(128);
@@ -591,11 +593,11 @@ static RoundedLine rounded_line(bool sparse, int64_t R, int64_t K, int64_t S, in
                                       {{0, 0, 0, 1.12, 1.203, 0, 1.32, 0, 1.537}, 4.17, -3.744, 0.921, 1.701, 5.284}};
         const Cost& c = costs[sparse];
         double best = 1e30;
-        int64_t best_tallest = 0, best_ks = 1;
-        for (const int64_t tallest : {128, 96, 64, 48}) {
+        int best_tallest = 0, best_ks = 1;
+        for (const int tallest : {128, 96, 64, 48}) {
             shape(tallest);
-            for (int64_t k = 1; k <= 16 && (k == 1 || units / k >= 8) && wgs * k <= 1024; ++k) {
-                const int64_t share = (units + k - 1) / k, rounds = (wgs * k + 255) / 256, last = wgs * k - (rounds - 1) * 256;
+            for (int k = 1; k <= 16 && (k == 1 || units >= 8 * k) && wgs * k <= 1024; ++k) {
+                const int share = (units + k - 1) / k, rounds = (wgs * k + 255) >> 8, last = wgs * k - (rounds - 1) * 256;
                 if (!fits(share)) continue;
                 const double t = rounds * (c.unit[tiles] * share + c.workgroup) + (k > 1 ? c.split + c.way * k + c.tile * tiles : 0.0) +
                                  (rounds > 1 ? c.last * last / 256.0 : 0.0);
@@ -605,7 +607,7 @@ static RoundedLine rounded_line(bool sparse, int64_t R, int64_t K, int64_t S, in
         if (best_tallest != 0) { shape(best_tallest); ks = best_ks; }
         else shape_and_split(48);
     }
-    const int64_t share = (units + ks - 1) / ks;
+    const int share = (units + ks - 1) / ks;
     ks = (units + share - 1) / share;
     if (!fits(share)) return none;
     // one round of two row blocks of the few-row kernel, or that kernel's own split of K
@@ -630,7 +632,7 @@ static RoundedLine rounded_line(bool sparse, int64_t R, int64_t K, int64_t S, in
                 : S > 8192 && S > (R <= 192 || (R <= 256 && K <= 4096) ? 32768 : R <= 256 ? 10240 : 8192);
     }
     if (few_row) return none;
-    return {true, ks > 1 ? (size_t)(wgs * ks * tiles * 16384) : 0};
+    return {true, ks > 1 ? (size_t)wgs * ks * tiles * 16384 : 0};
 }
 
 static bool needs_admission(int64_t R, RowsCall call) { return (R <= FEW_ROWS_MAX || call == FOR_MATVEC) && tuning(TUNE_NO_WIDE) < 2; }
