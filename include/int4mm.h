@@ -33,17 +33,24 @@
  *   multiplier, outs        : fp16 [B, M, K] and [B, M, S], contiguous.
  *
  * Numerics of the products.  "Bit-exact" above is about the formats and the helpers
- * (pack, unpack, dequantize).  int4mm_matmul with 17 or more rows of states multiplies
- * exactly those fp16 weights and accumulates in fp32.  int4mm_matvec and the few-row
- * kernels behind both products (2..16 rows, and up to 96 on some shapes) do not round
- * per weight: they accumulate sum(x * q) and sum(x) in fp32 and apply scale and zero
- * once per group, y += s * (sum(x * q) - z * sum(x)), which is the exact value of
- * sum(x * (q - z) * s) up to fp32 rounding -- closer to the true product than the
- * reference's fp16(fp16(q - z) * s) weights, but not the same bits.  A single row through
+ * (pack, unpack, dequantize).  Two classes of sums, both accumulated in fp32:
+ *  - rounded weights: exactly those fp16 weights are multiplied (error against float64
+ *    about 3.2e-4 of the result, 2-norm).  int4mm_matmul with more than 96 rows of states,
+ *    and some products of 17..96 rows through either entry and of more batch entries through
+ *    int4mm_matvec, on outputs of whole 256 columns and with the workspace that
+ *    int4mm_matmul_workspace_bytes asks for;
+ *  - exact codes: sum(x * q) and sum(x) are accumulated and scale and zero applied
+ *    once per group, y += s * (sum(x * q) - z * sum(x)), the exact value of
+ *    sum(x * (q - z) * s) up to fp32 rounding (2.1e-4, the fp16 result's own) -- closer to the
+ *    true product than the reference's fp16(fp16(q - z) * s) weights, but not the same bits.
+ *    One row, 2..16 rows, and every other product of up to 96 rows or of int4mm_matvec.
+ *    (2..96 rows in one launch: columns that share a strip with a negative scale are of rounded weights.)
+ * int4mm_describe_launch names the kernel: wide_rows_kernel and matmul_kernel* round their
+ * weights, skinny_kernel and matvec_kernel sum exact codes.  A single row through
  * int4mm_matmul is served by the matvec kernel as well (overwriting outs, as the matmul
  * does): bit for bit int4mm_matvec's result on zeroed outs, as long as the workspace holds
  * the matvec's part (int4mm_workspace_bytes); without it a tile kernel takes the row.  Results are a
- * deterministic function of the inputs and the shape (no atomics on data).
+ * deterministic function of the inputs, the shape and the workspace's size (no atomics on data).
  */
 #ifndef INT4MM_H
 #define INT4MM_H
@@ -83,8 +90,8 @@ INT4MM_API int int4mm_abi_version(void);
  * heuristic for the calling host thread (value 0 restores the default).  key 0 = waves per
  * workgroup of the matvec and few-row kernels, 1 = matvec 64-row units per lane
  * group, 2 = matvec lane groups per wave / few-row kernel columns per lane (1, 2, 4), 3 = matmul kernel variant
- * (5 / 6 / 7 = pipelined 256x128 / 256x256 / 128x256 tiles, 9 = 256x256 without
- * the two-phase order; a forced variant also keeps the product away from the
+ * (1 / 3 = general 128x128 / 128x256 tiles, 5 / 6 / 7 / 8 = pipelined 256x128 / 256x256 / 128x256 /
+ * 192x256 tiles, 9 = 256x256 without the two-phase order; a forced variant also keeps the product away from the
  * few-row kernels), 4 = matvec: 1 disables prefetch,
  * 5 = 1 disables the few-row (2..512 rows) kernels, 6 = split-K factor of the
  * matmul and few-row kernels (1 = never split, 2..8 = that factor where the
@@ -154,9 +161,12 @@ INT4MM_API int int4mm_describe_launch(int product, int bits, const int4mm_shape*
  * over several workgroups per output tile (shapes with so few tiles that most of
  * the GPU would idle, or whose last round of tiles would leave half of it idle; `sparse` != 0 for the 16:32 format), or
  * a few-row product share its column strips out evenly over the workgroups (more strips than compute units) -- also
- * int4mm_matvec with 2 and more batch entries, which takes the few-row kernels (in chunks of up to 512); never less than
- * int4mm_workspace_bytes(shape->out_size).  A smaller workspace is not an error:
- * the product then runs unsplit.  Same zero-fill rule as above.  No counterpart in
+ * int4mm_matvec with 2 and more batch entries, which takes the few-row kernels (in chunks of up to 512 where weights rounded to
+ * fp16 may serve it, else of up to 96); never less than int4mm_workspace_bytes(shape->out_size).  It is what the launch uses, not a bound;
+ * matrix_rows and group_size may be 0 if not known (the most of any format and group then).  A smaller workspace is not an error:
+ * the product then runs with the splits that fit or unsplit, and one of up to 96 rows (int4mm_matvec: any batch) whose rounded
+ * weights would have needed the room with sums of exact codes.
+ * Same zero-fill rule as above.  No counterpart in
  * the reference, whose matmul (matmul_kernel.cu:375-459) uses no scratch. */
 INT4MM_API size_t int4mm_matmul_workspace_bytes(const int4mm_shape* shape, int sparse);
 
@@ -186,7 +196,8 @@ INT4MM_API int int4mm_matvec_overwrite(int bits, void* outs, const void* matrix,
  * that allows the same launch plan: always for one row of states; for several batch entries
  * when that workspace has int4mm_matmul_workspace_bytes() and the few-row kernels' partial
  * sums fit the array's scratch half (8.4 MB) -- a smaller workspace, or larger partials, makes
- * one of the two run unsplit, which changes the summation order, not the accuracy class.  The
+ * one of the two run with another split or, from 17 batch entries on, with sums of exact codes where the
+ * other rounds its weights.  The
  * hand-over slots and split-K partials live in a 16.8 MB device array built into the library (each GPU the library
  * runs on holds its copy until the process ends), which covers out_size <= 32768; a wider
  * product returns INT4MM_ERR_WORKSPACE.  The call allocates and frees nothing.  Its first

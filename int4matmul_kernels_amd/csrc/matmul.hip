@@ -1237,9 +1237,9 @@ static void launch(MatmulArgs a, int64_t B, hipStream_t st, void* workspace, siz
         a.part = reinterpret_cast<float*>(wsp.scratch);
     }
     // 192 x 256 tiles instead of whole 256 x 256 ones, where they take no more rounds of 256 workgroups and pad no more
-    // rows: a round of them costs five sixths to seven eighths (us, 256 / 192 rows: int3, K=4096, S=11008, 777 rows 104 / 97; int4,
-    // S=20480, 520 rows 132 / 103; 1152 rows -- two rounds both ways -- 227 / 205; K=S=8192, 1300 rows 216 / 192; 16:32,
-    // K=8192, S=20480, 520 rows 269 / 234; a round more loses up to a third: int3, K=4096, S=11008, 1152 rows 115 / 175).  A grid
+    // rows: a round of them costs five sixths to nine tenths (us, 256 / 192 rows, one run: int3, K=4096, S=11008, 777 rows 100 / 91;
+    // int4, S=20480, 520 rows 115 / 95; 1152 rows -- two rounds both ways -- 205 / 186; K=S=8192, 1300 rows 193 / 174; 16:32,
+    // K=8192, S=20480, 520 rows 247 / 210; a round more loses: int3, K=4096, S=11008, 1152 rows 110 / 172).  A grid
     // whose last round is split along K keeps the large tiles, 1 - 15 % faster.
     if (variant == 6 && tuning(TUNE_MM_VARIANT) == 0 && a.ksplit == 1) {
         const int64_t rows_192 = (a.M + 191) / 192, t256 = m_pad / 256 * ((a.S + 255) / 256) * B, t192 = rows_192 * ((a.S + 255) / 256) * B;

@@ -1,4 +1,5 @@
-// Products of 17 ... 512 rows, every format, S a multiple of 256 (more than 96 rows: of 64): wide_rows_kernel.  Every weight is dequantised once per
+// Products of 17 ... 512 rows, every format, S a multiple of 256 (more than 96 rows: of 64): wide_rows_kernel, for the products of the
+// matmul entry and, within a line of precision (rounded_line), for up to 96 rows and for the matvec entry's batches.  Every weight is dequantised once per
 // block of up to 128 rows, with the reference's own two roundings fp16(fp16(q - z) s) (matmul.cuh:115-125) or, in exponent
 // mode, its single-rounded fma (matmul.cuh:127-136), and multiplied on v_mfma_f32_32x32x16_f16 into accumulators that hold
 // the product itself.
@@ -10,9 +11,9 @@
 // through LDS and, where K is also split across workgroups (blockIdx.z), through the workspace: a workgroup stores its fp32
 // tile write-through, counts itself in, and the last to arrive adds the others' up in split order, its own from registers.
 //
-// What bounds it is the issue of vector instructions, at the 1.9 GHz that the power limit leaves (counters at 64 rows:
-// VALU 42 % of the SIMD's cycles over the whole launch, 73 % in the loop; MFMA 29 %): an instruction with three operands or
-// packed halves takes 4.3 cycles of a SIMD, a plain and / shift 2.4, an MFMA 8.6 of the same port.  Hence
+// What bounds it is the issue of vector instructions, at the 2 GHz that the power limit leaves, and beside the loop the first
+// loads and the hand-over (counters of a launch of 64 rows at K=5120, S=20480: VALU 36 % of the SIMDs' cycles, MFMA 26 %, no bank
+// conflicts; 16:32, 45 rows at K=S=8192: 44 % and 16 %; int2, 200 rows at K=11008, S=4096: 49 % and 33 %).  Hence
 //  * 32x32x16 MFMAs: half the instructions of 16x16x32 for the same product;
 //  * 64 columns per wave: a fragment of states that is read from LDS serves two operands;
 //  * int4 codes become halves through the 8-bit float conversion: the byte q < 16 is q 2^-9 in e4m3, so mask, shift, mask and
@@ -523,8 +524,9 @@ static constexpr size_t wide_lds_bytes(int mt, int wn) {
 //     + (ksplit > 1: split + way x ksplit)
 // with the steps of a workgroup (units of its share / K groups), fill = the share of the 256 CUs that get a workgroup and
 // rounds of 256 workgroups (two of the smallest ones share a CU: their second round is cheaper).  Fitted per format and kernel
-// to 930 ... 2440 timed launches each (K = 1024 ... 20480, S = 1024 ... 28672, 24 ... 512 rows, every candidate, cold weights): 3 ...
-// 5 % off, and its pick 0.2 ... 0.8 % off the best measured candidate on average, 12 - 20 % at worst.
+// to 930 ... 2440 timed launches each (K = 1024 ... 20480, S = 1024 ... 28672, 24 ... 512 rows, cold weights).  On 30 other random shapes
+// of that range per format its pick was the best measured candidate on half of them and 1.1 / 1.8 / 1.0 / 0 % off it on
+// average (int4, int3, int2, 16:32), 12 / 21 / 23 / 8 % at worst.
 struct WidePlan { bool use; int mt, wn, row_blocks, ksplit, units_per_split; size_t part_bytes; };
 struct WideCost { int mt, wn; double step, filled, more_step, workgroup, more_workgroup, split, way, last; };
 static const WideCost wide_cost[4][6] = {             // int4, int3, int2, 16:32
@@ -554,9 +556,9 @@ static const WideCost wide_cost[4][6] = {             // int4, int3, int2, 16:32
      {4, 4, 1.76, 0.352, 1.84, 7.15, 6.6, 2.45, 1.26, 5.45}}};
 constexpr int64_t WIDE_MAX_SPLIT_WGS = 512;              // workgroups of a launch that splits K (bounds its partial tiles)
 
-// Which products of up to 96 rows, and which of the matvec entry, may take the kernel above.  Elsewhere they are sums of the exact codes, scale and zero applied in
-// fp32; here each weight is rounded to fp16 twice (error against float64, 2-norm: 2.1e-4 of the result there, 3.2e-4 here).
-// Hence this is a line of precision and not of speed, and is not to be fitted to timings: it admits what an earlier form of
+// Which products of up to 96 rows, and which of the matvec entry, may take the kernel above.  Elsewhere they are sums of the
+// exact codes, scale and zero applied in fp32; here each weight is rounded to fp16 twice (error against float64, 2-norm, 90
+// rows at K=5120, S=2560: 2.07e-4 of the result there -- all of it the fp16 output's --, 3.23e-4 here).  Hence this is a line of precision and not of speed, and is not to be fitted to timings: it admits what an earlier form of
 // the kernel took -- with its split of K, if its partial tiles have `room` in the workspace and a share's scales have room in the
 // LDS, as that form kept them there -- so that no product that had the exact codes' sums loses them.
 struct RoundedLine { bool admitted; size_t room; };

@@ -105,7 +105,7 @@ TOL_MEAN = 0.1
 
 def matmul_kind(p):
     """tolerance class of a matmul call: "mtx" when a kernel that dequantises its weights (tile
-    kernels, the 17 .. 256 row kernel) serves the shape, "vec" when the 2 .. 96 row kernel does,
+    kernels, the 17 .. 512 row kernel) serves the shape, "vec" when the 2 .. 96 row kernel does,
     which -- like the matvec -- applies scale and zero per group in fp32"""
     line = capi.describe_launch("mtx", p["bits"], p["B"], p["M"], p["K"], p["S"], p["group_size"], p["sparse_mask"] is not None)
     return "vec" if line.startswith("skinny_kernel") or p["B"] * p["M"] == 1 else "mtx"
