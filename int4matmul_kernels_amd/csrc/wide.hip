@@ -657,9 +657,9 @@ static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S
     const int64_t few = (R + 127) / 128, tallest = ((R + few - 1) / few + 31) / 32;
     double best = 1e30;
     for (const WideCost& c : wide_cost[sparse ? 3 : 4 - bits]) {
-        // (a block of rows that would hold no row more than the one below; up to K = 512 below 1024 columns, where nothing
-        // was fitted either, the fewest blocks)
-        if (32 * (c.mt - 1) >= R || (R > 64 && units <= 8 && S < 1024 && c.mt != tallest)) continue;
+        // (a block of rows that would hold no row more than the one below; 65 ... 256 rows up to K = 512 and 1024 columns keep the
+        // fewest blocks, through which the tests of tall blocks go: K=S=512, 100 rows 12.0 us, 10.1 by the model's choice)
+        if (32 * (c.mt - 1) >= R || (R > 64 && R <= 256 && units <= 8 && S <= 1024 && c.mt != tallest)) continue;
         // (49 ... 64 rows on 2048 ... 4096 columns and a long K: two blocks of 32 rows)
         if (!sparse && R > 48 && R <= 64 && S > 2048 && S <= 4096 && K > 8192 && forced < 1 && (c.mt != 1 || c.wn != 4)) continue;
         const int64_t blocks = (R + 32 * c.mt - 1) / (32 * c.mt), tiles = wide_strips(S, c.wn) * blocks;
