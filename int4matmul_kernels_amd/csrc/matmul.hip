@@ -1324,7 +1324,8 @@ extern "C" size_t int4mm_matmul_workspace_bytes(const int4mm_shape* shape, int s
     int64_t B = shape->batch, M = shape->seq_len;
     const int64_t K = shape->in_size, S = shape->out_size;
     size_t need = int4mm_workspace_bytes(S);
-    if (B <= 0 || M <= 0 || K < 64 || S < 64) return need;
+    // (below 128 columns two to four rows keep the launches that they have with the matvec's workspace)
+    if (B <= 0 || M <= 0 || K < 64 || S < (B * M < 5 ? 128 : 64)) return need;
     if (B > 1 && B * M <= ((int64_t)1 << 31) - 256) { M *= B; B = 1; }           // (as int4mm_matmul does)
     // (a caller who asks with the sizes alone leaves matrix_rows or group_size 0)
     int bits = 0;
