@@ -136,8 +136,9 @@ bool noting(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
 bool is_noting();
 
 // Few-row product (2 .. 96 rows, 17 .. 512 through csrc/wide.hip; sparse_mask != nullptr: 16:32 int4); false = shape not taken, use
-// the general kernels.  FOR_MATVEC: beyond 96 rows too only where weights rounded to fp16 may serve; EXACT_SUMS: never those
-enum RowsCall { FOR_MATMUL, FOR_MATVEC, EXACT_SUMS };
+// the general kernels.  FOR_MATVEC: beyond 96 rows too only where weights rounded to fp16 may serve; EXACT_SUMS: never those;
+// ROUNDED: those wherever the plan takes them
+enum RowsCall { FOR_MATMUL, FOR_MATVEC, EXACT_SUMS, ROUNDED };
 bool skinny_rows(int bits, _Float16* outs, const uint32_t* matrix, const _Float16* x, const _Float16* scales,
                  const _Float16* zeros, int64_t R, int64_t K, int64_t S, int64_t group_size, bool accumulate,
                  hipStream_t st, const uint32_t* sparse_mask, void* workspace, size_t workspace_bytes, RowsCall call);

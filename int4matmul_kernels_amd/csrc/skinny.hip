@@ -642,16 +642,20 @@ __global__ __launch_bounds__(512) void skinny_kernel(const uint32_t* pre_matrix,
     }
 }
 
+// LDS of the unsplit kernel: per wave its units, then the scales and zeros of all of the strip's groups
+static size_t skinny_lds_bytes(int cw, int waves, int groups) { return (size_t)waves * SK_WAVE_LDS + 16 + (size_t)groups * 16 * cw * 4; }
+static constexpr size_t skinny_lds_limit(bool sparse) { return 150 * 1024 - (sparse ? 4096 : 0); }      // (16:32: 4 KB of static LDS for the selector table)
+
 template <int BITS, int CW, bool SPARSE>
 static bool launch_skinny(const SkinnyArgs& a, int waves, int ksplit, bool plain, hipStream_t st) {
     const int strips = a.S / (16 * CW);
     const int rt = ((a.R > 32 ? 32 : a.R) + 7) / 8;
     int groups = (a.K / 64 + a.group_units - 1) / a.group_units;
     if (ksplit > 1) groups = std::min(groups, (a.units_per_split + a.group_units - 1) / a.group_units + 1);
-    size_t lds = (size_t)waves * SK_WAVE_LDS + 16 + (size_t)groups * 16 * CW * 4;
+    size_t lds = skinny_lds_bytes(CW, waves, groups);
     const size_t red = (size_t)(waves / 2) * (rt <= 2 ? 1 : 2) * 16 * 16 * CW * 4;
     if (red > lds) lds = red;
-    if (lds > 150 * 1024 - (SPARSE ? 4096 : 0)) return false;      // (16:32: 4 KB of static LDS for the selector table)
+    if (lds > skinny_lds_limit(SPARSE)) return false;
     const dim3 grid(strips, (a.R + 31) / 32, ksplit), block(waves * 64);
     plain = plain && rt > 2;
     if (noting("skinny_kernel<bits=%d,%s,columns_per_lane=%d,row_tiles=%d%s> strips=%d row_blocks=%u ksplit=%d waves=%d", BITS,
@@ -839,7 +843,11 @@ static SkinnySplit plan_skinny_split(int64_t R, int64_t K, int64_t S, bool spars
 
 size_t skinny_workspace_bytes(int bits, int64_t R, int64_t K, int64_t S, bool sparse, int64_t group_units, RowsCall call) {
     const SkinnySplit p = plan_skinny_split(R, K, S, sparse);
-    const size_t wide = wide_workspace_bytes(bits, R, K, S, sparse, group_units, call);
+    size_t wide = wide_workspace_bytes(bits, R, K, S, sparse, group_units, call);
+    // (a product that falls through skinny_rows; a group that is not known: the smallest)
+    if (call == FOR_MATMUL && wide == 0 && p.ksplit <= 1 && R <= FEW_ROWS_MAX &&
+        skinny_lds_bytes(unsplit_cw(R, S, sparse), 8, (int)(K / 64 / std::max<int64_t>(1, group_units))) > skinny_lds_limit(sparse))
+        wide = wide_workspace_bytes(bits, R, K, S, sparse, group_units, ROUNDED);
     const size_t balanced = balanced_shape(R, K, S) ? skinny_balanced_part_bytes(S) : 0;
     return std::max(std::max<size_t>(p.ksplit > 1 ? p.part_bytes : 0, wide), balanced);
 }
@@ -919,7 +927,9 @@ bool skinny_rows(int bits, h16* outs, const uint32_t* matrix, const h16* x, cons
         a.counters = nullptr;
         a.part = nullptr;
     }
-    return launch(cw, waves, 1);
+    if (launch(cw, waves, 1)) return true;
+    // a long K with small groups, whose scales do not fit the LDS: the matmul entry's tile kernels round the weights too
+    return call == FOR_MATMUL && wide_rows(bits, a, ROUNDED, workspace, workspace_bytes, st);
 }
 
 }  // namespace i4

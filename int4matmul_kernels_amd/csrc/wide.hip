@@ -637,7 +637,9 @@ static RoundedLine rounded_line(bool sparse, int64_t R, int64_t K, int64_t S, in
     return {true, ks > 1 ? (size_t)wgs * ks * tiles * 16384 : 0};
 }
 
-static bool needs_admission(int64_t R, RowsCall call) { return (R <= FEW_ROWS_MAX || call == FOR_MATVEC) && tuning(TUNE_NO_WIDE) < 2; }
+static bool needs_admission(int64_t R, RowsCall call) {
+    return (R <= FEW_ROWS_MAX || call == FOR_MATVEC) && call != ROUNDED && tuning(TUNE_NO_WIDE) < 2;
+}
 
 // Whole strips of 256 columns; beyond 96 rows, which the few-row kernel does not take, any number of whole 64 (the general
 // tiles that served them cannot split K: int2, K=9280, S=1600, 220 rows 238 us there, 21 here).

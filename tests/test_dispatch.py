@@ -126,6 +126,17 @@ def test_few_rows_keep_the_sums_of_exact_codes(product, bits, sparse, rows, k, s
         assert d("mtx", bits, 1, rows, k, s, g, sparse).startswith("wide_rows_kernel")
 
 
+# ---- a long K with so many groups that the few-row kernel has no room for their scales: the matmul entry, whose tile kernels round the
+# weights as well, has the kernel with shared staging for it, with or without a workspace
+@pytest.mark.parametrize("bits,rows,k,s,g", [(4, 34, 23296, 25600, 64), (4, 17, 28672, 28672, 64), (3, 34, 28672, 14336, 64),
+                                             (2, 61, 28672, 16384, 64), (4, 50, 46656, 8192, 128), (4, 96, 20480, 25600, 64)])
+def test_few_rows_on_many_groups_are_not_left_to_the_tiles(bits, rows, k, s, g):
+    for ws in (None, 0, 1 << 34):
+        assert d("mtx", bits, 1, rows, k, s, g, workspace_bytes=ws).startswith("wide_rows_kernel")
+    nbytes = capi.matmul_workspace_bytes(1, rows, k, s)
+    assert d("mtx", bits, 1, rows, k, s, g) == d("mtx", bits, 1, rows, k, s, g, False, 1 << 34) == d("mtx", bits, 1, rows, k, s, g, False, nbytes)
+
+
 # ---- the matvec entry with more batch elements than the few-row kernel takes at once: the kernel with rounded weights where it is
 # admitted, else shares of at most 96 elements with sums of exact codes; never a launch per element
 @pytest.mark.parametrize("bits,sparse,batch,k,s", [(4, False, 256, 5120, 20480), (4, False, 256, 8192, 28672), (4, False, 300, 4096, 11008),
