@@ -163,6 +163,12 @@ inline int64_t exact_sums_at_once(int64_t left, int64_t S) {
     const int64_t chunks = (left + FEW_ROWS_MAX - 1) / FEW_ROWS_MAX;
     return (left + chunks - 1) / chunks;
 }
+// bytes of partial tiles that such a chunk's line asks for; group_units = 0, not known: the least (SIZE_MAX: never admitted) or the most
+size_t rounded_room(bool sparse, int64_t R, int64_t K, int64_t S, int64_t group_units, bool least);
+// The last chunk, of n elements, of a batch of more than 512.  Its line of precision can ask for a split of K that the chunks of 512 do
+// not; it sums exact codes then (false), however much room the workspace has: K=1344, S=5888, 619 elements lost the exact sums of the
+// last 107 when the query made that room.  The limit is what a workspace has that was made for chunks of 512 and for the tile kernels
+bool last_chunk_as_others(bool sparse, int64_t B, int64_t n, int64_t K, int64_t S, int64_t group_units);
 // bytes of partial tiles with which such a product splits K across workgroups (0: no split); bits = 0, group_units = 0: not known
 size_t skinny_workspace_bytes(int bits, int64_t R, int64_t K, int64_t S, bool sparse, int64_t group_units, RowsCall call);
 

@@ -1317,6 +1317,19 @@ extern "C" int int4mm_matmul(int bits, void* outs, const void* matrix, const voi
     return check_launch("matmul");
 }
 
+bool i4::last_chunk_as_others(bool sparse, int64_t B, int64_t n, int64_t K, int64_t S, int64_t group_units) {
+    if (tuning(TUNE_NO_WIDE) >= 2) return true;
+    if (rounded_room(sparse, SK_WIDE_MAX_ROWS, K, S, group_units, true) == SIZE_MAX) return false;
+    const size_t room = rounded_room(sparse, n, K, S, group_units, true);
+    if (room == 0 || room == SIZE_MAX) return true;                      // (never admitted: nothing to decide)
+    const SplitPlan sp = plan_split(sparse, 1, B, K, S);
+    const TailPlan tp = plan_tail(sparse, 1, B, K, S);
+    size_t bytes = int4mm_workspace_bytes(S) + 2 * round_to_page(std::max(rounded_room(sparse, SK_WIDE_MAX_ROWS, K, S, 0, false),
+                                                                          sp.ksplit > 1 ? (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes) : 0));
+    if (sp.ksplit == 1 && tp.ksplit > 1) bytes += 2 * round_to_page((size_t)(tp.tiles * tp.ksplit * (256 * 256 * 4)));
+    return room <= bytes - ((bytes / 2) & ~size_t(4095));
+}
+
 // Workspace with which int4mm_matmul may split K for this shape: what the matvec needs, plus room for
 // the partial tiles in the scratch half.  A smaller workspace is not an error: the product then runs unsplit.
 extern "C" size_t int4mm_matmul_workspace_bytes(const int4mm_shape* shape, int sparse) {
@@ -1340,9 +1353,11 @@ extern "C" size_t int4mm_matmul_workspace_bytes(const int4mm_shape* shape, int s
     if (B * M > FEW_ROWS_MAX && (shape->seq_len == 1 || B * M <= SK_WIDE_MAX_ROWS))
         for (const int64_t n : {std::min<int64_t>(B * M, SK_WIDE_MAX_ROWS), B * M > SK_WIDE_MAX_ROWS ? B * M % SK_WIDE_MAX_ROWS : 0}) {
             if (n < 2) continue;
-            few_rows = std::max(few_rows, few(n, FOR_MATVEC));
+            const bool as_others = B * M <= SK_WIDE_MAX_ROWS || n == SK_WIDE_MAX_ROWS || last_chunk_as_others(sparse != 0, B * M, n, K, S, group_units);
+            if (as_others) few_rows = std::max(few_rows, few(n, FOR_MATVEC));
             for (const int64_t share : {exact_sums_at_once(n, S), exact_sums_at_once(B * M, S)})
-                if (n > FEW_ROWS_MAX && share > 2) few_rows = std::max({few_rows, few(share, EXACT_SUMS), few(share - 1, EXACT_SUMS)});
+                if ((n > FEW_ROWS_MAX || !as_others) && share >= 2)
+                    few_rows = std::max({few_rows, few(share, EXACT_SUMS), few(std::max<int64_t>(2, share - 1), EXACT_SUMS)});
         }
     if (B * M <= FEW_ROWS_MAX) return need + 2 * round_to_page(few_rows);
     const SplitPlan sp = plan_split(sparse != 0, B, M, K, S);

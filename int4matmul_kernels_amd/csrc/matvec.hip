@@ -1055,6 +1055,10 @@ static int matvec_impl(int bits, void* outs, const void* matrix, const void* mul
     while (B - done >= 2 && !tuning(TUNE_NO_SKINNY)) {
         const int64_t left = B - done, n = call == FOR_MATVEC ? std::min<int64_t>(left, SK_WIDE_MAX_ROWS) : exact_sums_at_once(left, S);
         if (n == 0) break;
+        if (call == FOR_MATVEC && done > 0 && n < SK_WIDE_MAX_ROWS && !last_chunk_as_others(sparse_mask != nullptr, B, n, K, S, g / 64)) {
+            call = EXACT_SUMS;
+            continue;
+        }
         if (!skinny_rows(bits, (h16*)outs + done * S, (const uint32_t*)matrix, (const h16*)multiplier + done * K, (const h16*)scales,
                          (const h16*)zeros, n, K, S, g, accumulate, (hipStream_t)stream, (const uint32_t*)sparse_mask, workspace,
                          workspace_bytes, call)) {

@@ -641,6 +641,19 @@ static bool needs_admission(int64_t R, RowsCall call) {
     return (R <= FEW_ROWS_MAX || call == FOR_MATVEC) && call != ROUNDED && tuning(TUNE_NO_WIDE) < 2;
 }
 
+// (groups of these units where the group is not known)
+static constexpr int64_t SOME_GROUPS[] = {1, 2, 3, 4, 6, 8, 16, 0x7FFFFFF};
+
+size_t rounded_room(bool sparse, int64_t R, int64_t K, int64_t S, int64_t group_units, bool least) {
+    size_t room = least ? SIZE_MAX : 0;
+    for (const int64_t units : SOME_GROUPS) {
+        const RoundedLine line = rounded_line(sparse, R, K, S, group_units > 0 ? group_units : units);
+        if (line.admitted) room = least ? std::min(room, line.room) : std::max(room, line.room);
+        if (group_units > 0) break;
+    }
+    return room;
+}
+
 // Whole strips of 256 columns; beyond 96 rows, which the few-row kernel does not take, any number of whole 64 (the general
 // tiles that served them cannot split K: int2, K=9280, S=1600, 220 rows 238 us there, 21 here).
 static bool wide_columns(int64_t R, int64_t S) { return S % 256 == 0 || (R > FEW_ROWS_MAX && S % 64 == 0); }
@@ -704,7 +717,7 @@ size_t wide_workspace_bytes(int bits, int64_t R, int64_t K, int64_t S, bool spar
     size_t need = 0;
     if (needs_admission(R, call)) {
         bool admitted = false;
-        for (const int64_t units : {1, 2, 3, 4, 6, 8, 16, 0x7FFFFFF}) {
+        for (const int64_t units : SOME_GROUPS) {
             const RoundedLine line = rounded_line(sparse, R, K, S, group_units > 0 ? group_units : units);
             admitted = admitted || line.admitted;
             need = std::max(need, line.room);

@@ -148,6 +148,19 @@ def test_many_batch_elements_keep_the_sums_of_exact_codes(bits, sparse, batch, k
     assert line.startswith("skinny_kernel") and "row_tiles=4,plain>" in line and "wide_rows" not in line, line
 
 
+@pytest.mark.parametrize("bits,batch,k,s,g", [(4, 619, 1344, 5888, 128), (2, 877, 19200, 3584, -1), (4, 1740, 1536, 8192, -1), (3, 625, 1024, 7424, 128)])
+def test_the_last_chunk_of_many_batch_elements_keeps_the_sums_of_exact_codes(bits, batch, k, s, g):
+    # it asks for a split of K that the chunks of 512 do not: whatever the workspace has room for
+    for ws in (None, 1 << 34):
+        lines = d("vec", bits, batch, 1, k, s, g, False, ws).split("; ")[:-1]
+        assert all(line.startswith("wide_rows_kernel") for line in lines[:batch // 512]), lines
+        assert lines[batch // 512:] and all(line.startswith("skinny_kernel") for line in lines[batch // 512:]), lines
+    # (no room is asked for a chunk that follows none of 512: 180 MB here)
+    assert capi.matmul_workspace_bytes(657, 1, 18176, 16896) < 10 << 20
+    # a last chunk that asks no more than those before it goes with them
+    assert d("vec", 4, 1000, 1, 4096, 4096, 128).count("wide_rows_kernel") == 2
+
+
 @pytest.mark.parametrize("bits,sparse", [(4, False), (3, False), (2, False), (4, True)])
 def test_many_batch_elements_never_run_one_by_one(bits, sparse):
     for k, s in ((512, 256), (4096, 512), (2048, 1600), (4096, 11008), (5120, 20480), (8192, 28672), (2048, 40960)):
