@@ -1319,9 +1319,9 @@ extern "C" int int4mm_matmul(int bits, void* outs, const void* matrix, const voi
 
 bool i4::last_chunk_as_others(bool sparse, int64_t B, int64_t n, int64_t K, int64_t S, int64_t group_units) {
     if (tuning(TUNE_NO_WIDE) >= 2) return true;
-    if (rounded_room(sparse, SK_WIDE_MAX_ROWS, K, S, group_units, true) == SIZE_MAX) return false;
-    const size_t room = rounded_room(sparse, n, K, S, group_units, true);
-    if (room == 0 || room == SIZE_MAX) return true;                      // (never admitted: nothing to decide)
+    const size_t others = rounded_room(sparse, SK_WIDE_MAX_ROWS, K, S, group_units, true), room = rounded_room(sparse, n, K, S, group_units, true);
+    if (others == SIZE_MAX) return false;
+    if (room <= others || room == SIZE_MAX) return true;                 // (never admitted: nothing to decide)
     const SplitPlan sp = plan_split(sparse, 1, B, K, S);
     const TailPlan tp = plan_tail(sparse, 1, B, K, S);
     size_t bytes = int4mm_workspace_bytes(S) + 2 * round_to_page(std::max(rounded_room(sparse, SK_WIDE_MAX_ROWS, K, S, 0, false),

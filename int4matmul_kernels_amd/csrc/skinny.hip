@@ -845,7 +845,7 @@ size_t skinny_workspace_bytes(int bits, int64_t R, int64_t K, int64_t S, bool sp
     const SkinnySplit p = plan_skinny_split(R, K, S, sparse);
     size_t wide = wide_workspace_bytes(bits, R, K, S, sparse, group_units, call);
     // (a product that falls through skinny_rows; a group that is not known: the smallest)
-    if (call == FOR_MATMUL && wide == 0 && p.ksplit <= 1 && R <= FEW_ROWS_MAX &&
+    if (call == FOR_MATMUL && wide == 0 && p.ksplit <= 1 && R >= 17 && R <= FEW_ROWS_MAX &&
         skinny_lds_bytes(unsplit_cw(R, S, sparse), 8, (int)(K / 64 / std::max<int64_t>(1, group_units))) > skinny_lds_limit(sparse))
         wide = wide_workspace_bytes(bits, R, K, S, sparse, group_units, ROUNDED);
     const size_t balanced = balanced_shape(R, K, S) ? skinny_balanced_part_bytes(S) : 0;
