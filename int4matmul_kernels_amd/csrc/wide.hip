@@ -685,7 +685,7 @@ static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S
         // (below 1024 columns, where nothing was fitted: as many ways as leave shares of eight units)
         int64_t only = forced >= 1 ? std::min<int64_t>(forced, std::max<int64_t>(1, units / 4))
                      : S < 1024 ? std::max<int64_t>(1, std::min<int64_t>({256 / tiles, units / 8, 16})) : 0;
-        while (too_large(only)) --only;
+        while (only > 1 && too_large(only)) --only;
         for (int64_t k = only ? only : 1; k <= 16; ++k) {
             if (k > 1 && (units / k < 4 || tiles * k > WIDE_MAX_SPLIT_WGS || too_large(k))) break;
             const int64_t share = (units + k - 1) / k, steps = (share * c.wn + 7) / 8, wgs = tiles * k, rounds = (wgs + 255) / 256;
