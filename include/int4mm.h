@@ -38,7 +38,8 @@
  *    about 3.2e-4 of the result, 2-norm).  int4mm_matmul with more than 96 rows of states,
  *    and some products of 17..96 rows through either entry and of more batch entries through
  *    int4mm_matvec, on outputs of whole 256 columns and with the workspace that
- *    int4mm_matmul_workspace_bytes asks for;
+ *    int4mm_matmul_workspace_bytes asks for.  Also 17..96 rows through int4mm_matmul on so many groups
+ *    (K of some 20 000 and more) that the kernel with exact codes has no room for their scales;
  *  - exact codes: sum(x * q) and sum(x) are accumulated and scale and zero applied
  *    once per group, y += s * (sum(x * q) - z * sum(x)), the exact value of
  *    sum(x * (q - z) * s) up to fp32 rounding (2.1e-4, the fp16 result's own) -- closer to the
