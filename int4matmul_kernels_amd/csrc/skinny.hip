@@ -927,7 +927,13 @@ bool skinny_rows(int bits, h16* outs, const uint32_t* matrix, const h16* x, cons
         a.counters = nullptr;
         a.part = nullptr;
     }
-    if (launch(cw, waves, 1)) return true;
+    // (so many groups that their scales do not fit the LDS beside the waves' units: narrower strips, where the matvec entry would run an
+    // element at a time else -- us, so / now: int4, g=64, K=25344, S=27648, 48 elements 2945 / 378, K=22784, S=18688, 368 elements
+    // 16601 / 1435; four waves on strips of 64 columns take 402 and 1447)
+    for (; cw >= 1; cw >>= 1) {
+        if (launch(cw, waves, 1)) return true;
+        if (call != EXACT_SUMS || R < 17) break;
+    }
     // a long K with small groups, whose scales do not fit the LDS: the matmul entry's tile kernels round the weights too
     return call == FOR_MATMUL && wide_rows(bits, a, ROUNDED, workspace, workspace_bytes, st);
 }

@@ -168,6 +168,11 @@ def test_many_batch_elements_never_run_one_by_one(bits, sparse):
             for ws in (None, capi.lib().int4mm_workspace_bytes(s)):
                 line = d("vec", bits, batch, 1, k, s, 64 if sparse else 128, sparse, ws)
                 assert line.startswith(("skinny_kernel", "wide_rows_kernel")), (batch, k, s, line)
+    # (so many groups that the strips have to be narrower for their scales)
+    for batch, k, s in ((368, 22784, 18688), (501, 19968, 15104), (48, 25344, 27648), (17, 28672, 28672), (90, 22400, 2752), (130, 57344, 17728)):
+        for ws in (None, capi.lib().int4mm_workspace_bytes(s)):
+            line = d("vec", bits, batch, 1, k, s, 64, sparse, ws)
+            assert line.startswith(("skinny_kernel", "wide_rows_kernel")) and "matvec" not in line, (batch, k, s, line)
 
 
 def test_many_rows_on_a_short_k_are_not_left_to_few_workgroups():

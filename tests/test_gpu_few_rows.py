@@ -804,6 +804,13 @@ def test_matvec_many_batch_elements_as_exact_as_one(H, bits, sparse, B, K, S, g,
     assert np.linalg.norm(got[:, 0] - want) / np.linalg.norm(want) < 2.0 ** -11 / 3 ** 0.5 + 5e-6
 
 
+@pytest.mark.parametrize("bits", [4, 3, 2])
+def test_matvec_batch_on_many_groups_as_exact_as_one(H, bits):
+    """350 groups, whose scales fit the LDS in strips of 32 columns instead of 64"""
+    assert "columns_per_lane=2," in H.capi.describe_launch("vec", bits, 90, 1, 22400, 2752, 64)
+    test_matvec_many_batch_elements_as_exact_as_one(H, bits, False, 90, 22400, 2752, 64, 0.05)
+
+
 @pytest.mark.parametrize("bits,sparse", [(4, False), (3, False), (2, False), (4, True)])
 @pytest.mark.parametrize("M,K", [(8, 16384), (44, 17728), (130, 2048), (401, 12352)])
 def test_one_strip_of_64_columns_splits_k(H, bits, sparse, M, K):
