@@ -65,6 +65,12 @@ __device__ __forceinline__ uint32_t in_vgpr(uint32_t literal) {
     return r;
 }
 
+// two 8-bit floats (4 exponent, 3 mantissa bits) -> halves times a power of two, exactly; a byte q < 16 is q 2^-9
+template <bool HI>
+__device__ __forceinline__ h16x2 from_fp8(uint32_t bytes, float scale) {
+    return bitcast<h16x2>(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)bytes, scale, HI));
+}
+
 // a / b for 0 <= a < 2^22, b >= 1 with b's magic number floor(2^32 / b) + 1 (2^32 - 1 for b = 1), which the host passes:
 // the high word of the product is the quotient or one off -- eight integer instructions where the compiler's exact
 // division by a run-time divisor takes ~35

@@ -7,7 +7,7 @@
 // made of whole tiles; matmul_kernel takes everything else.  Common to both: one
 // workgroup owns a tile of outs; per K step the packed weights of the tile are
 // read from HBM once, decoded and dequantised to fp16 ONCE by the workgroup and
-// stored to LDS in the operand layout of v_mfma_f32_32x32x16_f16: 16-byte chunks
+// stored to LDS in MFMA operand layout: 16-byte chunks
 // of 8 consecutive k for one column, chunk (kc, n) at kc*BN + n, which both the
 // writes (lanes along n) and the MFMA operand reads (lanes along n) touch
 // without bank conflicts.  The states tile is stored row-major with an XOR
@@ -110,37 +110,104 @@ __device__ __forceinline__ void dequant_cell_generic(const Cell<BITS, SPARSE>& c
     }
 }
 
-// Fast linear-mode decode of one dense int4 word into 8 fp16 weights in natural
-// k order, bit-exact: the word's low (high) two bytes are replicated into both
-// halves of a register, so that mask-and-OR yields the half2 {1024 + q_even,
-// 64 + q_odd}; subtracting {1024, 64} is exact, then the reference's own two
-// roundings follow: fp16(q - z), fp16(. * s).
-// (mask / magic constants are held in registers, in_vgpr, so that v_and_or_b32 is selected)
-
-__device__ __forceinline__ h16x8 dequant_word_int4(uint32_t u, h16x2 negz, h16x2 s2) {
-    const uint32_t MSK = in_vgpr(0x00F0000Fu), MAGIC = in_vgpr(0x54006400u);
-    const h16x2 unmagic = {(h16)-1024.0f, (h16)-64.0f};
-    const uint32_t lo = __builtin_amdgcn_perm(u, u, 0x01000100u);    // bytes B0 B1 B0 B1
-    const uint32_t hi = __builtin_amdgcn_perm(u, u, 0x03020302u);    // bytes B2 B3 B2 B3
-    const uint32_t h[4] = {(lo & MSK) | MAGIC, ((lo >> 8) & MSK) | MAGIC,
-                           (hi & MSK) | MAGIC, ((hi >> 8) & MSK) | MAGIC};
-    u32x4 r;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        h16x2 q = as_h2(h[i]) + unmagic;       // exact: {q_even, q_odd}
-        h16x2 d = q + negz;                    // fp16 subtract, one rounding
-        r[i] = as_u32(d * s2);                 // fp16 multiply, one rounding
+// ---- decodes of a chunk, 8 consecutive k of one column, bit-exact and in natural k order
+// The coefficients of a column's group: {s, s}, {z, z} or what the decode makes of them.
+// Linear mode: the reference's own two roundings, fp16(q - z), fp16(. * s).
+struct LinearCoef {
+    h16x2 s, z;
+    __device__ __forceinline__ void set(h16x2 s2, h16x2 z2) { s = s2; z = z2; }
+    __device__ __forceinline__ uint32_t weight(h16x2 q) const { return as_u32((q - z) * s); }
+};
+// Either mode, chosen per thread (a thread decodes whole columns, and the mode belongs to a (group, column)), without a branch:
+//     A = P + N (one rounding),  w = fma(A, B, C) (one rounding)
+// linear:   P = q, N = -z, B = s, C = -0:  fp16(q - z), then fp16(. * s) -- adding -0 changes nothing
+// exponent: P = +-2^e, N = -0, B = -s, C = z:  the reference's single-rounded fma (matmul.cuh:127-136)
+struct TwoModeCoef {
+    uint32_t m;                                  // all ones in exponent mode (bit picks: a selection came out as a branch)
+    h16x2 N, B, C;
+    float scale;                                 // of the 8-bit floats: 2^9 for q, 1 for +-2^e
+    __device__ __forceinline__ uint32_t pick(uint32_t e, uint32_t l) const { return (e & m) | (l & ~m); }
+    __device__ __forceinline__ void set(h16x2 s2, h16x2 z2) {
+        m = s2.x >= (h16)0.0f ? 0u : 0xFFFFFFFFu;
+        N = as_h2(pick(0x80008000u, as_u32(z2) ^ 0x80008000u));
+        B = as_h2(as_u32(s2) ^ (m & 0x80008000u));
+        C = as_h2(pick(as_u32(z2), 0x80008000u));
+        scale = bitcast<float>(pick(0x3F800000u, 0x44000000u));
     }
-    return bitcast<h16x8>(r);
+    __device__ __forceinline__ uint32_t weight(h16x2 P) const { return as_u32(__builtin_elementwise_fma(P + N, B, C)); }
+    // four codes as bytes -> the 8-bit floats of q 2^-9 or +-2^e
+    __device__ __forceinline__ uint32_t powers(uint32_t b) const {
+        return pick(((b & 0x08080808u) << 4) | (((b & 0x07070707u) << 3) + 0x38383838u), b);
+    }
+};
+// int2: the group's four weights, in either mode, are a v_perm table
+struct Int2Coef {
+    uint32_t T0, T1;
+    __device__ __forceinline__ void set(h16x2 s2, h16x2 z2) {
+        TwoModeCoef c;
+        c.set(s2, z2);
+        T0 = c.weight(as_h2(c.pick(0x40003C00u, 0x3C000000u)));
+        T1 = c.weight(as_h2(c.pick(0xC000BC00u, 0x42004000u)));
+    }
+};
+// int3: the eight values' upper bytes are one (their lower ones are 0)
+struct Int3Coef : TwoModeCoef {
+    uint32_t T0, T1;
+    __device__ __forceinline__ void set(h16x2 s2, h16x2 z2) {
+        TwoModeCoef::set(s2, z2);
+        T0 = pick(0x4844403Cu, 0x42403C00u);
+        T1 = pick(0xC8C4C0BCu, 0x47464544u);
+    }
+};
+template <int BITS, bool TWO_MODES>
+using Coef = std::conditional_t<BITS == 2, Int2Coef, std::conditional_t<BITS == 3, Int3Coef, std::conditional_t<TWO_MODES, TwoModeCoef, LinearCoef>>>;
+
+// four codes of a word as bytes -> eight weights: a byte q < 16 is the 8-bit float q 2^-9
+template <class C>
+__device__ __forceinline__ h16x8 weights_of_bytes(uint32_t b03, uint32_t b47, const C& c) {
+    float scale = 512.f;
+    if constexpr (std::is_same_v<C, TwoModeCoef>) {
+        b03 = c.powers(b03);
+        b47 = c.powers(b47);
+        scale = c.scale;
+    }
+    return bitcast<h16x8>(u32x4{c.weight(from_fp8<false>(b03, scale)), c.weight(from_fp8<true>(b03, scale)),
+                                c.weight(from_fp8<false>(b47, scale)), c.weight(from_fp8<true>(b47, scale))});
+}
+
+// `bits`: the chunk's codes, LSB first, BITS bits apart (bits above 8 * BITS are ignored).  17 (int4), 17 (int2) and 24 (int3)
+// instructions; with magic numbers and their removal 20, 24 and 24, and twice as many for either mode
+template <int BITS, class C>
+__device__ __forceinline__ h16x8 dequant_chunk(uint32_t bits, const C& c) {
+    if constexpr (BITS == 4) {
+        const uint32_t even = bits & 0x0F0F0F0Fu, odd = (bits >> 4) & 0x0F0F0F0Fu;
+        return weights_of_bytes(__builtin_amdgcn_perm(odd, even, 0x05010400u), __builtin_amdgcn_perm(odd, even, 0x07030602u), c);
+    } else if constexpr (BITS == 2) {
+        const uint32_t v = (bits & 0xFFFFu) | (bits << 14);               // code 2 j at bit 4 j, code 2 j + 1 at 16 + 4 j
+        u32x4 r;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            r[j] = __builtin_amdgcn_perm(c.T1, c.T0, __umul24((v >> (4 * j)) & 0x00030003u, 0x0202u) + 0x01000100u);
+        return bitcast<h16x8>(r);
+    } else {
+        const uint32_t u = bits & 0xFFFFFFu;
+        const uint32_t v = (u & 0xFFFFu) | ((u << 13) & 0xFFFF0000u);      // codes 0, 2, 4 at bits 0, 6, 12, codes 1, 3, 5 at 16, 22, 28
+        const uint32_t y = u >> 10;                                       // code 6 at bit 8, code 7 at 11
+        const uint32_t sel[4] = {v << 8, v << 2, v >> 4, (y << 13) | y};
+        u32x4 r;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r[j] = c.weight(as_h2(__builtin_amdgcn_perm(c.T1, c.T0, (sel[j] & 0x07000700u) | 0x000C000Cu)));
+        return bitcast<h16x8>(r);
+    }
 }
 
 template <int BITS, bool SPARSE>
 __device__ __forceinline__ void dequant_cell(const Cell<BITS, SPARSE>& c, h16 sc, h16 ze, h16x8 out[4]) {
     if constexpr (BITS == 4 && !SPARSE) {
         if (sc >= (h16)0.0f) {
-            const h16x2 negz = {-ze, -ze}, s2 = {sc, sc};
+            const LinearCoef co = {{sc, sc}, {ze, ze}};
 #pragma unroll
-            for (int i = 0; i < 4; ++i) out[i] = dequant_word_int4(c.w[i], negz, s2);
+            for (int i = 0; i < 4; ++i) out[i] = dequant_chunk<4>(c.w[i], co);
             return;
         }
     }
@@ -268,106 +335,33 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 2) void matmul_kernel(M
         }
 }
 
-// ---- pipelined variant for dense int4: (TM * 64) x (NW * 64) tile, 2 x NW waves
-// of (TM * 32) x 64, K steps of 32, three LDS stages of each operand.  With
-// NW = 2 (256 x 128 tile, 72 KB of LDS, four waves) two workgroups share a CU
-// and fill each other's barrier and latency bubbles.
-//  * states go global -> registers three steps ahead and are stored to the LDS
-//    stage of step k+2 during step k;
-//  * packed weights go global -> registers four steps ahead and are decoded
-//    into the LDS stage of step k+2 one word at a time between the MFMAs of
-//    step k, so VALU, LDS and the matrix core overlap inside a wave;
-//  * MFMA operand fragments are fetched one 16-wide k slice ahead, ACROSS step
-//    boundaries: everything a step reads was complete one barrier earlier, so
-//    the barrier that closes a step orders buffer reuse only and the MFMA
-//    stream never drains while waves wait for each other.
-// The steady-state loop body has no branches; a tile that contains exponent-mode
-// groups takes a second pipelined loop whose decode serves either mode (dense formats, 256-column
-// tiles) or a plain two-stage loop with that decode (the others).
+// ---- the pipelined kernel: (TM * 32) x (NW * 64) tiles, 2 x NW waves of (TM * 16) x 64, K steps of 32.
+//
+// What bounds it is the power limit: at full load the clock falls to what the work of a K step allows, so energy per step counts,
+// and beside it the step's length.  Hence
+//  * v_mfma_f32_16x16x32_f16: a loop of nothing but MFMAs and their LDS reads, on all CUs and random data, does 1710 TFLOP/s where
+//    32x32x16 ones do 1530 (a third less accumulator traffic per flop); at zeros, which cost no power, both do 2260;
+//  * the states go from global memory straight to LDS, A_AHEAD steps ahead (six stages), which leaves the registers alone;
+//  * decodes of 17 (int4, int2) and 24 (int3) instructions per chunk through the 8-bit float conversion and v_perm tables;
+//  * scales and zeros are asked for once per pair of steps, int4's words of two columns in one load;
+//  * the two halves of the workgroup run a step in opposite phases (PING): a SIMD holds a wave of each, one on the matrix
+//    pipe, its decode in the shadow of its MFMAs, while the other does everything that touches the LDS or memory.  A wave's own
+//    LDS stores between its MFMAs would hold these up (40 cycles each, on a step of 1024), and just before the barrier the
+//    barrier; so what phase 1 stores at a step's start was decoded in the step before.  (1330 cycles a step with the
+//    stores between the MFMAs, 1200 with those of the decode at its end, 1050 so, in a loop without global loads.)
+// A tile of int4 or 16:32 that contains exponent-mode groups takes a second copy of the loop whose decode serves either mode;
+// int2 and int3 have one decode for both.
+//
+// Measured, before (32x32x16 MFMAs, states through registers, magic-number decodes) / so, us: K=5120, S=20480, 2048 rows int4 398 /
+// 351, int3 402 / 363, int2 394 / 340, 16:32 437 / 407, one group in 40 in exponent mode 464 / 380, int3 468 / 363; K=8192,
+// S=28672, 4096 rows 1663 / 1453 (1.32 PFLOP/s); K=S=8192, 768 rows 125 / 109; K=20480, S=5120, 1024 rows 250 / 222.
 constexpr int PK = 32;            // K per step of the pipelined kernel
-
-// One 16-byte chunk = 8 consecutive k of one column; `bits` holds its 8 codes, LSB first, BITS bits apart (bits
-// above 8 * BITS are ignored).  Linear-mode fast decode of such a chunk, bit-exact.  The two codes of a pair
-// are brought to the low bits of the two halves of a register; mask-and-OR with
-// a magic exponent turns them into {2^a + q_even, 2^b + q_odd}, whose offsets
-// are then subtracted exactly before the reference's two roundings.
-template <int BITS>
-__device__ __forceinline__ h16x8 dequant_chunk_fast(uint32_t bits, h16x2 negz, h16x2 s2) {
-    if constexpr (BITS == 4) {
-        return dequant_word_int4(bits, negz, s2);
-    } else {
-        // int2: pair j = bits 4j .. 4j+3 of the 16 code bits, replicated into both halves:
-        //       low half keeps bits 0-1 (ulp 1 at 2^10), high half bits 2-3 (ulp 1/4 at 2^8).
-        // int3: pair j = bits 6j .. 6j+5: low half bits 0-2 (2^10), high half bits 3-5 (ulp 1/8 at 2^7).
-        constexpr uint32_t MSK = BITS == 2 ? 0x000C0003u : 0x00380007u;
-        constexpr uint32_t MAGIC = BITS == 2 ? 0x5C006400u : 0x58006400u;
-        const h16x2 unmagic = {(h16)-1024.0f, BITS == 2 ? (h16)-256.0f : (h16)-128.0f};
-        u32x4 r;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t u = bits >> (2 * BITS * j);
-            const uint32_t v = __builtin_amdgcn_perm(u, u, 0x01000100u);     // low 16 bits in both halves
-            h16x2 q = as_h2((v & MSK) | MAGIC) + unmagic;      // exact: {q_even, q_odd}
-            h16x2 d = q + negz;                                // fp16 subtract, one rounding
-            r[j] = as_u32(d * s2);                             // fp16 multiply, one rounding
-        }
-        return bitcast<h16x8>(r);
-    }
-}
-
-// Either mode, chosen per thread (a thread decodes one column, and the mode belongs to a
-// (group, column)), without a branch: bit-exact with dequant_code in both.  Shared tail
-//     A = P + N (one rounding),  w = fma(A, B, C) (one rounding)
-// linear:   P = q, N = -z, B = s, C = -0:  fp16(q - z), then fp16(. * s) -- adding -0 changes nothing
-// exponent: P = +-2^e, N = -0, B = -s, C = z:  the reference's single-rounded fma (matmul.cuh:127-136)
-// +-2^e comes from the pair's magic-number word {2^a | q_even, 2^b | q_odd << BITS}: a packed
-// 16-bit multiply moves both codes to bits 10.. of their halves (the magic bits leave through the
-// top), the low BITS - 1 bits are the exponent field's increment over 15, the top bit is the sign.
-template <int BITS>
-__device__ __forceinline__ h16x2 expo_pair(uint32_t h) {
-    return as_h2(expo_operand<BITS>(h, off2(1024u, 1u << (10 - BITS))));
-}
-
-template <int BITS>
-__device__ __forceinline__ h16x8 dequant_chunk_mixed(uint32_t bits, bool expo, h16x2 negz, h16x2 s2) {
-    const h16x2 minus0 = as_h2(0x80008000u);
-    const h16x2 N = expo ? minus0 : negz, B = expo ? -s2 : s2, C = expo ? -negz : minus0;
-    uint32_t h[4];
-    h16x2 unmagic;
-    if constexpr (BITS == 4) {
-        const uint32_t MSK = in_vgpr(0x00F0000Fu), MAGIC = in_vgpr(0x54006400u);
-        unmagic = h16x2{(h16)-1024.0f, (h16)-64.0f};
-        const uint32_t lo = __builtin_amdgcn_perm(bits, bits, 0x01000100u);
-        const uint32_t hi = __builtin_amdgcn_perm(bits, bits, 0x03020302u);
-        h[0] = (lo & MSK) | MAGIC; h[1] = ((lo >> 8) & MSK) | MAGIC;
-        h[2] = (hi & MSK) | MAGIC; h[3] = ((hi >> 8) & MSK) | MAGIC;
-    } else {
-        constexpr uint32_t MSK = BITS == 2 ? 0x000C0003u : 0x00380007u;
-        constexpr uint32_t MAGIC = BITS == 2 ? 0x5C006400u : 0x58006400u;
-        unmagic = h16x2{(h16)-1024.0f, BITS == 2 ? (h16)-256.0f : (h16)-128.0f};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t u = bits >> (2 * BITS * j);
-            h[j] = (__builtin_amdgcn_perm(u, u, 0x01000100u) & MSK) | MAGIC;
-        }
-    }
-    u32x4 r;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const h16x2 q = as_h2(h[j]) + unmagic;             // exact: {q_even, q_odd}
-        const h16x2 P = expo ? expo_pair<BITS>(h[j]) : q;
-        const h16x2 A = P + N;
-        r[j] = as_u32(__builtin_elementwise_fma(A, B, C));
-    }
-    return bitcast<h16x8>(r);
-}
 
 // 16:32 sparse int4.  `v` holds the (up to 8) kept codes of one 8-row chunk as
 // consecutive nibbles, `m8` the chunk's mask bits.  A 256-entry table in LDS
 // (8 words per mask byte: four words of per-half keep masks, two v_perm
 // selectors) spreads the kept codes to their rows: the even / odd nibbles are
-// separated into bytes, v_perm picks for every row the byte of its rank, a
-// second v_perm widens byte pairs to {0x6400 | q, 0x6400 | q'}.  Dropped rows
+// separated into bytes, v_perm picks for every row the byte of its rank.  Dropped rows
 // are cleared at the end, so they are exactly zero.
 constexpr int SPARSE_LUT_WORDS = 256 * 8;
 
@@ -385,51 +379,14 @@ __device__ __forceinline__ void sparse_lut_entry(uint32_t e, uint32_t out[8]) {
     out[4] = sel[0]; out[5] = sel[1]; out[6] = 0; out[7] = 0;
 }
 
-__device__ __forceinline__ h16x8 dequant_chunk_sparse_fast(uint32_t v, uint32_t m8, const uint32_t* lut,
-                                                           h16x2 negz, h16x2 s2) {
+template <class C>
+__device__ __forceinline__ h16x8 dequant_chunk_sparse(uint32_t v, uint32_t m8, const uint32_t* lut, const C& c) {
     const u32x4 keep = *reinterpret_cast<const u32x4*>(lut + m8 * 8);
     const u32x2 sel = *reinterpret_cast<const u32x2*>(lut + m8 * 8 + 4);
     const uint32_t even = v & 0x0F0F0F0Fu, odd = (v >> 4) & 0x0F0F0F0Fu;
-    const uint32_t c03 = __builtin_amdgcn_perm(odd, even, sel.x);       // codes of rows 0..3, one per byte
-    const uint32_t c47 = __builtin_amdgcn_perm(odd, even, sel.y);
-    const uint32_t MAGIC = 0x64006400u;
-    const uint32_t h[4] = {__builtin_amdgcn_perm(c03, MAGIC, 0x01050104u), __builtin_amdgcn_perm(c03, MAGIC, 0x01070106u),
-                           __builtin_amdgcn_perm(c47, MAGIC, 0x01050104u), __builtin_amdgcn_perm(c47, MAGIC, 0x01070106u)};
-    const h16x2 unmagic = {(h16)-1024.0f, (h16)-1024.0f};
-    u32x4 r;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        h16x2 q = as_h2(h[i]) + unmagic;       // exact
-        h16x2 d = q + negz;                    // fp16 subtract, one rounding
-        r[i] = as_u32(d * s2) & keep[i];       // fp16 multiply, one rounding; dropped rows -> +0
-    }
-    return bitcast<h16x8>(r);
+    const u32x4 r = bitcast<u32x4>(weights_of_bytes(__builtin_amdgcn_perm(odd, even, sel.x), __builtin_amdgcn_perm(odd, even, sel.y), c));
+    return bitcast<h16x8>(r & keep);             // (dropped rows -> +0)
 }
-
-// Either mode per thread without a branch (see dequant_chunk_mixed): the rows' codes ride on 1024 in both halves of
-// a pair, so the packed multiply that moves them to bits 10.. is by 1024 for both.
-__device__ __forceinline__ h16x8 dequant_chunk_sparse_mixed(uint32_t v, uint32_t m8, const uint32_t* lut, bool expo,
-                                                            h16x2 negz, h16x2 s2) {
-    const u32x4 keep = *reinterpret_cast<const u32x4*>(lut + m8 * 8);
-    const u32x2 sel = *reinterpret_cast<const u32x2*>(lut + m8 * 8 + 4);
-    const uint32_t even = v & 0x0F0F0F0Fu, odd = (v >> 4) & 0x0F0F0F0Fu;
-    const uint32_t c03 = __builtin_amdgcn_perm(odd, even, sel.x);
-    const uint32_t c47 = __builtin_amdgcn_perm(odd, even, sel.y);
-    const uint32_t MAGIC = 0x64006400u;
-    const uint32_t h[4] = {__builtin_amdgcn_perm(c03, MAGIC, 0x01050104u), __builtin_amdgcn_perm(c03, MAGIC, 0x01070106u),
-                           __builtin_amdgcn_perm(c47, MAGIC, 0x01050104u), __builtin_amdgcn_perm(c47, MAGIC, 0x01070106u)};
-    const h16x2 unmagic = {(h16)-1024.0f, (h16)-1024.0f}, minus0 = as_h2(0x80008000u);
-    const h16x2 N = expo ? minus0 : negz, B = expo ? -s2 : s2, C = expo ? -negz : minus0;
-    u32x4 r;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const h16x2 q = as_h2(h[i]) + unmagic;             // exact
-        const h16x2 P = expo ? as_h2(expo_operand<4>(h[i], off2(1024u, 1024u))) : q;
-        r[i] = as_u32(__builtin_elementwise_fma(P + N, B, C)) & keep[i];      // dropped rows -> +0
-    }
-    return bitcast<h16x8>(r);
-}
-
 
 // Per-format constants of the pipelined kernel: packed rows per 32-row block and
 // the number of packed words a thread loads per K step for its two chunks.
@@ -440,32 +397,37 @@ template <> struct PipeFmt<2, false> { static constexpr int ROWS = 2, NWORDS = 1
 template <> struct PipeFmt<4, true> { static constexpr int ROWS = 2, NWORDS = 2; };
 
 constexpr int P_STAGES = 3;
+constexpr int pipe_a_stages(int nw) { return nw == 4 ? 6 : P_STAGES; }
+constexpr int A_AHEAD = 5;                 // steps that the states loaded straight to LDS are ahead
+// immediate of s_waitcnt: at most so many vector memory and LDS operations outstanding
+constexpr int wait_counts(int vm, int lgkm) { return (vm & 15) | 0x70 | lgkm << 8 | (vm >> 4) << 14; }
 
-// PING: the waves of the first half ("compute first") run a step as its 16 MFMAs back to back
-// and then everything else; the waves of the second half run everything else first and the MFMAs
-// last.  A SIMD holds one wave of each kind, so its matrix pipe is fed by one wave at a time while
-// the other loads, decodes and stores -- instead of both competing for it and the younger one
-// finishing the step alone.
+// Swizzle of the states stage: row m's 16-byte chunk c stands at c ^ pipe_swz(m).  A 16-byte LDS read is served in
+// groups of lanes 0-3, 12-15, 20-27 and 4-11, 16-19, 28-31 (of each half wave); with lane = row + 16 chunk each group then
+// touches all 64 banks once (247 bytes a cycle and CU; with (m >> 2) & 3, which suits 32 rows x 2 chunks, 127).
+__device__ __forceinline__ int pipe_swz(int m) { return ((m >> 3) & 1) | (((m >> 1 ^ m >> 2) & 2)); }
+
+// PING: the waves of the first half run phase 0, MFMAs first and then everything else; those of the second half phase 1,
+// everything else first and the MFMAs last.  Without it all waves run phase 1, which is what the 128-column kernel does: its two
+// workgroups per CU drift apart by themselves.
 template <int BITS, bool SPARSE, int TM, int NW, bool PING, bool SPLIT>
 __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, const int s0, const h16* x,
-                                          h16* outs, h16* As, h16* Bs, uint32_t* lut, const int tile, const int split,
+                                          h16* outs, h16* const (&As)[pipe_a_stages(NW)], h16* Bs, uint32_t* lut, const int tile, const int split,
                                           const int nsplit) {
-    constexpr int BM = TM * 64, BN = NW * 64, WM = TM * 32, WN = 64, TN = 2, T = 2 * NW * 64;
+    constexpr int BM = TM * 32, BN = NW * 64, WM = TM * 16, WN = 64, TN = 4, T = 2 * NW * 64;
     constexpr int A_ROWS = T / 4;                                  // rows covered by one 16-byte load per thread
     constexpr int A_LOADS = (BM + A_ROWS - 1) / A_ROWS;            // such loads per thread and step (192 rows: the second half full)
-    constexpr int A_STAGE = A_LOADS * A_ROWS * PK, B_STAGE = PK * BN;            // halves per stage
+    constexpr int B_STAGE = PK * BN;                               // halves per stage
+    constexpr bool DMA = NW == 4;
 
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm0 = (wave / NW) * WM, wn0 = (wave % NW) * WN;
 
-    // states stage: row m at m * 64 bytes, 16-byte chunk c of the row stored at
-    // c ^ ((m >> 2) & 3): sixteen consecutive rows read the same logical chunk
-    // from sixteen different bank groups.  Thread t moves chunk t % 4 of rows
-    // t / 4 + A_ROWS * i through registers (rows >= M re-read row M - 1 and are
-    // dropped at the store).  The tile's columns lie inside the matrix
-    // (launcher's duty).
+    // states stage: row m at m * 64 bytes, 16-byte chunk c of the row at c ^ pipe_swz(m).  Thread t fills position t % 4 of rows
+    // t / 4 + A_ROWS * i (rows >= M re-read row M - 1 and are dropped at the store), from global memory straight to LDS or, in the
+    // 128-column kernel, whose two workgroups per CU leave no LDS for that many stages, through registers.
     struct AStage { u32x4 v[A_LOADS]; };
-    const int a_row = t >> 2, a_chunk = t & 3;
+    const int a_row = t >> 2, a_chunk = (t & 3) ^ pipe_swz(a_row);            // (rows + A_ROWS: same swizzle)
     // every global address is a buffer resource (the tile's rows of states; the whole
     // of the packed matrix, mask, scales, zeros) plus a per-lane 32-bit byte offset that
     // never changes plus a workgroup-uniform 32-bit offset that moves with the K step:
@@ -478,36 +440,49 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
 #pragma unroll
     for (int i = 0; i < A_LOADS; ++i)
         a_off[i] = (uint32_t)((min(a_row + A_ROWS * i, min(a.M - m0, BM) - 1) * a.K + a_chunk * 8) * 2);
-    const int a_dst = a_row * PK + ((a_chunk ^ ((a_row >> 2) & 3)) << 3);       // halves; rows + A_ROWS: same swizzle
     auto load_a = [&](AStage& r, uint32_t step_off) {
 #pragma unroll
         for (int i = 0; i < A_LOADS; ++i) r.v[i] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_off[i], step_off, 0);
     };
     auto write_a = [&](const AStage& r, int stage) {
 #pragma unroll
+        for (int i = 0; i < A_LOADS; ++i) *reinterpret_cast<u32x4*>(&As[stage][i * A_ROWS * PK + t * 8]) = r.v[i];
+    };
+    auto dma_a = [&](int stage, uint32_t step_off) {
+#pragma unroll
         for (int i = 0; i < A_LOADS; ++i)
-            *reinterpret_cast<u32x4*>(&As[stage * A_STAGE + i * A_ROWS * PK + a_dst]) = r.v[i];
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (__attribute__((address_space(3))) void*)&As[stage][i * A_ROWS * PK + wave * 512], 16,
+                                                     a_off[i], step_off, 0, 0);
     };
 
-    // weights: thread owns column bn and packed rows 2 bhb, 2 bhb + 1 of every K step.
-    // scale / zero travel as the aligned 32-bit word that holds the column's half
-    // (sub-dword loads make the compiler wait for every outstanding load); `half_sel`
-    // replicates the wanted half into both lanes of a packed register.
-    // Thread (bn, bhb) decodes rows 16 bhb .. 16 bhb + 15 of the step's 32-row block:
-    // int4 words 2 bhb, 2 bhb + 1; int2 word bhb; int3 words bhb, bhb + 1 (bits
-    // 48 bhb .. 48 bhb + 47 of the block's 96-bit stream); 16:32 sparse: both words
-    // and the mask word of the block.
+    // weights: a thread decodes two chunks of 8 rows of every K step.
+    // int4: word `row` of two adjacent columns, one 8-byte load; the others: column bn, rows 16 bhb .. 16 bhb + 15 of the
+    // step's 32-row block: int2 word bhb; int3 words bhb, bhb + 1 (bits 48 bhb .. 48 bhb + 47 of the block's 96-bit stream); 16:32
+    // sparse: both words and the mask word of the block.
+    // Column 4 n + j of a wave's 64 stands at position 16 j + (n ^ 8 (j / 2)) of its row of chunks: an MFMA tile takes every fourth
+    // column, so that the four tiles leave a lane with four adjacent columns of a row, an 8-byte store; the fragment reads and
+    // the stores of either mapping touch all banks once.
+    // (a last tile that is not full: the columns beyond the last repeat the last 64 and are not written)
     using F = PipeFmt<BITS, SPARSE>;
     constexpr int NWORDS = F::NWORDS;
-    const int bn = t % BN, bhb = t / BN;
-    // (a last tile that is not full: the columns beyond the last repeat the last 64 and are not written)
-    const int bcol = min(s0 + bn, a.S - 64 + (bn & 63));
-    struct Stage { uint32_t w[NWORDS]; uint32_t m; uint32_t sc, ze; };
-    const uint32_t half_sel = (bcol & 1) ? 0x03020302u : 0x01000100u;
-    uint32_t b_off[NWORDS];
+    constexpr bool PAIR = BITS == 4 && !SPARSE;
+    constexpr int W_LOADS = PAIR ? 1 : NWORDS + (SPARSE ? 1 : 0);
+    constexpr int VALU = (72 + TM * TN - 1) / (TM * TN);          // other vector instructions behind an MFMA
+    const int bn = PAIR ? t % (BN / 2) * 2 : t % BN, bhb = PAIR ? t / (BN / 2) : t / BN;
+    const int bcol = min(s0 + (bn & ~63), a.S - 64) + (PAIR ? bn & 63 : 4 * ((bn & 15) ^ (bn >> 2 & 8)) + (bn >> 4 & 3));
+    int b_chunk[2];                                      // where the two chunks go (halves)
 #pragma unroll
-    for (int i = 0; i < NWORDS; ++i)
-        b_off[i] = (uint32_t)((((SPARSE ? 0 : BITS == 4 ? 2 * bhb : bhb) + i) * a.S + bcol) * 4);
+    for (int q = 0; q < 2; ++q)
+        b_chunk[q] = 8 * (PAIR ? bhb * BN + (bn & ~63) + 16 * ((bn & 2) + q) + ((bn >> 2 & 15) ^ (bn << 2 & 8)) : (bhb * 2 + q) * BN + bn);
+    struct Stage { uint32_t w[NWORDS]; uint32_t m; };
+    // scale / zero travel as the aligned 32-bit word that holds the column's half
+    // (sub-dword loads make the compiler wait for every outstanding load); `half_sel`
+    // replicates the wanted half into both lanes of a packed register
+    const uint32_t half_sel = (bcol & 1) ? 0x03020302u : 0x01000100u;
+    uint32_t b_off[W_LOADS];
+#pragma unroll
+    for (int i = 0; i < (PAIR ? 1 : NWORDS); ++i)
+        b_off[i] = (uint32_t)((((SPARSE ? 0 : bhb) + i) * a.S + bcol) * 4);
     const uint32_t m_off = (uint32_t)(bcol * 4);
     const uint32_t m_step = 4u * a.S;                    // bytes of one row of mask words
     const uint32_t sz_off = (uint32_t)((bcol & ~1) * 2);
@@ -528,16 +503,30 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
         const int gu = a.group_units * 2, group = kt / gu;
         return Cursor{kt * b_step, SPARSE ? kt * m_step : 0u, group * g_step, kt, gu - kt % gu};
     };
-    auto load_b = [&](Stage& s, const Cursor& c) {
+    // scale and zero of the thread's column: of the pair of steps that is decoded, and as loaded for the next one (a group is
+    // whole pairs of steps, and a workgroup starts with one)
+    uint32_t next_s, next_z;
+    auto load_b = [&](Stage& s, const Cursor& c, bool first_of_pair) {
+        if constexpr (PAIR) {
+            const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(w_rsrc, b_off[0], c.w, 0);
+            s.w[0] = v.x;
+            s.w[1] = v.y;
+        } else {
 #pragma unroll
-        for (int i = 0; i < NWORDS; ++i) s.w[i] = __builtin_amdgcn_raw_buffer_load_b32(w_rsrc, b_off[i], c.w, 0);
+            for (int i = 0; i < NWORDS; ++i) s.w[i] = __builtin_amdgcn_raw_buffer_load_b32(w_rsrc, b_off[i], c.w, 0);
+        }
         if constexpr (SPARSE) s.m = __builtin_amdgcn_raw_buffer_load_b32(m_rsrc, m_off, c.m, 0);
-        s.sc = __builtin_amdgcn_raw_buffer_load_b32(sc_rsrc, sz_off, c.sz, 0);
-        s.ze = __builtin_amdgcn_raw_buffer_load_b32(ze_rsrc, sz_off, c.sz, 0);
+        if (first_of_pair) {
+            next_s = __builtin_amdgcn_raw_buffer_load_b32(sc_rsrc, sz_off, c.sz, 0);
+            next_z = __builtin_amdgcn_raw_buffer_load_b32(ze_rsrc, sz_off, c.sz, 0);
+        }
     };
-    auto stage_scale = [&](const Stage& s) { return as_h2(__builtin_amdgcn_perm(s.sc, s.sc, half_sel)); };
-    auto stage_negzero = [&](const Stage& s) {
-        return as_h2(__builtin_amdgcn_perm(s.ze, s.ze, half_sel) ^ 0x80008000u);
+    auto take_sz = [&](auto (&co)[PAIR ? 2 : 1]) {
+#pragma unroll
+        for (int q = 0; q < (PAIR ? 2 : 1); ++q) {
+            const uint32_t sel = !PAIR ? half_sel : q ? 0x03020302u : 0x01000100u;
+            co[q].set(as_h2(__builtin_amdgcn_perm(next_s, next_s, sel)), as_h2(__builtin_amdgcn_perm(next_z, next_z, sel)));
+        }
     };
     // the 8 codes of the thread's chunk q (rows 16 bhb + 8 q .. + 7), LSB first
     const int i3_shift = 16 * bhb;
@@ -557,54 +546,54 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
         const uint64_t st = ((uint64_t)s.w[1] << 32) | s.w[0];
         v = (uint32_t)((st >> (2 * skip)) >> (2 * skip));
     };
-    auto write_b_fast = [&](const Stage& s, int stage, int q) {
-        h16x8 w;
-        if constexpr (SPARSE) {
-            uint32_t v, m8;
-            sparse_chunk(s, q, v, m8);
-            w = dequant_chunk_sparse_fast(v, m8, lut, stage_negzero(s), stage_scale(s));
-        } else {
-            w = dequant_chunk_fast<BITS>(chunk_bits(s, q), stage_negzero(s), stage_scale(s));
+    auto decode = [&](const Stage& st, const auto (&co)[PAIR ? 2 : 1], h16x8 (&w)[2]) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const auto& c = co[PAIR ? q : 0];
+            if constexpr (SPARSE) {
+                uint32_t v, m8;
+                sparse_chunk(st, q, v, m8);
+                w[q] = dequant_chunk_sparse(v, m8, lut, c);
+            } else {
+                w[q] = dequant_chunk<BITS>(chunk_bits(st, q), c);
+            }
         }
-        *reinterpret_cast<h16x8*>(&Bs[stage * B_STAGE + ((bhb * 2 + q) * BN + bn) * 8]) = w;
     };
-    f32x16 acc[TM][TN];
+    auto write_b = [&](const h16x8 (&w)[2], int stage) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) *reinterpret_cast<h16x8*>(&Bs[stage * B_STAGE + b_chunk[q]]) = w[q];
+    };
+    f32x4 acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // fragment addresses (halves, inside a stage); k slice ks selects chunk 2 ks + lane / 32
-    int a_frag[TM], b_frag[TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) a_frag[i] = (wm0 + i * 32 + (lane & 31)) * PK;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) b_frag[j] = (wn0 + j * 32 + (lane & 31)) * 8;
-    const int a_sw = (lane >> 2) & 3;                 // row offsets are multiples of 32: same swizzle
-    auto load_frags = [&](int stage, int ks, h16x8 fa[TM], h16x8 fb[TN]) {
-        const int kc = 2 * ks + (lane >> 5);
+    // fragment addresses (halves, inside a stage); a step's 32 k are four chunks, one per lane group of 16
+    // (row offsets are multiples of 16: the same swizzle for all of a lane's rows)
+    const int a_frag = (wm0 + (lane & 15)) * PK + (((lane >> 4) ^ pipe_swz(lane)) << 3);
+    const int b_frag[2] = {((lane >> 4) * BN + wn0 + (lane & 15)) * 8, ((lane >> 4) * BN + wn0 + ((lane & 15) ^ 8)) * 8};
+    auto load_frags = [&](int a_stage, int stage, h16x8 fa[TM], h16x8 fb[TN]) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
-            fa[i] = *reinterpret_cast<const h16x8*>(&As[stage * A_STAGE + a_frag[i] + ((kc ^ a_sw) << 3)]);
+            fa[i] = *reinterpret_cast<const h16x8*>(&As[a_stage][a_frag + i * 16 * PK]);
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-            fb[j] = *reinterpret_cast<const h16x8*>(&Bs[stage * B_STAGE + kc * BN * 8 + b_frag[j]]);
+            fb[j] = *reinterpret_cast<const h16x8*>(&Bs[stage * B_STAGE + b_frag[j >> 1] + j * 128]);
     };
-    auto mfma_slice = [&](const h16x8 fa[TM], const h16x8 fb[TN]) {
+    auto mfma_step = [&](const h16x8 fa[TM], const h16x8 fb[TN]) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[i], fb[j], acc[i][j], 0, 0, 0);
     };
 
     // K steps kt0 .. last of the matrix belong to this workgroup (all of them unless SPLIT)
     const int ksteps = a.K / PK;
-    const int per_split = SPLIT ? (ksteps + nsplit - 1) / nsplit : ksteps;
-    const int kt0 = SPLIT ? split * per_split : 0;
-    const int ktiles = SPLIT ? min(ksteps, kt0 + per_split) - kt0 : ksteps;
+    // (whole pairs of steps; a share has at least four)
+    const int kt0 = SPLIT ? ksteps / 2 * split / nsplit * 2 : 0;
+    const int ktiles = (SPLIT ? ksteps / 2 * (split + 1) / nsplit * 2 : ksteps) - kt0;
     const int last = kt0 + ktiles - 1;
 
     // Cursors of the loads: weights run four K steps ahead of the MFMAs, states
@@ -634,298 +623,155 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
     };
     Stage r[3];
     AStage ra[2];
-    // the first two steps' operands are requested before the look at the scales below, whose
+    // the first steps' operands are requested before the look at the scales below, whose
     // round trip to memory they then share
-    load_a(ra[0], a_cur); advance_a();
-    load_a(ra[1], a_cur); advance_a();
-    load_b(r[0], cur); advance();
-    load_b(r[1], cur); advance();
+    if constexpr (!DMA) {
+        load_a(ra[0], a_cur); advance_a();
+        load_a(ra[1], a_cur); advance_a();
+    }
+    load_b(r[0], cur, true); advance();
+    load_b(r[1], cur, false); advance();
+    if constexpr (DMA) {
+#pragma unroll
+        for (int i = 0; i < A_AHEAD; ++i) { dma_a(i, a_cur); advance_a(); }
+    }
 
     // Does any (group, column) of this tile use exponent quantisation (scale < 0
     // or NaN)?  One pass over the tile's scales (a few KB); the answer is
     // workgroup-uniform and selects between the pipelined loop, whose decode is
-    // the branch-free linear one, and the loops that also serve exponent groups.
-    int& any_expo = *reinterpret_cast<int*>(Bs);          // borrowed before the pipeline starts
-    __syncthreads();
-    if constexpr (SPARSE) {
-        if (t < 256) {
-            uint32_t e[8];
-            sparse_lut_entry(t, e);
-            *reinterpret_cast<u32x4*>(lut + t * 8) = u32x4{e[0], e[1], e[2], e[3]};
-            *reinterpret_cast<u32x4*>(lut + t * 8 + 4) = u32x4{e[4], e[5], e[6], e[7]};
-        }
-    }
-    if (t == 0) any_expo = 0;
-    __syncthreads();
-    {
-        // the tile's scales are `groups` rows of BN / 2 aligned 32-bit words; the threads share them
-        // out and fetch four words each per trip, all in flight together (one round trip to
-        // memory instead of one per group)
-        bool bad = false;
-        const int groups = (ksteps + a.group_units * 2 - 1) / (a.group_units * 2);
-        const int total = groups * (BN / 2);
-        const uint32_t* tile_scales = reinterpret_cast<const uint32_t*>(a.scales + s0);
-        const int64_t row_words = a.S / 2;
-        const int last_word = (a.S - s0) / 2 - 1;
-        for (int i0 = t; i0 < total; i0 += 4 * T) {
-            uint32_t v[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int i = min(i0 + k * T, total - 1);
-                v[k] = tile_scales[(int64_t)(i / (BN / 2)) * row_words + min(i % (BN / 2), last_word)];
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const h16x2 h = as_h2(v[k]);
-                bad |= !(h.x >= (h16)0.0f) | !(h.y >= (h16)0.0f);
+    // the linear one, and the one that also serves exponent groups.  (int2 and int3 have one decode for both.)
+    bool tile_has_expo = false;
+    if constexpr (BITS == 4) {
+        int& any_expo = *reinterpret_cast<int*>(Bs);          // borrowed before the pipeline starts
+        __syncthreads();
+        if constexpr (SPARSE) {
+            if (t < 256) {
+                uint32_t e[8];
+                sparse_lut_entry(t, e);
+                *reinterpret_cast<u32x4*>(lut + t * 8) = u32x4{e[0], e[1], e[2], e[3]};
+                *reinterpret_cast<u32x4*>(lut + t * 8 + 4) = u32x4{e[4], e[5], e[6], e[7]};
             }
         }
-        if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) any_expo = 1;
+        if (t == 0) any_expo = 0;
+        __syncthreads();
+        {
+            // the tile's scales are `groups` rows of BN / 2 aligned 32-bit words; the threads share them
+            // out and fetch four words each per trip, all in flight together (one round trip to
+            // memory instead of one per group)
+            bool bad = false;
+            const int groups = (ksteps + a.group_units * 2 - 1) / (a.group_units * 2);
+            const int total = groups * (BN / 2);
+            const uint32_t* tile_scales = reinterpret_cast<const uint32_t*>(a.scales + s0);
+            const int64_t row_words = a.S / 2;
+            const int last_word = (a.S - s0) / 2 - 1;
+            for (int i0 = t; i0 < total; i0 += 4 * T) {
+                uint32_t v[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int i = min(i0 + k * T, total - 1);
+                    v[k] = tile_scales[(int64_t)(i / (BN / 2)) * row_words + min(i % (BN / 2), last_word)];
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const h16x2 h = as_h2(v[k]);
+                    bad |= !(h.x >= (h16)0.0f) | !(h.y >= (h16)0.0f);
+                }
+            }
+            if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) any_expo = 1;
+        }
+        __syncthreads();
+        tile_has_expo = any_expo != 0;
+        __syncthreads();
     }
-    __syncthreads();
-    const bool tile_has_expo = any_expo != 0;
-    __syncthreads();
 
-    if (!tile_has_expo) {
-        h16x8 fa[2][TM], fb[2][TN];         // fragments of the current and the next k slice
-        // Step kt, u = kt % 6, stage b = kt % 3.  On entry: states and decoded weights
-        // of steps kt, kt+1 are complete in stages b, b+1; ra[kt % 2] holds the states
-        // and r[(kt+2) % 3] the packed weights of step kt+2, which this step moves
-        // into stage b+2; the fragments of slice (kt, 0) are in fa[0] / fb[0].  The
-        // step loads states kt+3 and weights kt+4 into the register sets it does not use.
-        auto body = [&](int b, AStage& ra_new, const AStage& ra_wr, Stage& r_new, const Stage& r_dec) {
-            const int b1 = (b + 1) % P_STAGES, b2 = (b + 2) % P_STAGES;
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                if (ks == 0) load_frags(b, 1, fa[1], fb[1]);
-                else load_frags(b1, 0, fa[0], fb[0]);
-                if (ks == 0) {
-                    load_a(ra_new, a_cur);             // step kt + 3
-                    load_b(r_new, cur);                // step kt + 4
-                    advance_a();
-                    advance();
-                }
-                if (ks == 0) { write_b_fast(r_dec, b2, 0); write_b_fast(r_dec, b2, 1); }
-                if (ks == 1) write_a(ra_wr, b2);
-                mfma_slice(fa[ks], fb[ks]);
-                // scheduling template.  First slice: the next slice's fragment reads, then
-                // every MFMA followed by decode instructions of both of the thread's chunks
-                // (and one of this step's global loads), the two LDS stores of the decoded
-                // chunks last.  Second slice: fragment reads, one MFMA, the LDS stores of the
-                // states, the remaining MFMAs -- every store of the step then has most of a
-                // slice to complete before the barrier asks for it.
-                if (ks == 0) {
-                    __builtin_amdgcn_sched_group_barrier(0x100, TM + TN + (SPARSE ? 4 : 0), 0);
-#pragma unroll
-                    for (int e = 0; e < TM * TN; ++e) {
-                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                        __builtin_amdgcn_sched_group_barrier(0x002, 24 / TM, 0);
-                        if (e < A_LOADS + NWORDS + (SPARSE ? 3 : 2)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-                    }
-                    __builtin_amdgcn_sched_group_barrier(0x200, 2, 0);
-                } else {
-                    __builtin_amdgcn_sched_group_barrier(0x100, TM + TN, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x200, A_LOADS, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x008, TM * TN - 1, 0);
-                }
-            }
-            // this step's LDS stores are complete; then all waves meet
-            __builtin_amdgcn_s_waitcnt(0xC07F);      // lgkmcnt(0) only
-            __builtin_amdgcn_s_barrier();
-        };
-        // the same step in the two orders of PING (phase = 0: MFMAs first; 1: MFMAs last).  Compute-first
-        // waves enter with the step's fragments (both slices) in registers and leave with the next step's;
-        // the others fetch the step's own fragments at its start.
-        auto body_ping = [&](auto phase_tag, int b, AStage& ra_new, const AStage& ra_wr, Stage& r_new, const Stage& r_dec) {
+    // Step kt, u = kt % 6, weights' stage b = kt % 3, states' stage u (registers: b).  On entry states and decoded weights of
+    // steps kt and kt + 1 are complete.  The step stores the decoded weights of step kt + 2 and asks for the packed ones of
+    // kt + 4 and the states of kt + A_AHEAD (registers: moves those of kt + 2 to LDS and asks for kt + 3).  Phase 0:
+    // MFMAs, on fragments fetched in the step before, beside the decode of step kt + 2's weights; then stores, loads, the next
+    // step's fragments.  Phase 1: the step's own fragments, stores of what the step before decoded, loads; then MFMAs
+    // beside the decode of step kt + 3's weights.
+    h16x8 fa[TM], fb[TN], dec[2];
+    auto walk = [&](auto mode) {
+        Coef<BITS, decltype(mode)::value> co[PAIR ? 2 : 1];
+        auto body = [&](auto phase_tag, int u, AStage& ra_new, const AStage& ra_wr, Stage& r_new, const Stage& r_dec) {
             constexpr int phase = decltype(phase_tag)::value;
-            const int b1 = (b + 1) % P_STAGES, b2 = (b + 2) % P_STAGES;
-            if constexpr (phase == 0) {
-                mfma_slice(fa[0], fb[0]);
-                mfma_slice(fa[1], fb[1]);
-            }
-            load_frags(phase == 0 ? b1 : b, 0, fa[0], fb[0]);
-            load_frags(phase == 0 ? b1 : b, 1, fa[1], fb[1]);
-            load_a(ra_new, a_cur);             // step kt + 3
-            load_b(r_new, cur);                // step kt + 4
-            advance_a();
-            advance();
-            write_b_fast(r_dec, b2, 0);
-            write_b_fast(r_dec, b2, 1);
-            write_a(ra_wr, b2);
+            const int b = u % P_STAGES, b1 = (u + 1) % P_STAGES, b2 = (u + 2) % P_STAGES;
+            auto stores_and_loads = [&]() {
+                write_b(dec, b2);
+                if constexpr (!DMA) write_a(ra_wr, b2);
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (DMA) dma_a((u + A_AHEAD) % 6, a_cur);
+                else load_a(ra_new, a_cur);
+                load_b(r_new, cur, u % 2 == 0);
+                advance_a();
+                advance();
+                __builtin_amdgcn_sched_barrier(0);
+            };
             if constexpr (phase == 1) {
-                mfma_slice(fa[0], fb[0]);
-                mfma_slice(fa[1], fb[1]);
+                load_frags(DMA ? u : b, b, fa, fb);
+                __builtin_amdgcn_sched_barrier(0);
+                stores_and_loads();
             }
-            // scheduling template: the MFMAs as one cluster with the decode instructions in their
-            // shadow (an MFMA occupies the pipe for 32 cycles, the wave issues three or four other
-            // instructions meanwhile); fragment reads, global loads and LDS stores outside it
+            if ((u + phase) % 2 == 0) take_sz(co);
+            decode(r_dec, co, dec);
+            mfma_step(fa, fb);
+            // (the decode in the shadow of the MFMAs: one occupies the pipe for 16 cycles, two waves of a SIMD issue two
+            // other vector instructions each meanwhile)
+#pragma unroll
+            for (int e = 0; e < TM * TN; ++e) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, decltype(mode)::value ? 2 * VALU : VALU, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (phase == 0) stores_and_loads();
+            // the step's stores are complete (lgkmcnt(0)) and, of the states loaded straight to LDS, all but the last two steps'
+            __builtin_amdgcn_s_waitcnt(DMA ? wait_counts(2 * (A_LOADS + W_LOADS) + 2, 0) : wait_counts(63, 0));
             if constexpr (phase == 0) {
-#pragma unroll
-                for (int e = 0; e < 2 * TM * TN; ++e) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, TM == 4 ? 3 : 4, 0);
-                }
-                __builtin_amdgcn_sched_group_barrier(0x100, 2 * (TM + TN) + (SPARSE ? 4 : 0), 0);
-                __builtin_amdgcn_sched_group_barrier(0x020, A_LOADS + NWORDS + (SPARSE ? 3 : 2), 0);
-                __builtin_amdgcn_sched_group_barrier(0x200, A_LOADS + 2, 0);
-            } else {
-                __builtin_amdgcn_sched_group_barrier(0x100, 2 * (TM + TN) + (SPARSE ? 4 : 0), 0);
-                __builtin_amdgcn_sched_group_barrier(0x020, A_LOADS + NWORDS + (SPARSE ? 3 : 2), 0);
-                __builtin_amdgcn_sched_group_barrier(0x200, A_LOADS, 0);
-#pragma unroll
-                for (int e = 0; e < 2 * TM * TN; ++e) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, TM == 4 ? 3 : 4, 0);
-                }
-                __builtin_amdgcn_sched_group_barrier(0x200, 2, 0);
+                load_frags(DMA ? (u + 1) % 6 : b1, b1, fa, fb);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            __builtin_amdgcn_sched_barrier(0);       // nothing of this step moves behind the barrier
-            __builtin_amdgcn_s_waitcnt(0xC07F);      // lgkmcnt(0) only
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
         };
-        write_a(ra[0], 0);
-        write_a(ra[1], 1);
-        load_a(ra[0], a_cur); advance_a();              // step 2
-#pragma unroll
-        for (int q = 0; q < 2; ++q) { write_b_fast(r[0], 0, q); write_b_fast(r[1], 1, q); }
-        load_b(r[2], cur); advance();                   // step 2
-        load_b(r[0], cur); advance();                   // step 3
+        if constexpr (!DMA) {
+            write_a(ra[0], 0);
+            write_a(ra[1], 1);
+            load_a(ra[0], a_cur); advance_a();              // step 2
+        }
+        take_sz(co);
+        decode(r[0], co, dec);
+        write_b(dec, 0);
+        decode(r[1], co, dec);
+        write_b(dec, 1);
+        if constexpr (DMA) __builtin_amdgcn_s_waitcnt(wait_counts(0, 15));         // steps 0 ... A_AHEAD - 1 of the states
+        load_b(r[2], cur, true); advance();             // step 2
+        load_b(r[0], cur, false); advance();            // step 3
         __syncthreads();
-        load_frags(0, 0, fa[0], fb[0]);
-        // LDS stages and weight registers rotate with period 3, state registers with
-        // period 2: six steps per trip, unrolled so that all of them are compile-time names
-        if constexpr (!PING) {
+        // LDS stages and weight registers rotate with period 3, states with 2 or 6: six steps per trip, unrolled so that
+        // all of them are compile-time names
+        auto run = [&](auto phase_tag) {
+            constexpr int ahead = 2 + decltype(phase_tag)::value;
             for (int kt = 0; kt < ktiles; kt += 6) {
 #pragma unroll
                 for (int u = 0; u < 6; ++u) {
                     if (u > 0 && kt + u >= ktiles) break;
-                    body(u % 3, ra[(u + 1) % 2], ra[u % 2], r[(u + 1) % 3], r[(u + 2) % 3]);
+                    body(phase_tag, u, ra[(u + 1) % 2], ra[u % 2], r[(u + 1) % 3], r[(u + ahead) % 3]);
                 }
             }
+        };
+        if (PING && wave < NW) {
+            load_frags(0, 0, fa, fb);
+            if constexpr (PING) run(std::integral_constant<int, 0>{});
         } else {
-            auto run = [&](auto phase_tag) {
-                for (int kt = 0; kt < ktiles; kt += 6) {
-#pragma unroll
-                    for (int u = 0; u < 6; ++u) {
-                        if (u > 0 && kt + u >= ktiles) break;
-                        body_ping(phase_tag, u % 3, ra[(u + 1) % 2], ra[u % 2], r[(u + 1) % 3], r[(u + 2) % 3]);
-                    }
-                }
-            };
-            if (__builtin_amdgcn_readfirstlane(wave) < NW) {
-                load_frags(0, 1, fa[1], fb[1]);
-                run(std::integral_constant<int, 0>{});
-            } else {
-                run(std::integral_constant<int, 1>{});
-            }
+            take_sz(co);
+            decode(r[2], co, dec);
+            run(std::integral_constant<int, 1>{});
         }
-    } else if constexpr (!SPARSE && NW == 4) {
-        // A tile with exponent-mode groups: the same three-stage pipeline (in the plain order of a
-        // step: fragments, loads, decode between the MFMAs, stores, barrier) with the decode that
-        // serves either mode per thread.  (256-column tiles only: in the 128-column kernel, which
-        // keeps two workgroups per compute unit, this loop does not fit the registers, and its
-        // spills slowed the linear loop down as well.)
-        auto write_b_mixed = [&](const Stage& s, int stage, int q) {
-            const h16x2 s2 = stage_scale(s);
-            const bool expo = !(s2.x >= (h16)0.0f);
-            const h16x8 w = dequant_chunk_mixed<BITS>(chunk_bits(s, q), expo, stage_negzero(s), s2);
-            *reinterpret_cast<h16x8*>(&Bs[stage * B_STAGE + ((bhb * 2 + q) * BN + bn) * 8]) = w;
-        };
-        h16x8 fa[2][TM], fb[2][TN];
-        auto body_mixed = [&](int b, AStage& ra_new, const AStage& ra_wr, Stage& r_new, const Stage& r_dec) {
-            const int b1 = (b + 1) % P_STAGES, b2 = (b + 2) % P_STAGES;
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                if (ks == 0) load_frags(b, 1, fa[1], fb[1]);
-                else load_frags(b1, 0, fa[0], fb[0]);
-                if (ks == 0) {
-                    load_a(ra_new, a_cur);             // step kt + 3
-                    load_b(r_new, cur);                // step kt + 4
-                    advance_a();
-                    advance();
-                    write_b_mixed(r_dec, b2, 0);
-                    write_b_mixed(r_dec, b2, 1);
-                } else {
-                    write_a(ra_wr, b2);
-                }
-                mfma_slice(fa[ks], fb[ks]);
-                if (ks == 0) {
-                    __builtin_amdgcn_sched_group_barrier(0x100, TM + TN, 0);
-#pragma unroll
-                    for (int e = 0; e < TM * TN; ++e) {
-                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                        __builtin_amdgcn_sched_group_barrier(0x002, TM == 4 ? 14 : TM == 3 ? 19 : 28, 0);
-                        if (e < A_LOADS + NWORDS + 2) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-                    }
-                    __builtin_amdgcn_sched_group_barrier(0x200, 2, 0);
-                } else {
-                    __builtin_amdgcn_sched_group_barrier(0x100, TM + TN, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x200, A_LOADS, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x008, TM * TN - 1, 0);
-                }
-            }
-            __builtin_amdgcn_s_waitcnt(0xC07F);      // lgkmcnt(0) only
-            __builtin_amdgcn_s_barrier();
-        };
-        write_a(ra[0], 0);
-        write_a(ra[1], 1);
-        load_a(ra[0], a_cur); advance_a();              // step 2
-#pragma unroll
-        for (int q = 0; q < 2; ++q) { write_b_mixed(r[0], 0, q); write_b_mixed(r[1], 1, q); }
-        load_b(r[2], cur); advance();                   // step 2
-        load_b(r[0], cur); advance();                   // step 3
-        __syncthreads();
-        load_frags(0, 0, fa[0], fb[0]);
-        for (int kt = 0; kt < ktiles; kt += 6) {
-#pragma unroll
-            for (int u = 0; u < 6; ++u) {
-                if (u > 0 && kt + u >= ktiles) break;
-                body_mixed(u % 3, ra[(u + 1) % 2], ra[u % 2], r[(u + 1) % 3], r[(u + 2) % 3]);
-            }
-        }
-    } else {
-        // A tile with exponent-mode groups, 16:32 and the 128-column tiles (whose registers do not hold a second copy
-        // of the pipelined loop): a plain loop over two LDS stages -- the step's operands, requested two steps
-        // earlier, are decoded (either mode per thread, without a branch) and stored, the operands of the step
-        // after next are requested, one barrier, the step's MFMAs.  (A stage is written again two steps later,
-        // and every wave has left its reads of it behind when it arrives at the barrier in between.)
-        auto write_b_two_modes = [&](const Stage& s, int stage, int q) {
-            const h16x2 s2 = stage_scale(s);
-            const bool expo = !(s2.x >= (h16)0.0f);
-            h16x8 w;
-            if constexpr (SPARSE) {
-                uint32_t v, m8;
-                sparse_chunk(s, q, v, m8);
-                w = dequant_chunk_sparse_mixed(v, m8, lut, expo, stage_negzero(s), s2);
-            } else {
-                w = dequant_chunk_mixed<BITS>(chunk_bits(s, q), expo, stage_negzero(s), s2);
-            }
-            *reinterpret_cast<h16x8*>(&Bs[stage * B_STAGE + ((bhb * 2 + q) * BN + bn) * 8]) = w;
-        };
-        h16x8 fa[TM], fb[TN];
-        for (int kt = 0; kt < ktiles; kt += 2) {
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                if (u > 0 && kt + u >= ktiles) break;
-                write_a(ra[u], u);
-                write_b_two_modes(r[u], u, 0);
-                write_b_two_modes(r[u], u, 1);
-                if (kt + u + 2 < ktiles) {
-                    load_a(ra[u], a_cur); advance_a();
-                    load_b(r[u], cur); advance();
-                }
-                __syncthreads();
-#pragma unroll
-                for (int ks = 0; ks < 2; ++ks) {
-                    load_frags(u, ks, fa, fb);
-                    mfma_slice(fa, fb);
-                }
-            }
-        }
-    }
+    };
+    if (BITS == 4 && tile_has_expo) walk(std::bool_constant<BITS == 4>{});
+    else walk(std::false_type{});
+    // (no load to LDS is in flight any more when the LDS is used otherwise or given back)
+    if constexpr (DMA) __builtin_amdgcn_s_waitcnt(wait_counts(0, 15));
     if (SPLIT && nsplit > 1) {
         // Every workgroup of the tile stores its partial accumulators (16 bytes per lane and
         // store: register group g of thread t at (g * T + t) * 16 -- whole cache lines per wave)
@@ -943,13 +789,9 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-                    __builtin_amdgcn_raw_buffer_store_b128(bitcast<u32x4>(v), mine, (((i * TN + j) * 4 + q) * T + t) * 16, 0, THROUGH);
-                }
+                __builtin_amdgcn_raw_buffer_store_b128(bitcast<u32x4>(acc[i][j]), mine, ((i * TN + j) * T + t) * 16, 0, THROUGH);
         __builtin_amdgcn_s_waitcnt(0);                 // every store of this thread has been acknowledged
-        int* const flag = reinterpret_cast<int*>(As);
+        int* const flag = reinterpret_cast<int*>(Bs);
         __syncthreads();
         if (t == 0) *flag = __hip_atomic_fetch_add(a.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
@@ -959,9 +801,7 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+                for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
         for (int sp = nsplit > 2 ? 0 : 1 - split; sp < (nsplit > 2 ? nsplit : 2 - split); ++sp) {
             const __amdgpu_buffer_rsrc_t theirs = __builtin_amdgcn_make_buffer_rsrc(
@@ -970,34 +810,30 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const f32x4 v = bitcast<f32x4>(__builtin_amdgcn_raw_buffer_load_b128(
-                            theirs, (((i * TN + j) * 4 + q) * T + t) * 16, 0, THROUGH));
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) acc[i][j][4 * q + e] += v[e];
-                    }
+                    acc[i][j] += bitcast<f32x4>(__builtin_amdgcn_raw_buffer_load_b128(theirs, ((i * TN + j) * T + t) * 16, 0, THROUGH));
         }
     }
     if (s0 + wn0 >= a.S) return;                       // (a wave's 64 columns are inside or outside as one)
+    // register r of tile (i, j) is row 16 i + 4 (lane / 16) + r, column 4 (lane % 16) + j of the wave's
+    h16* const out = outs + (int64_t)(m0 + wm0 + 4 * (lane >> 4)) * a.S + s0 + wn0 + 4 * (lane & 15);
+    const int rows = a.M - (m0 + wm0 + 4 * (lane >> 4));
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const int col = s0 + wn0 + j * 32 + (lane & 31);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = m0 + wm0 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (row < a.M) outs[(int64_t)row * a.S + col] = (h16)acc[i][j][r];
-            }
-        }
+        for (int r = 0; r < 4; ++r)
+            if (16 * i + r < rows)
+                *reinterpret_cast<h16x4*>(out + (int64_t)(16 * i + r) * a.S) =
+                    h16x4{(h16)acc[i][0][r], (h16)acc[i][1][r], (h16)acc[i][2][r], (h16)acc[i][3][r]};
 }
 
 template <int BITS, bool SPARSE, int NW, int TM, bool PING, bool SPLIT>
 __global__ __launch_bounds__(NW * 128, NW == 2 ? 2 : 1) void matmul_kernel_pipe(MatmulArgs a) {
-    constexpr int BM = TM * 64, BN = NW * 64;
+    constexpr int BM = TM * 32, BN = NW * 64;
     constexpr int A_ROWS = NW * 32;
-    __shared__ __attribute__((aligned(16))) h16 As[P_STAGES * ((BM + A_ROWS - 1) / A_ROWS) * A_ROWS * PK];
+    // (each stage of the states an array of its own: in one array every fragment read would wait for all loads in flight)
+    constexpr int A_HALVES = (BM + A_ROWS - 1) / A_ROWS * A_ROWS * PK;
+    __shared__ __attribute__((aligned(16))) h16 A0[A_HALVES], A1[A_HALVES], A2[A_HALVES];
+    __shared__ __attribute__((aligned(16))) h16 A3[NW == 4 ? A_HALVES : 8], A4[NW == 4 ? A_HALVES : 8], A5[NW == 4 ? A_HALVES : 8];
     __shared__ __attribute__((aligned(16))) h16 Bs[P_STAGES * PK * BN];
     __shared__ __attribute__((aligned(16))) uint32_t Lut[SPARSE ? SPARSE_LUT_WORDS : 4];
     // (split-K: the workgroups of a tile are neighbours in the grid, so they run at about the same time;
@@ -1034,21 +870,25 @@ __global__ __launch_bounds__(NW * 128, NW == 2 ? 2 : 1) void matmul_kernel_pipe(
         tile_m = bid % a.tiles_m, tile_n = bid / a.tiles_m;
     }
     const int64_t boff = blockIdx.z;
+    h16* As[pipe_a_stages(NW)];
+    As[0] = A0; As[1] = A1; As[2] = A2;
+    if constexpr (NW == 4) { As[3] = A3; As[4] = A4; As[5] = A5; }
     pipe_tile<BITS, SPARSE, TM, NW, PING, SPLIT>(a, tile_m * BM, tile_n * BN, a.x + boff * a.M * (int64_t)a.K,
                                           a.outs + boff * a.M * (int64_t)a.S, As, Bs, Lut, slot, split, nsplit);
 }
 
-template <int BITS, bool SPARSE, int NW, int TM = 4, bool PING = false>
+template <int BITS, bool SPARSE, int NW, int TM = 8, bool PING = false>
 static void launch_pipe(MatmulArgs a, int64_t B, hipStream_t st) {
-    a.tiles_m = (a.M + TM * 64 - 1) / (TM * 64);
+    a.tiles_m = (a.M + TM * 32 - 1) / (TM * 32);
     a.tiles_n = (a.S + NW * 64 - 1) / (NW * 64);
     const int total = a.tiles_m * a.tiles_n;
     const dim3 grid(a.split_from + (total - a.split_from) * a.ksplit, 1, (unsigned)B), block(NW * 128);
     a.by_columns = a.tiles_n % 8 == 0;
+    // (the word behind the tile tells the dense formats' variants 6 and 9 apart; other tiles read `plain` whatever their order)
     if (noting("matmul_kernel_pipe<bits=%d,%s,tile=%dx%d,%s> tiles=%d ksplit=%d split_from=%d workgroups=%u batch=%d", BITS,
-               SPARSE ? "16:32" : "dense", TM * 64, NW * 64, PING ? "two-phase" : "plain", total, a.ksplit, a.split_from, grid.x, (int)B))
+               SPARSE ? "16:32" : "dense", TM * 32, NW * 64, PING && !SPARSE && TM > 4 ? "two-phase" : "plain", total, a.ksplit, a.split_from, grid.x, (int)B))
         return;
-    if constexpr (TM != 3) {
+    if constexpr (TM != 6) {
         if (a.ksplit > 1) {
             hipLaunchKernelGGL((matmul_kernel_pipe<BITS, SPARSE, NW, TM, PING, true>), grid, block, 0, st, a);
             return;
@@ -1247,11 +1087,10 @@ static void launch(MatmulArgs a, int64_t B, hipStream_t st, void* workspace, siz
     }
     if (variant == 1) launch_tile<BITS, SPARSE, 128, 128, 64, 64>(a, B, st);
     else if (variant == 3) launch_tile<BITS, SPARSE, 128, 256, 128, 64>(a, B, st);
-    // (256 x 256: the dense formats run the two halves of the workgroup in opposite phases, 2-3 %
-    // faster; the 16:32 decode has no registers to spare for it.  Variant 9 forces the plain order.)
-    else if (variant == 7) launch_pipe<BITS, SPARSE, 4, 2>(a, B, st);
-    else if (variant == 8) launch_pipe<BITS, SPARSE, 4, 3, !SPARSE>(a, B, st);
-    else if (variant == 6 && !SPARSE) launch_pipe<BITS, SPARSE, 4, 4, true>(a, B, st);
+    // (variant 9 forces 256 x 256 without the two phases: 9 % slower, 16:32 4 %)
+    else if (variant == 7) launch_pipe<BITS, SPARSE, 4, 4, true>(a, B, st);
+    else if (variant == 8) launch_pipe<BITS, SPARSE, 4, 6, true>(a, B, st);
+    else if (variant == 6) launch_pipe<BITS, SPARSE, 4, 8, true>(a, B, st);
     else if (variant == 6 || variant == 9) launch_pipe<BITS, SPARSE, 4>(a, B, st);
     else if constexpr (!SPARSE) launch_pipe<BITS, false, 2>(a, B, st);
 }

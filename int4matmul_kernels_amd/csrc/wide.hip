@@ -41,12 +41,6 @@ namespace i4 {
 constexpr int RSRC_FLAGS = 0x00020000;                // raw buffer, 32-bit data format
 constexpr uint32_t BEYOND = 0x80000000u;              // ORed into a lane's offset: beyond every buffer here, the load returns 0
 
-// two 8-bit floats (4 exponent, 3 mantissa bits) -> halves times a power of two, exactly; a byte q < 16 is q 2^-9
-template <bool HI>
-__device__ __forceinline__ h16x2 from_fp8(uint32_t bytes, float scale) {
-    return bitcast<h16x2>(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)bytes, scale, HI));
-}
-
 // packed rows of a 64-row unit, and words per column that a lane loads of it
 template <int BITS, bool SPARSE> struct WideFmt;
 template <> struct WideFmt<4, false> { static constexpr int ROWS = 8, WORDS = 4; };
