@@ -888,30 +888,87 @@ static void launch_pipe(MatmulArgs a, int64_t B, hipStream_t st) {
     if (noting("matmul_kernel_pipe<bits=%d,%s,tile=%dx%d,%s> tiles=%d ksplit=%d split_from=%d workgroups=%u batch=%d", BITS,
                SPARSE ? "16:32" : "dense", TM * 32, NW * 64, PING && !SPARSE && TM > 4 ? "two-phase" : "plain", total, a.ksplit, a.split_from, grid.x, (int)B))
         return;
-    if constexpr (TM != 6) {
-        if (a.ksplit > 1) {
-            hipLaunchKernelGGL((matmul_kernel_pipe<BITS, SPARSE, NW, TM, PING, true>), grid, block, 0, st, a);
-            return;
-        }
-    }
-    hipLaunchKernelGGL((matmul_kernel_pipe<BITS, SPARSE, NW, TM, PING, false>), grid, block, 0, st, a);
+    if (a.ksplit > 1) hipLaunchKernelGGL((matmul_kernel_pipe<BITS, SPARSE, NW, TM, PING, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((matmul_kernel_pipe<BITS, SPARSE, NW, TM, PING, false>), grid, block, 0, st, a);
 }
 
-// The pipelined kernel takes any whole number of 64 columns; the last tile may be partly empty, up to an eighth of the
-// columns in all (16:32: half, its general tiles are the slowest).  Before, such outputs went to the general tiles, which hide
+// The pipelined kernel takes any whole number of 64 columns; the last tile may be partly empty, up to half of the
+// columns in all (its 128-column form: an eighth).  Before, such outputs went to the general tiles, which hide
 // less of their loads and cannot split K (us, general / here: int4, K=9280, S=1600, 700 rows 135 / 54, S=14400, 1100 rows 422 /
 // 351; int2 there 239 / 54 and 699 / 341; 16:32 280 / 73 and 846 / 385; int4, K=9280, S=9344 -- 256 x 128 tiles before --
 // 1100 rows 280 / 214).
-static bool tile_columns(int64_t S, int width, bool sparse) {
-    return S % 64 == 0 && (S + width - 1) / width * width * 8 <= S * (sparse ? 12 : 9);
+static bool tile_columns(int64_t S, int width, bool half) {
+    return S % 64 == 0 && (S + width - 1) / width * width * 8 <= S * (half ? 12 : 9);
 }
 
-// ---- split-K plan.  Shapes with at most 128 tiles of 256 x 256 leave more than half of the GPU
-// idle; they run as 256 x 128 tiles (16:32: 256 x 256) with `ksplit` workgroups per tile.  The factor
-// minimises a cost in K steps fitted to measurements (K = 4096 ... 20480, 32 ... 240 tiles):
-// rounds of 256 workgroups x (steps per workgroup + 20 for its prologue and hand-over) + 6 per split.
 constexpr int64_t MM_SPLIT_MAX_TILES = 1024;             // counters: one int per tile in 4 KB
 constexpr int64_t MM_SPLIT_MAX_BYTES = 192ll << 20;      // cap of the partial tiles
+
+// ---- plan of the tiles.  Heights of 128 ... 256 rows in steps of 32, all 256 columns wide, one workgroup per CU, each K split
+// `ksplit` ways or not, or only the tiles of a last, partly filled round (from `split_from` on): the candidate that a cost model
+// finds cheapest, in us,
+//     rounds of 256 workgroups, each  steps x step(height) x (1 + fill x share of the CUs^3) + fixed(height)      (*)
+//     + (split: (way x ways + hand x share of the CUs) x height / 256)
+// the last of several rounds with its share of the CUs raised towards 1 by `last`, full ones times `round`.  (*) is the power limit:
+// a GPU filled to the last CU runs its K steps 40 % slower than an almost empty one.  Fitted per format to 870 ... 2050 timed
+// launches (K = 1024 ... 28672, S = 1024 ... 28672, 257 ... 4096 rows); on these shapes its pick is 1.0 - 1.2 % off the best
+// candidate on average, 9 - 16 % at worst.  Before, a tree of rules chose among 128, 192 and 256 rows and 256 x 128 tiles, of which
+// the last are the best candidate on none of 210 shapes: above 512 rows this plan takes 10 % (int4), 15 % (int3), 14 % (int2) and
+// 11 % (16:32) less time on average, at most 3 % more on a shape (us: int4, K=16128, S=3072, 1411 rows 217 / 151; K=9216, S=2304, 1151
+// rows 98 / 70; int3, K=28096, S=2176, 880 rows 201 / 134; K=S=4096, 777 rows on S=11008 77 / 72).
+struct TileCost { double step[5], fixed[5], fill, way, hand, round, last; };
+static const TileCost tile_cost[4] = {                // int4, int3, int2, 16:32
+    {{0.373, 0.434, 0.466, 0.521, 0.555}, {4.151, 4.233, 4.77, 4.391, 5.388}, 0.369, 2.82, 19.858, 1.065, 0.292},
+    {{0.405, 0.462, 0.493, 0.536, 0.58}, {3.632, 4.086, 3.915, 4.283, 5.317}, 0.406, 2.965, 19.124, 1.027, 0.321},
+    {{0.376, 0.423, 0.463, 0.515, 0.544}, {2.878, 3.789, 3.887, 3.45, 5.247}, 0.344, 2.974, 18.171, 1.042, 0.363},
+    {{0.59, 0.659, 0.686, 0.759, 0.817}, {5.287, 5.577, 5.793, 5.759, 6.161}, 0.131, 3.381, 18.391, 1.061, 0.347}};
+struct TilePlan { int tm; int ksplit; int64_t split_from, tiles; size_t part_bytes; double us; };
+// `only`: this height alone (0: any); `scratch`: bytes for partial tiles, splits that need more are no candidates
+static TilePlan plan_tiles(int bits, bool sparse, int64_t M, int64_t K, int64_t S, size_t scratch, int only) {
+    TilePlan best{0, 1, 0, 0, 0, 1e30};
+    const TileCost& c = tile_cost[sparse ? 3 : 4 - bits];
+    const int64_t columns = (S + 255) / 256, steps = K / 32, forced = tuning(TUNE_MM_SPLIT), tail_knob = tuning(TUNE_MM_TAIL);
+    const int64_t room = (int64_t)std::min<size_t>(scratch, MM_SPLIT_MAX_BYTES);
+    for (int tm = 4; tm <= 8; ++tm) {
+        if (only != 0 && tm != only) continue;
+        const int64_t total = (M + 32 * tm - 1) / (32 * tm) * columns, tile_bytes = 32 * 256 * 4 * (int64_t)tm;
+        const double share = tm / 8.0;
+        auto one = [&](double n, double fill) { return n * c.step[tm - 4] * (1.0 + c.fill * fill * fill * fill) + c.fixed[tm - 4]; };
+        auto take = [&](double us, int64_t ks, int64_t from) {
+            if (us < best.us) best = TilePlan{tm, (int)ks, from, total, ks > 1 ? (size_t)((total - from) * ks * tile_bytes) : 0, us};
+        };
+        // (16:32 in tiles of 224 rows is not split: K=4096, S=8192, 896 rows keep 256 rows two ways, 86 us to 79)
+        for (int64_t ks = 1; ks <= (sparse && tm == 7 ? 1 : 8); ++ks) {
+            if (ks > 1 && (steps / ks < 8 || total > MM_SPLIT_MAX_TILES || total * ks * tile_bytes > room || forced == 1)) break;
+            const int64_t wgs = total * ks, rounds = (wgs + 255) / 256;
+            const double n = (double)steps / ks, last = (wgs - (rounds - 1) * 256) / 256.0;
+            double us = (rounds - 1) * c.round * one(n, 1.0) + one(n, rounds > 1 ? last + (1.0 - last) * c.last : last);
+            if (ks > 1) us += (c.way * ks + c.hand * (rounds - 1 + last)) * share;
+            // (256 rows: preferred within 6 % where they pad none and are not split, K=20480, S=5120, 2048 rows 382 us, 374 in tiles of 192;
+            // split 16:32 tiles come out 8 % too high)
+            if (tm == 8 && ks == 1 && M % 256 == 0) us /= 1.06;
+            if (tm == 8 && ks > 1 && sparse) us /= 1.05;
+            take(forced >= 2 && ks == forced ? 0.0 : us, ks, 0);
+        }
+        // the tiles of the last round alone, over at most half of the GPU (two ways from 64 tiles on, where the second adds the first
+        // one's partial tile to its registers and nothing else is read back) in shares of at least 32 steps (K=4096, S=8192, 2304 rows,
+        // 32 tiles in the tail: eight ways 197 us, four ways 170)
+        const int64_t tail = total % 256;
+        if (tm != 8 || total <= 256 || tail == 0 || tail > 128 || tail_knob == 1 || (tail > 96 && K < 3072)) continue;
+        const int64_t ks = std::min<int64_t>({std::max<int64_t>(2, 128 / tail), tail_knob >= 2 ? tail_knob : 8, steps / 32});
+        if (ks < 2 || tail * ks * tile_bytes > room) continue;
+        const double fill = tail * ks / 256.0;
+        const double us = total / 256 * c.round * one(steps, 1.0) + one((double)steps / ks, fill + (1.0 - fill) * c.last) + (c.way * ks + c.hand * fill) * share;
+        // (preferred within 5 %: the model has few of these to go by)
+        take(us / 1.05, ks, total - tail);
+    }
+    best.us += 2.0;
+    return best;
+}
+
+// ---- what earlier forms of the tile kernels split along K.  It decides still which workspaces the last chunk of a large batch is taken
+// to have (last_chunk_as_others, a line of precision) and the ways of the 128-column tiles.  Shapes with at most 128 tiles of 256 x 256:
+// 256 x 128 tiles (16:32: 256 x 256) with `ksplit` workgroups per tile, by a cost in K steps.
 struct SplitPlan { int ksplit; int64_t tiles; int64_t tile_bytes; };
 static SplitPlan plan_split(bool sparse, int64_t B, int64_t M, int64_t K, int64_t S) {
     const SplitPlan none{1, 0, 0};
@@ -921,11 +978,6 @@ static SplitPlan plan_split(bool sparse, int64_t B, int64_t M, int64_t K, int64_
     SplitPlan p{1, m_pad / 256 * ((S + (sparse ? 255 : 127)) / (sparse ? 256 : 128)) * B, sparse ? 256 * 256 * 4 : 256 * 128 * 4};
     if (p.tiles > MM_SPLIT_MAX_TILES) return none;
     const int64_t steps = K / 32, forced = tuning(TUNE_MM_SPLIT);
-    // (16:32, whose 256 x 256 tiles run one per CU: a GPU filled to the last CU runs its K steps 39 % slower than a
-    // nearly empty one -- the power limit --, three quarters full 15 % slower; fitted to 320 timed launches, K = 2048 ...
-    // 14336, 16 ... 128 tiles, 1 ... 8 ways: 64 tiles at K=4096 four ways 79 us, three ways 68; 32 tiles at K=14336 eight
-    // ways 125, six ways 106.  Its pick is within 1 % of the best measured factor on average, 10 % at worst; without
-    // the term 3 % / 20 %.  The dense formats' 256 x 128 tiles, two workgroups per CU, are within 1.4 % / 11 % as is.)
     auto cost = [&](int64_t ks) -> double {
         const int64_t wgs = p.tiles * ks, rounds = (wgs + 255) / 256;
         const double own = (double)(rounds * ((steps + ks - 1) / ks + 20));
@@ -944,20 +996,13 @@ static SplitPlan plan_split(bool sparse, int64_t B, int64_t M, int64_t K, int64_
     return p;
 }
 
-// ---- split of the last round.  256 x 256 tiles run one per CU, in rounds of 256; when the last round
-// would fill at most half of the GPU, its tiles -- and only they -- are split along K over as many
-// workgroups as fit half of the GPU (at least two per tile, at least 32 K steps each).
+// and the tiles of a last round of 256 x 256 ones that fills at most half of the GPU
 struct TailPlan { int ksplit; int64_t split_from, tiles; };
 static TailPlan plan_tail(bool sparse, int64_t B, int64_t M, int64_t K, int64_t S) {
     const TailPlan none{1, 0, 0};
     if (B != 1 || !tile_columns(S, 256, sparse) || tuning(TUNE_MM_TAIL) == 1) return none;
     const int64_t total = (M + 255) / 256 * ((S + 255) / 256), tail = total % 256;
     if (total <= 256 || tail == 0 || tail > 128) return none;
-    // (measured, K = 2048 ... 8192, tails of 16 ... 128 tiles: the split pays while its workgroups fill at most half of
-    // the GPU -- two per tile from 64 tiles on, where the second adds the first one's partial tile to its registers
-    // and nothing else is read back -- and while a share keeps 32 K steps: K=4096, S=8192, 2304 rows, 32 tiles in
-    // the tail: eight ways 197 us, four ways 170; K=2048, S=8192, 2560 rows, 64 tiles: four ways 121, two ways 101,
-    // unsplit 107; a tail of 97 ... 128 tiles on K = 2048 is better left whole, 110 against 117)
     if (tail > 96 && K < 3072) return none;
     const int64_t cap = tuning(TUNE_MM_TAIL) >= 2 ? tuning(TUNE_MM_TAIL) : 8;
     const int64_t ks = std::min<int64_t>({std::max<int64_t>(2, 128 / tail), cap, K / 32 / 32});
@@ -974,125 +1019,72 @@ static void launch_tile(MatmulArgs a, int64_t B, hipStream_t st) {
     hipLaunchKernelGGL((matmul_kernel<BITS, SPARSE, BM, BN, WM, WN>), grid, block, 0, st, a);
 }
 
+// (the kernel addresses with 32-bit byte offsets into buffer resources: 256 rows of states,
+// the whole packed matrix and the whole of scales / zeros have to stay below 2 GB each)
+static bool pipe_shape(int bits, bool sparse, int64_t K, int64_t S, int64_t group_units) {
+    const int64_t w_bytes = K / 32 * (sparse ? 2 : bits) * 4 * S, sz_bytes = (K / 64 + group_units - 1) / group_units * S * 2;
+    return K <= (1 << 22) && S <= (1 << 27) && w_bytes < (1ll << 31) && sz_bytes < (1ll << 31);
+}
+// (a short K on a small dense grid: the pipelined kernel's prologue costs more than its faster steps return: 2048 rows,
+// K=S=128 8.7 -> 5.3 us; 512 rows, K=512, S=1024 14.6 -> 10.7; from K = 1024 on there is nothing in it)
+static bool takes_tiles(int bits, bool sparse, int64_t M, int64_t K, int64_t S, int64_t group_units) {
+    return pipe_shape(bits, sparse, K, S, group_units) && tile_columns(S, 256, true) &&
+           (sparse || K >= 1024 || (M + 255) / 256 * ((S + 255) / 256) > 128);
+}
+
+double tiles_us(int bits, bool sparse, int64_t M, int64_t K, int64_t S, int64_t group_units, size_t scratch) {
+    return takes_tiles(bits, sparse, M, K, S, group_units) ? plan_tiles(bits, sparse, M, K, S, scratch, 0).us : 1e30;
+}
+
+// height of a forced variant's tiles, in 32 rows (0: none)
+static int forced_height(int64_t variant) {
+    static const int heights[12] = {0, 0, 0, 0, 0, 0, 8, 4, 6, 8, 5, 7};
+    return variant >= 0 && variant < 12 ? heights[variant] : 0;
+}
+
 template <int BITS, bool SPARSE>
 static void launch(MatmulArgs a, int64_t B, hipStream_t st, void* workspace, size_t workspace_bytes) {
-    // variant 0 = automatic.  Shapes that fill their tiles well enough take the pipelined kernel, as
-    // 256 x 256 tiles (one eight-wave workgroup per CU) or 256 x 128 tiles (two
-    // four-wave workgroups per CU).  Measured on MI355X (K = 4096 ... 20480, S = 5120
-    // ... 28672, M = 256 ... 4096): the small tiles win when at most half of the CUs
-    // would get a large tile, and in the second round of large tiles while it is at
-    // most three eighths full; the large ones everywhere else.  The 16:32 format always takes the large tiles (its decode
-    // needs more registers than the four-wave shape leaves).  Everything else:
-    // 128 x 256 tiles, and 128 x 128 for narrow outputs or few rows.
-    int variant = (int)tuning(TUNE_MM_VARIANT);
-    // (M is padded to whole tiles of 256 rows; measured worth it up to half as many rows again
-    // -- the general kernel reaches about 60 % of the pipelined one's rate -- and for a single
-    // row of tiles from 129 rows on, where the general kernel would need two rows of its 128-row tiles)
-    const int64_t m_pad = (a.M + 255) / 256 * 256;
-    // (97 ... 128 rows: the general kernel's single row of 128 x 128 tiles cannot split K; the padded
-    // pipelined kernel can, and wins when K is long -- 16:32: from K = 1024; dense: from K = 2048 on
-    // outputs too narrow to give the general kernel a tile per CU and a half)
-    const bool pad_97_128 = a.M > 96 && a.M <= 128 && (SPARSE ? a.K >= 1024 : (a.K >= 2048 && a.S <= 12288));
-    // (the kernel addresses with 32-bit byte offsets into buffer resources: 256 rows of states,
-    // the whole packed matrix and the whole of scales / zeros have to stay below 2 GB each)
-    const int64_t w_bytes = (int64_t)a.K / 32 * PipeFmt<BITS, SPARSE>::ROWS * 4 * a.S;
-    const int64_t sz_bytes = ((int64_t)a.K / 64 + a.group_units - 1) / a.group_units * a.S * 2;
-    const bool shape_ok = a.K <= (1 << 22) && a.S <= (1 << 27) && w_bytes < (1ll << 31) && sz_bytes < (1ll << 31);
-    // (257 ... 341 rows, padded by half and more: still better than the general kernel where split-K makes up
-    // for a small grid, and for 16:32 everywhere -- its general decode is slow; measured K >= 2048)
-    const bool pad_257_341 = a.M > 256 && a.M < 342 && a.K >= 2048 &&
-                             (SPARSE || m_pad / 256 * ((a.S + 255) / 256) * B <= 128);
-    const bool m_ok = (m_pad * 2 <= a.M * 3 || (a.M > 128 && a.M <= 256) || pad_97_128 || pad_257_341) && shape_ok;
-    // An odd number of 128-row tile rows (257 ... 384 rows, 513 ... 640, ... up to 1152): 128 x 256 tiles (the
-    // same kernel with half the rows per wave) instead of 256 x 256 tiles padded by another 128 rows -- when
-    // they give the GPU at most one round of at least half (16:32: three quarters) of its CUs; smaller grids
-    // are better off with split-K
-    const int64_t rows_128 = (a.M + 127) / 128, tiles_128 = rows_128 * ((a.S + 255) / 256) * B;
-    // (dense: also with an even number of rows when the 128 x 256 tiles fill nine sixteenths of the GPU and more --
-    // better than half as many 256 x 256 tiles or 256 x 128 tiles with split-K, by 5 - 10 %)
-    // (K=S=3072, eleven to thirteen rows of 128: 132 - 156 tiles of 128 x 256 in 49 - 50 us against 56 - 59 for the
-    // 256 x 128 tiles that used to serve 1408 ... 1664 rows there)
-    const bool odd_rows = rows_128 % 2 == 1 && rows_128 <= (SPARSE ? 9 : 13);
-    const bool three_rows = a.M > 256 && shape_ok && tile_columns(a.S, 256, SPARSE) && tiles_128 <= 256 &&
-                            (SPARSE ? odd_rows && tiles_128 >= 192 : tiles_128 >= (odd_rows ? 128 : 144));
-    const bool pipe2_ok = !SPARSE && m_ok && tile_columns(a.S, 128, SPARSE);
-    const bool pipe4_ok = m_ok && tile_columns(a.S, 256, SPARSE);
-    if (variant != 1 && variant != 3 && variant != 5 && variant != 6 && variant != 7 && variant != 8 && variant != 9) variant = 0;
-    if ((variant == 5 && !pipe2_ok) || ((variant == 6 || variant == 9) && !pipe4_ok) ||
-        ((variant == 7 || variant == 8) && !(shape_ok && tile_columns(a.S, 256, SPARSE)))) variant = 0;
-    // (a last round of large tiles that fills at most half of the GPU is split along K when the
-    // workspace has room for its partial tiles: better than small tiles then)
-    const TailPlan tp = plan_tail(SPARSE, B, a.M, a.K, a.S);
+    // variant 0 = automatic: the plan of the pipelined kernel's tiles; where that kernel does not take the shape its 128-column form
+    // or the general tiles, 128 x 256, and 128 x 128 for narrow outputs or few rows
+    const int variant = (int)tuning(TUNE_MM_VARIANT);
     const WorkspaceParts wsp = workspace_parts(workspace, workspace_bytes);
-    const bool tail_ok = pipe4_ok && tp.ksplit > 1 && wsp.counters != nullptr &&
-                         wsp.scratch_bytes >= (size_t)(tp.tiles * tp.ksplit * (256 * 256 * 4));
-    if (variant == 0) {
-        const int64_t tiles4 = m_pad / 256 * ((a.S + 255) / 256) * B;
-        const int64_t last = tiles4 % 256;
-        const bool small_better = tiles4 <= 128 || (!tail_ok && tiles4 > 256 && tiles4 < 512 && last > 0 && last <= 96);
-        // (a grid that fills at most half of the GPU with a short K: the pipelined kernel's prologue -- three
-        // stages, the scan of the scales -- costs more than its faster steps return; measured K <= 1024)
-        // (a long K on a narrow output: 256 x 128 tiles split three ways and more along K, in shares of at least
-        // 140 steps, beat one round of unsplit 128 x 256 tiles -- K=20480, S=5120: 769 rows 283 -> 240 us, 1024 rows
-        // 279 -> 252 us; K=14336, S=4096, 1280 rows 198 -> 187 us; shorter shares lose: K=S=8192, 1024 rows 147 / 159)
-        bool long_k_split = false;
-        if (!SPARSE && three_rows && pipe2_ok) {
-            const SplitPlan sp = plan_split(false, B, a.M, a.K, a.S);
-            long_k_split = sp.ksplit >= 3 && a.K / 32 / sp.ksplit >= 140 && wsp.counters != nullptr &&
-                           wsp.scratch_bytes >= (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes);
-        }
-        // (16:32 with at most 128 padded 256-row tiles: those, split along K, beat the 128-row tiles from K = 4096 on --
-        // K=S=8192, 896 rows: 182 -> 163 us; K=8192, S=10240, 640 rows: 178 -> 155; K=16384, S=7168, 800 rows: 346 -> 271;
-        // K=4096: 0 - 12 %; at K=2048 the unsplit 128-row tiles still win by 1 - 7 %)
-        bool sparse_split = false;
-        if (SPARSE && three_rows && pipe4_ok && tiles4 <= 128 && a.K >= 4096) {
-            const SplitPlan sp = plan_split(true, B, a.M, a.K, a.S);
-            sparse_split = sp.ksplit > 1 && wsp.counters != nullptr && sp.tiles <= 1024 &&
-                           wsp.scratch_bytes >= (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes);
-        }
-        if (!SPARSE && tiles4 <= 128 && a.K <= 1024) variant = 1;
-        else if (long_k_split) variant = 5;
-        else if (three_rows && !sparse_split) variant = 7;
-        else if (pipe4_ok && (SPARSE || !pipe2_ok || !small_better)) variant = 6;
-        else if (pipe2_ok) variant = 5;
-        else if (a.M > 512 && a.S >= 256) variant = 3;
-        else variant = 1;
+    const size_t scratch = wsp.counters != nullptr && B == 1 ? wsp.scratch_bytes : 0;
+    a.counters = reinterpret_cast<int*>(wsp.counters);
+    a.part = reinterpret_cast<float*>(wsp.scratch);
+    const bool shape_ok = pipe_shape(BITS, SPARSE, a.K, a.S, a.group_units);
+    // the 128-column form: where rows of 256 pad less than half (or would leave the general tiles a second row); and 513 ... 1152
+    // rows that are a whole odd number of 128s on a K so long that three ways leave shares of 140 steps, for which its tests
+    // ask (int4, K=14336, S=4096, 1152 rows 166 us; 192 x 256 two ways 136)
+    bool narrow = false;
+    if constexpr (!SPARSE) {
+        const int64_t m_pad = (a.M + 255) / 256 * 256, rows_128 = (a.M + 127) / 128, tiles_128 = rows_128 * ((a.S + 255) / 256);
+        const bool fits = shape_ok && B == 1 && tile_columns(a.S, 128, false) && (m_pad * 2 <= a.M * 3 || (a.M > 128 && a.M <= 256));
+        const SplitPlan sp = plan_split(false, B, a.M, a.K, a.S);
+        const bool split = sp.ksplit > 1 && scratch >= (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes);
+        const bool long_k = a.M > 512 && a.M % 256 == 128 && a.M <= 1152 && tiles_128 >= 128 && tiles_128 <= 256 && sp.ksplit >= 3 && a.K / 32 / sp.ksplit >= 140;
+        narrow = fits && (variant == 5 || (variant == 0 && ((split && long_k) || (!tile_columns(a.S, 256, true) && a.K > 1024))));
+        if (narrow && split) a.ksplit = sp.ksplit;
     }
-    // split-K where the plan asks for it and the scratch half of the caller's workspace has room for
-    // the partial tiles (the per-tile counters sit in the last page of the half that is kept zero)
-    if ((SPARSE && (variant == 6 || variant == 9)) || (!SPARSE && variant == 5)) {
-        const SplitPlan sp = plan_split(SPARSE, B, a.M, a.K, a.S);
-        const WorkspaceParts ws = workspace_parts(workspace, workspace_bytes);
-        if (sp.ksplit > 1 && ws.counters != nullptr && sp.tiles <= 1024 &&
-            ws.scratch_bytes >= (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes)) {
-            a.ksplit = sp.ksplit;
-            a.counters = reinterpret_cast<int*>(ws.counters);
-            a.part = reinterpret_cast<float*>(ws.scratch);
-        }
+    const int only = forced_height(variant);
+    const bool tiles = !narrow && (variant == 0 ? takes_tiles(BITS, SPARSE, a.M, a.K, a.S, a.group_units) : only != 0 && shape_ok && tile_columns(a.S, 256, true));
+    if (narrow) {
+        if constexpr (!SPARSE) launch_pipe<BITS, false, 2>(a, B, st);
+    } else if (tiles) {
+        const TilePlan p = plan_tiles(BITS, SPARSE, a.M, a.K, a.S, scratch, only);
+        a.ksplit = p.ksplit;
+        a.split_from = (int)p.split_from;
+        // (variant 9 forces 256 x 256 without the two phases: 9 % slower, 16:32 4 %)
+        if (variant == 9) launch_pipe<BITS, SPARSE, 4>(a, B, st);
+        else if (p.tm == 4) launch_pipe<BITS, SPARSE, 4, 4, true>(a, B, st);
+        else if (p.tm == 5) launch_pipe<BITS, SPARSE, 4, 5, true>(a, B, st);
+        else if (p.tm == 6) launch_pipe<BITS, SPARSE, 4, 6, true>(a, B, st);
+        else if (p.tm == 7) launch_pipe<BITS, SPARSE, 4, 7, true>(a, B, st);
+        else launch_pipe<BITS, SPARSE, 4, 8, true>(a, B, st);
+    } else if (variant == 3 || (variant != 1 && a.M > 512 && a.S >= 256 && !(!SPARSE && a.K <= 1024))) {
+        launch_tile<BITS, SPARSE, 128, 256, 128, 64>(a, B, st);
+    } else {
+        launch_tile<BITS, SPARSE, 128, 128, 64, 64>(a, B, st);
     }
-    if (a.ksplit == 1 && (variant == 6 || variant == 9) && tail_ok) {
-        a.ksplit = tp.ksplit;
-        a.split_from = (int)tp.split_from;
-        a.counters = reinterpret_cast<int*>(wsp.counters);
-        a.part = reinterpret_cast<float*>(wsp.scratch);
-    }
-    // 192 x 256 tiles instead of whole 256 x 256 ones, where they take no more rounds of 256 workgroups and pad no more
-    // rows: a round of them costs five sixths to nine tenths (us, 256 / 192 rows, one run: int3, K=4096, S=11008, 777 rows 100 / 91;
-    // int4, S=20480, 520 rows 115 / 95; 1152 rows -- two rounds both ways -- 205 / 186; K=S=8192, 1300 rows 193 / 174; 16:32,
-    // K=8192, S=20480, 520 rows 247 / 210; a round more loses: int3, K=4096, S=11008, 1152 rows 110 / 172).  A grid
-    // whose last round is split along K keeps the large tiles, 1 - 15 % faster.
-    if (variant == 6 && tuning(TUNE_MM_VARIANT) == 0 && a.ksplit == 1) {
-        const int64_t rows_192 = (a.M + 191) / 192, t256 = m_pad / 256 * ((a.S + 255) / 256) * B, t192 = rows_192 * ((a.S + 255) / 256) * B;
-        if (rows_192 * 192 <= m_pad && (t192 + 255) / 256 == (t256 + 255) / 256) variant = 8;
-    }
-    if (variant == 1) launch_tile<BITS, SPARSE, 128, 128, 64, 64>(a, B, st);
-    else if (variant == 3) launch_tile<BITS, SPARSE, 128, 256, 128, 64>(a, B, st);
-    // (variant 9 forces 256 x 256 without the two phases: 9 % slower, 16:32 4 %)
-    else if (variant == 7) launch_pipe<BITS, SPARSE, 4, 4, true>(a, B, st);
-    else if (variant == 8) launch_pipe<BITS, SPARSE, 4, 6, true>(a, B, st);
-    else if (variant == 6) launch_pipe<BITS, SPARSE, 4, 8, true>(a, B, st);
-    else if (variant == 6 || variant == 9) launch_pipe<BITS, SPARSE, 4>(a, B, st);
-    else if constexpr (!SPARSE) launch_pipe<BITS, false, 2>(a, B, st);
 }
 
 }  // namespace i4
@@ -1199,10 +1191,19 @@ extern "C" size_t int4mm_matmul_workspace_bytes(const int4mm_shape* shape, int s
                     few_rows = std::max({few_rows, few(share, EXACT_SUMS), few(std::max<int64_t>(2, share - 1), EXACT_SUMS)});
         }
     if (B * M <= FEW_ROWS_MAX) return need + 2 * round_to_page(few_rows);
+    size_t part = few_rows;
     const SplitPlan sp = plan_split(sparse != 0, B, M, K, S);
-    if (sp.ksplit > 1 || few_rows > 0)
-        need += 2 * round_to_page(std::max(few_rows, sp.ksplit > 1 ? (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes) : 0));
-    const TailPlan tp = plan_tail(sparse != 0, B, M, K, S);
-    if (sp.ksplit == 1 && tp.ksplit > 1) need += 2 * round_to_page((size_t)(tp.tiles * tp.ksplit * (256 * 256 * 4)));
-    return need;
+    const bool chunks = shape->seq_len == 1 && B * M > SK_WIDE_MAX_ROWS;           // (of the matvec entry: last_chunk_as_others)
+    if (sp.ksplit > 1 && chunks) part = std::max(part, (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes));
+    if (chunks && sp.ksplit == 1) {
+        const TailPlan tp = plan_tail(sparse != 0, B, M, K, S);
+        if (tp.ksplit > 1) part = round_to_page(part) + (size_t)(tp.tiles * tp.ksplit * (256 * 256 * 4));
+    }
+    for (const int b : {4, 3, 2}) {
+        const int64_t gu = group_units > 0 ? group_units : 1, variant = tuning(TUNE_MM_VARIANT);
+        if (B != 1 || (sparse ? b != 4 : bits != 0 && b != bits) || (M <= SK_WIDE_MAX_ROWS && variant == 0 && !tuning(TUNE_NO_SKINNY) && wide_serves(b, sparse != 0, M, K, S, gu))) continue;
+        if (variant != 0 || takes_tiles(b, sparse != 0, M, K, S, gu)) part = std::max(part, plan_tiles(b, sparse != 0, M, K, S, SIZE_MAX, forced_height(variant)).part_bytes);
+        if (!sparse && sp.ksplit > 1) part = std::max(part, (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes));        // (the 128-column tiles)
+    }
+    return need + 2 * round_to_page(part);
 }

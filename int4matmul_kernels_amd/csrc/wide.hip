@@ -521,7 +521,7 @@ static constexpr size_t wide_lds_bytes(int mt, int wn) {
 // to 930 ... 2440 timed launches each (K = 1024 ... 20480, S = 1024 ... 28672, 24 ... 512 rows, cold weights).  On 30 other random shapes
 // of that range per format its pick was the best measured candidate on half of them and 1.1 / 1.8 / 1.0 / 0 % off it on
 // average (int4, int3, int2, 16:32), 12 / 21 / 23 / 8 % at worst.
-struct WidePlan { bool use; int mt, wn, row_blocks, ksplit, units_per_split; size_t part_bytes; };
+struct WidePlan { bool use; int mt, wn, row_blocks, ksplit, units_per_split; size_t part_bytes; double us; };
 struct WideCost { int mt, wn; double step, filled, more_step, workgroup, more_workgroup, split, way, last; };
 static const WideCost wide_cost[4][6] = {             // int4, int3, int2, 16:32
     {{1, 2, 0.736, 0.148, 0.824, 4.36, 2.51, 0.847, 0.445, 1.3},
@@ -655,7 +655,7 @@ static int64_t wide_strips(int64_t S, int wn) { return (S + 64 * wn - 1) / (64 *
 
 // `scratch`: bytes for partial tiles; the splits that need more are no candidates
 static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S, size_t scratch) {
-    WidePlan p{false, 0, 0, 0, 1, 0, 0};
+    WidePlan p{false, 0, 0, 0, 1, 0, 0, 0.0};
     // (knob: 1 = never, n >= 2 = from n rows on whatever the shape)
     const int64_t knob = tuning(TUNE_NO_WIDE), min_rows = knob >= 2 ? knob : 17, forced = tuning(TUNE_MM_SPLIT);
     if (R < min_rows || R > SK_WIDE_MAX_ROWS || !wide_columns(R, S) || K % 64 != 0 || knob == 1) return p;
@@ -700,8 +700,21 @@ static WidePlan plan_wide(int bits, bool sparse, int64_t R, int64_t K, int64_t S
         if (best > 5.0 + flops / (wide_strips(S, p.wn) * p.row_blocks > 256 ? 1.05e9 : 0.75e9)) return p;
     }
     p.part_bytes = p.ksplit > 1 ? (size_t)p.ksplit * p.row_blocks * p.mt * wide_strips(S, p.wn) * p.wn * 8192 : 0;
+    p.us = best;
     p.use = true;
     return p;
+}
+
+// More than 256 rows through the matmul entry: the tile kernels where they are faster, by both models (us, here / there: int4, K=6656, S=14592,
+// 306 rows 86 / 75; K=16000, S=14208, 432 rows 230 / 189; int3, K=2816, S=8448, 462 rows 47 / 39)
+static bool tiles_instead(int bits, bool sparse, int64_t R, int64_t K, int64_t S, int64_t group_units, size_t scratch, const WidePlan& p) {
+    return R > 256 && tuning(TUNE_NO_WIDE) < 2 && tuning(TUNE_MM_SPLIT) < 1 && tiles_us(bits, sparse, R, K, S, group_units, scratch) < 0.95 * p.us;
+}
+
+// Does the matmul entry leave a product of 97 ... 512 rows to this kernel, given room for any split?
+bool wide_serves(int bits, bool sparse, int64_t R, int64_t K, int64_t S, int64_t group_units) {
+    const WidePlan p = plan_wide(bits, sparse, R, K, S, SIZE_MAX);
+    return p.use && !tiles_instead(bits, sparse, R, K, S, group_units, SIZE_MAX, p);
 }
 
 // What the plan's partial tiles take with room for any split and, where a product has to be admitted, the room that it takes to be;
@@ -772,6 +785,7 @@ bool wide_rows(int bits, const SkinnyArgs& args, RowsCall call, void* workspace,
     }
     const WidePlan p = plan_wide(bits, sparse, args.R, args.K, args.S, ws.scratch_bytes);
     if (!p.use) return false;
+    if (call == FOR_MATMUL && tiles_instead(bits, sparse, args.R, args.K, args.S, args.group_units, ws.counters != nullptr ? ws.scratch_bytes : 0, p)) return false;
     SkinnyArgs a = args;
     a.counters = reinterpret_cast<int*>(ws.counters);
     a.part = reinterpret_cast<float*>(ws.scratch);

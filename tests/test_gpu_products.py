@@ -371,6 +371,36 @@ def test_matmul_tiles_of_192_rows_default_rule(H, bits, sparse):
     H.assert_product_close(got, exact, f32, kind="mtx")
 
 
+# ---- every height of the pipelined tiles (tuning key 3: 128, 160, 192, 224, 256 rows), K split and not: one to nine pairs of K steps
+# (the ring of states is six steps long), shares of unequal length, a row more and a row less than a tile, exponent-mode groups in
+# one tile column.  Unsplit, an element's sum has one order whatever the height: the same bits.
+@pytest.mark.parametrize("bits,sparse", FORMATS)
+@pytest.mark.parametrize("M,K,S,g,ksplit", [(161, 64, 256, 64, 1), (223, 128, 256, 64, 1), (159, 192, 512, 64, 1), (1, 320, 256, 64, 1),
+                                            (225, 576, 448, 192, 1), (161, 1088, 256, 64, 2), (225, 832, 512, 128, 3), (300, 2112, 256, -1, 8)])
+def test_every_tile_height(H, bits, sparse, M, K, S, g, ksplit):
+    p = _problem(bits, sparse, K=K, S=S, M=M, group_size=g, seed=M + K)
+    sc = p["scales"].reshape(-1, S)
+    sc[sc.shape[0] // 2, S - 60:S - 50] *= np.float16(-1)
+    d = H.dev_problem(p)
+    exact, f32 = H.oracles(p)
+    runs = []
+    for variant in (6, 7, 8, 10, 11):
+        try:
+            H.capi.tune(3, variant)
+            H.capi.tune(6, ksplit)
+            line = H.capi.describe_launch("mtx", bits, 1, M, K, S, g, sparse)
+            assert f"tile={32 * {6: 8, 7: 4, 8: 6, 10: 5, 11: 7}[variant]}x256" in line, line
+            assert f"ksplit={1 if sparse and variant == 11 else ksplit} " in line, line
+            runs.append(H.run_capi(p, d, "mtx", outs_init=np.full((1, M, S), 4.0, np.float16)))
+        finally:
+            H.capi.tune(3, 0)
+            H.capi.tune(6, 0)
+        H.assert_product_close(runs[-1], exact, f32, kind="mtx")
+    if ksplit == 1:
+        for r in runs[1:]:
+            assert np.array_equal(r.view(np.uint16), runs[0].view(np.uint16))
+
+
 # ---- a last strip or tile that is partly beyond the last column (S a multiple of 64, not of the strip's 128 or 256): one to three
 # quarters of it full, K split and not, exponent-mode groups in the last columns, and 0 = whatever the dispatch picks
 @pytest.mark.parametrize("bits,sparse", FORMATS)
