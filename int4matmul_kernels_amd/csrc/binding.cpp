@@ -26,10 +26,10 @@
 
 namespace {
 
-#define TENSOR_MULT_ARGS                                                         \
-    torch::Tensor outs, torch::Tensor matrix, torch::Tensor multiplier,          \
-        torch::Tensor scales, torch::Tensor zeros, int group_size,               \
-        c10::optional<torch::Tensor> sparse_mask
+#define TENSOR_MULT_ARGS                                                                    \
+    const torch::Tensor &outs, const torch::Tensor &matrix, const torch::Tensor &multiplier, \
+        const torch::Tensor &scales, const torch::Tensor &zeros, int group_size,             \
+        const c10::optional<torch::Tensor>& sparse_mask
 #define TENSOR_MULT_PASS outs, matrix, multiplier, scales, zeros, group_size, sparse_mask
 
 void check_rc(int rc, const char* what) {
@@ -55,8 +55,8 @@ std::mutex g_mu;
 std::map<std::pair<int, int64_t>, Scratch> g_scratch;
 
 torch::Tensor workspace_for(const c10::Device& dev, c10::hip::HIPStream stream, const int4mm_shape& shape, bool sparse) {
-    // (covers the matvec's need; more when a matmul of this shape wants to split K)
-    const size_t need = int4mm_matmul_workspace_bytes(&shape, sparse ? 1 : 0);
+    // (covers the matvec's need, which is all of a single row's; more when a matmul of this shape wants to split K)
+    const size_t need = shape.batch * shape.seq_len == 1 ? int4mm_workspace_bytes(shape.out_size) : int4mm_matmul_workspace_bytes(&shape, sparse ? 1 : 0);
     std::lock_guard<std::mutex> lock(g_mu);
     auto key = std::make_pair((int)dev.index(), (int64_t)stream.id());
     auto it = g_scratch.find(key);
@@ -180,14 +180,16 @@ void quant_matmul(uint32_t bits, TENSOR_MULT_ARGS) {
 // the output zeroed / unfilled: sixteen 1024 x 1024 matvecs 221 / 179 / 119; four layers of K = 5120, S = 20480 with one token
 // 56 / 56 / 48, 8 tokens 88 / 88 / 72, 64 tokens 154 / 153 / 118; one with 2048 rows 410 / 410 / 399: where kernels are long the
 // gain is the fill alone.
-torch::Tensor linear_forward(uint32_t bits, int64_t out_size, torch::Tensor matrix, torch::Tensor multiplier,
-                             torch::Tensor scales, torch::Tensor zeros, int group_size,
-                             c10::optional<torch::Tensor> sparse_mask) {
-    TORCH_CHECK(multiplier.defined() && multiplier.dim() == 3, "multiplier must be 3-D");
-    TORCH_CHECK(multiplier.is_cuda(), "multiplier must be a GPU tensor");
-    c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(multiplier.device());
-    if (multiplier.scalar_type() != torch::kHalf || !multiplier.is_contiguous())
-        multiplier = multiplier.contiguous().to(torch::kHalf);
+torch::Tensor linear_forward(uint32_t bits, int64_t out_size, const torch::Tensor& matrix, const torch::Tensor& states,
+                             const torch::Tensor& scales, const torch::Tensor& zeros, int group_size,
+                             const c10::optional<torch::Tensor>& sparse_mask) {
+    TORCH_CHECK(states.defined() && states.dim() == 3, "multiplier must be 3-D");
+    TORCH_CHECK(states.is_cuda(), "multiplier must be a GPU tensor");
+    c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(states.device());
+    torch::Tensor converted;
+    if (states.scalar_type() != torch::kHalf || !states.is_contiguous())
+        converted = states.contiguous().to(torch::kHalf);
+    const torch::Tensor& multiplier = converted.defined() ? converted : states;
     const bool vec = multiplier.size(1) == 1;
     auto outs = at::empty({multiplier.size(0), multiplier.size(1), out_size},
                           torch::TensorOptions().dtype(torch::kHalf).device(multiplier.device()));
