@@ -232,6 +232,11 @@ INT4MM_API int int4mm_matmul(int bits, void* outs, const void* matrix, const voi
 INT4MM_API int int4mm_sparse_pack(void* wt_outs, void* msk_outs, const void* wt_in, const void* msk_in,
                        int64_t out_size, int64_t in_size, void* bad_blocks, void* stream);
 
+/* The same, waiting for it: *bad_blocks (host memory) is the number of 32-row
+ * blocks that do not keep exactly 16 rows.  Not capturable. */
+INT4MM_API int int4mm_sparse_pack_checked(void* wt_outs, void* msk_outs, const void* wt_in, const void* msk_in,
+                                          int64_t out_size, int64_t in_size, int* bad_blocks, void* stream);
+
 /* Dense packer for int4/int3/int2: codes uint8 [K, S] (row = k) -> matrix
  * int32 [K*bits/32, S].  The reference packs dense weights with Python loops
  * (kernel_test.py:60-123); this is the on-device equivalent of those loops. */

@@ -16,7 +16,7 @@ EXPORTS = [
     "int4mm_error_string", "int4mm_last_hip_error", "int4mm_abi_version", "int4mm_tune",
     "int4mm_workspace_bytes", "int4mm_workspace_init", "int4mm_matmul_workspace_bytes", "int4mm_matvec", "int4mm_matmul",
     "int4mm_matvec_overwrite", "int4mm_matvec_static", "int4mm_workspace_status", "int4mm_describe_launch",
-    "int4mm_sparse_pack", "int4mm_dense_pack", "int4mm_unpack", "int4mm_dequantize",
+    "int4mm_sparse_pack", "int4mm_sparse_pack_checked", "int4mm_dense_pack", "int4mm_unpack", "int4mm_dequantize",
 ]
 
 

@@ -38,6 +38,11 @@ int check_launch(const char*) {
     return INT4MM_OK;
 }
 
+int launch_error() {
+    g_last_hip_error = (int)hipGetLastError();
+    return INT4MM_ERR_LAUNCH;
+}
+
 int64_t tuning(int key) { return (key >= 0 && key < TUNE_COUNT) ? g_tuning[key] : 0; }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }

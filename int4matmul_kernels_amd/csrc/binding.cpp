@@ -203,8 +203,8 @@ torch::Tensor linear_forward(uint32_t bits, int64_t out_size, const torch::Tenso
 }
 
 // int4matmul.cpp:50-63, utils_kernel.cu:67-119
-void weight_matrix_packing(torch::Tensor wt_outs, torch::Tensor msk_outs, torch::Tensor wt_in,
-                           torch::Tensor msk_in) {
+void weight_matrix_packing(const torch::Tensor& wt_outs, const torch::Tensor& msk_outs, const torch::Tensor& wt_in,
+                           const torch::Tensor& msk_in) {
     TORCH_CHECK(wt_outs.defined() && wt_outs.is_cuda(), "wt_outs must be a GPU tensor");
     const c10::Device dev = wt_outs.device();
     c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(dev);
@@ -220,11 +220,10 @@ void weight_matrix_packing(torch::Tensor wt_outs, torch::Tensor msk_outs, torch:
     TORCH_CHECK(wt_outs.size(0) * 16 == K && wt_outs.size(1) == S, "wt_outs must be [", K / 16, ", ", S, "]");
     TORCH_CHECK(msk_outs.size(0) * 32 == K && msk_outs.size(1) == S, "msk_outs must be [", K / 32, ", ", S, "]");
     auto stream = c10::hip::getCurrentHIPStream(dev.index());
-    auto bad = torch::zeros({1}, torch::TensorOptions().dtype(torch::kInt).device(dev));
-    check_rc(int4mm_sparse_pack(wt_outs.data_ptr(), msk_outs.data_ptr(), wt_in.data_ptr(),
-                                msk_in.data_ptr(), S, K, bad.data_ptr(), (void*)stream.stream()),
+    int n_bad = 0;                          // packing is an offline step: synchronising is fine
+    check_rc(int4mm_sparse_pack_checked(wt_outs.data_ptr(), msk_outs.data_ptr(), wt_in.data_ptr(), msk_in.data_ptr(), S, K, &n_bad,
+                                        (void*)stream.stream()),
              "weight_matrix_packing");
-    const int n_bad = bad.item<int>();      // packing is an offline step: synchronising is fine
     TORCH_CHECK(n_bad == 0, "weight_matrix_packing: ", n_bad,
                 " 32-row blocks do not keep exactly 16 rows");
 }

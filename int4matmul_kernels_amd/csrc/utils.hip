@@ -5,6 +5,7 @@
 #include "common.h"
 
 #include <algorithm>
+#include <mutex>
 
 namespace i4 {
 
@@ -171,7 +172,7 @@ __global__ __launch_bounds__(256) void sparse_pack_kernel(uint32_t* __restrict__
                                                           const uint8_t* __restrict__ wt_in,
                                                           const uint8_t* __restrict__ msk_in,
                                                           int64_t S, int64_t K, int64_t s_first, uint32_t k_tiles,
-                                                          int* __restrict__ bad_blocks) {
+                                                          int* __restrict__ bad_blocks, int* bad_flag) {
     constexpr int PASSES = sparse_pack_passes(LANES), CELLS = LANES / 2, COLS_PASS = 256 / LANES, COLS = sparse_pack_cols(LANES);
     // compaction table: for a byte of eight keep flags, the v_perm selectors that move the kept rows' code bytes to
     // the front in row order (0 ... 7: that row of the eight; 0x0C: a zero byte)
@@ -255,19 +256,68 @@ __global__ __launch_bounds__(256) void sparse_pack_kernel(uint32_t* __restrict__
         wt_outs[(2 * blk + 1) * S + s] = tile[1][c][col];
         msk_outs[blk * S + s] = tile[2][c][col];
     }
-    if (bad && bad_blocks) atomicAdd(bad_blocks, bad);
+    if (bad && bad_blocks) {
+        atomicAdd(bad_blocks, bad);
+        // (pinned host memory: a plain store, which every bus carries)
+        if (bad_flag) __hip_atomic_store(bad_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 static dim3 cell_grid(int64_t S, int64_t K) { return dim3((unsigned)((S + 255) / 256), (unsigned)(K / 32)); }
 
-}  // namespace i4
+// What a checked packing reports through: a device counter that is 0 between calls, and a word of pinned host memory that the kernel
+// sets when it counts.  A call takes one for itself and gives it back; MOST are kept.
+struct PackReport { int device; int* count; int* flag; };
+constexpr int MOST_REPORTS = 16;
+static std::mutex g_reports_mutex;
+static PackReport g_reports[MOST_REPORTS];
+static int g_n_reports = 0;
 
-using namespace i4;
+static bool clear_count(const PackReport& r) {
+    const int zero = 0;
+    return hipMemcpy(r.count, &zero, sizeof(int), hipMemcpyHostToDevice) == hipSuccess;
+}
+static void free_report(const PackReport& r) {
+    if (r.count) (void)hipFree(r.count);
+    if (r.flag) (void)hipHostFree(r.flag);
+}
 
-extern "C" {
+static bool take_report(PackReport& r) {
+    r = PackReport{0, nullptr, nullptr};
+    if (hipGetDevice(&r.device) != hipSuccess) return false;
+    {
+        std::lock_guard<std::mutex> lock(g_reports_mutex);
+        for (int i = 0; i < g_n_reports; ++i)
+            if (g_reports[i].device == r.device) {
+                r = g_reports[i];
+                g_reports[i] = g_reports[--g_n_reports];
+                return true;
+            }
+    }
+    // (another thread may be capturing a graph, which allocations must not end)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const bool ok = hipMalloc(&r.count, sizeof(int)) == hipSuccess && hipHostMalloc(&r.flag, sizeof(int), hipHostMallocDefault) == hipSuccess &&
+                    clear_count(r);
+    if (ok) *r.flag = 0;
+    else free_report(r);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return ok;
+}
 
-int int4mm_sparse_pack(void* wt_outs, void* msk_outs, const void* wt_in, const void* msk_in,
-                       int64_t out_size, int64_t in_size, void* bad_blocks, void* stream) {
+static void give_back(const PackReport& r) {
+    {
+        std::lock_guard<std::mutex> lock(g_reports_mutex);
+        if (g_n_reports < MOST_REPORTS) {
+            g_reports[g_n_reports++] = r;
+            return;
+        }
+    }
+    free_report(r);
+}
+
+static int sparse_pack(void* wt_outs, void* msk_outs, const void* wt_in, const void* msk_in,
+                       int64_t out_size, int64_t in_size, int* bad_blocks, int* bad_flag, void* stream) {
     if (out_size < 0 || in_size < 0 || in_size % 32 != 0) return INT4MM_ERR_SHAPE;
     if (in_size / 32 > 65535) return INT4MM_ERR_SHAPE;
     if (out_size == 0 || in_size == 0) return INT4MM_OK;
@@ -283,7 +333,7 @@ int int4mm_sparse_pack(void* wt_outs, void* msk_outs, const void* wt_in, const v
             hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(256), 0,
                                (hipStream_t)stream, (uint32_t*)wt_outs, (uint32_t*)msk_outs,
                                (const uint8_t*)wt_in, (const uint8_t*)msk_in, out_size, in_size, s_first,
-                               (uint32_t)k_tiles, (int*)bad_blocks);
+                               (uint32_t)k_tiles, bad_blocks, bad_flag);
         };
         switch (lanes) {
             case 2: launch(sparse_pack_kernel<2>); break;
@@ -294,6 +344,43 @@ int int4mm_sparse_pack(void* wt_outs, void* msk_outs, const void* wt_in, const v
         }
     }
     return check_launch("sparse_pack");
+}
+
+}  // namespace i4
+
+using namespace i4;
+
+extern "C" {
+
+int int4mm_sparse_pack(void* wt_outs, void* msk_outs, const void* wt_in, const void* msk_in,
+                       int64_t out_size, int64_t in_size, void* bad_blocks, void* stream) {
+    return sparse_pack(wt_outs, msk_outs, wt_in, msk_in, out_size, in_size, (int*)bad_blocks, nullptr, stream);
+}
+
+// Nothing runs before the kernel and nothing but the wait after it: a fill that clears a counter and a copy that reads it back
+// make a call at 16384 x 16384 134 us instead of 129.
+int int4mm_sparse_pack_checked(void* wt_outs, void* msk_outs, const void* wt_in, const void* msk_in,
+                               int64_t out_size, int64_t in_size, int* bad_blocks, void* stream) {
+    if (bad_blocks == nullptr) return INT4MM_ERR_NULL;
+    *bad_blocks = 0;
+    PackReport r;
+    if (!take_report(r)) return launch_error();
+    const int rc = sparse_pack(wt_outs, msk_outs, wt_in, msk_in, out_size, in_size, r.count, r.flag, stream);
+    if (hipStreamSynchronize((hipStream_t)stream) != hipSuccess) {          // (the kernel may still write: the report is not used again)
+        const int failed = launch_error();
+        return rc != INT4MM_OK ? rc : failed;
+    }
+    bool clean = true;
+    if (*(volatile int*)r.flag != 0) {
+        clean = hipMemcpy(bad_blocks, r.count, sizeof(int), hipMemcpyDeviceToHost) == hipSuccess && clear_count(r);
+        *r.flag = 0;
+    }
+    if (!clean) {
+        free_report(r);
+        return launch_error();
+    }
+    give_back(r);
+    return rc;
 }
 
 int int4mm_dense_pack(int bits, void* matrix_out, const void* codes_in, int64_t in_size,

@@ -95,6 +95,37 @@ def test_sparse_pack_bit_exact_capi_and_extension(H):
         assert np.array_equal(m.cpu().numpy(), want_m)
 
 
+@pytest.mark.parametrize("S,K", [(1, 32), (300, 96), (4096, 1024)])
+def test_weight_matrix_packing_counts_bad_blocks_anew_each_time(H, S, K):
+    """the report of a bad packing does not reach the next one, on whichever stream or thread that runs"""
+    from concurrent.futures import ThreadPoolExecutor
+    ext = H.pkg.load_extension()
+    codes = torch.full((S, K), 5, dtype=torch.uint8, device=H.DEV)
+    good = (torch.arange(K, device=H.DEV) % 2).to(torch.uint8).repeat(S, 1).contiguous()
+    torch.cuda.synchronize()
+
+    def pack(bad):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            keep = good.clone()
+            if bad > 0:
+                keep.view(-1, 32)[:bad, 0] = 1                # 17 rows of 32
+            w = torch.empty((K // 16, S), dtype=torch.int32, device=H.DEV)
+            m = torch.empty((K // 32, S), dtype=torch.int32, device=H.DEV)
+            if bad == 0:
+                ext.weight_matrix_packing(w, m, codes, keep)
+                assert int((m != -0x55555556).sum()) == 0
+            else:
+                with pytest.raises(RuntimeError, match=f" {bad} 32-row blocks"):
+                    ext.weight_matrix_packing(w, m, codes, keep)
+
+    most = S * K // 32
+    counts = [0, 1, most, 0, min(2, most), 0]
+    for n in counts:
+        pack(n)
+    with ThreadPoolExecutor(4) as pool:
+        list(pool.map(pack, counts * 4))
+
+
 @pytest.mark.parametrize("S,K", [(64, 64), (63, 96), (65, 512), (1, 544), (128, 1056), (200, 480), (320, 1600)])
 def test_sparse_pack_tile_edges(H, S, K):
     """edges of the packer's tiles; cells that keep more or fewer than 16 rows are counted once each"""
