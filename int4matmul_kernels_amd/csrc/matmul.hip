@@ -467,7 +467,6 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
     constexpr int NWORDS = F::NWORDS;
     constexpr bool PAIR = BITS == 4 && !SPARSE;
     constexpr int W_LOADS = PAIR ? 1 : NWORDS + (SPARSE ? 1 : 0);
-    constexpr int VALU = (72 + TM * TN - 1) / (TM * TN);          // other vector instructions behind an MFMA
     const int bn = PAIR ? t % (BN / 2) * 2 : t % BN, bhb = PAIR ? t / (BN / 2) : t / BN;
     const int bcol = min(s0 + (bn & ~63), a.S - 64) + (PAIR ? bn & 63 : 4 * ((bn & 15) ^ (bn >> 2 & 8)) + (bn >> 4 & 3));
     int b_chunk[2];                                      // where the two chunks go (halves)
@@ -715,12 +714,19 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
             if ((u + phase) % 2 == 0) take_sz(co);
             decode(r_dec, co, dec);
             mfma_step(fa, fb);
-            // (the decode in the shadow of the MFMAs: one occupies the pipe for 16 cycles, two waves of a SIMD issue two
-            // other vector instructions each meanwhile)
+            // (the decode in the shadow of the MFMAs: one occupies the pipe for 16 cycles, and up to two other vector instructions per
+            // MFMA go beside it.  Spread over the last two thirds, so that the packed words need not have arrived yet: 261 us where
+            // three behind each of the first MFMAs take 288, 16 tiles at K = 16384; at full load 2 - 3 %)
+            constexpr int MFMAS = TM * TN, LATE = MFMAS / 3, DECODE = (SPARSE ? 64 : BITS == 3 ? 52 : 40) + (decltype(mode)::value ? 26 : 0);
 #pragma unroll
-            for (int e = 0; e < TM * TN; ++e) {
+            for (int e = 0; e < MFMAS; ++e) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, decltype(mode)::value ? 2 * VALU : VALU, 0);
+                const int n = e < LATE ? 0 : (e - LATE + 1) * DECODE / (MFMAS - LATE) - (e - LATE) * DECODE / (MFMAS - LATE);
+                if (n == 1) __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
+                else if (n == 2) __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+                else if (n == 3) __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+                else if (n == 4) __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+                else if (n > 4) __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (phase == 0) stores_and_loads();
