@@ -459,20 +459,21 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
     // int4: word `row` of two adjacent columns, one 8-byte load; the others: column bn, rows 16 bhb .. 16 bhb + 15 of the
     // step's 32-row block: int2 word bhb; int3 words bhb, bhb + 1 (bits 48 bhb .. 48 bhb + 47 of the block's 96-bit stream); 16:32
     // sparse: both words and the mask word of the block.
-    // Column 4 n + j of a wave's 64 stands at position 16 j + (n ^ 8 (j / 2)) of its row of chunks: an MFMA tile takes every fourth
-    // column, so that the four tiles leave a lane with four adjacent columns of a row, an 8-byte store; the fragment reads and
-    // the stores of either mapping touch all banks once.
+    // Column 4 n + j of a wave's 64 stands at position 16 j + (n ^ 4 (j / 2)) of its row of chunks: an MFMA tile takes every fourth
+    // column, so that the four tiles leave a lane with four adjacent columns of a row, an 8-byte store.  The fragment reads, 256 bytes
+    // a cycle, and the stores of either mapping, 128 bytes of eight lanes a cycle, touch every bank once (with n ^ 8 the stores of
+    // int4 met twice on every second one: 16 conflict cycles per wave and step).
     // (a last tile that is not full: the columns beyond the last repeat the last 64 and are not written)
     using F = PipeFmt<BITS, SPARSE>;
     constexpr int NWORDS = F::NWORDS;
     constexpr bool PAIR = BITS == 4 && !SPARSE;
     constexpr int W_LOADS = PAIR ? 1 : NWORDS + (SPARSE ? 1 : 0);
     const int bn = PAIR ? t % (BN / 2) * 2 : t % BN, bhb = PAIR ? t / (BN / 2) : t / BN;
-    const int bcol = min(s0 + (bn & ~63), a.S - 64) + (PAIR ? bn & 63 : 4 * ((bn & 15) ^ (bn >> 2 & 8)) + (bn >> 4 & 3));
+    const int bcol = min(s0 + (bn & ~63), a.S - 64) + (PAIR ? bn & 63 : 4 * ((bn & 15) ^ (bn >> 3 & 4)) + (bn >> 4 & 3));
     int b_chunk[2];                                      // where the two chunks go (halves)
 #pragma unroll
     for (int q = 0; q < 2; ++q)
-        b_chunk[q] = 8 * (PAIR ? bhb * BN + (bn & ~63) + 16 * ((bn & 2) + q) + ((bn >> 2 & 15) ^ (bn << 2 & 8)) : (bhb * 2 + q) * BN + bn);
+        b_chunk[q] = 8 * (PAIR ? bhb * BN + (bn & ~63) + 16 * ((bn & 2) + q) + ((bn >> 2 & 15) ^ (bn << 1 & 4)) : (bhb * 2 + q) * BN + bn);
     struct Stage { uint32_t w[NWORDS]; uint32_t m; };
     // scale / zero travel as the aligned 32-bit word that holds the column's half
     // (sub-dword loads make the compiler wait for every outstanding load); `half_sel`
@@ -571,7 +572,7 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
     // fragment addresses (halves, inside a stage); a step's 32 k are four chunks, one per lane group of 16
     // (row offsets are multiples of 16: the same swizzle for all of a lane's rows)
     const int a_frag = (wm0 + (lane & 15)) * PK + (((lane >> 4) ^ pipe_swz(lane)) << 3);
-    const int b_frag[2] = {((lane >> 4) * BN + wn0 + (lane & 15)) * 8, ((lane >> 4) * BN + wn0 + ((lane & 15) ^ 8)) * 8};
+    const int b_frag[2] = {((lane >> 4) * BN + wn0 + (lane & 15)) * 8, ((lane >> 4) * BN + wn0 + ((lane & 15) ^ 4)) * 8};
     auto load_frags = [&](int a_stage, int stage, h16x8 fa[TM], h16x8 fb[TN]) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
