@@ -273,16 +273,17 @@ static std::mutex g_reports_mutex;
 static PackReport g_reports[MOST_REPORTS];
 static int g_n_reports = 0;
 
-static bool clear_count(const PackReport& r) {
-    const int zero = 0;
-    return hipMemcpy(r.count, &zero, sizeof(int), hipMemcpyHostToDevice) == hipSuccess;
+// (on the caller's stream: a copy on the null stream would wait for, or under a capture elsewhere be refused because of, other streams)
+static bool clear_count(const PackReport& r, hipStream_t stream) {
+    static const int zero = 0;
+    return hipMemcpyAsync(r.count, &zero, sizeof(int), hipMemcpyHostToDevice, stream) == hipSuccess;
 }
 static void free_report(const PackReport& r) {
     if (r.count) (void)hipFree(r.count);
     if (r.flag) (void)hipHostFree(r.flag);
 }
 
-static bool take_report(PackReport& r) {
+static bool take_report(PackReport& r, hipStream_t stream) {
     r = PackReport{0, nullptr, nullptr};
     if (hipGetDevice(&r.device) != hipSuccess) return false;
     {
@@ -298,7 +299,7 @@ static bool take_report(PackReport& r) {
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     (void)hipThreadExchangeStreamCaptureMode(&mode);
     const bool ok = hipMalloc(&r.count, sizeof(int)) == hipSuccess && hipHostMalloc(&r.flag, sizeof(int), hipHostMallocDefault) == hipSuccess &&
-                    clear_count(r);
+                    clear_count(r, stream);
     if (ok) *r.flag = 0;
     else free_report(r);
     (void)hipThreadExchangeStreamCaptureMode(&mode);
@@ -364,7 +365,7 @@ int int4mm_sparse_pack_checked(void* wt_outs, void* msk_outs, const void* wt_in,
     if (bad_blocks == nullptr) return INT4MM_ERR_NULL;
     *bad_blocks = 0;
     PackReport r;
-    if (!take_report(r)) return launch_error();
+    if (!take_report(r, (hipStream_t)stream)) return launch_error();
     const int rc = sparse_pack(wt_outs, msk_outs, wt_in, msk_in, out_size, in_size, r.count, r.flag, stream);
     if (hipStreamSynchronize((hipStream_t)stream) != hipSuccess) {          // (the kernel may still write: the report is not used again)
         const int failed = launch_error();
@@ -372,7 +373,8 @@ int int4mm_sparse_pack_checked(void* wt_outs, void* msk_outs, const void* wt_in,
     }
     bool clean = true;
     if (*(volatile int*)r.flag != 0) {
-        clean = hipMemcpy(bad_blocks, r.count, sizeof(int), hipMemcpyDeviceToHost) == hipSuccess && clear_count(r);
+        clean = hipMemcpyAsync(bad_blocks, r.count, sizeof(int), hipMemcpyDeviceToHost, (hipStream_t)stream) == hipSuccess &&
+                clear_count(r, (hipStream_t)stream) && hipStreamSynchronize((hipStream_t)stream) == hipSuccess;
         *r.flag = 0;
     }
     if (!clean) {
