@@ -153,6 +153,7 @@ bool skinny_rows(int bits, _Float16* outs, const uint32_t* matrix, const _Float1
 bool matvec_rows(int bits, _Float16* outs, const uint32_t* matrix, const _Float16* x, const _Float16* scales,
                  const _Float16* zeros, int64_t R, int64_t K, int64_t S, int64_t group_size, bool accumulate,
                  hipStream_t st, void* workspace, size_t workspace_bytes);
+bool matvec_takes_rows(int64_t R, int64_t K, int64_t S);        // is it a shape that the above takes, given a workspace?
 // a single row through the matmul entry (overwrites outs); *rc is the launch's result when the shape is taken
 bool matvec_one_row(int bits, _Float16* outs, const uint32_t* matrix, const uint32_t* sparse_mask, const _Float16* x,
                     const _Float16* scales, const _Float16* zeros, int64_t K, int64_t S, int64_t group_size, hipStream_t st,
@@ -180,6 +181,9 @@ size_t rounded_room(bool sparse, int64_t R, int64_t K, int64_t S, int64_t group_
 // not; it sums exact codes then (false), however much room the workspace has: K=1344, S=5888, 619 elements lost the exact sums of the
 // last 107 when the query made that room.  The limit is what a workspace has that was made for chunks of 512 and for the tile kernels
 bool last_chunk_as_others(bool sparse, int64_t B, int64_t n, int64_t K, int64_t S, int64_t group_units);
+// does the matmul entry leave a product of 2 ... 96 rows to these kernels, given room for any split?  (not: a long K in so many groups that
+// a strip's scales do not fit the LDS, and no whole strips for the kernel with shared staging or fewer rows than it takes)
+bool few_rows_serve(int bits, bool sparse, int64_t R, int64_t K, int64_t S, int64_t group_units);
 // bytes of partial tiles with which such a product splits K across workgroups (0: no split); bits = 0, group_units = 0: not known
 size_t skinny_workspace_bytes(int bits, int64_t R, int64_t K, int64_t S, bool sparse, int64_t group_units, RowsCall call);
 

@@ -1055,7 +1055,8 @@ static void launch(MatmulArgs a, int64_t B, hipStream_t st, void* workspace, siz
     // or the general tiles, 128 x 256, and 128 x 128 for narrow outputs or few rows
     const int variant = (int)tuning(TUNE_MM_VARIANT);
     const WorkspaceParts wsp = workspace_parts(workspace, workspace_bytes);
-    const size_t scratch = wsp.counters != nullptr && B == 1 ? wsp.scratch_bytes : 0;
+    // (a single row comes here where its matvec has a group longer than a launch covers: the size query asks nothing for it)
+    const size_t scratch = wsp.counters != nullptr && B == 1 && (a.M > 1 || variant != 0) ? wsp.scratch_bytes : 0;
     a.counters = reinterpret_cast<int*>(wsp.counters);
     a.part = reinterpret_cast<float*>(wsp.scratch);
     const bool shape_ok = pipe_shape(BITS, SPARSE, a.K, a.S, a.group_units);
@@ -1197,19 +1198,26 @@ extern "C" size_t int4mm_matmul_workspace_bytes(const int4mm_shape* shape, int s
                 if ((n > FEW_ROWS_MAX || !as_others) && share >= 2)
                     few_rows = std::max({few_rows, few(share, EXACT_SUMS), few(std::max<int64_t>(2, share - 1), EXACT_SUMS)});
         }
-    if (B * M <= FEW_ROWS_MAX) return need + 2 * round_to_page(few_rows);
     size_t part = few_rows;
-    const SplitPlan sp = plan_split(sparse != 0, B, M, K, S);
+    const SplitPlan sp = B * M > FEW_ROWS_MAX ? plan_split(sparse != 0, B, M, K, S) : SplitPlan{1, 0, 0};
     const bool chunks = shape->seq_len == 1 && B * M > SK_WIDE_MAX_ROWS;           // (of the matvec entry: last_chunk_as_others)
     if (sp.ksplit > 1 && chunks) part = std::max(part, (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes));
     if (chunks && sp.ksplit == 1) {
         const TailPlan tp = plan_tail(sparse != 0, B, M, K, S);
         if (tp.ksplit > 1) part = round_to_page(part) + (size_t)(tp.tiles * tp.ksplit * (256 * 256 * 4));
     }
+    // (rows that the few-row kernels leave to the tiles are asked for as well: what a product is split into, and with it the order of its
+    // sums, may not hang on what a workspace was made for)
+    const int64_t variant = tuning(TUNE_MM_VARIANT);
+    auto others_serve = [&](int b) {
+        if (variant != 0 || tuning(TUNE_NO_SKINNY) || B != 1 || M > SK_WIDE_MAX_ROWS) return false;
+        if (M <= FEW_ROWS_MAX) return M == 1 || few_rows_serve(b, sparse != 0, M, K, S, group_units);
+        return wide_serves(b, sparse != 0, M, K, S, std::max<int64_t>(1, group_units));
+    };
     for (const int b : {4, 3, 2}) {
-        const int64_t gu = group_units > 0 ? group_units : 1, variant = tuning(TUNE_MM_VARIANT);
-        if (B != 1 || (sparse ? b != 4 : bits != 0 && b != bits) || (M <= SK_WIDE_MAX_ROWS && variant == 0 && !tuning(TUNE_NO_SKINNY) && wide_serves(b, sparse != 0, M, K, S, gu))) continue;
-        if (variant != 0 || takes_tiles(b, sparse != 0, M, K, S, gu)) part = std::max(part, plan_tiles(b, sparse != 0, M, K, S, SIZE_MAX, forced_height(variant)).part_bytes);
+        if (B != 1 || (sparse ? b != 4 : bits != 0 && b != bits) || others_serve(b)) continue;
+        if (variant != 0 || takes_tiles(b, sparse != 0, M, K, S, std::max<int64_t>(1, group_units)))
+            part = std::max(part, plan_tiles(b, sparse != 0, M, K, S, SIZE_MAX, forced_height(variant)).part_bytes);
         if (!sparse && sp.ksplit > 1) part = std::max(part, (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes));        // (the 128-column tiles)
     }
     return need + 2 * round_to_page(part);

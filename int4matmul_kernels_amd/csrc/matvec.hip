@@ -946,11 +946,9 @@ static MatvecShape plan_matvec(int64_t S, int units_total) {
 
 // Two to four rows of states (a matmul with that many rows in all, or a matvec with that many batch
 // elements), dense formats: the matvec kernel with a row per MFMA result register -- one pass over the
-// weights at the matvec's rate.  Returns false when it does not take the shape (the few-row kernels do then):
-// the hand-over needs four slot rows per split, the staged states four times the LDS.
-bool i4::matvec_rows(int bits, h16* outs, const uint32_t* matrix, const h16* x, const h16* scales, const h16* zeros,
-                     int64_t R, int64_t K, int64_t S, int64_t group_size, bool accumulate, hipStream_t st,
-                     void* workspace, size_t workspace_bytes) {
+// weights at the matvec's rate.  Not for every shape (the few-row kernels take the others): the hand-over needs four slot
+// rows per split, the staged states four times the LDS.
+static bool rows_shape(int64_t R, int64_t K, int64_t S, MatvecShape& ms) {
     if (R < 2 || R > 4 || K % 64 != 0 || S % 4 != 0) return false;
     // measured against the few-row kernel (S = 11008 ... 32768, warm weights): 10 - 26 % faster up to K = 5120
     // (K=5120, S=20480: 2 / 3 / 4 rows 14.0 / 15.4 / 17.1 against 18.4 / 18.1 / 18.3 us; K=4096, S=11008: 9.5 / 11.1 /
@@ -968,10 +966,23 @@ bool i4::matvec_rows(int bits, h16* outs, const uint32_t* matrix, const h16* x, 
     if (R > 2 && S <= 16384) return false;
     if (R > 2 && (K > 5120 || K < 4096)) return false;
     const int units_total = (int)(K / 64);
-    const MatvecShape ms = plan_matvec(S, units_total);
+    ms = plan_matvec(S, units_total);
     const int nr = R <= 2 ? 2 : 4;
     if (ms.splits * nr > MV_MAX_SPLITS || ms.upwg * nr > MV_MAX_UNITS_WG) return false;
     if (R == 2 && K > 5120 && ms.splits > 5) return false;
+    return true;
+}
+bool i4::matvec_takes_rows(int64_t R, int64_t K, int64_t S) {
+    MatvecShape ms;
+    return rows_shape(R, K, S, ms);
+}
+
+bool i4::matvec_rows(int bits, h16* outs, const uint32_t* matrix, const h16* x, const h16* scales, const h16* zeros,
+                     int64_t R, int64_t K, int64_t S, int64_t group_size, bool accumulate, hipStream_t st,
+                     void* workspace, size_t workspace_bytes) {
+    MatvecShape ms;
+    if (!rows_shape(R, K, S, ms)) return false;
+    const int units_total = (int)(K / 64), nr = R <= 2 ? 2 : 4;
     const WorkspaceParts ws = workspace_parts(workspace, workspace_bytes);
     if (ms.splits > 1 && ws.slots_bytes < matvec_slots_bytes(S)) return false;
     const bool pf = ms.upwg >= 3 * ms.waves * ms.lk && tuning(TUNE_MV_NOPF) == 0;

@@ -841,12 +841,39 @@ static SkinnySplit plan_skinny_split(int64_t R, int64_t K, int64_t S, bool spars
     return p;
 }
 
+// Waves of the unsplit kernel.  Four split K when there are more workgroups than CUs (three of them fit a CU) and K
+// is short (each wave should walk a dozen units or more), eight otherwise -- also at exactly one
+// workgroup per CU, where eight waves keep twice the bytes in flight (K=5120, S=16384, 8 rows:
+// 14.6 -> 12.0 us; K=S=8192: 16.5 -> 12.3 us; 320 and 448 strips: 17.7 against 22.2, 27 against 32)
+static int unsplit_waves(int64_t S, int cw, int64_t units) { return S / (16 * cw) > 256 && units < 160 ? 4 : 8; }
+
+// Do the scales of a strip's groups, or of those of a share of K, leave the LDS room for the waves' units?  (a group that is not known: the
+// smallest)
+static bool few_row_groups_fit(int64_t R, int64_t K, int64_t S, bool sparse, int64_t group_units) {
+    const int64_t units = K / 64, gu = std::max<int64_t>(1, std::min(group_units, units)), groups = (units + gu - 1) / gu;
+    auto fits = [&](int cw, int waves, int64_t n) { return skinny_lds_bytes(cw, waves, (int)n) <= skinny_lds_limit(sparse); };
+    const SkinnySplit p = plan_skinny_split(R, K, S, sparse);
+    if (p.ksplit > 1) {
+        const int64_t share = (units + p.ksplit - 1) / p.ksplit;
+        if (fits(p.cw, 8, std::min(groups, (share + gu - 1) / gu + 1))) return true;
+    }
+    const int cw = unsplit_cw(R, S, sparse);
+    return fits(cw, unsplit_waves(S, cw, units), groups);
+}
+
+bool few_rows_serve(int bits, bool sparse, int64_t R, int64_t K, int64_t S, int64_t group_units) {
+    if (!sparse && matvec_takes_rows(R, K, S)) return true;
+    if (few_row_groups_fit(R, K, S, sparse, group_units)) return true;
+    for (const int b : {4, 3, 2})
+        if ((sparse ? b == 4 : bits == 0 || b == bits) && (R < 17 || !wide_serves(b, sparse, R, K, S, std::max<int64_t>(1, group_units)))) return false;
+    return true;
+}
+
 size_t skinny_workspace_bytes(int bits, int64_t R, int64_t K, int64_t S, bool sparse, int64_t group_units, RowsCall call) {
     const SkinnySplit p = plan_skinny_split(R, K, S, sparse);
     size_t wide = wide_workspace_bytes(bits, R, K, S, sparse, group_units, call);
-    // (a product that falls through skinny_rows; a group that is not known: the smallest)
-    if (call == FOR_MATMUL && wide == 0 && p.ksplit <= 1 && R >= 17 && R <= FEW_ROWS_MAX &&
-        skinny_lds_bytes(unsplit_cw(R, S, sparse), 8, (int)(K / 64 / std::max<int64_t>(1, group_units))) > skinny_lds_limit(sparse))
+    // (a product that falls through skinny_rows)
+    if (call == FOR_MATMUL && wide == 0 && R >= 17 && R <= FEW_ROWS_MAX && !few_row_groups_fit(R, K, S, sparse, group_units))
         wide = wide_workspace_bytes(bits, R, K, S, sparse, group_units, ROUNDED);
     const size_t balanced = balanced_shape(R, K, S) ? skinny_balanced_part_bytes(S) : 0;
     return std::max(std::max<size_t>(p.ksplit > 1 ? p.part_bytes : 0, wide), balanced);
@@ -873,10 +900,6 @@ bool skinny_rows(int bits, h16* outs, const uint32_t* matrix, const h16* x, cons
     // 17 rows and more: the kernel whose waves share the staged states, where its plan says so
     if (wide_rows(bits, a, call, workspace, workspace_bytes, st)) return true;
     if (R > FEW_ROWS_MAX) return false;
-    // four waves split K when there are more workgroups than CUs (three of them fit a CU) and K
-    // is short (each wave should walk a dozen units or more), eight otherwise -- also at exactly one
-    // workgroup per CU, where eight waves keep twice the bytes in flight (K=5120, S=16384, 8 rows:
-    // 14.6 -> 12.0 us; K=S=8192: 16.5 -> 12.3 us; 320 and 448 strips: 17.7 against 22.2, 27 against 32)
     int cw = unsplit_cw(R, S, sparse_mask != nullptr);
     {   // (tuning: columns per lane of the few-row kernel where the shape allows them)
         const int64_t forced_cw = tuning(TUNE_MV_LK);
@@ -885,7 +908,7 @@ bool skinny_rows(int bits, h16* outs, const uint32_t* matrix, const h16* x, cons
     }
     const int units = (int)(K / 64);
     int waves = (int)tuning(TUNE_MV_WAVES);
-    if (waves != 2 && waves != 4 && waves != 8) waves = S / (16 * cw) > 256 && units < 160 ? 4 : 8;
+    if (waves != 2 && waves != 4 && waves != 8) waves = unsplit_waves(S, cw, units);
     while (waves > 1 && units < 2 * waves) waves >>= 1;
     auto launch = [&](int cw_, int waves_, int ksplit_) {
         a.units_per_wave = (a.units_per_split + waves_ - 1) / waves_;

@@ -243,6 +243,22 @@ def test_the_workspace_asked_for_is_all_that_a_product_uses(s):
             assert capi.matmul_workspace_bytes(1, rows, 8192, s) == capi.lib().int4mm_workspace_bytes(s)
 
 
+@pytest.mark.parametrize("bits,sparse,rows,k,s,g", [(4, False, 75, 20864, 17856, 64), (4, True, 14, 23232, 10944, 64), (4, False, 16, 28672, 9216, 64),
+                                                    (2, False, 72, 43776, 10048, 64), (3, False, 2, 40960, 9216, 64), (4, True, 27, 49472, 4736, 64),
+                                                    (4, True, 2, 46720, 27264, 128), (2, False, 5, 21376, 34560, 64), (3, False, 96, 20480, 12352, 64),
+                                                    (4, False, 1, 917504, 1024, 524288)])
+def test_few_rows_that_are_left_to_the_tiles_are_split_alike_on_any_workspace(bits, sparse, rows, k, s, g):
+    # so many groups that their scales do not fit the few-row kernel's LDS (and a single row with a group longer than a launch of the
+    # matvec covers): the launch with the workspace that the query asks for, knowing the group or not, is the launch with any amount
+    # more, which other products on the stream may have left there
+    plenty = d("mtx", bits, 1, rows, k, s, g, sparse, 1 << 34)
+    assert d("mtx", bits, 1, rows, k, s, g, sparse) == plenty
+    nbytes = capi.matmul_workspace_bytes(1, rows, k, s, sparse)
+    assert d("mtx", bits, 1, rows, k, s, g, sparse, nbytes) == plenty
+    name, f, line = fields(plenty)
+    assert name == "matmul_kernel_pipe" and (f["ksplit"] > 1) == (rows > 1), line
+
+
 def test_matvec_of_a_k_beyond_one_launch():
     # 32 x 224 units of 64 rows is what one launch covers: a longer K runs as several launches (one line each)
     line = d("vec", 4, 1, 1, 1 << 20, 256, 128)

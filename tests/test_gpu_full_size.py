@@ -187,3 +187,29 @@ def test_long_k_narrow_output_takes_split_small_tiles(H, bits):
     finally:
         H.capi.tune(6, 0)
     assert O.max_rel_error(ref.astype(np.float64), out) < H.TOL_EXACT_MTX
+
+
+@pytest.mark.parametrize("bits,sparse,M", [(4, False, 16), (3, False, 5), (2, False, 75), (4, True, 14)])
+def test_few_rows_in_many_groups_on_any_workspace(H, bits, sparse, M):
+    """321 groups, whose scales do not fit the few-row kernel's LDS: tiles split seven ways along K, the last one three quarters
+    full.  The same bits on the workspace that is asked for and on a larger one; the first and the last columns against the oracle."""
+    K, S, g = 20544, 8384, 64
+    line = H.capi.describe_launch("mtx", bits, 1, M, K, S, g, sparse)
+    assert line.startswith("matmul_kernel_pipe") and "ksplit=7" in line, line
+    rng = np.random.default_rng(M)
+    rows = K // 16 if sparse else K * bits // 32
+    mask = np.array([0x0F0F3355, 0x5555AAAA, 0x00FFFF00, 0xFFFF0000], np.uint32)[rng.integers(0, 4, (K // 32, S))].view(np.int32) if sparse else None
+    p = dict(bits=bits, B=1, M=M, K=K, S=S, group_size=g, sparse_mask=mask,
+             matrix=rng.integers(-2**31, 2**31, (rows, S), dtype=np.int32),
+             states=rng.standard_normal((1, M, K), dtype=np.float32).astype(np.float16),
+             scales=rng.uniform(0.001, 0.02, (K // g, S)).astype(np.float16),
+             zeros=rng.uniform(0, 2**bits - 1, (K // g, S)).astype(np.float16))
+    d = H.dev_problem(p)
+    got = H.run_capi(p, d, "mtx", outs_init=np.full((1, M, S), 3.0, np.float16))
+    larger = torch.full((1, M, S), 7.0, dtype=torch.float16, device=H.DEV)
+    ws = torch.zeros(1 << 28, dtype=torch.uint8, device=H.DEV)
+    H.capi.matmul(bits, larger, d["matrix"], d["states"], d["scales"], d["zeros"], g, d["mask"], ws)
+    assert np.array_equal(got.view(np.uint16), larger.cpu().numpy().view(np.uint16))
+    for cols in (slice(0, 320), slice(S - 320, S)):
+        w16 = O.dequantize_matrix(bits, p["matrix"][:, cols], p["scales"][:, cols], p["zeros"][:, cols], g, None if mask is None else mask[:, cols])
+        assert O.max_rel_error(O.matmul_exact(p["states"][0], w16), got[0][:, cols], floor_frac=H.FLOOR_EXACT_MTX) < H.TOL_EXACT_MTX
