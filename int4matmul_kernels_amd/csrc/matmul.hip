@@ -1060,17 +1060,14 @@ static void launch(MatmulArgs a, int64_t B, hipStream_t st, void* workspace, siz
     a.counters = reinterpret_cast<int*>(wsp.counters);
     a.part = reinterpret_cast<float*>(wsp.scratch);
     const bool shape_ok = pipe_shape(BITS, SPARSE, a.K, a.S, a.group_units);
-    // the 128-column form: where rows of 256 pad less than half (or would leave the general tiles a second row); and 513 ... 1152
-    // rows that are a whole odd number of 128s on a K so long that three ways leave shares of 140 steps, for which its tests
-    // ask (int4, K=14336, S=4096, 1152 rows 166 us; 192 x 256 two ways 136)
+    // the 128-column form: outputs of 128 columns where rows of 256 pad less than half (or would leave the general tiles a second row)
     bool narrow = false;
     if constexpr (!SPARSE) {
-        const int64_t m_pad = (a.M + 255) / 256 * 256, rows_128 = (a.M + 127) / 128, tiles_128 = rows_128 * ((a.S + 255) / 256);
+        const int64_t m_pad = (a.M + 255) / 256 * 256;
         const bool fits = shape_ok && B == 1 && tile_columns(a.S, 128, false) && (m_pad * 2 <= a.M * 3 || (a.M > 128 && a.M <= 256));
         const SplitPlan sp = plan_split(false, B, a.M, a.K, a.S);
         const bool split = sp.ksplit > 1 && scratch >= (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes);
-        const bool long_k = a.M > 512 && a.M % 256 == 128 && a.M <= 1152 && tiles_128 >= 128 && tiles_128 <= 256 && sp.ksplit >= 3 && a.K / 32 / sp.ksplit >= 140;
-        narrow = fits && (variant == 5 || (variant == 0 && ((split && long_k) || (!tile_columns(a.S, 256, true) && a.K > 1024))));
+        narrow = fits && (variant == 5 || (variant == 0 && !tile_columns(a.S, 256, true) && a.K > 1024));
         if (narrow && split) a.ksplit = sp.ksplit;
     }
     const int only = forced_height(variant);

@@ -259,6 +259,14 @@ def test_few_rows_that_are_left_to_the_tiles_are_split_alike_on_any_workspace(bi
     assert name == "matmul_kernel_pipe" and (f["ksplit"] > 1) == (rows > 1), line
 
 
+@pytest.mark.parametrize("bits", [4, 3, 2])
+def test_a_row_more_or_fewer_takes_the_same_tiles(bits):
+    # 640 and 1152 rows on a long K are no rule of their own: the tiles that their neighbours take (rows padded to the same height)
+    for rows, k, s in ((640, 28672, 3840), (1152, 14336, 4096), (1152, 20480, 4096), (1152, 28672, 2048)):
+        line = d("mtx", bits, 1, rows, k, s, 128)
+        assert "x256," in line and line == d("mtx", bits, 1, rows - 1, k, s, 128), line
+
+
 def test_matvec_of_a_k_beyond_one_launch():
     # 32 x 224 units of 64 rows is what one launch covers: a longer K runs as several launches (one line each)
     line = d("vec", 4, 1, 1, 1 << 20, 256, 128)

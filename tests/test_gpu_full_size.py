@@ -167,13 +167,14 @@ def test_mixed_quantisation_modes_matvec_full_size(H, bits):
 
 
 @pytest.mark.parametrize("bits", [4, 3])
-def test_long_k_narrow_output_takes_split_small_tiles(H, bits):
+def test_long_k_narrow_output_takes_split_tiles(H, bits):
     """K=14336, S=4096, 1152 rows: nine rows of 128 x 256 tiles would fill the GPU once; the long K makes
-    256 x 128 tiles split three ways along K the faster choice.  Sampled rows against the oracle, the whole
-    output against the unsplit kernel."""
+    256 x 256 tiles split three ways along K the faster choice, as for one row fewer.  The 128-column tiles, which served whole odd
+    numbers of 128 rows before and took longer, are forced with the same split.  Sampled rows against the oracle, the whole
+    outputs against the unsplit kernel."""
     K, S, g, M = 14336, 4096, 128, 1152
     tiles = H.capi.describe_launch("mtx", bits, 1, M, K, S, g)
-    assert "tile=256x128,plain> tiles=160 ksplit=3" in tiles, tiles
+    assert "tile=256x256,two-phase> tiles=80 ksplit=3" in tiles and tiles == H.capi.describe_launch("mtx", bits, 1, M - 1, K, S, g), tiles
     kw = {} if bits == 4 else dict(scale_range=(0.004, 0.08), zero_const=3.5)
     p = O.make_problem(K=K, S=S, M=1, bits=bits, group_size=g, seed=3, **kw)
     xs = np.random.default_rng(6).standard_normal((1, M, K), dtype=np.float32).astype(np.float16)
@@ -181,12 +182,17 @@ def test_long_k_narrow_output_takes_split_small_tiles(H, bits):
     d = H.dev_problem(pm)
     out = H.run_capi(pm, d, "mtx", outs_init=np.full((1, M, S), 5.0, np.float16))
     _matmul_rows_against_oracle(H, pm, out, np.array([0, 1, 127, 128, 255, 256, 511, 512, 767, 1023, 1024, 1150, 1151]))
-    H.capi.tune(6, 1)
     try:
+        H.capi.tune(6, 1)
         ref = H.run_capi(pm, d, "mtx")
+        H.capi.tune(3, 5)
+        H.capi.tune(6, 3)
+        narrow = H.run_capi(pm, d, "mtx", outs_init=np.full((1, M, S), 5.0, np.float16))
     finally:
+        H.capi.tune(3, 0)
         H.capi.tune(6, 0)
     assert O.max_rel_error(ref.astype(np.float64), out) < H.TOL_EXACT_MTX
+    assert O.max_rel_error(ref.astype(np.float64), narrow) < H.TOL_EXACT_MTX
 
 
 @pytest.mark.parametrize("bits,sparse,M", [(4, False, 16), (3, False, 5), (2, False, 75), (4, True, 14)])
