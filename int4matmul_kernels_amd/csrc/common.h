@@ -160,8 +160,8 @@ bool matvec_one_row(int bits, _Float16* outs, const uint32_t* matrix, const uint
                     void* workspace, size_t workspace_bytes, int* rc);
 // what the tile kernels' plan takes for a product, by its cost model (1e30: they do not take the shape)
 double tiles_us(int bits, bool sparse, int64_t M, int64_t K, int64_t S, int64_t group_units, size_t scratch);
-// does the matmul entry leave a product of 97 ... 512 rows to the kernel with shared staging, given room for any split?
-bool wide_serves(int bits, bool sparse, int64_t R, int64_t K, int64_t S, int64_t group_units);
+// does the matmul entry leave a product of 97 ... 512 rows to the kernel with shared staging, given room for any split?  *part_bytes: that room
+bool wide_serves(int bits, bool sparse, int64_t R, int64_t K, int64_t S, int64_t group_units, size_t* part_bytes = nullptr);
 // most rows the few-row path takes (beyond 96: only its kernel with shared staging, for the shapes it serves)
 constexpr int SK_WIDE_MAX_ROWS = 512;
 constexpr int FEW_ROWS_MAX = 96;                     // rows that the few-row kernel with its sums of exact codes takes at once

@@ -1039,6 +1039,13 @@ static bool takes_tiles(int bits, bool sparse, int64_t M, int64_t K, int64_t S, 
            (sparse || K >= 1024 || (M + 255) / 256 * ((S + 255) / 256) > 128);
 }
 
+// the 128-column form: outputs of 128 columns where rows of 256 pad less than half (or would leave the general tiles a second row)
+static bool takes_narrow_tiles(int bits, bool sparse, int64_t M, int64_t K, int64_t S, int64_t group_units) {
+    const int64_t variant = tuning(TUNE_MM_VARIANT), m_pad = (M + 255) / 256 * 256;
+    return !sparse && pipe_shape(bits, sparse, K, S, group_units) && tile_columns(S, 128, false) && (m_pad * 2 <= M * 3 || (M > 128 && M <= 256)) &&
+           (variant == 5 || (variant == 0 && K > 1024 && !tile_columns(S, 256, true)));
+}
+
 double tiles_us(int bits, bool sparse, int64_t M, int64_t K, int64_t S, int64_t group_units, size_t scratch) {
     return takes_tiles(bits, sparse, M, K, S, group_units) ? plan_tiles(bits, sparse, M, K, S, scratch, 0).us : 1e30;
 }
@@ -1059,19 +1066,13 @@ static void launch(MatmulArgs a, int64_t B, hipStream_t st, void* workspace, siz
     const size_t scratch = wsp.counters != nullptr && B == 1 && (a.M > 1 || variant != 0) ? wsp.scratch_bytes : 0;
     a.counters = reinterpret_cast<int*>(wsp.counters);
     a.part = reinterpret_cast<float*>(wsp.scratch);
-    const bool shape_ok = pipe_shape(BITS, SPARSE, a.K, a.S, a.group_units);
-    // the 128-column form: outputs of 128 columns where rows of 256 pad less than half (or would leave the general tiles a second row)
-    bool narrow = false;
-    if constexpr (!SPARSE) {
-        const int64_t m_pad = (a.M + 255) / 256 * 256;
-        const bool fits = shape_ok && B == 1 && tile_columns(a.S, 128, false) && (m_pad * 2 <= a.M * 3 || (a.M > 128 && a.M <= 256));
+    const bool narrow = B == 1 && takes_narrow_tiles(BITS, SPARSE, a.M, a.K, a.S, a.group_units);
+    if (narrow) {
         const SplitPlan sp = plan_split(false, B, a.M, a.K, a.S);
-        const bool split = sp.ksplit > 1 && scratch >= (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes);
-        narrow = fits && (variant == 5 || (variant == 0 && !tile_columns(a.S, 256, true) && a.K > 1024));
-        if (narrow && split) a.ksplit = sp.ksplit;
+        if (sp.ksplit > 1 && scratch >= (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes)) a.ksplit = sp.ksplit;
     }
     const int only = forced_height(variant);
-    const bool tiles = !narrow && (variant == 0 ? takes_tiles(BITS, SPARSE, a.M, a.K, a.S, a.group_units) : only != 0 && shape_ok && tile_columns(a.S, 256, true));
+    const bool tiles = !narrow && (variant == 0 ? takes_tiles(BITS, SPARSE, a.M, a.K, a.S, a.group_units) : only != 0 && pipe_shape(BITS, SPARSE, a.K, a.S, a.group_units) && tile_columns(a.S, 256, true));
     if (narrow) {
         if constexpr (!SPARSE) launch_pipe<BITS, false, 2>(a, B, st);
     } else if (tiles) {
@@ -1182,7 +1183,7 @@ extern "C" size_t int4mm_matmul_workspace_bytes(const int4mm_shape* shape, int s
         if (shape->matrix_rows * 32 == K * b) bits = b;
     const int64_t g = shape->group_size, group_units = g < 0 ? ONE_GROUP / 64 : g / 64;
     auto few = [&](int64_t rows, RowsCall call) { return skinny_workspace_bytes(bits, rows, K, S, sparse != 0, group_units, call); };
-    size_t few_rows = B * M <= SK_WIDE_MAX_ROWS ? few(B * M, FOR_MATMUL) : 0;
+    size_t few_rows = B * M <= FEW_ROWS_MAX ? few(B * M, FOR_MATMUL) : 0;
     // (the matvec entry takes many batch elements of one row in chunks through the few-row kernels: as many as the kernel
     // for more rows takes, else even shares, which may be one fewer towards the end; its callers may ask with the flattened
     // shape too)
@@ -1209,13 +1210,17 @@ extern "C" size_t int4mm_matmul_workspace_bytes(const int4mm_shape* shape, int s
     auto others_serve = [&](int b) {
         if (variant != 0 || tuning(TUNE_NO_SKINNY) || B != 1 || M > SK_WIDE_MAX_ROWS) return false;
         if (M <= FEW_ROWS_MAX) return M == 1 || few_rows_serve(b, sparse != 0, M, K, S, group_units);
-        return wide_serves(b, sparse != 0, M, K, S, std::max<int64_t>(1, group_units));
+        size_t bytes = 0;
+        if (!wide_serves(b, sparse != 0, M, K, S, std::max<int64_t>(1, group_units), &bytes)) return false;
+        part = std::max(part, bytes);
+        return true;
     };
     for (const int b : {4, 3, 2}) {
         if (B != 1 || (sparse ? b != 4 : bits != 0 && b != bits) || others_serve(b)) continue;
-        if (variant != 0 || takes_tiles(b, sparse != 0, M, K, S, std::max<int64_t>(1, group_units)))
-            part = std::max(part, plan_tiles(b, sparse != 0, M, K, S, SIZE_MAX, forced_height(variant)).part_bytes);
-        if (!sparse && sp.ksplit > 1) part = std::max(part, (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes));        // (the 128-column tiles)
+        const int64_t gu = std::max<int64_t>(1, group_units);
+        if (takes_narrow_tiles(b, sparse != 0, M, K, S, gu)) {
+            if (sp.ksplit > 1) part = std::max(part, (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes));
+        } else if (variant != 0 || takes_tiles(b, sparse != 0, M, K, S, gu)) part = std::max(part, plan_tiles(b, sparse != 0, M, K, S, SIZE_MAX, forced_height(variant)).part_bytes);
     }
     return need + 2 * round_to_page(part);
 }

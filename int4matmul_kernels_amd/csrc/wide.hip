@@ -712,8 +712,9 @@ static bool tiles_instead(int bits, bool sparse, int64_t R, int64_t K, int64_t S
 }
 
 // Does the matmul entry leave a product of 97 ... 512 rows to this kernel, given room for any split?
-bool wide_serves(int bits, bool sparse, int64_t R, int64_t K, int64_t S, int64_t group_units) {
+bool wide_serves(int bits, bool sparse, int64_t R, int64_t K, int64_t S, int64_t group_units, size_t* part_bytes) {
     const WidePlan p = plan_wide(bits, sparse, R, K, S, SIZE_MAX);
+    if (part_bytes) *part_bytes = p.part_bytes;
     return p.use && !tiles_instead(bits, sparse, R, K, S, group_units, SIZE_MAX, p);
 }
 

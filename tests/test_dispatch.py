@@ -267,6 +267,18 @@ def test_a_row_more_or_fewer_takes_the_same_tiles(bits):
         assert "x256," in line and line == d("mtx", bits, 1, rows - 1, k, s, 128), line
 
 
+@pytest.mark.parametrize("bits,rows,k,s,g", [(3, 546, 30272, 8832, 128), (4, 703, 31104, 9088, -1), (2, 2643, 31872, 2432, -1), (3, 293, 23936, 13568, -1),
+                                             (4, 289, 24320, 13440, 128), (4, 2048, 8192, 128, 128), (2, 600, 4096, 128, 64), (4, 1152, 14336, 4096, 128)])
+def test_the_workspace_asked_for_is_the_partial_tiles_of_the_launch(bits, rows, k, s, g):
+    # not what a kernel that the product does not go to would split into (int3, K=23936, S=13568, 293 rows asked for 340 MB and used 35)
+    name, f, line = fields(d("mtx", bits, 1, rows, k, s, g))
+    tm, tn = (int(v) for v in line.split("tile=")[1].split(",")[0].split("x"))
+    assert name == "matmul_kernel_pipe" and f["ksplit"] > 1, line
+    used = (f["tiles"] - f["split_from"]) * f["ksplit"] * tm * tn * 4
+    sh = capi.Shape(1, rows, k, s, k * bits // 32, 1 if g < 0 else -(-k // g), g)
+    assert capi.lib().int4mm_matmul_workspace_bytes(sh, 0) - capi.lib().int4mm_workspace_bytes(s) == 2 * (-(-used // 4096) * 4096)
+
+
 def test_matvec_of_a_k_beyond_one_launch():
     # 32 x 224 units of 64 rows is what one launch covers: a longer K runs as several launches (one line each)
     line = d("vec", 4, 1, 1, 1 << 20, 256, 128)
