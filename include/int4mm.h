@@ -91,7 +91,7 @@ INT4MM_API int int4mm_abi_version(void);
  * heuristic for the calling host thread (value 0 restores the default).  key 0 = waves per
  * workgroup of the matvec and few-row kernels, 1 = matvec 64-row units per lane
  * group, 2 = matvec lane groups per wave / few-row kernel columns per lane (1, 2, 4), 3 = matmul kernel variant
- * (1 / 3 = general 128x128 / 128x256 tiles, 5 / 6 / 7 / 8 = pipelined 256x128 / 256x256 / 128x256 /
+ * (1 / 3 = general 128x128 / 128x256 tiles, 5 / 6 / 7 / 8 = pipelined 128x128 / 256x256 / 128x256 /
  * 192x256 tiles, 9 = 256x256 without the two-phase order, 10 / 11 = 160x256 / 224x256; a forced variant also keeps the product away from the
  * few-row kernels), 4 = matvec: 1 disables prefetch,
  * 5 = 1 disables the few-row (2..512 rows) kernels, 6 = split-K factor of the

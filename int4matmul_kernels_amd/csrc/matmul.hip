@@ -396,9 +396,8 @@ template <> struct PipeFmt<3, false> { static constexpr int ROWS = 3, NWORDS = 2
 template <> struct PipeFmt<2, false> { static constexpr int ROWS = 2, NWORDS = 1; };
 template <> struct PipeFmt<4, true> { static constexpr int ROWS = 2, NWORDS = 2; };
 
-constexpr int P_STAGES = 3;
-constexpr int pipe_a_stages(int nw) { return nw == 4 ? 6 : P_STAGES; }
-constexpr int A_AHEAD = 5;                 // steps that the states loaded straight to LDS are ahead
+constexpr int P_STAGES = 3, A_STAGES = 6;  // of the weights, of the states
+constexpr int A_AHEAD = 5;                 // steps that the states are ahead
 // immediate of s_waitcnt: at most so many vector memory and LDS operations outstanding
 constexpr int wait_counts(int vm, int lgkm) { return (vm & 15) | 0x70 | lgkm << 8 | (vm >> 4) << 14; }
 
@@ -408,25 +407,21 @@ constexpr int wait_counts(int vm, int lgkm) { return (vm & 15) | 0x70 | lgkm << 
 __device__ __forceinline__ int pipe_swz(int m) { return ((m >> 3) & 1) | (((m >> 1 ^ m >> 2) & 2)); }
 
 // PING: the waves of the first half run phase 0, MFMAs first and then everything else; those of the second half phase 1,
-// everything else first and the MFMAs last.  Without it all waves run phase 1, which is what the 128-column kernel does: its two
-// workgroups per CU drift apart by themselves.
+// everything else first and the MFMAs last.  Without it all waves run phase 1.
 template <int BITS, bool SPARSE, int TM, int NW, bool PING, bool SPLIT>
 __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, const int s0, const h16* x,
-                                          h16* outs, h16* const (&As)[pipe_a_stages(NW)], h16* Bs, uint32_t* lut, const int tile, const int split,
+                                          h16* outs, h16* const (&As)[A_STAGES], h16* Bs, uint32_t* lut, const int tile, const int split,
                                           const int nsplit) {
     constexpr int BM = TM * 32, BN = NW * 64, WM = TM * 16, WN = 64, TN = 4, T = 2 * NW * 64;
     constexpr int A_ROWS = T / 4;                                  // rows covered by one 16-byte load per thread
     constexpr int A_LOADS = (BM + A_ROWS - 1) / A_ROWS;            // such loads per thread and step (192 rows: the second half full)
     constexpr int B_STAGE = PK * BN;                               // halves per stage
-    constexpr bool DMA = NW == 4;
 
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm0 = (wave / NW) * WM, wn0 = (wave % NW) * WN;
 
     // states stage: row m at m * 64 bytes, 16-byte chunk c of the row at c ^ pipe_swz(m).  Thread t fills position t % 4 of rows
-    // t / 4 + A_ROWS * i (rows >= M re-read row M - 1 and are dropped at the store), from global memory straight to LDS or, in the
-    // 128-column kernel, whose two workgroups per CU leave no LDS for that many stages, through registers.
-    struct AStage { u32x4 v[A_LOADS]; };
+    // t / 4 + A_ROWS * i (rows >= M re-read row M - 1 and are dropped at the store), from global memory straight to LDS.
     const int a_row = t >> 2, a_chunk = (t & 3) ^ pipe_swz(a_row);            // (rows + A_ROWS: same swizzle)
     // every global address is a buffer resource (the tile's rows of states; the whole
     // of the packed matrix, mask, scales, zeros) plus a per-lane 32-bit byte offset that
@@ -440,14 +435,6 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
 #pragma unroll
     for (int i = 0; i < A_LOADS; ++i)
         a_off[i] = (uint32_t)((min(a_row + A_ROWS * i, min(a.M - m0, BM) - 1) * a.K + a_chunk * 8) * 2);
-    auto load_a = [&](AStage& r, uint32_t step_off) {
-#pragma unroll
-        for (int i = 0; i < A_LOADS; ++i) r.v[i] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_off[i], step_off, 0);
-    };
-    auto write_a = [&](const AStage& r, int stage) {
-#pragma unroll
-        for (int i = 0; i < A_LOADS; ++i) *reinterpret_cast<u32x4*>(&As[stage][i * A_ROWS * PK + t * 8]) = r.v[i];
-    };
     auto dma_a = [&](int stage, uint32_t step_off) {
 #pragma unroll
         for (int i = 0; i < A_LOADS; ++i)
@@ -597,7 +584,7 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
     const int last = kt0 + ktiles - 1;
 
     // Cursors of the loads: weights run four K steps ahead of the MFMAs, states
-    // three; both stop at the last step (the surplus loads re-read it, unused).
+    // A_AHEAD; both stop at the last step (the surplus loads re-read it, unused).
     Cursor cur = cursor_at(kt0);
     // (selects instead of branches: a branch here would split the scheduling
     // region of the step and invite the compiler to reuse the previous step's
@@ -622,19 +609,12 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
         a_cur += more * (PK * 2);
     };
     Stage r[3];
-    AStage ra[2];
     // the first steps' operands are requested before the look at the scales below, whose
     // round trip to memory they then share
-    if constexpr (!DMA) {
-        load_a(ra[0], a_cur); advance_a();
-        load_a(ra[1], a_cur); advance_a();
-    }
     load_b(r[0], cur, true); advance();
     load_b(r[1], cur, false); advance();
-    if constexpr (DMA) {
 #pragma unroll
-        for (int i = 0; i < A_AHEAD; ++i) { dma_a(i, a_cur); advance_a(); }
-    }
+    for (int i = 0; i < A_AHEAD; ++i) { dma_a(i, a_cur); advance_a(); }
 
     // Does any (group, column) of this tile use exponent quantisation (scale < 0
     // or NaN)?  One pass over the tile's scales (a few KB); the answer is
@@ -684,31 +664,29 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
         __syncthreads();
     }
 
-    // Step kt, u = kt % 6, weights' stage b = kt % 3, states' stage u (registers: b).  On entry states and decoded weights of
+    // Step kt, u = kt % 6, weights' stage b = kt % 3, states' stage u.  On entry states and decoded weights of
     // steps kt and kt + 1 are complete.  The step stores the decoded weights of step kt + 2 and asks for the packed ones of
-    // kt + 4 and the states of kt + A_AHEAD (registers: moves those of kt + 2 to LDS and asks for kt + 3).  Phase 0:
+    // kt + 4 and the states of kt + A_AHEAD.  Phase 0:
     // MFMAs, on fragments fetched in the step before, beside the decode of step kt + 2's weights; then stores, loads, the next
     // step's fragments.  Phase 1: the step's own fragments, stores of what the step before decoded, loads; then MFMAs
     // beside the decode of step kt + 3's weights.
     h16x8 fa[TM], fb[TN], dec[2];
     auto walk = [&](auto mode) {
         Coef<BITS, decltype(mode)::value> co[PAIR ? 2 : 1];
-        auto body = [&](auto phase_tag, int u, AStage& ra_new, const AStage& ra_wr, Stage& r_new, const Stage& r_dec) {
+        auto body = [&](auto phase_tag, int u, Stage& r_new, const Stage& r_dec) {
             constexpr int phase = decltype(phase_tag)::value;
             const int b = u % P_STAGES, b1 = (u + 1) % P_STAGES, b2 = (u + 2) % P_STAGES;
             auto stores_and_loads = [&]() {
                 write_b(dec, b2);
-                if constexpr (!DMA) write_a(ra_wr, b2);
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (DMA) dma_a((u + A_AHEAD) % 6, a_cur);
-                else load_a(ra_new, a_cur);
+                dma_a((u + A_AHEAD) % A_STAGES, a_cur);
                 load_b(r_new, cur, u % 2 == 0);
                 advance_a();
                 advance();
                 __builtin_amdgcn_sched_barrier(0);
             };
             if constexpr (phase == 1) {
-                load_frags(DMA ? u : b, b, fa, fb);
+                load_frags(u, b, fa, fb);
                 __builtin_amdgcn_sched_barrier(0);
                 stores_and_loads();
             }
@@ -731,30 +709,25 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
             }
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (phase == 0) stores_and_loads();
-            // the step's stores are complete (lgkmcnt(0)) and, of the states loaded straight to LDS, all but the last two steps'
-            __builtin_amdgcn_s_waitcnt(DMA ? wait_counts(2 * (A_LOADS + W_LOADS) + 2, 0) : wait_counts(63, 0));
+            // the step's stores are complete (lgkmcnt(0)) and, of the loads, all but the last two steps'
+            __builtin_amdgcn_s_waitcnt(wait_counts(2 * (A_LOADS + W_LOADS) + 2, 0));
             if constexpr (phase == 0) {
-                load_frags(DMA ? (u + 1) % 6 : b1, b1, fa, fb);
+                load_frags((u + 1) % A_STAGES, b1, fa, fb);
                 __builtin_amdgcn_sched_barrier(0);
             }
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
         };
-        if constexpr (!DMA) {
-            write_a(ra[0], 0);
-            write_a(ra[1], 1);
-            load_a(ra[0], a_cur); advance_a();              // step 2
-        }
         take_sz(co);
         decode(r[0], co, dec);
         write_b(dec, 0);
         decode(r[1], co, dec);
         write_b(dec, 1);
-        if constexpr (DMA) __builtin_amdgcn_s_waitcnt(wait_counts(0, 15));         // steps 0 ... A_AHEAD - 1 of the states
+        __builtin_amdgcn_s_waitcnt(wait_counts(0, 15));         // steps 0 ... A_AHEAD - 1 of the states
         load_b(r[2], cur, true); advance();             // step 2
         load_b(r[0], cur, false); advance();            // step 3
         __syncthreads();
-        // LDS stages and weight registers rotate with period 3, states with 2 or 6: six steps per trip, unrolled so that
+        // weight stages and registers rotate with period 3, the states' stages with 6: six steps per trip, unrolled so that
         // all of them are compile-time names
         auto run = [&](auto phase_tag) {
             constexpr int ahead = 2 + decltype(phase_tag)::value;
@@ -762,7 +735,7 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
 #pragma unroll
                 for (int u = 0; u < 6; ++u) {
                     if (u > 0 && kt + u >= ktiles) break;
-                    body(phase_tag, u, ra[(u + 1) % 2], ra[u % 2], r[(u + 1) % 3], r[(u + ahead) % 3]);
+                    body(phase_tag, u, r[(u + 1) % 3], r[(u + ahead) % 3]);
                 }
             }
         };
@@ -778,7 +751,7 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
     if (BITS == 4 && tile_has_expo) walk(std::bool_constant<BITS == 4>{});
     else walk(std::false_type{});
     // (no load to LDS is in flight any more when the LDS is used otherwise or given back)
-    if constexpr (DMA) __builtin_amdgcn_s_waitcnt(wait_counts(0, 15));
+    __builtin_amdgcn_s_waitcnt(wait_counts(0, 15));
     if (SPLIT && nsplit > 1) {
         // Every workgroup of the tile stores its partial accumulators (16 bytes per lane and
         // store: register group g of thread t at (g * T + t) * 16 -- whole cache lines per wave)
@@ -839,8 +812,7 @@ __global__ __launch_bounds__(NW * 128, NW == 2 ? 2 : 1) void matmul_kernel_pipe(
     constexpr int A_ROWS = NW * 32;
     // (each stage of the states an array of its own: in one array every fragment read would wait for all loads in flight)
     constexpr int A_HALVES = (BM + A_ROWS - 1) / A_ROWS * A_ROWS * PK;
-    __shared__ __attribute__((aligned(16))) h16 A0[A_HALVES], A1[A_HALVES], A2[A_HALVES];
-    __shared__ __attribute__((aligned(16))) h16 A3[NW == 4 ? A_HALVES : 8], A4[NW == 4 ? A_HALVES : 8], A5[NW == 4 ? A_HALVES : 8];
+    __shared__ __attribute__((aligned(16))) h16 A0[A_HALVES], A1[A_HALVES], A2[A_HALVES], A3[A_HALVES], A4[A_HALVES], A5[A_HALVES];
     __shared__ __attribute__((aligned(16))) h16 Bs[P_STAGES * PK * BN];
     __shared__ __attribute__((aligned(16))) uint32_t Lut[SPARSE ? SPARSE_LUT_WORDS : 4];
     // (split-K: the workgroups of a tile are neighbours in the grid, so they run at about the same time;
@@ -877,9 +849,7 @@ __global__ __launch_bounds__(NW * 128, NW == 2 ? 2 : 1) void matmul_kernel_pipe(
         tile_m = bid % a.tiles_m, tile_n = bid / a.tiles_m;
     }
     const int64_t boff = blockIdx.z;
-    h16* As[pipe_a_stages(NW)];
-    As[0] = A0; As[1] = A1; As[2] = A2;
-    if constexpr (NW == 4) { As[3] = A3; As[4] = A4; As[5] = A5; }
+    h16* const As[A_STAGES] = {A0, A1, A2, A3, A4, A5};
     pipe_tile<BITS, SPARSE, TM, NW, PING, SPLIT>(a, tile_m * BM, tile_n * BN, a.x + boff * a.M * (int64_t)a.K,
                                           a.outs + boff * a.M * (int64_t)a.S, As, Bs, Lut, slot, split, nsplit);
 }
@@ -900,7 +870,7 @@ static void launch_pipe(MatmulArgs a, int64_t B, hipStream_t st) {
 }
 
 // The pipelined kernel takes any whole number of 64 columns; the last tile may be partly empty, up to half of the
-// columns in all (its 128-column form: an eighth).  Before, such outputs went to the general tiles, which hide
+// columns in all (128-column tiles: an eighth).  Before, such outputs went to the general tiles, which hide
 // less of their loads and cannot split K (us, general / here: int4, K=9280, S=1600, 700 rows 135 / 54, S=14400, 1100 rows 422 /
 // 351; int2 there 239 / 54 and 699 / 341; 16:32 280 / 73 and 846 / 385; int4, K=9280, S=9344 -- 256 x 128 tiles before --
 // 1100 rows 280 / 214).
@@ -974,8 +944,8 @@ static TilePlan plan_tiles(int bits, bool sparse, int64_t M, int64_t K, int64_t 
 }
 
 // ---- what earlier forms of the tile kernels split along K.  It decides still which workspaces the last chunk of a large batch is taken
-// to have (last_chunk_as_others, a line of precision) and the ways of the 128-column tiles.  Shapes with at most 128 tiles of 256 x 256:
-// 256 x 128 tiles (16:32: 256 x 256) with `ksplit` workgroups per tile, by a cost in K steps.
+// to have (last_chunk_as_others, a line of precision), and nothing else.  Shapes with at most 128 tiles of 256 x 256: 256 x 128 tiles
+// (16:32: 256 x 256) with `ksplit` workgroups per tile, by a cost in K steps.
 struct SplitPlan { int ksplit; int64_t tiles; int64_t tile_bytes; };
 static SplitPlan plan_split(bool sparse, int64_t B, int64_t M, int64_t K, int64_t S) {
     const SplitPlan none{1, 0, 0};
@@ -1039,11 +1009,28 @@ static bool takes_tiles(int bits, bool sparse, int64_t M, int64_t K, int64_t S, 
            (sparse || K >= 1024 || (M + 255) / 256 * ((S + 255) / 256) > 128);
 }
 
-// the 128-column form: outputs of 128 columns where rows of 256 pad less than half (or would leave the general tiles a second row)
+// ---- outputs of 128 columns, of which a tile of 256 would leave half empty: tiles of 128 x 128, two workgroups of four waves per CU, in the
+// two phases as well.  On many rows the states' reads are the bound, 5.1 TB/s at 65536 rows.  K is split as many ways as fit 256 workgroups, in
+// shares of 16 steps and more (int4, us: K=8192, 128 tiles 95 unsplit, two ways 69, three 73, four 75; 80 tiles three ways 38, four
+// 44), or 512 where these are filled better (160 tiles, K=4096: one way 44, three 41; 96 tiles, K=16384: two ways 134, five 110) or the
+// states are more than the 256 MB of the cache beside memory (110 tiles, K=28672: two ways 217, four 195).  Before, 256 x 128 tiles with
+// the states through registers, whose decode spilled (int4, us, so / now: K=8192, 2048 rows 41.4 / 23.7, without room for a split 146 /
+// 76, 65536 rows 249 / 211; K=4096, 600 rows 31.5 / 17.0; with 32x32x16 MFMAs and no spill 39.7, 126, 233, 30.4).
 static bool takes_narrow_tiles(int bits, bool sparse, int64_t M, int64_t K, int64_t S, int64_t group_units) {
-    const int64_t variant = tuning(TUNE_MM_VARIANT), m_pad = (M + 255) / 256 * 256;
-    return !sparse && pipe_shape(bits, sparse, K, S, group_units) && tile_columns(S, 128, false) && (m_pad * 2 <= M * 3 || (M > 128 && M <= 256)) &&
+    const int64_t variant = tuning(TUNE_MM_VARIANT);
+    return !sparse && M > 128 && pipe_shape(bits, sparse, K, S, group_units) && tile_columns(S, 128, false) &&
            (variant == 5 || (variant == 0 && K > 1024 && !tile_columns(S, 256, true)));
+}
+struct NarrowPlan { int ksplit; size_t part_bytes; };
+static NarrowPlan plan_narrow(int64_t M, int64_t K, int64_t S, size_t scratch) {
+    const int64_t tiles = (M + 127) / 128 * ((S + 127) / 128), steps = K / 32, forced = tuning(TUNE_MM_SPLIT), tile_bytes = 128 * 128 * 4;
+    const int64_t room = (int64_t)std::min<size_t>(scratch, MM_SPLIT_MAX_BYTES);
+    auto ways = [&](int64_t workgroups) { return std::max<int64_t>(1, std::min<int64_t>({8, workgroups / tiles, steps / 16})); };
+    int64_t ks = forced >= 1 ? std::min(forced, steps / 8) : ways(256);
+    if (forced < 1 && (ways(512) * 10 > ks * 22 || M * K * 2 > 256ll << 20)) ks = ways(512);
+    if (tiles > MM_SPLIT_MAX_TILES) ks = 1;
+    while (ks > 1 && tiles * ks * tile_bytes > room) --ks;
+    return ks > 1 ? NarrowPlan{(int)ks, (size_t)(tiles * ks * tile_bytes)} : NarrowPlan{1, 0};
 }
 
 double tiles_us(int bits, bool sparse, int64_t M, int64_t K, int64_t S, int64_t group_units, size_t scratch) {
@@ -1058,23 +1045,21 @@ static int forced_height(int64_t variant) {
 
 template <int BITS, bool SPARSE>
 static void launch(MatmulArgs a, int64_t B, hipStream_t st, void* workspace, size_t workspace_bytes) {
-    // variant 0 = automatic: the plan of the pipelined kernel's tiles; where that kernel does not take the shape its 128-column form
-    // or the general tiles, 128 x 256, and 128 x 128 for narrow outputs or few rows
+    // variant 0 = automatic: the plan of the pipelined kernel's tiles; where that kernel does not take the shape its 128 x 128 tiles
+    // or the general ones, 128 x 256, and 128 x 128 for narrow outputs or few rows
     const int variant = (int)tuning(TUNE_MM_VARIANT);
     const WorkspaceParts wsp = workspace_parts(workspace, workspace_bytes);
     // (a single row comes here where its matvec has a group longer than a launch covers: the size query asks nothing for it)
     const size_t scratch = wsp.counters != nullptr && B == 1 && (a.M > 1 || variant != 0) ? wsp.scratch_bytes : 0;
     a.counters = reinterpret_cast<int*>(wsp.counters);
     a.part = reinterpret_cast<float*>(wsp.scratch);
+    const bool shape_ok = pipe_shape(BITS, SPARSE, a.K, a.S, a.group_units);
     const bool narrow = B == 1 && takes_narrow_tiles(BITS, SPARSE, a.M, a.K, a.S, a.group_units);
-    if (narrow) {
-        const SplitPlan sp = plan_split(false, B, a.M, a.K, a.S);
-        if (sp.ksplit > 1 && scratch >= (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes)) a.ksplit = sp.ksplit;
-    }
     const int only = forced_height(variant);
-    const bool tiles = !narrow && (variant == 0 ? takes_tiles(BITS, SPARSE, a.M, a.K, a.S, a.group_units) : only != 0 && pipe_shape(BITS, SPARSE, a.K, a.S, a.group_units) && tile_columns(a.S, 256, true));
+    const bool tiles = !narrow && (variant == 0 ? takes_tiles(BITS, SPARSE, a.M, a.K, a.S, a.group_units) : only != 0 && shape_ok && tile_columns(a.S, 256, true));
     if (narrow) {
-        if constexpr (!SPARSE) launch_pipe<BITS, false, 2>(a, B, st);
+        a.ksplit = plan_narrow(a.M, a.K, a.S, scratch).ksplit;
+        if constexpr (!SPARSE) launch_pipe<BITS, false, 2, 4, true>(a, B, st);
     } else if (tiles) {
         const TilePlan p = plan_tiles(BITS, SPARSE, a.M, a.K, a.S, scratch, only);
         a.ksplit = p.ksplit;
@@ -1197,12 +1182,11 @@ extern "C" size_t int4mm_matmul_workspace_bytes(const int4mm_shape* shape, int s
                     few_rows = std::max({few_rows, few(share, EXACT_SUMS), few(std::max<int64_t>(2, share - 1), EXACT_SUMS)});
         }
     size_t part = few_rows;
-    const SplitPlan sp = B * M > FEW_ROWS_MAX ? plan_split(sparse != 0, B, M, K, S) : SplitPlan{1, 0, 0};
-    const bool chunks = shape->seq_len == 1 && B * M > SK_WIDE_MAX_ROWS;           // (of the matvec entry: last_chunk_as_others)
-    if (sp.ksplit > 1 && chunks) part = std::max(part, (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes));
-    if (chunks && sp.ksplit == 1) {
+    if (shape->seq_len == 1 && B * M > SK_WIDE_MAX_ROWS) {           // (chunks of the matvec entry: last_chunk_as_others)
+        const SplitPlan sp = plan_split(sparse != 0, B, M, K, S);
         const TailPlan tp = plan_tail(sparse != 0, B, M, K, S);
-        if (tp.ksplit > 1) part = round_to_page(part) + (size_t)(tp.tiles * tp.ksplit * (256 * 256 * 4));
+        if (sp.ksplit > 1) part = std::max(part, (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes));
+        else if (tp.ksplit > 1) part = round_to_page(part) + (size_t)(tp.tiles * tp.ksplit * (256 * 256 * 4));
     }
     // (rows that the few-row kernels leave to the tiles are asked for as well: what a product is split into, and with it the order of its
     // sums, may not hang on what a workspace was made for)
@@ -1218,9 +1202,8 @@ extern "C" size_t int4mm_matmul_workspace_bytes(const int4mm_shape* shape, int s
     for (const int b : {4, 3, 2}) {
         if (B != 1 || (sparse ? b != 4 : bits != 0 && b != bits) || others_serve(b)) continue;
         const int64_t gu = std::max<int64_t>(1, group_units);
-        if (takes_narrow_tiles(b, sparse != 0, M, K, S, gu)) {
-            if (sp.ksplit > 1) part = std::max(part, (size_t)(sp.tiles * sp.ksplit * sp.tile_bytes));
-        } else if (variant != 0 || takes_tiles(b, sparse != 0, M, K, S, gu)) part = std::max(part, plan_tiles(b, sparse != 0, M, K, S, SIZE_MAX, forced_height(variant)).part_bytes);
+        if (takes_narrow_tiles(b, sparse != 0, M, K, S, gu)) part = std::max(part, plan_narrow(M, K, S, SIZE_MAX).part_bytes);
+        else if (variant != 0 || takes_tiles(b, sparse != 0, M, K, S, gu)) part = std::max(part, plan_tiles(b, sparse != 0, M, K, S, SIZE_MAX, forced_height(variant)).part_bytes);
     }
     return need + 2 * round_to_page(part);
 }

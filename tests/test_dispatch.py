@@ -279,6 +279,18 @@ def test_the_workspace_asked_for_is_the_partial_tiles_of_the_launch(bits, rows, 
     assert capi.lib().int4mm_matmul_workspace_bytes(sh, 0) - capi.lib().int4mm_workspace_bytes(s) == 2 * (-(-used // 4096) * 4096)
 
 
+@pytest.mark.parametrize("bits", [4, 3, 2])
+def test_outputs_of_128_columns_take_tiles_of_128(bits):
+    for rows, k, want in ((513, 1088, 2), (600, 4096, 8), (4096, 2048, 4), (10240, 8192, 3), (16384, 8192, 2), (20480, 4096, 3), (24576, 4096, 1),
+                          (12288, 16384, 5), (32768, 16384, 2), (65536, 8192, 1)):
+        line = d("mtx", bits, 1, rows, k, 128, 128)
+        assert line.startswith("matmul_kernel_pipe") and "tile=128x128," in line and f"tiles={-(-rows // 128)} ksplit={want} " in line, line
+        assert "ksplit=1 " in d("mtx", bits, 1, rows, k, 128, 128, workspace_bytes=0)
+    # up to 512 rows the kernel with shared staging, on a short K the general tiles
+    assert d("mtx", bits, 1, 512, 8192, 128, 128).startswith("wide_rows_kernel")
+    assert d("mtx", bits, 1, 2048, 1024, 128, 128).startswith("matmul_kernel<")
+
+
 def test_matvec_of_a_k_beyond_one_launch():
     # 32 x 224 units of 64 rows is what one launch covers: a longer K runs as several launches (one line each)
     line = d("vec", 4, 1, 1, 1 << 20, 256, 128)

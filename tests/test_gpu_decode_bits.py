@@ -60,7 +60,7 @@ def test_tile_kernels_return_the_dequantised_weights(H, bits, sparse, variant, e
     `mixed`: every tile holds groups of both modes and takes the loop (or, for the 128-column and
     16:32 tiles, the plain loop) that decodes either."""
     if variant == 5 and sparse:
-        pytest.skip("256 x 128 tiles serve the dense formats only")
+        pytest.skip("128 x 128 tiles serve the dense formats only")
     K, S, g = 512, 512, 128
     p = _problem(bits, sparse, K, S, g, seed=70 + bits, expo=expo)
     want = O.dequantize_matrix(bits, p["matrix"], p["scales"], p["zeros"], g, p["sparse_mask"])

@@ -262,7 +262,7 @@ def test_full_size_matvec_and_matmul_c2_c3(H):
 @pytest.mark.parametrize("M,K,S,g,B", [(256, 512, 512, 128, 1), (512, 192, 256, 64, 2), (256, 2048, 256, -1, 1),
                                        (512, 448, 512, 64, 1)])
 def test_pipelined_matmul_with_exponent_groups(H, bits, sparse, variant, M, K, S, g, B):
-    """tile-aligned dense shapes take the pipelined kernel (variant 5: 256 x 128
+    """tile-aligned dense shapes take the pipelined kernel (variant 5: 128 x 128
     tiles, variant 6: 256 x 256 with the two halves of the workgroup in opposite
     phases for the dense formats, variant 9: 256 x 256 in the plain order); negative
     scales in a few columns force its general loop for the tiles that contain them.
@@ -399,6 +399,34 @@ def test_every_tile_height(H, bits, sparse, M, K, S, g, ksplit):
     if ksplit == 1:
         for r in runs[1:]:
             assert np.array_equal(r.view(np.uint16), runs[0].view(np.uint16))
+
+
+# ---- 128 x 128 tiles, which outputs of 128 columns take from 513 rows and K = 1088 on (tuning key 3 = 5 forces them): a row more and
+# fewer than whole tiles, 34 K steps and more, shares of unequal length, exponent-mode groups in one tile
+@pytest.mark.parametrize("bits", [4, 3, 2])
+@pytest.mark.parametrize("M,K,S,g,variant,ksplit", [(513, 1088, 128, 64, 0, 0), (640, 2112, 128, -1, 0, 0), (1025, 4160, 128, 192, 0, 1),
+                                                    (129, 512, 256, 128, 5, 2), (255, 64, 128, 64, 5, 0), (300, 832, 384, 64, 5, 3)])
+@pytest.mark.parametrize("expo", [False, True], ids=["linear", "mixed"])
+def test_tiles_of_128_columns(H, bits, M, K, S, g, variant, ksplit, expo):
+    p = _problem(bits, False, K=K, S=S, M=M, group_size=g, seed=M + K)
+    if expo:
+        sc = p["scales"].reshape(-1, S)
+        sc[sc.shape[0] // 2, S - 70:S - 50] *= np.float16(-1)
+    d = H.dev_problem(p)
+    exact, f32 = H.oracles(p)
+    try:
+        H.capi.tune(3, variant)
+        H.capi.tune(6, ksplit)
+        line = H.capi.describe_launch("mtx", bits, 1, M, K, S, g)
+        assert "tile=128x128," in line and line.startswith("matmul_kernel_pipe"), line
+        assert f"ksplit={ksplit or {1088: 2, 2112: 4, 64: 1}[K]} " in line, line
+        got = H.run_capi(p, d, "mtx", outs_init=np.full((1, M, S), 4.0, np.float16))
+        again = H.run_capi(p, d, "mtx")
+    finally:
+        H.capi.tune(3, 0)
+        H.capi.tune(6, 0)
+    H.assert_product_close(got, exact, f32, kind="mtx")
+    assert np.array_equal(got.view(np.uint16), again.view(np.uint16))
 
 
 # ---- a last strip or tile that is partly beyond the last column (S a multiple of 64, not of the strip's 128 or 256): one to three
