@@ -892,7 +892,9 @@ constexpr int64_t MM_SPLIT_MAX_BYTES = 192ll << 20;      // cap of the partial t
 // candidate on average, 9 - 16 % at worst.  Before, a tree of rules chose among 128, 192 and 256 rows and 256 x 128 tiles, of which
 // the last are the best candidate on none of 210 shapes: above 512 rows this plan takes 10 % (int4), 15 % (int3), 14 % (int2) and
 // 11 % (16:32) less time on average, at most 3 % more on a shape (us: int4, K=16128, S=3072, 1411 rows 217 / 151; K=9216, S=2304, 1151
-// rows 98 / 70; int3, K=28096, S=2176, 880 rows 201 / 134; K=S=4096, 777 rows on S=11008 77 / 72).
+// rows 98 / 70; int3, K=28096, S=2176, 880 rows 201 / 134; K=S=4096, 777 rows on S=11008 77 / 72).  Preferences on top of the model -- whole
+// 256-row tiles, 16:32 split in 256 rows and never in 224 -- had single shapes' sake and cost 2 % (90 random products of multiples
+// of 256 rows; int4, K=20480, S=5120, 2048 rows 420 / 373) and 4 % (121 of 16:32; K=4096, S=8192, 896 rows 79.5 / 74.9).
 struct TileCost { double step[5], fixed[5], fill, way, hand, round, last; };
 static const TileCost tile_cost[4] = {                // int4, int3, int2, 16:32
     {{0.373, 0.434, 0.466, 0.521, 0.555}, {4.151, 4.233, 4.77, 4.391, 5.388}, 0.369, 2.82, 19.858, 1.065, 0.292},
@@ -914,17 +916,12 @@ static TilePlan plan_tiles(int bits, bool sparse, int64_t M, int64_t K, int64_t 
         auto take = [&](double us, int64_t ks, int64_t from) {
             if (us < best.us) best = TilePlan{tm, (int)ks, from, total, ks > 1 ? (size_t)((total - from) * ks * tile_bytes) : 0, us};
         };
-        // (16:32 in tiles of 224 rows is not split: K=4096, S=8192, 896 rows keep 256 rows two ways, 86 us to 79)
-        for (int64_t ks = 1; ks <= (sparse && tm == 7 ? 1 : 8); ++ks) {
+        for (int64_t ks = 1; ks <= 8; ++ks) {
             if (ks > 1 && (steps / ks < 8 || total > MM_SPLIT_MAX_TILES || total * ks * tile_bytes > room || forced == 1)) break;
             const int64_t wgs = total * ks, rounds = (wgs + 255) / 256;
             const double n = (double)steps / ks, last = (wgs - (rounds - 1) * 256) / 256.0;
             double us = (rounds - 1) * c.round * one(n, 1.0) + one(n, rounds > 1 ? last + (1.0 - last) * c.last : last);
             if (ks > 1) us += (c.way * ks + c.hand * (rounds - 1 + last)) * share;
-            // (256 rows: preferred within 6 % where they pad none and are not split, K=20480, S=5120, 2048 rows 382 us, 374 in tiles of 192;
-            // split 16:32 tiles come out 8 % too high)
-            if (tm == 8 && ks == 1 && M % 256 == 0) us /= 1.06;
-            if (tm == 8 && ks > 1 && sparse) us /= 1.05;
             take(forced >= 2 && ks == forced ? 0.0 : us, ks, 0);
         }
         // the tiles of the last round alone, over at most half of the GPU (two ways from 64 tiles on, where the second adds the first

@@ -44,7 +44,8 @@ def test_dense_matmul_m2048(bits):
 
 
 def test_other_matmul_configurations():
-    assert d("mtx", 4, 1, 2048, S, K, 128).startswith("matmul_kernel_pipe<bits=4,dense,tile=256x256,two-phase> tiles=160")
+    # eleven rows of 192-row tiles, the last a third empty, fill the GPU better than eight rows of whole 256-row ones
+    assert d("mtx", 4, 1, 2048, S, K, 128).startswith("matmul_kernel_pipe<bits=4,dense,tile=192x256,two-phase> tiles=220")
     # C3 small: one group, 16 tiles of the general kernel (the pipelined kernel's prologue would dominate)
     assert d("mtx", 4, 1, 2048, 128, 128, 128).startswith("matmul_kernel<bits=4,dense,tile=128x128> tiles=16")
     # C4: the 16:32 format keeps the plain order (its decode has no registers to spare)
@@ -259,12 +260,16 @@ def test_few_rows_that_are_left_to_the_tiles_are_split_alike_on_any_workspace(bi
     assert name == "matmul_kernel_pipe" and (f["ksplit"] > 1) == (rows > 1), line
 
 
-@pytest.mark.parametrize("bits", [4, 3, 2])
-def test_a_row_more_or_fewer_takes_the_same_tiles(bits):
-    # 640 and 1152 rows on a long K are no rule of their own: the tiles that their neighbours take (rows padded to the same height)
-    for rows, k, s in ((640, 28672, 3840), (1152, 14336, 4096), (1152, 20480, 4096), (1152, 28672, 2048)):
-        line = d("mtx", bits, 1, rows, k, s, 128)
-        assert "x256," in line and line == d("mtx", bits, 1, rows - 1, k, s, 128), line
+@pytest.mark.parametrize("bits,sparse", [(4, False), (3, False), (2, False), (4, True)])
+def test_a_row_more_or_fewer_takes_the_same_tiles(bits, sparse):
+    # 640 and 1152 rows on a long K, multiples of 256 rows, and 224-row tiles of 16:32 are no rules of their own: the tiles that a row
+    # fewer takes (which is padded to the same height)
+    for rows, k, s in ((640, 28672, 3840), (1152, 14336, 4096), (1152, 20480, 4096), (1152, 28672, 2048), (2048, 20480, 5120), (1024, 8192, 9216),
+                       (1536, 4096, 6400), (896, 4096, 8192), (672, 14336, 6144)):
+        line = d("mtx", bits, 1, rows, k, s, 64, sparse)
+        assert "x256," in line and line == d("mtx", bits, 1, rows - 1, k, s, 64, sparse), line
+    if sparse:
+        assert "tile=224x256," in d("mtx", 4, 1, 896, 4096, 8192, 64, True) and "ksplit=2 " in d("mtx", 4, 1, 896, 4096, 8192, 64, True)
 
 
 @pytest.mark.parametrize("bits,rows,k,s,g", [(3, 546, 30272, 8832, 128), (4, 703, 31104, 9088, -1), (2, 2643, 31872, 2432, -1), (3, 293, 23936, 13568, -1),

@@ -390,7 +390,7 @@ def test_every_tile_height(H, bits, sparse, M, K, S, g, ksplit):
             H.capi.tune(6, ksplit)
             line = H.capi.describe_launch("mtx", bits, 1, M, K, S, g, sparse)
             assert f"tile={32 * {6: 8, 7: 4, 8: 6, 10: 5, 11: 7}[variant]}x256" in line, line
-            assert f"ksplit={1 if sparse and variant == 11 else ksplit} " in line, line
+            assert f"ksplit={ksplit} " in line, line
             runs.append(H.run_capi(p, d, "mtx", outs_init=np.full((1, M, S), 4.0, np.float16)))
         finally:
             H.capi.tune(3, 0)
