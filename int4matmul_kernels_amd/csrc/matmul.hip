@@ -861,9 +861,8 @@ static void launch_pipe(MatmulArgs a, int64_t B, hipStream_t st) {
     const int total = a.tiles_m * a.tiles_n;
     const dim3 grid(a.split_from + (total - a.split_from) * a.ksplit, 1, (unsigned)B), block(NW * 128);
     a.by_columns = a.tiles_n % 8 == 0;
-    // (the word behind the tile tells the dense formats' variants 6 and 9 apart; other tiles read `plain` whatever their order)
     if (noting("matmul_kernel_pipe<bits=%d,%s,tile=%dx%d,%s> tiles=%d ksplit=%d split_from=%d workgroups=%u batch=%d", BITS,
-               SPARSE ? "16:32" : "dense", TM * 32, NW * 64, PING && !SPARSE && TM > 4 ? "two-phase" : "plain", total, a.ksplit, a.split_from, grid.x, (int)B))
+               SPARSE ? "16:32" : "dense", TM * 32, NW * 64, PING ? "two-phase" : "plain", total, a.ksplit, a.split_from, grid.x, (int)B))
         return;
     if (a.ksplit > 1) hipLaunchKernelGGL((matmul_kernel_pipe<BITS, SPARSE, NW, TM, PING, true>), grid, block, 0, st, a);
     else hipLaunchKernelGGL((matmul_kernel_pipe<BITS, SPARSE, NW, TM, PING, false>), grid, block, 0, st, a);

@@ -48,9 +48,18 @@ def test_other_matmul_configurations():
     assert d("mtx", 4, 1, 2048, S, K, 128).startswith("matmul_kernel_pipe<bits=4,dense,tile=192x256,two-phase> tiles=220")
     # C3 small: one group, 16 tiles of the general kernel (the pipelined kernel's prologue would dominate)
     assert d("mtx", 4, 1, 2048, 128, 128, 128).startswith("matmul_kernel<bits=4,dense,tile=128x128> tiles=16")
-    # C4: the 16:32 format keeps the plain order (its decode has no registers to spare)
+    # C4: the 16:32 format, in the two phases as well
     assert d("mtx", 4, 1, 2048, K, S, 64, sparse=True).startswith(
-        "matmul_kernel_pipe<bits=4,16:32,tile=256x256,plain> tiles=640 ksplit=2 split_from=512 workgroups=768")
+        "matmul_kernel_pipe<bits=4,16:32,tile=256x256,two-phase> tiles=640 ksplit=2 split_from=512 workgroups=768")
+    # every height and format runs the two phases; tuning key 3 = 9 forces 256 x 256 tiles without them
+    for variant, order in ((5, "two-phase"), (6, "two-phase"), (7, "two-phase"), (8, "two-phase"), (9, "plain"), (10, "two-phase"), (11, "two-phase")):
+        capi.tune(3, variant)
+        try:
+            for bits, sparse in ((4, False), (3, False), (2, False), (4, True)):
+                if variant != 5 or not sparse:
+                    assert f",{order}> " in d("mtx", bits, 1, 2048, K, S, 128, sparse), (variant, bits, sparse)
+        finally:
+            capi.tune(3, 0)
 
 
 def test_baseline_shape_with_few_rows():

@@ -57,8 +57,8 @@ def _assert_same_bits(got, want, what):
 @pytest.mark.parametrize("expo", [False, True], ids=["linear", "mixed"])
 def test_tile_kernels_return_the_dequantised_weights(H, bits, sparse, variant, expo):
     """`linear`: no exponent group anywhere, so the pipelined kernels run their linear-only loop;
-    `mixed`: every tile holds groups of both modes and takes the loop (or, for the 128-column and
-    16:32 tiles, the plain loop) that decodes either."""
+    `mixed`: every tile holds groups of both modes and takes the copy of the loop that decodes either
+    (int2 and int3 have one loop for both)."""
     if variant == 5 and sparse:
         pytest.skip("128 x 128 tiles serve the dense formats only")
     K, S, g = 512, 512, 128

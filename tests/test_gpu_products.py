@@ -263,9 +263,9 @@ def test_full_size_matvec_and_matmul_c2_c3(H):
                                        (512, 448, 512, 64, 1)])
 def test_pipelined_matmul_with_exponent_groups(H, bits, sparse, variant, M, K, S, g, B):
     """tile-aligned dense shapes take the pipelined kernel (variant 5: 128 x 128
-    tiles, variant 6: 256 x 256 with the two halves of the workgroup in opposite
-    phases for the dense formats, variant 9: 256 x 256 in the plain order); negative
-    scales in a few columns force its general loop for the tiles that contain them.
+    tiles, variant 6: 256 x 256, both with the two halves of the workgroup in opposite
+    phases, variant 9: 256 x 256 in the plain order); negative scales in a few columns force
+    the loop that decodes either mode for the tiles that contain them.
     K = 192 is six K steps (one trip of the unrolled loop), K = 448 fourteen (two trips
     and a remainder), K = 2048 with a single group runs many trips."""
     from int4matmul_kernels_amd import capi
