@@ -233,7 +233,8 @@ INT4MM_API int int4mm_sparse_pack(void* wt_outs, void* msk_outs, const void* wt_
                        int64_t out_size, int64_t in_size, void* bad_blocks, void* stream);
 
 /* The same, waiting for it: *bad_blocks (host memory) is the number of 32-row
- * blocks that do not keep exactly 16 rows.  Not capturable. */
+ * blocks that do not keep exactly 16 rows.  A stream that is being captured is
+ * refused (INT4MM_ERR_LAUNCH), with nothing recorded. */
 INT4MM_API int int4mm_sparse_pack_checked(void* wt_outs, void* msk_outs, const void* wt_in, const void* msk_in,
                                           int64_t out_size, int64_t in_size, int* bad_blocks, void* stream);
 

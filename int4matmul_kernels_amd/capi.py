@@ -70,6 +70,8 @@ def lib():
     L.int4mm_describe_launch.argtypes = [C.c_int, C.c_int, C.POINTER(Shape), C.c_int, sz, C.c_char_p, sz]
     L.int4mm_sparse_pack.restype = C.c_int
     L.int4mm_sparse_pack.argtypes = [vp, vp, vp, vp, i64, i64, vp, vp]
+    L.int4mm_sparse_pack_checked.restype = C.c_int
+    L.int4mm_sparse_pack_checked.argtypes = [vp, vp, vp, vp, i64, i64, C.POINTER(C.c_int), vp]
     L.int4mm_dense_pack.restype = C.c_int
     L.int4mm_dense_pack.argtypes = [C.c_int, vp, vp, i64, i64, vp]
     L.int4mm_unpack.restype = C.c_int
@@ -183,6 +185,15 @@ def sparse_pack(wt_outs, msk_outs, wt_in, msk_in, bad_blocks=None):
     S, K = wt_in.shape
     _check(lib().int4mm_sparse_pack(_ptr(wt_outs), _ptr(msk_outs), _ptr(wt_in), _ptr(msk_in), S, K,
                                     _ptr(bad_blocks), _stream()), "int4mm_sparse_pack")
+
+
+def sparse_pack_checked(wt_outs, msk_outs, wt_in, msk_in) -> int:
+    """the same, waiting for it: the number of 32-row blocks that do not keep exactly 16 rows"""
+    S, K = wt_in.shape
+    bad = C.c_int(0)
+    _check(lib().int4mm_sparse_pack_checked(_ptr(wt_outs), _ptr(msk_outs), _ptr(wt_in), _ptr(msk_in), S, K,
+                                            C.byref(bad), _stream()), "int4mm_sparse_pack_checked")
+    return bad.value
 
 
 def dense_pack(bits, matrix_out, codes_in):

@@ -38,8 +38,8 @@ int check_launch(const char*) {
     return INT4MM_OK;
 }
 
-int launch_error() {
-    g_last_hip_error = (int)hipGetLastError();
+int launch_error(hipError_t e) {
+    g_last_hip_error = (int)(e != hipSuccess ? e : hipGetLastError());
     return INT4MM_ERR_LAUNCH;
 }
 

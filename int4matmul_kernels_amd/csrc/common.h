@@ -128,7 +128,7 @@ __device__ __forceinline__ float code_value(uint32_t q, bool exponent_mode) {
 struct LaunchStatus { int code; hipError_t hip; };
 
 int check_launch(const char* what);           // returns INT4MM_OK or INT4MM_ERR_LAUNCH
-int launch_error();                           // notes the runtime's last error, INT4MM_ERR_LAUNCH
+int launch_error(hipError_t e = hipSuccess);  // notes e or else the runtime's last error, INT4MM_ERR_LAUNCH
 int validate_product(int bits, const void* outs, const void* matrix, const void* multiplier,
                      const void* scales, const void* zeros, const void* sparse_mask,
                      const int4mm_shape* sh, bool matvec);

@@ -317,13 +317,19 @@ static void give_back(const PackReport& r) {
     free_report(r);
 }
 
-static int sparse_pack(void* wt_outs, void* msk_outs, const void* wt_in, const void* msk_in,
-                       int64_t out_size, int64_t in_size, int* bad_blocks, int* bad_flag, void* stream) {
+static int validate_pack(const void* wt_outs, const void* msk_outs, const void* wt_in, const void* msk_in, int64_t out_size, int64_t in_size) {
     if (out_size < 0 || in_size < 0 || in_size % 32 != 0) return INT4MM_ERR_SHAPE;
     if (in_size / 32 > 65535) return INT4MM_ERR_SHAPE;
     if (out_size == 0 || in_size == 0) return INT4MM_OK;
     if (!wt_outs || !msk_outs || !wt_in || !msk_in) return INT4MM_ERR_NULL;
     if (((uintptr_t)wt_in | (uintptr_t)msk_in) & 15u) return INT4MM_ERR_ALIGN;
+    return INT4MM_OK;
+}
+
+static int sparse_pack(void* wt_outs, void* msk_outs, const void* wt_in, const void* msk_in,
+                       int64_t out_size, int64_t in_size, int* bad_blocks, int* bad_flag, void* stream) {
+    const int wrong = validate_pack(wt_outs, msk_outs, wt_in, msk_in, out_size, in_size);
+    if (wrong != INT4MM_OK || out_size == 0 || in_size == 0) return wrong;
     int lanes = 2;
     while (lanes < SPARSE_PACK_MAX_LANES && 16 * lanes < in_size) lanes *= 2;
     const int64_t k_tiles = (in_size + 16 * lanes - 1) / (16 * lanes);
@@ -364,6 +370,12 @@ int int4mm_sparse_pack_checked(void* wt_outs, void* msk_outs, const void* wt_in,
                                int64_t out_size, int64_t in_size, int* bad_blocks, void* stream) {
     if (bad_blocks == nullptr) return INT4MM_ERR_NULL;
     *bad_blocks = 0;
+    const int wrong = validate_pack(wt_outs, msk_outs, wt_in, msk_in, out_size, in_size);
+    if (wrong != INT4MM_OK || out_size == 0 || in_size == 0) return wrong;
+    // (refused before anything is enqueued: a recorded kernel would go on reporting into what the next call takes)
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing((hipStream_t)stream, &capture) != hipSuccess) return launch_error();
+    if (capture != hipStreamCaptureStatusNone) return launch_error(hipErrorStreamCaptureUnsupported);
     PackReport r;
     if (!take_report(r, (hipStream_t)stream)) return launch_error();
     const int rc = sparse_pack(wt_outs, msk_outs, wt_in, msk_in, out_size, in_size, r.count, r.flag, stream);

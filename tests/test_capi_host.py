@@ -68,6 +68,13 @@ def test_argument_validation_happens_on_the_host():
     assert lib.int4mm_dense_pack(5, vp(16), vp(16), 64, 64, None) == 1
     assert lib.int4mm_dense_pack(4, vp(16), vp(16), 48, 64, None) == 3
     assert lib.int4mm_sparse_pack(vp(16), vp(16), vp(16), vp(16), 64, 48, None, None) == 3
+    # (the packing that waits and counts: before it takes anything from the device)
+    bad = C.c_int(9)
+    checked = lambda k, *p, s=64: lib.int4mm_sparse_pack_checked(*(vp(q) for q in p), s, k, C.byref(bad), None)
+    assert lib.int4mm_sparse_pack_checked(vp(16), vp(16), vp(16), vp(16), 64, 64, None, None) == 5
+    assert checked(48, 16, 16, 16, 16) == 3 and checked(65536 * 32, 16, 16, 16, 16) == 3
+    assert checked(64, 16, 16, None, 16) == 5 and checked(64, 16, 16, 16, 8) == 8
+    assert bad.value == 0 and checked(64, None, None, None, None, s=0) == 0
     assert lib.int4mm_unpack(3, vp(16), None, vp(16), vp(16), 64, 64, None) == 2
     assert lib.int4mm_dequantize(4, vp(16), vp(16), vp(16), vp(16), None, 64, 64, 1, 32, None) == 4
     assert lib.int4mm_dequantize(4, None, vp(16), vp(16), vp(16), None, 64, 64, 1, 64, None) == 5

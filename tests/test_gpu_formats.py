@@ -118,12 +118,44 @@ def test_weight_matrix_packing_counts_bad_blocks_anew_each_time(H, S, K):
                 with pytest.raises(RuntimeError, match=f" {bad} 32-row blocks"):
                     ext.weight_matrix_packing(w, m, codes, keep)
 
+    def pack_through_the_c_api(bad):
+        # (ctypes lets go of the interpreter's lock: several reports are out at once)
+        with torch.cuda.stream(torch.cuda.Stream()):
+            keep = good.clone()
+            keep.view(-1, 32)[:bad, 0] = 1
+            w = torch.empty((K // 16, S), dtype=torch.int32, device=H.DEV)
+            m = torch.empty((K // 32, S), dtype=torch.int32, device=H.DEV)
+            for _ in range(4):
+                assert H.capi.sparse_pack_checked(w, m, codes, keep) == bad
+
     most = S * K // 32
     counts = [0, 1, most, 0, min(2, most), 0]
     for n in counts:
         pack(n)
     with ThreadPoolExecutor(4) as pool:
-        list(pool.map(pack, counts * 4))
+        list(pool.map(pack_through_the_c_api, counts * 4))
+
+
+def test_checked_packing_is_refused_on_a_stream_that_is_being_captured(H):
+    """with nothing recorded: the capture goes on, and the packing after it counts as ever"""
+    codes = torch.full((64, 64), 5, dtype=torch.uint8, device=H.DEV)
+    keep = (torch.arange(64, device=H.DEV) % 2).to(torch.uint8).repeat(64, 1).contiguous()
+    keep[0, 0] = 1
+    w = torch.full((4, 64), 3, dtype=torch.int32, device=H.DEV)
+    m = torch.empty((2, 64), dtype=torch.int32, device=H.DEV)
+    x = torch.zeros(4, device=H.DEV)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        x.add_(1.0)
+        with pytest.raises(H.capi.Int4mmError) as e:
+            H.capi.sparse_pack_checked(w, m, codes, keep)
+        assert e.value.code == 7
+    for n in range(1, 4):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert x.tolist() == [float(n)] * 4 and bool((w == 3).all())
+    assert H.capi.sparse_pack_checked(w, m, codes, keep) == 1
 
 
 @pytest.mark.parametrize("S,K", [(64, 64), (63, 96), (65, 512), (1, 544), (128, 1056), (200, 480), (320, 1600)])
