@@ -176,10 +176,10 @@ void quant_matmul(uint32_t bits, TENSOR_MULT_ARGS) {
 // The product of a layer that holds its weights: [batch, seq_len, in_size] states to a new [batch, seq_len, out_size]
 // tensor.  Both products overwrite, so the output is allocated without a fill: the products' kernels are the same as
 // quant_matmul's on a zeroed tensor, one launch less per call and, with the checks and allocation in one native call, less
-// host time.  QuantLinear, us per pass, conversions, zeros and quant_matmul called one by one from Python / in this one call with
-// the output zeroed / unfilled: sixteen 1024 x 1024 matvecs 221 / 179 / 119; four layers of K = 5120, S = 20480 with one token
-// 56 / 56 / 48, 8 tokens 88 / 88 / 72, 64 tokens 154 / 153 / 118; one with 2048 rows 410 / 410 / 399: where kernels are long the
-// gain is the fill alone.
+// host time.  QuantLinear, us per pass: sixteen 1024 x 1024 matvecs 84 - 95, four layers of K = 5120, S = 20480 with one token
+// 48, 8 tokens 71, 64 tokens 100, one with 2048 rows 346.  (When this call was introduced, conversions, zeros and quant_matmul
+// called one by one from Python took 221, 56, 88, 154 and 410 where it took 119, 48, 72, 118 and 399: where kernels are long
+// the gain is the fill alone.)
 torch::Tensor linear_forward(uint32_t bits, int64_t out_size, const torch::Tensor& matrix, const torch::Tensor& states,
                              const torch::Tensor& scales, const torch::Tensor& zeros, int group_size,
                              const c10::optional<torch::Tensor>& sparse_mask) {

@@ -3,8 +3,9 @@
 // where w16 is the fp16 matrix the reference's unpack step builds (two fp16
 // roundings per weight in linear mode, one fused multiply-add in exponent mode).
 //
-// Two kernels.  matmul_kernel_pipe (further down) is the fast one for shapes
-// made of whole tiles; matmul_kernel takes everything else.  Common to both: one
+// Two kernels.  matmul_kernel_pipe (further down) is the fast one, for any number of
+// rows and outputs whose columns fill at least two thirds of whole tiles;
+// matmul_kernel takes everything else.  Common to both: one
 // workgroup owns a tile of outs; per K step the packed weights of the tile are
 // read from HBM once, decoded and dequantised to fp16 ONCE by the workgroup and
 // stored to LDS in MFMA operand layout: 16-byte chunks
@@ -353,8 +354,9 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 2) void matmul_kernel(M
 // int2 and int3 have one decode for both.
 //
 // Measured, before (32x32x16 MFMAs, states through registers, magic-number decodes) / so, us: K=5120, S=20480, 2048 rows int4 398 /
-// 351, int3 402 / 363, int2 394 / 340, 16:32 437 / 407, one group in 40 in exponent mode 464 / 380, int3 468 / 363; K=8192,
-// S=28672, 4096 rows 1663 / 1453 (1.32 PFLOP/s); K=S=8192, 768 rows 125 / 109; K=20480, S=5120, 1024 rows 250 / 222.
+// 346, int3 402 / 359, int2 394 / 337, 16:32 437 / 400, one group in 40 in exponent mode 464 / 369, int3 468 / 359; K=8192,
+// S=28672, 4096 rows 1663 / 1430 (1.35 PFLOP/s); with the plan of the tiles below K=S=8192, 768 rows 146 / 107; K=20480, S=5120, 1024
+// rows 265 / 206.
 constexpr int PK = 32;            // K per step of the pipelined kernel
 
 // 16:32 sparse int4.  `v` holds the (up to 8) kept codes of one 8-row chunk as
@@ -427,7 +429,7 @@ __device__ __forceinline__ void pipe_tile(const MatmulArgs& a, const int m0, con
     // of the packed matrix, mask, scales, zeros) plus a per-lane 32-bit byte offset that
     // never changes plus a workgroup-uniform 32-bit offset that moves with the K step:
     // buffer loads add the three themselves, no address arithmetic is left to the VALU
-    // (the launcher admits only shapes whose tensors stay below 4 GB)
+    // (the launcher admits only shapes whose tensors stay below 2 GB: pipe_shape)
     constexpr int RSRC_FLAGS = 0x00020000;               // raw buffer, 32-bit data format
     const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<h16*>(x + (int64_t)m0 * a.K), 0, min(a.M - m0, BM) * a.K * 2, RSRC_FLAGS);
@@ -892,7 +894,7 @@ constexpr int64_t MM_SPLIT_MAX_BYTES = 192ll << 20;      // cap of the partial t
 // the last are the best candidate on none of 210 shapes: above 512 rows this plan takes 10 % (int4), 15 % (int3), 14 % (int2) and
 // 11 % (16:32) less time on average, at most 3 % more on a shape (us: int4, K=16128, S=3072, 1411 rows 217 / 151; K=9216, S=2304, 1151
 // rows 98 / 70; int3, K=28096, S=2176, 880 rows 201 / 134; K=S=4096, 777 rows on S=11008 77 / 72).  Preferences on top of the model -- whole
-// 256-row tiles, 16:32 split in 256 rows and never in 224 -- had single shapes' sake and cost 2 % (90 random products of multiples
+// 256-row tiles, 16:32 split in 256 rows and never in 224 -- were made for single shapes and cost 2 % (90 random products of multiples
 // of 256 rows; int4, K=20480, S=5120, 2048 rows 420 / 373) and 4 % (121 of 16:32; K=4096, S=8192, 896 rows 79.5 / 74.9).
 struct TileCost { double step[5], fixed[5], fill, way, hand, round, last; };
 static const TileCost tile_cost[4] = {                // int4, int3, int2, 16:32
