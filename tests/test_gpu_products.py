@@ -284,8 +284,8 @@ def test_pipelined_matmul_with_exponent_groups(H, bits, sparse, variant, M, K, S
         capi.tune(3, 0)
 
 
-# ---- 257 ... 384 rows: three rows of 128 x 256 tiles of the pipelined kernel (tuning key 3 = 7 forces them), and the
-# padded 256-row tiles that serve 257 ... 341 rows on small grids and for 16:32
+# ---- 257 ... 384 rows: three rows of 128 x 256 tiles of the pipelined kernel (tuning key 3 = 7 forces them), and what the
+# dispatch picks without the kernel with shared staging
 @pytest.mark.parametrize("bits,sparse", FORMATS)
 @pytest.mark.parametrize("M,K,S,g", [(384, 512, 512, 128), (300, 2048, 256, 64), (257, 1024, 768, -1), (341, 2560, 256, 128)])
 def test_matmul_three_rows_of_128_row_tiles(H, bits, sparse, M, K, S, g):
@@ -309,8 +309,8 @@ def test_matmul_three_rows_of_128_row_tiles(H, bits, sparse, M, K, S, g):
 
 @pytest.mark.parametrize("bits,sparse", [(4, False), (4, True)])
 def test_matmul_three_rows_default_rule_and_exponent_groups(H, bits, sparse):
-    """M=300 against S=11264 (44 tile columns: 132 tiles of 128 x 256) takes the variant by default for the dense
-    format; some exponent-mode groups on top"""
+    """M=300 against S=11264 (44 tile columns: 132 tiles of 128 x 256) takes the variant by default, in
+    every format; some exponent-mode groups on top"""
     p = _problem(bits, sparse, K=1024, S=11264, M=300, group_size=128, seed=12)
     p["scales"][2, 100:108] *= np.float16(-1)
     p["scales"][5, 7000] *= np.float16(-1)
